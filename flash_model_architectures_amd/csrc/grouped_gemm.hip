@@ -739,6 +739,7 @@ int xma_grouped_gemm(const xma_grouped_gemm_args* args, void* stream_) {
     // a gated tile of the vector kernels pairs whole 16-byte chunks of the two halves
     const bool paired_tail = (a.epilogue == XMA_EPI_SWIGLU || a.epilogue == XMA_EPI_GLU) && a.n % (2 * pv) != 0;
     const bool elementwise = ragged || paired_tail;
+    if (!elementwise && skinny_gemm_supports(a)) return launch_skinny_gemm(a, stream);
     if (!elementwise && dma_gemm_supports(a)) return launch_dma_gemm(a, stream);
     switch (a.dtype) {
         case XMA_F32:

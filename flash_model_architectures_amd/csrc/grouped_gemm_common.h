@@ -257,6 +257,45 @@ inline int64_t grid_for_tiles(int64_t row_tiles, int64_t col_tiles) {
 
 inline int64_t max_row_tiles(int64_t rows, int E, int BM) { return rows / BM + E; }
 
+// ---- row tiles without a table ---------------------------------------------------------------------------------
+// Inclusive prefix sum over the 64 lanes of a wave (data-parallel moves: no LDS round trips).
+__device__ __forceinline__ int32_t wave_inclusive_sum(int32_t v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1, missing lanes read 0
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+// Expert e owns ceil(count_e / bm) consecutive row tiles.  Which expert and rows `tile` has, found by one wave from the
+// offsets (64 experts at a time); false when there are fewer tiles.  Costs a load and some thirty instructions per 64
+// experts, against a launch of its own (3-6 us) for a table of tiles.
+constexpr int kMaxScannedExperts = 512;
+__device__ __forceinline__ bool find_row_tile(const int32_t* __restrict__ offsets, int E, int bm, int tile, int lane,
+                                              int& expert, int32_t& row0, int32_t& row_end) {
+    int before = 0;
+    for (int e0 = 0; e0 < E; e0 += kWaveSize) {
+        const int e = e0 + lane;
+        const int32_t begin = offsets[e < E ? e : E], end = offsets[e < E ? e + 1 : E];
+        const int32_t mine = (end - begin + bm - 1) / bm;
+        const int32_t upto = before + wave_inclusive_sum(mine);
+        const uint64_t holder = __ballot(tile < upto);  // lanes at or after the expert that has the tile
+        if (holder != 0) {
+            const int l = __ffsll((unsigned long long)holder) - 1;
+            expert = e0 + l;
+            const int first = __builtin_amdgcn_readlane(upto - mine, l);
+            row0 = __builtin_amdgcn_readlane(begin, l) + (tile - first) * bm;
+            const int32_t last = __builtin_amdgcn_readlane(end, l);
+            row_end = row0 + bm < last ? row0 + bm : last;
+            return true;
+        }
+        before = __builtin_amdgcn_readlane(upto, kWaveSize - 1);
+    }
+    return false;
+}
+
 // The MFMA instruction of the register-staged kernel for 16-bit types: acc(32x32) += X(32 x 16) * Y(32 x 16)^T,
 // lane l supplies row l%32 and the 8 reduction elements 8*(l/32)..8*(l/32)+7 of both operands.
 template <typename T>
@@ -315,5 +354,16 @@ void fill_params(const xma_grouped_gemm_args& a, GemmParams& P);
 // The LDS-DMA pipelined kernel for 16-bit element types (grouped_gemm_dma.hip).
 bool dma_gemm_supports(const xma_grouped_gemm_args& a);
 int launch_dma_gemm(const xma_grouped_gemm_args& a, hipStream_t stream);
+
+// The weight-streaming kernel for few routed rows per expert (grouped_gemm_skinny.hip).
+// Taken up to kSkinnyRows routed rows per expert on average: with every further row tile of an expert its weights are
+// streamed once more.  Measured, bf16, up + down projection: H 4096, I 14336, E 8 at 16 / 24 / 32 rows per expert 595 /
+// 652 / 857 us against 668 / 670 / 671 us of the 256 x 256 kernel; H 2048, I 1024, E 64 at 12 / 28 rows 162 / 212 us against
+// 214 / 217 us.  Row tiles of 16 up to kSkinnyOneBlock rows on average, of 32 beyond (fewer loads of the routed rows
+// per weight, but twice the registers: at 2 rows 5 % slower, at 12 rows 10 % faster).
+constexpr int kSkinnyRows = 24;
+constexpr int kSkinnyOneBlock = 8;
+bool skinny_gemm_supports(const xma_grouped_gemm_args& a);
+int launch_skinny_gemm(const xma_grouped_gemm_args& a, hipStream_t stream);
 
 }  // namespace xma

@@ -1,0 +1,275 @@
+// Forward projections (TN) over few routed rows per expert: a decoded token, a serving batch, a short prompt.
+//
+//   C[p, n] = sum_k A[row(p), k] * W[e][n, k] (+ bias[e][n])     plain, tanh-GELU or gated epilogue
+//
+// Bound by reading the weights of the experts that are hit, once, from HBM.  The tiled kernels give a compute unit
+// 256 weight rows and one wave per SIMD, so a call with a few row tiles leaves most of the device idle and every
+// tile waits for its own prologue.  Here a work-group owns 16 * NF weight rows and 16 * RF routed rows and its four
+// waves SPLIT THE REDUCTION: each streams its quarter of the weight rows straight from memory into matrix-instruction
+// operands (no LDS, no barrier, U * NF 16-byte loads of weights in flight per lane and several work-groups per compute
+// unit), and the four partial tiles are added in wave order through LDS.  Many small work-groups keep HBM busy
+// whatever the number of experts that are hit.
+//
+// Measured against the 256 x 256 kernel, up + down projection, inputs changing from call to call: H 2048, I 1024, E 64,
+// k 6, one token (6 experts, 75 MB of weights) 21 us instead of 82; 16 tokens 112 us instead of 192 (5.7 TB/s of
+// weights); H 4096, I 14336, E 8, k 2, 8 tokens 418 us instead of 594 (5.6 TB/s), 32 tokens 560 us instead of 667.
+// In fp32 (the 128 x 128 register-staged kernel before) one token 38 us instead of 248.
+// What was chosen by measurement: four waves (eight: 2-5 % slower); U = 2 for 2 x 1 blocks (4: 5-10 % slower at
+// H 2048, 8: 40 % slower, the registers of the longer batches cost wavefronts); streaming loads of the weights 7-10 %
+// slower.
+//
+// Which rows a work-group has is found by each wave on its own from the expert offsets (find_row_tile), so there is
+// no table to build in a launch of its own.
+#include <type_traits>
+
+#include "grouped_gemm_common.h"
+
+namespace xma {
+namespace skinny {
+
+constexpr int THREADS = 256, WAVES = THREADS / kWaveSize;
+
+// acc(16 x 16) += W(16 weight rows x 4 chunks) * X(16 routed rows x 4 chunks)^T where lane l supplies the 16-byte chunk
+// l / 16 of row l % 16 of both operands; register r of lane l is [weight row 4 * (l / 16) + r][routed row l % 16].
+// The order in which a chunk's elements meet the matrix instruction's reduction slots does not matter as long as it is
+// the same for both operands.
+template <typename T>
+__device__ __forceinline__ void mma(const uint4& w, const uint4& x, f32x4_t& acc) {
+    if constexpr (std::is_same<T, float>::value) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w.x), __uint_as_float(x.x), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w.y), __uint_as_float(x.y), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w.z), __uint_as_float(x.z), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w.w), __uint_as_float(x.w), acc, 0, 0, 0);
+    } else if constexpr (std::is_same<T, bf16_t>::value) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x),
+                                                      acc, 0, 0, 0);
+    } else {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, w), __builtin_bit_cast(f16x8_t, x), acc,
+                                                     0, 0, 0);
+    }
+}
+
+// value as the layer's type holds it
+template <typename T>
+__device__ __forceinline__ float rounded(float v) {
+    if constexpr (std::is_same<T, float>::value) return v;
+    T t;
+    Elem<T>::store(&t, v);
+    return Elem<T>::load(&t);
+}
+
+template <typename T>
+__device__ __forceinline__ void store4(T* p, const float (&v)[4]) {
+    if constexpr (std::is_same<T, float>::value)
+        *reinterpret_cast<uint4*>(p) = Elem<float>::pack(v);
+    else
+        *reinterpret_cast<uint2*>(p) = make_uint2(Elem<T>::pack2(v[0], v[1]), Elem<T>::pack2(v[2], v[3]));
+}
+template <typename T>
+__device__ __forceinline__ void load4(const T* p, float (&v)[4]) {
+    if constexpr (std::is_same<T, float>::value) {
+        Elem<float>::unpack(*reinterpret_cast<const uint4*>(p), v);
+    } else {
+        const uint2 raw = *reinterpret_cast<const uint2*>(p);
+        float u[8];
+        Elem<T>::unpack(make_uint4(raw.x, raw.y, 0u, 0u), u);
+        for (int q = 0; q < 4; ++q) v[q] = u[q];
+    }
+}
+
+// NF: 16-row blocks of weights per work-group; a gated tile (EPI_PAIRED) takes NF / 2 blocks of each half.
+// RF: 16-row blocks of routed rows.  U: 64-byte steps of every row requested together.
+template <typename T, int NF, int RF, int EPI, int U>
+__global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(const GemmParams P, int64_t rows) {
+    constexpr int PV = Elem<T>::kPerVec;
+    constexpr int STEP = 4 * PV;  // reduction elements of one 64-byte step
+    constexpr bool PAIRED = EPI == EPI_PAIRED;
+    constexpr int NF_OUT = PAIRED ? NF / 2 : NF;  // blocks of output columns
+    constexpr int BM = 16 * RF, BN_OUT = 16 * NF_OUT;
+    static_assert(!PAIRED || NF % 2 == 0, "a gated tile pairs blocks");
+    __shared__ __attribute__((aligned(16))) f32x4_t partial[WAVES][NF * RF][kWaveSize];
+
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWaveSize);
+    const int row_tile = blockIdx.x / P.col_tiles;
+    const int col_tile = blockIdx.x - row_tile * P.col_tiles;
+
+    int expert = 0;
+    int32_t m_begin, m_end;
+    if (P.offsets == nullptr) {  // one group: a plain product
+        m_begin = row_tile * BM;
+        m_end = m_begin + BM < rows ? m_begin + BM : (int32_t)rows;
+    } else if (!find_row_tile(P.offsets, P.num_experts, BM, row_tile, lane, expert, m_begin, m_end)) {
+        return;  // (the same for every wave of the work-group)
+    }
+
+    const T* A = reinterpret_cast<const T*>(P.a);
+    const T* W = reinterpret_cast<const T*>(P.b) + (int64_t)expert * P.b_expert_stride;
+    const int64_t n_out = PAIRED ? P.n / 2 : P.n;
+    const int64_t n0 = (int64_t)col_tile * BN_OUT;
+    const int row16 = lane & 15, quarter = lane >> 4;
+
+    // Rows past the end of the tile or of the weights read an existing row: their results are dropped.
+    const T* xp[RF];
+    const T* wp[NF];
+#pragma unroll
+    for (int r = 0; r < RF; ++r) {
+        int64_t p = m_begin + r * 16 + row16;
+        p = p < m_end ? p : m_end - 1;
+        const int64_t src = P.in_index ? source_row(P, p) : p;
+        xp[r] = A + src * P.lda + quarter * PV;
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        int64_t n = n0 + (f % NF_OUT) * 16 + row16;
+        n = n < n_out ? n : n_out - 1;
+        wp[f] = W + (n + (f >= NF_OUT ? n_out : 0)) * P.ldb + quarter * PV;
+    }
+
+    f32x4_t acc[NF][RF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int r = 0; r < RF; ++r) acc[f][r] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // this wave's steps, in whole 128-byte lines
+    const int steps = (int)((P.k + STEP - 1) / STEP);
+    const int per_wave = ((steps + WAVES - 1) / WAVES + 1) / 2 * 2;
+    const int first = wave * per_wave < steps ? wave * per_wave : steps;
+    const int last = first + per_wave < steps ? first + per_wave : steps;
+    const int whole = P.k % STEP == 0 ? last : (last < steps ? last : steps - 1);  // steps without missing elements
+    const int batches = whole > first ? (whole - first) / U : 0;
+
+    uint4 w[2][U][NF], x[2][U][RF];
+    auto load_batch = [&](int set, int step) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t k = (int64_t)(step + u) * STEP;
+#pragma unroll
+            for (int f = 0; f < NF; ++f) w[set][u][f] = *reinterpret_cast<const uint4*>(wp[f] + k);
+#pragma unroll
+            for (int r = 0; r < RF; ++r) x[set][u][r] = *reinterpret_cast<const uint4*>(xp[r] + k);
+        }
+    };
+    auto multiply_batch = [&](int set) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+#pragma unroll
+                for (int r = 0; r < RF; ++r) mma<T>(w[set][u][f], x[set][u][r], acc[f][r]);
+    };
+    if (batches > 0) load_batch(0, first);
+    for (int b = 0; b < batches; b += 2) {
+        if (b + 1 < batches) load_batch(1, first + (b + 1) * U);
+        multiply_batch(0);
+        if (b + 1 < batches) {
+            if (b + 2 < batches) load_batch(0, first + (b + 2) * U);
+            multiply_batch(1);
+        }
+    }
+    // the remaining steps one by one; elements past the end of the reduction are zero in both operands
+    for (int s = first + batches * U; s < last; ++s) {
+        const int64_t k = (int64_t)s * STEP;
+        const bool exists = k + quarter * PV < P.k;
+        const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+        uint4 wv[NF], xv[RF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) wv[f] = exists ? *reinterpret_cast<const uint4*>(wp[f] + k) : zero;
+#pragma unroll
+        for (int r = 0; r < RF; ++r) xv[r] = exists ? *reinterpret_cast<const uint4*>(xp[r] + k) : zero;
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+            for (int r = 0; r < RF; ++r) mma<T>(wv[f], xv[r], acc[f][r]);
+    }
+
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int r = 0; r < RF; ++r) partial[wave][f * RF + r][lane] = acc[f][r];
+    __syncthreads();
+
+    // epilogue: a thread owns four adjacent columns of one row (for a gated tile, of both halves)
+    T* C = reinterpret_cast<T*>(P.c);
+    T* H = reinterpret_cast<T*>(P.aux);
+    for (int item = threadIdx.x; item < NF_OUT * RF * kWaveSize; item += THREADS) {
+        const int block = item / kWaveSize, l = item % kWaveSize;
+        const int f = block / RF, r = block % RF;
+        const int64_t p = m_begin + r * 16 + (l & 15);
+        const int64_t n = n0 + f * 16 + 4 * (l >> 4);
+        if (p >= m_end || n >= n_out) continue;
+        auto sum_of = [&](int frag, int64_t column, float (&v)[4]) {
+            f32x4_t s = partial[0][frag * RF + r][l];
+#pragma unroll
+            for (int wv = 1; wv < WAVES; ++wv) s += partial[wv][frag * RF + r][l];
+            for (int q = 0; q < 4; ++q) v[q] = s[q];
+            if (P.bias != nullptr) {
+                float b[4];
+                load4(reinterpret_cast<const T*>(P.bias) + (int64_t)expert * P.ld_bias + column, b);
+                for (int q = 0; q < 4; ++q) v[q] += b[q];
+            }
+        };
+        const int64_t out_row = P.out_index ? load_index(P.out_index, P.idx_is_i64, p) : p;
+        constexpr bool FAST = !std::is_same<T, float>::value;
+        float v[4], o[4];
+        sum_of(f, n, v);
+        if constexpr (PAIRED) {
+            float g[4];
+            sum_of(f + NF_OUT, n_out + n, g);
+            if (H) {
+                store4(H + p * P.ld_aux + n, v);
+                store4(H + p * P.ld_aux + n_out + n, g);
+            }
+            for (int q = 0; q < 4; ++q) o[q] = gated_forward<FAST>(P.act, rounded<T>(v[q]), rounded<T>(g[q]));
+            store4(C + out_row * P.ldc + n, o);
+        } else if (P.act == ACT_GELU_TANH) {
+            if (H) store4(H + p * P.ld_aux + n, v);
+            for (int q = 0; q < 4; ++q) o[q] = gelu_tanh_forward<FAST>(rounded<T>(v[q]));
+            store4(C + out_row * P.ldc + n, o);
+        } else {
+            store4(C + out_row * P.ldc + n, v);
+        }
+    }
+}
+
+template <typename T, int NF, int RF, int EPI, int U>
+static int launch(const GemmParams& params, int64_t rows, hipStream_t stream) {
+    GemmParams P = params;
+    const int64_t n_out = EPI == EPI_PAIRED ? P.n / 2 : P.n;
+    P.col_tiles = (int32_t)ceil_div(n_out, EPI == EPI_PAIRED ? 8 * NF : 16 * NF);
+    const int64_t row_tiles =
+        P.offsets == nullptr ? ceil_div(rows, 16 * RF) : rows / (16 * RF) + (rows < P.num_experts ? rows : P.num_experts);
+    const int64_t grid = row_tiles * P.col_tiles;
+    XMA_REQUIRE(grid < ((int64_t)1 << 31), "xma_grouped_gemm: %lld tiles exceed the grid limit", (long long)grid);
+    hipLaunchKernelGGL((skinny_gemm_kernel<T, NF, RF, EPI, U>), dim3((unsigned)grid), dim3(THREADS), 0, stream, P, rows);
+    return check_launch("xma_grouped_gemm");
+}
+
+template <typename T>
+static int dispatch(const xma_grouped_gemm_args& a, const GemmParams& P, hipStream_t stream) {
+    int shape = EPI_PLAIN, act = ACT_NONE;
+    split_epilogue(a.epilogue, shape, act);
+    const bool one_block = a.rows <= kSkinnyOneBlock * (int64_t)a.num_experts;
+    if (shape == EPI_PAIRED)
+        return one_block ? launch<T, 2, 1, EPI_PAIRED, 2>(P, a.rows, stream)
+                         : launch<T, 4, 2, EPI_PAIRED, 1>(P, a.rows, stream);
+    return one_block ? launch<T, 2, 1, EPI_PLAIN, 2>(P, a.rows, stream)
+                     : launch<T, 4, 2, EPI_PLAIN, 1>(P, a.rows, stream);
+}
+
+}  // namespace skinny
+
+bool skinny_gemm_supports(const xma_grouped_gemm_args& a) {
+    return a.kind == XMA_GEMM_TN && a.k > 0 && a.num_experts <= kMaxScannedExperts &&
+           a.rows <= kSkinnyRows * (int64_t)a.num_experts;
+}
+
+int launch_skinny_gemm(const xma_grouped_gemm_args& a, hipStream_t stream) {
+    GemmParams P;
+    fill_params(a, P);
+    if (a.dtype == XMA_F32) return skinny::dispatch<float>(a, P, stream);
+    return a.dtype == XMA_BF16 ? skinny::dispatch<bf16_t>(a, P, stream) : skinny::dispatch<f16_t>(a, P, stream);
+}
+
+}  // namespace xma

@@ -185,6 +185,51 @@ def test_fused_activations_and_bias(case, activation, dtype):
     assert_close(d_pre, leaf.grad, tol, f"fused {activation} backward")
 
 
+FEW_ROWS = [
+    # rows per expert, reduction, columns of the gated projection
+    ([1], 8, 16),  # one row, one 16-byte chunk of reduction, half a block of columns
+    ([0, 1, 0, 16, 0, 17, 2], 2048, 272),  # empty experts in between; one block exactly, one row more
+    ([15, 33, 1, 32, 31] + [0] * 70 + [7], 520, 144),  # beyond 64 experts; reduction ends inside a step
+    ([20, 24, 9, 31, 5], 424, 80),  # row tiles of 32; reduction shorter than two steps of every wave
+    ([100, 3], 1096, 112),  # many row tiles of one expert
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("sizes,K,N", FEW_ROWS)
+def test_forward_with_few_rows_per_expert(sizes, K, N, dtype):
+    """The weight-streaming kernel of the forward projections at the edges of its row tiles (16 and 32), of its
+    64-byte steps and of its 16-column blocks: gathered rows and gated epilogue, scattered rows with a bias."""
+
+    E, M, dev = len(sizes), sum(sizes), "cuda"
+    g = torch.Generator().manual_seed(M + K + N)
+    off_list = [0] + torch.tensor(sizes).cumsum(0).tolist()
+    off = torch.tensor(off_list, dtype=torch.int32, device=dev)
+    se = torch.repeat_interleave(torch.arange(E), torch.tensor(sizes))
+    idx = torch.randperm(M, generator=g)
+    x = torch.randn(M, K, generator=g).to(dtype)
+    w = (torch.randn(E, N, K, generator=g) * 0.05).to(dtype)
+    b = (torch.randn(E, N, generator=g) * 0.5).to(dtype)
+    product = torch.cat([x[idx][off_list[e] : off_list[e + 1]].float() @ w[e].float().T for e in range(E)])
+    product = product + b.float()[se]
+    elem = GEMM_ELEM_TOL[dtype]
+
+    act = torch.empty(M, N // 2, dtype=dtype, device=dev)
+    pre = torch.full((M, N), float("nan"), dtype=dtype, device=dev)
+    args = (x.to(dev), w.to(dev), idx.to(dev).int(), off)
+    ops.up_projection_fused(*args, act, pre, 1, "swiglu", b.to(dev))
+    assert_close(pre, product, TOL[dtype], "pre-activation, few rows", elem_tol=elem)
+    assert_close(act, to.swiglu_packed(pre.float().cpu()), TOL[dtype], "swiglu, few rows")
+
+    out = torch.full((M, N), float("nan"), dtype=dtype, device=dev)
+    xg = x[idx].to(dev)
+    ops.scatter2scatter(xg, w.to(dev).permute(0, 2, 1), se.to(dev).int(), idx.to(dev).int(), out, 1, True, False, off,
+                        b.to(dev))
+    want = torch.empty(M, N)
+    want[idx] = product
+    assert_close(out, want, TOL[dtype], "scattered rows, few rows", elem_tol=elem)
+
+
 def test_full_length_reductions_dense():
     """Every layout once at the row counts of the benchmark layer (16384 routed rows over 8 experts, about 2048 per
     expert) with DENSE operands, so that the weight-gradient kernel's reductions run over ~2048 non-zero rows (32
