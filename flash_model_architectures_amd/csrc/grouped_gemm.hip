@@ -13,8 +13,8 @@
 // the epilogue stages the tile in LDS again so that HBM sees full 16-byte row-wise stores
 // (optionally fused with SwiGLU forward / backward, row scatter).
 //
-// Work-group -> tile mapping: a prologue kernel expands the expert offsets into a list of row
-// tiles (expert, first row), so ragged and empty groups cost nothing; the main kernel renumbers
+// Work-group -> tile mapping: every wave finds its row tile (expert, first row) from the expert offsets,
+// so ragged and empty groups cost nothing; the kernel renumbers
 // work-groups so that each of the 8 XCDs (private L2 each) owns a contiguous range of tiles, and
 // walks tiles in bands of 4 row tiles x all column tiles to reuse both panels from L2.
 #include <cstddef>
@@ -233,7 +233,11 @@ __global__ __launch_bounds__(TileCfg<T>::THREADS) void grouped_gemm_kernel(const
     const int wn0 = (wave % Cfg::WAVES_N) * WN;
 
     // ---- which tile ----
-    const int row_tiles = KIND == XMA_GEMM_MT ? P.row_tiles_max * P.num_experts : P.tile_count[0];
+    // the row tiles present: from the table, or from the offsets when there is none
+    const bool table = KIND == XMA_GEMM_MT || P.tile_count != nullptr;
+    const RowTileScan tiles(P.offsets, table ? 0 : P.num_experts, BM, lane);
+    const int row_tiles =
+        KIND == XMA_GEMM_MT ? P.row_tiles_max * P.num_experts : table ? P.tile_count[0] : tiles.total;
     int row_tile, col_tile;
     if (!locate_tile<KIND == XMA_GEMM_MT>(row_tiles, P.col_tiles, row_tile, col_tile)) return;
 
@@ -253,10 +257,17 @@ __global__ __launch_bounds__(TileCfg<T>::THREADS) void grouped_gemm_kernel(const
         red_len = m_end - m_begin;
         n0 = (int64_t)col_tile * BN;
     } else {
-        expert = P.tile_expert[row_tile];
-        m_begin = P.tile_row0[row_tile];
-        const int64_t e_end = P.offsets[expert + 1];
-        m_end = m_begin + BM < e_end ? m_begin + BM : e_end;
+        if (table) {
+            expert = P.tile_expert[row_tile];
+            m_begin = P.tile_row0[row_tile];
+            const int64_t e_end = P.offsets[expert + 1];
+            m_end = m_begin + BM < e_end ? m_begin + BM : e_end;
+        } else {
+            int32_t row0, row_end;
+            tiles.find(row_tile, expert, row0, row_end);
+            m_begin = row0;
+            m_end = row_end;
+        }
         red_len = P.k;
         n0 = (int64_t)col_tile * BN_OUT;
     }
@@ -562,17 +573,19 @@ static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
         grid = grid_for_tiles((int64_t)P.row_tiles_max * a.num_experts, P.col_tiles);
     } else {
         const int64_t rt = max_row_tiles(a.rows, a.num_experts, Cfg::BM);
-        int32_t* ws = reinterpret_cast<int32_t*>(a.workspace);
-        P.tile_count = ws;
-        P.tile_expert = ws + 4;
-        P.tile_row0 = ws + 4 + rt;
         P.row_tiles_max = (int32_t)rt;
         const int bn_out = EPI == EPI_PAIRED ? Cfg::BN / 2 : Cfg::BN;
         const int64_t n_out = EPI == EPI_PAIRED ? a.n / 2 : a.n;
         P.col_tiles = (int32_t)ceil_div(n_out, bn_out);
         grid = grid_for_tiles(rt, P.col_tiles);
-        hipLaunchKernelGGL(build_row_tiles_kernel, dim3(1), dim3(1024), 0, stream, a.expert_offsets, a.num_experts,
-                           Cfg::BM, ws + 4, ws + 4 + rt, ws, nullptr);
+        if (a.num_experts > kMaxScannedExperts) {
+            int32_t* ws = reinterpret_cast<int32_t*>(a.workspace);
+            P.tile_count = ws;
+            P.tile_expert = ws + 4;
+            P.tile_row0 = ws + 4 + rt;
+            hipLaunchKernelGGL(build_row_tiles_kernel, dim3(1), dim3(1024), 0, stream, a.expert_offsets, a.num_experts,
+                               Cfg::BM, ws + 4, ws + 4 + rt, ws, nullptr);
+        }
     }
     XMA_REQUIRE(grid < ((int64_t)1 << 31), "xma_grouped_gemm: %lld tiles exceed the grid limit", (long long)grid);
     (void)PV;

@@ -24,9 +24,9 @@ struct GemmParams {
     const int32_t* offsets;
     const void* in_index;
     const void* out_index;
-    const int32_t* tile_expert;  // [row tiles] expert of each row tile (TN/NN)
+    const int32_t* tile_expert;  // [row tiles] expert of each row tile (TN/NN; only beyond kMaxScannedExperts experts)
     const int32_t* tile_row0;    // [row tiles] first grouped row of each row tile
-    const int32_t* tile_count;   // [1] number of row tiles actually present
+    const int32_t* tile_count;   // [1] number of row tiles actually present; nullptr: no table
     int64_t lda, ldb, ldc, ld_aux, b_expert_stride, c_expert_stride;
     int64_t n, k;
     int32_t num_experts, in_fan_out, idx_is_i64;
@@ -269,32 +269,51 @@ __device__ __forceinline__ int32_t wave_inclusive_sum(int32_t v) {
     return v;
 }
 
-// Expert e owns ceil(count_e / bm) consecutive row tiles.  Which expert and rows `tile` has, found by one wave from the
-// offsets (64 experts at a time); false when there are fewer tiles.  Costs a load and some thirty instructions per 64
-// experts, against a launch of its own (3-6 us) for a table of tiles.
-constexpr int kMaxScannedExperts = 512;
-__device__ __forceinline__ bool find_row_tile(const int32_t* __restrict__ offsets, int E, int bm, int tile, int lane,
-                                              int& expert, int32_t& row0, int32_t& row_end) {
-    int before = 0;
-    for (int e0 = 0; e0 < E; e0 += kWaveSize) {
-        const int e = e0 + lane;
-        const int32_t begin = offsets[e < E ? e : E], end = offsets[e < E ? e + 1 : E];
-        const int32_t mine = (end - begin + bm - 1) / bm;
-        const int32_t upto = before + wave_inclusive_sum(mine);
-        const uint64_t holder = __ballot(tile < upto);  // lanes at or after the expert that has the tile
-        if (holder != 0) {
-            const int l = __ffsll((unsigned long long)holder) - 1;
-            expert = e0 + l;
-            const int first = __builtin_amdgcn_readlane(upto - mine, l);
-            row0 = __builtin_amdgcn_readlane(begin, l) + (tile - first) * bm;
-            const int32_t last = __builtin_amdgcn_readlane(end, l);
-            row_end = row0 + bm < last ? row0 + bm : last;
-            return true;
+// Expert e owns ceil(count_e / bm) consecutive row tiles.  How many there are and which expert and rows a tile has, found
+// by each wave on its own from the offsets: lane l adds up the tiles of the l-th run of consecutive experts, one prefix
+// sum over the lanes.  Costs a load and some thirty instructions, against a launch of its own (3-6 us and the gap
+// before the next) for a table of tiles.
+constexpr int kMaxScannedExperts = 512;  // up to eight experts per lane
+struct RowTileScan {
+    const int32_t* offsets;
+    int experts, per_lane, bm;
+    int first_tile;  // of the lane's run
+    int upto;        // first_tile + the run's tiles
+    int total;
+
+    __device__ __forceinline__ int tiles_of(int32_t begin, int32_t end) const { return (end - begin + bm - 1) / bm; }
+    __device__ __forceinline__ RowTileScan(const int32_t* __restrict__ expert_offsets, int E, int tile_rows, int lane)
+        : offsets(expert_offsets), experts(E), per_lane((E + kWaveSize - 1) / kWaveSize), bm(tile_rows) {
+        const int e0 = lane * per_lane;
+        int32_t begin = offsets[e0 < E ? e0 : E];
+        int mine = 0;
+        for (int i = 1; i <= per_lane; ++i) {
+            const int32_t end = offsets[e0 + i < E ? e0 + i : E];
+            mine += tiles_of(begin, end);
+            begin = end;
         }
-        before = __builtin_amdgcn_readlane(upto, kWaveSize - 1);
+        upto = wave_inclusive_sum(mine);
+        first_tile = upto - mine;
+        total = __builtin_amdgcn_readlane(upto, kWaveSize - 1);
     }
-    return false;
-}
+    // tile < total
+    __device__ __forceinline__ void find(int tile, int& expert, int32_t& row0, int32_t& row_end) const {
+        const int l = __ffsll((unsigned long long)__ballot(tile < upto)) - 1;
+        int before = __builtin_amdgcn_readlane(first_tile, l);
+        expert = l * per_lane;
+        int32_t begin = offsets[expert], end = offsets[expert + 1];
+        for (int i = 1; i < per_lane && tile >= before + tiles_of(begin, end); ++i) {
+            before += tiles_of(begin, end);
+            ++expert;
+            begin = end;
+            end = offsets[expert + 1];
+        }
+        // (the compiler does not see that these are the same in every lane)
+        expert = __builtin_amdgcn_readfirstlane(expert);
+        row0 = __builtin_amdgcn_readfirstlane(begin + (tile - before) * bm);
+        row_end = __builtin_amdgcn_readfirstlane(row0 + bm < end ? row0 + bm : end);
+    }
+};
 
 // The MFMA instruction of the register-staged kernel for 16-bit types: acc(32x32) += X(32 x 16) * Y(32 x 16)^T,
 // lane l supplies row l%32 and the 8 reduction elements 8*(l/32)..8*(l/32)+7 of both operands.
@@ -347,6 +366,10 @@ struct Mma<float> {
         acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(x.w), __uint_as_float(y.w), acc, 0, 0, 0);
     }
 };
+
+// a launch splits the tiles of its last round only when a part keeps kSplitMinStages stages
+inline bool may_split(int64_t reduction) { return (reduction + 63) / 64 >= 2 * kSplitMinStages; }
+static __global__ void clear_split_counters_kernel(int32_t* counters) { counters[threadIdx.x] = 0; }
 
 // Fills the fields of GemmParams that do not depend on the tile shape.
 void fill_params(const xma_grouped_gemm_args& a, GemmParams& P);

@@ -513,21 +513,37 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
     k.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     int row_tile, col_tile;
+    int tile_expert = 0;
+    int64_t m_begin, m_end, tile_i0 = 0, n0;
     TileWork work;
     work.parts = 1;
     if constexpr (KIND == XMA_GEMM_MT) {
         if (!locate_tile<true>(P.row_tiles_max * P.num_experts, P.col_tiles, row_tile, col_tile)) return;
     } else {
-        if (!locate_work(P.tile_count[0], P.col_tiles, P.num_cu, (P.k + K::BK - 1) / K::BK, work)) return;
+        // the row tiles present and this one's rows: from the table, or from the offsets when there is none
+        const bool table = P.tile_count != nullptr;
+        const RowTileScan tiles(P.offsets, table ? 0 : P.num_experts, BM, k.lane);
+        const int64_t stages = (P.k + K::BK - 1) / K::BK;
+        if (!locate_work(table ? P.tile_count[0] : tiles.total, P.col_tiles, P.num_cu, stages, work)) return;
         row_tile = work.row_tile;
         col_tile = work.col_tile;
+        int32_t row0, row_end;
+        if (table) {
+            tile_expert = P.tile_expert[row_tile];
+            row0 = P.tile_row0[row_tile];
+            const int32_t last = P.offsets[tile_expert + 1];
+            row_end = row0 + BM < last ? row0 + BM : last;
+        } else {
+            tiles.find(row_tile, tile_expert, row0, row_end);
+        }
+        m_begin = row0;
+        m_end = row_end;
     }
 
     const T* A = reinterpret_cast<const T*>(P.a);
     const T* B = reinterpret_cast<const T*>(P.b);
 
     int expert;
-    int64_t m_begin, m_end, tile_i0 = 0, n0;
     if constexpr (KIND == XMA_GEMM_MT) {
         const int slot = row_tile / P.row_tiles_max;
         tile_i0 = (int64_t)(row_tile % P.row_tiles_max) * BM;
@@ -544,10 +560,7 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
         k.red_len = m_end - m_begin;
         n0 = (int64_t)col_tile * BN;
     } else {
-        expert = P.tile_expert[row_tile];
-        m_begin = P.tile_row0[row_tile];
-        const int64_t e_end = P.offsets[expert + 1];
-        m_end = m_begin + BM < e_end ? m_begin + BM : e_end;
+        expert = tile_expert;
         k.red_len = P.k;
         n0 = (int64_t)col_tile * BN_OUT;
     }
@@ -1010,9 +1023,6 @@ static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
     } else {
         const int64_t rt = max_row_tiles(a.rows, a.num_experts, BM);
         int32_t* ws = reinterpret_cast<int32_t*>(a.workspace);
-        P.tile_count = ws;
-        P.tile_expert = ws + 4;
-        P.tile_row0 = ws + 4 + rt;
         P.row_tiles_max = (int32_t)rt;
         // the split-K region is the tail of the workspace
         char* split = reinterpret_cast<char*>(a.workspace) +
@@ -1024,8 +1034,15 @@ static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
         const int64_t n_out = EPI == EPI_PAIRED ? a.n / 2 : a.n;
         P.col_tiles = (int32_t)ceil_div(n_out, bn_out);
         grid = grid_for_work(rt * P.col_tiles);
-        hipLaunchKernelGGL(build_row_tiles_kernel, dim3(1), dim3(1024), 0, stream, a.expert_offsets, a.num_experts, BM,
-                           ws + 4, ws + 4 + rt, ws, P.split_counters);
+        if (a.num_experts > kMaxScannedExperts) {
+            P.tile_count = ws;
+            P.tile_expert = ws + 4;
+            P.tile_row0 = ws + 4 + rt;
+            hipLaunchKernelGGL(build_row_tiles_kernel, dim3(1), dim3(1024), 0, stream, a.expert_offsets, a.num_experts,
+                               BM, ws + 4, ws + 4 + rt, ws, P.split_counters);
+        } else if (may_split(a.k)) {
+            hipLaunchKernelGGL(clear_split_counters_kernel, dim3(1), dim3(kSplitSlots), 0, stream, P.split_counters);
+        }
     }
     XMA_REQUIRE(grid < ((int64_t)1 << 31), "xma_grouped_gemm: %lld tiles exceed the grid limit", (long long)grid);
     hipLaunchKernelGGL((grouped_gemm_dma_kernel<T, KIND, EPI, Pipe>), dim3((unsigned)grid), dim3(THREADS), 0, stream, P);

@@ -18,7 +18,7 @@
 // H 2048, 8: 40 % slower, the registers of the longer batches cost wavefronts); streaming loads of the weights 7-10 %
 // slower.
 //
-// Which rows a work-group has is found by each wave on its own from the expert offsets (find_row_tile), so there is
+// Which rows a work-group has is found by each wave on its own from the expert offsets (RowTileScan), so there is
 // no table to build in a launch of its own.
 #include <type_traits>
 
@@ -73,6 +73,7 @@ __device__ __forceinline__ void load4(const T* p, float (&v)[4]) {
         const uint2 raw = *reinterpret_cast<const uint2*>(p);
         float u[8];
         Elem<T>::unpack(make_uint4(raw.x, raw.y, 0u, 0u), u);
+#pragma unroll
         for (int q = 0; q < 4; ++q) v[q] = u[q];
     }
 }
@@ -99,8 +100,10 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(const GemmParams P
     if (P.offsets == nullptr) {  // one group: a plain product
         m_begin = row_tile * BM;
         m_end = m_begin + BM < rows ? m_begin + BM : (int32_t)rows;
-    } else if (!find_row_tile(P.offsets, P.num_experts, BM, row_tile, lane, expert, m_begin, m_end)) {
-        return;  // (the same for every wave of the work-group)
+    } else {
+        const RowTileScan tiles(P.offsets, P.num_experts, BM, lane);
+        if (row_tile >= tiles.total) return;  // (the same for every wave of the work-group)
+        tiles.find(row_tile, expert, m_begin, m_end);
     }
 
     const T* A = reinterpret_cast<const T*>(P.a);
@@ -203,10 +206,12 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(const GemmParams P
             f32x4_t s = partial[0][frag * RF + r][l];
 #pragma unroll
             for (int wv = 1; wv < WAVES; ++wv) s += partial[wv][frag * RF + r][l];
+#pragma unroll
             for (int q = 0; q < 4; ++q) v[q] = s[q];
             if (P.bias != nullptr) {
                 float b[4];
                 load4(reinterpret_cast<const T*>(P.bias) + (int64_t)expert * P.ld_bias + column, b);
+#pragma unroll
                 for (int q = 0; q < 4; ++q) v[q] += b[q];
             }
         };
@@ -221,10 +226,12 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(const GemmParams P
                 store4(H + p * P.ld_aux + n, v);
                 store4(H + p * P.ld_aux + n_out + n, g);
             }
+#pragma unroll
             for (int q = 0; q < 4; ++q) o[q] = gated_forward<FAST>(P.act, rounded<T>(v[q]), rounded<T>(g[q]));
             store4(C + out_row * P.ldc + n, o);
         } else if (P.act == ACT_GELU_TANH) {
             if (H) store4(H + p * P.ld_aux + n, v);
+#pragma unroll
             for (int q = 0; q < 4; ++q) o[q] = gelu_tanh_forward<FAST>(rounded<T>(v[q]));
             store4(C + out_row * P.ldc + n, o);
         } else {

@@ -230,6 +230,31 @@ def test_forward_with_few_rows_per_expert(sizes, K, N, dtype):
     assert_close(out, want, TOL[dtype], "scattered rows, few rows", elem_tol=elem)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("E", [65, 130, 600])
+def test_row_tiles_of_many_experts(E, dtype):
+    """More experts than lanes in a wave (two and three per lane in the prefix sum that finds a work-group's rows) and
+    more than the kernels look up themselves (a table of tiles), with empty experts and one many tiles long, at row
+    counts the tiled kernels take (more than 24 per expert on average)."""
+
+    dev, K, N = "cuda", 64, 72
+    g = torch.Generator().manual_seed(E)
+    sizes = torch.randint(0, 60, (E,), generator=g)
+    sizes[::7] = 0
+    sizes[E // 2], sizes[E - 1] = 2000, 1
+    assert int(sizes.sum()) > 24 * E
+    M = int(sizes.sum())
+    off_list = [0] + sizes.cumsum(0).tolist()
+    off = torch.tensor(off_list, dtype=torch.int32, device=dev)
+    x = torch.randn(M, K, generator=g).to(dtype)
+    w = (torch.randn(E, N, K, generator=g) * 0.1).to(dtype)
+    idx, se = torch.arange(M), torch.repeat_interleave(torch.arange(E), sizes)
+    out = torch.full((M, N), float("nan"), dtype=dtype, device=dev)
+    ops.scatter2scatter(x.to(dev), w.to(dev).permute(0, 2, 1), se.to(dev).int(), idx.to(dev).int(), out, 1, True, True, off)
+    want = torch.cat([x[off_list[e] : off_list[e + 1]].float() @ w[e].float().T for e in range(E)])
+    assert_close(out, want, TOL[dtype], "many experts", elem_tol=GEMM_ELEM_TOL[dtype])
+
+
 def test_full_length_reductions_dense():
     """Every layout once at the row counts of the benchmark layer (16384 routed rows over 8 experts, about 2048 per
     expert) with DENSE operands, so that the weight-gradient kernel's reductions run over ~2048 non-zero rows (32
