@@ -1,4 +1,7 @@
-// Ragged (per-expert) GEMM for gfx950 with MFMA and fp32 accumulation.
+// Ragged (per-expert) GEMM for gfx950 with MFMA and fp32 accumulation: the form that takes any size and alignment
+// (element-wise accesses, RAGGED), and the 16-bit weight gradient with a fused row gather.  Whole, aligned vectors go to
+// grouped_gemm_dma.hip (16-bit), grouped_gemm_f32.hip and grouped_gemm_skinny.hip (few rows per expert); the entry point
+// that chooses is here.
 //
 // One kernel body serves the three operand layouts of the MoE layer; they differ only in how a
 // tile is fetched from HBM:
@@ -633,28 +636,25 @@ void fill_params(const xma_grouped_gemm_args& a, GemmParams& P) {
     P.col_tiles = 0;
 }
 
-template <typename T, bool RAGGED>
-static int dispatch_kind(const xma_grouped_gemm_args& a, hipStream_t stream) {
+// Whole vectors only reach this kernel for the 16-bit weight gradient with a fused row gather; everything else that does
+// is ragged.
+template <typename T>
+static int dispatch_kind(const xma_grouped_gemm_args& a, bool ragged, hipStream_t stream) {
     int shape = EPI_PLAIN, act = ACT_NONE;
     split_epilogue(a.epilogue, shape, act);
     switch (a.kind) {
         case XMA_GEMM_TN:
-            if (shape == EPI_PAIRED) return launch<T, XMA_GEMM_TN, EPI_PAIRED, RAGGED>(a, stream);
-            return launch<T, XMA_GEMM_TN, EPI_PLAIN, RAGGED>(a, stream);
+            if (shape == EPI_PAIRED) return launch<T, XMA_GEMM_TN, EPI_PAIRED, true>(a, stream);
+            return launch<T, XMA_GEMM_TN, EPI_PLAIN, true>(a, stream);
         case XMA_GEMM_NN:
-            if (shape == EPI_BACKWARD) return launch<T, XMA_GEMM_NN, EPI_BACKWARD, RAGGED>(a, stream);
-            return launch<T, XMA_GEMM_NN, EPI_PLAIN, RAGGED>(a, stream);
+            if (shape == EPI_BACKWARD) return launch<T, XMA_GEMM_NN, EPI_BACKWARD, true>(a, stream);
+            return launch<T, XMA_GEMM_NN, EPI_PLAIN, true>(a, stream);
         default:
-            return launch<T, XMA_GEMM_MT, EPI_PLAIN, RAGGED>(a, stream);
+            if constexpr (sizeof(T) == 2)
+                if (!ragged) return launch<T, XMA_GEMM_MT, EPI_PLAIN, false>(a, stream);
+            return launch<T, XMA_GEMM_MT, EPI_PLAIN, true>(a, stream);
     }
 }
-template <typename T>
-static int dispatch_kind(const xma_grouped_gemm_args& a, bool ragged, hipStream_t stream) {
-    return ragged ? dispatch_kind<T, true>(a, stream) : dispatch_kind<T, false>(a, stream);
-}
-
-static int largest_bm() { return TileCfg<bf16_t>::BM > TileCfg<float>::BM ? TileCfg<bf16_t>::BM : TileCfg<float>::BM; }
-static int smallest_bm() { return TileCfg<bf16_t>::BM < TileCfg<float>::BM ? TileCfg<bf16_t>::BM : TileCfg<float>::BM; }
 
 }  // namespace xma
 
@@ -664,9 +664,8 @@ extern "C" {
 
 int64_t xma_grouped_gemm_workspace_bytes(int32_t num_experts, int64_t rows) {
     if (num_experts < 1 || rows < 0) return -1;
-    (void)largest_bm();
     // tile tables (sized for the smallest tile height of any kernel), then the split-K counters and partials
-    const int64_t rt = max_row_tiles(rows, num_experts, smallest_bm());
+    const int64_t rt = max_row_tiles(rows, num_experts, kSmallestTileRows);
     return tile_table_bytes(rt) + split_region_bytes();
 }
 
@@ -753,10 +752,11 @@ int xma_grouped_gemm(const xma_grouped_gemm_args* args, void* stream_) {
     const bool paired_tail = (a.epilogue == XMA_EPI_SWIGLU || a.epilogue == XMA_EPI_GLU) && a.n % (2 * pv) != 0;
     const bool elementwise = ragged || paired_tail;
     if (!elementwise && skinny_gemm_supports(a)) return launch_skinny_gemm(a, stream);
+    if (!elementwise && a.dtype == XMA_F32) return launch_f32_gemm(a, stream);
     if (!elementwise && dma_gemm_supports(a)) return launch_dma_gemm(a, stream);
     switch (a.dtype) {
         case XMA_F32:
-            return dispatch_kind<float>(a, elementwise, stream);
+            return dispatch_kind<float>(a, true, stream);
         case XMA_F16:
             return dispatch_kind<f16_t>(a, elementwise, stream);
         default:

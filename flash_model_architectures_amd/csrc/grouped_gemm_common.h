@@ -255,6 +255,7 @@ inline int64_t grid_for_tiles(int64_t row_tiles, int64_t col_tiles) {
     return ceil_div(bands, kNumXcd) * kNumXcd * kBandTiles * col_tiles;
 }
 
+constexpr int kSmallestTileRows = 32;  // of any kernel that may use a table of tiles
 inline int64_t max_row_tiles(int64_t rows, int E, int BM) { return rows / BM + E; }
 
 // ---- row tiles without a table ---------------------------------------------------------------------------------
@@ -378,11 +379,14 @@ void fill_params(const xma_grouped_gemm_args& a, GemmParams& P);
 bool dma_gemm_supports(const xma_grouped_gemm_args& a);
 int launch_dma_gemm(const xma_grouped_gemm_args& a, hipStream_t stream);
 
+// The kernel for fp32 operands in whole, aligned vectors (grouped_gemm_f32.hip).
+int launch_f32_gemm(const xma_grouped_gemm_args& a, hipStream_t stream);
+
 // The weight-streaming kernel for few routed rows per expert (grouped_gemm_skinny.hip).
 // Taken up to kSkinnyRows routed rows per expert on average: with every further row tile of an expert its weights are
 // streamed once more.  Measured, bf16, up + down projection: H 4096, I 14336, E 8 at 16 / 24 / 32 rows per expert 595 /
 // 652 / 857 us against 668 / 670 / 671 us of the 256 x 256 kernel; H 2048, I 1024, E 64 at 12 / 28 rows 162 / 212 us against
-// 214 / 217 us.  Row tiles of 16 up to kSkinnyOneBlock rows on average, of 32 beyond (fewer loads of the routed rows
+// 214 / 217 us.  In fp32, at 19 / 28 rows, 421 / 504 us against 562 / 405 us.  Row tiles of 16 up to kSkinnyOneBlock rows on average, of 32 beyond (fewer loads of the routed rows
 // per weight, but twice the registers: at 2 rows 5 % slower, at 12 rows 10 % faster).
 constexpr int kSkinnyRows = 24;
 constexpr int kSkinnyOneBlock = 8;

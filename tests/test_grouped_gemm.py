@@ -255,6 +255,53 @@ def test_row_tiles_of_many_experts(E, dtype):
     assert_close(out, want, TOL[dtype], "many experts", elem_tol=GEMM_ELEM_TOL[dtype])
 
 
+FP32_TILES = [
+    # rows per expert, K, N: tiles of 32 rows (few of them), of 64 and of 128 (enough output columns to fill the device)
+    ([1, 0, 31, 32, 33], 4, 4),
+    ([65, 40, 2], 36, 200),
+    ([64, 65, 129, 300], 68, 8192),
+    ([127, 128, 129, 97, 33, 0, 700], 100, 8196),
+    ([257, 900], 32, 8320),
+]
+
+
+@pytest.mark.parametrize("sizes,K,N", FP32_TILES)
+def test_fp32_tiles(sizes, K, N):
+    """The fp32 kernel at the edges of its tile heights (32, 64, 128 rows; 32-row blocks left out of an expert's last
+    tile), of its 32-deep stages (one, a partial one, two and three of them) and of its 128 columns, in all three
+    layouts, the weight gradient with and without the fused row gather.  Checker: float64 products."""
+
+    E, M, dev, dt = len(sizes), sum(sizes), "cuda", torch.float32
+    g = torch.Generator().manual_seed(M + K + N)
+    off_list = [0] + torch.tensor(sizes).cumsum(0).tolist()
+    off = torch.tensor(off_list, dtype=torch.int32, device=dev)
+    se = torch.repeat_interleave(torch.arange(E), torch.tensor(sizes)).int().to(dev)
+    idx = torch.randperm(M, generator=g).int().to(dev)
+    x = torch.randn(M, K, generator=g).to(dev)
+    w = torch.randn(E, N, K, generator=g).to(dev)
+    dy = torch.randn(M, N, generator=g).to(dev)
+    rows = [slice(off_list[e], off_list[e + 1]) for e in range(E)]
+    elem = GEMM_ELEM_TOL[dt]
+    xg = x[idx.long()]
+
+    out = torch.full((M, N), float("nan"), device=dev)
+    ops.scatter2scatter(x, w.permute(0, 2, 1), se, idx, out, 1, False, True, off)
+    want = torch.cat([xg[r].double() @ w[e].double().T for e, r in enumerate(rows)])
+    assert_close(out, want.float(), TOL[dt], "TN", elem_tol=elem)
+
+    dx = torch.full((M, K), float("nan"), device=dev)
+    ops.scatter2scatter(dy, w, se, idx, dx, 1, True, False, off)
+    want = torch.empty(M, K, dtype=torch.float64, device=dev)
+    want[idx.long()] = torch.cat([dy[r].double() @ w[e].double() for e, r in enumerate(rows)])
+    assert_close(dx, want.float(), TOL[dt], "NN", elem_tol=elem)
+
+    want = torch.stack([dy[r].double().T @ xg[r].double() for r in rows]).float()
+    for source, index in ((xg, None), (x, idx)):
+        dw = torch.full((E, N, K), float("nan"), device=dev)
+        ops.group_bwd_W(dy, source, off, dw.permute(0, 2, 1), E, index)
+        assert_close(dw, want, TOL[dt], "MT", elem_tol=elem)
+
+
 def test_full_length_reductions_dense():
     """Every layout once at the row counts of the benchmark layer (16384 routed rows over 8 experts, about 2048 per
     expert) with DENSE operands, so that the weight-gradient kernel's reductions run over ~2048 non-zero rows (32
