@@ -2,13 +2,14 @@
 
 `xma_op` registers a Python function that mutates its output arguments as a
 `torch.library.custom_op` in the `xma::` namespace, so the HIP-backed operators are opaque,
-traceable nodes for `torch.compile(fullgraph=True)`.  `CustomOp` is the autograd.Function base
-whose `run()` resolves the backend and bumps the call counter.
+traceable nodes for `torch.compile(fullgraph=True)`.  `direct_xma_op` adds a short way for plain eager calls on device
+tensors.  `CustomOp` is the autograd.Function base whose `run()` resolves the backend and bumps the call counter.
 """
 
 from __future__ import annotations
 
 import inspect
+from functools import lru_cache
 from typing import Any, Callable, Iterable, Sequence
 
 import torch
@@ -63,6 +64,134 @@ def xma_op(
         call.__name__ = func.__name__
         call.__doc__ = func.__doc__
         call._custom_op = op
+        return call
+
+    return decorator
+
+
+# annotation -> the exact types a direct call takes; anything else goes to the operator, whose schema judges it
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+_DIRECT_TYPES = {
+    "torch.Tensor": _TENSORS,
+    "torch.Tensor | None": (*_TENSORS, type(None)),
+    "int": (int,),
+    "bool": (bool,),
+    "str": (str,),
+}
+
+
+def _eager() -> bool:
+    """True when nothing observes or transforms operator calls: no compiler, tracer, profiler, dispatch or function
+    mode, functorch transform (vmap, grad, jvp, functionalization) or forward-mode level is active."""
+
+    return not (
+        torch.compiler.is_compiling()
+        or torch._C._len_torch_dispatch_stack()
+        or torch._C._len_torch_function_stack()
+        or torch._C._functorch.peek_interpreter_stack() is not None
+        or torch._C._autograd._profiler_enabled()
+        or torch.autograd.forward_ad._current_level >= 0
+        or torch._C._get_tracing_state() is not None
+    )
+
+
+@lru_cache
+def _plain_keys(inference: bool) -> "torch._C.DispatchKeySet":
+    """Dispatch keys of an ordinary dense device tensor (created in inference mode or outside it)."""
+
+    with torch.inference_mode(inference):
+        return torch._C._dispatch_keys(torch.empty(0, device="cuda"))
+
+
+class _NoGraph:
+    """Stands for an autograd context where no graph is recorded."""
+
+    def __init__(self, inputs: int) -> None:
+        self.needs_input_grad = (False,) * inputs
+
+    def save_for_backward(self, *tensors) -> None:
+        pass
+
+    def mark_non_differentiable(self, *tensors) -> None:
+        pass
+
+
+def apply_function(function: type[torch.autograd.Function], *args) -> Any:
+    """`function.apply(*args)`; a plain eager call that records no graph runs `function.forward` itself, without the
+    10 us of host time that `apply` takes.  `function` must return new tensors and use no more of its context than
+    `_NoGraph` has."""
+
+    if _eager():
+        grad = torch.is_grad_enabled()
+        for value in args:
+            if isinstance(value, torch.Tensor) and (type(value) not in _TENSORS or (grad and value.requires_grad)):
+                break
+        else:
+            return function.forward(_NoGraph(len(args)), *args)
+    return function.apply(*args)
+
+
+def direct_xma_op(mutates_args: Iterable[str]) -> Callable:
+    """`xma_op` for the package's own operators, with a short way past the dispatcher.
+
+    The returned callable runs the function itself when a call can mean nothing else: nothing observes or transforms
+    operator calls (`_eager`), every argument has exactly the type its annotation names, and every tensor is an ordinary
+    device tensor (by its dispatch keys: no subclass, wrapper, sparse layout, negated or conjugated view) that is not to
+    be differentiated through.  It then bumps the version counters of the mutated tensors, as the operator does.  Every
+    other call goes to the operator and is traced, transformed or refused there.
+
+    Measured, host-bound calls with and without the two short ways (this and `apply_function`): one decoded token
+    through the layer (H 2048, I 1024, E 64, k 6) 141 us against 212, a full-precision forward pass of 1024 tokens
+    (H 256, I 512) 139 against 215, a training step of 3001 tokens (H 512, I 1024) 696 against 865, the routing of 2^20
+    ids 47 against 61.
+    """
+
+    mutated = frozenset(mutates_args)
+
+    def decorator(func: Callable) -> Callable:
+        op = xma_op(mutates_args=mutates_args)(func)
+        parameters = inspect.signature(func).parameters
+        names = tuple(parameters)
+        types = {name: _DIRECT_TYPES[p.annotation] for name, p in parameters.items()}
+
+        def written_tensors(args: tuple, kwargs: dict) -> list[torch.Tensor] | None:
+            """The mutated tensors of a call that may run directly, None when it has to go through the operator."""
+
+            if len(args) > len(names):
+                return None
+            grad, inference = torch.is_grad_enabled(), torch.is_inference_mode_enabled()
+            written = []
+            for name, value in (*zip(names, args), *kwargs.items()):
+                kind = type(value)
+                if kind not in types.get(name, ()):
+                    return None
+                if kind in _TENSORS:
+                    if not value.is_cuda or (grad and value.requires_grad):
+                        return None
+                    is_inference = value.is_inference()
+                    if torch._C._dispatch_keys(value) != _plain_keys(is_inference):
+                        return None
+                    if name in mutated:
+                        if not is_inference:
+                            written.append(value)
+                        elif not inference:  # refused by the operator
+                            return None
+            return written
+
+        def call(*args, **kwargs):
+            if _eager():
+                written = written_tensors(args, kwargs)
+                if written is not None:
+                    func(*args, **kwargs)
+                    if written:
+                        torch.autograd.graph.increment_version(written)
+                    return None
+            return op(*args, **kwargs)
+
+        call.__signature__ = op.__signature__
+        call.__name__ = op.__name__
+        call.__doc__ = op.__doc__
+        call._custom_op = op._custom_op
         return call
 
     return decorator

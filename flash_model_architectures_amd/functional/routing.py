@@ -12,6 +12,7 @@ from typing import NamedTuple
 import torch
 
 from ..accelerator import KernelBackend, resolve_backend
+from ..custom_op import apply_function
 from ..ops import route_build_rocm, topk_softmax_backward_rocm, topk_softmax_rocm
 
 
@@ -51,7 +52,7 @@ def topk_softmax(
     assert logits.dim() == 2, "logits should be [tokens, experts]"
     if logits.stride(1) != 1:
         logits = logits.contiguous()
-    return _TopkSoftmax.apply(logits, k, index_dtype)
+    return apply_function(_TopkSoftmax, logits, k, index_dtype)
 
 
 class Routing(NamedTuple):

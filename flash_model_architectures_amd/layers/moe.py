@@ -21,6 +21,7 @@ import torch
 import torch.nn as nn
 
 from ..accelerator import KernelBackend, resolve_backend
+from ..custom_op import apply_function
 from ..functional.routing import route_tokens, topk_softmax
 from ..functional.swiglu_packed import swiglu_packed
 from ..ops import (
@@ -68,7 +69,7 @@ class _Gate(nn.Linear):
     def forward(self, input: torch.Tensor) -> torch.Tensor:
         if self.bias is not None or input.dim() != 2:
             return super().forward(input)
-        return _GateLinear.apply(input, self.weight)
+        return apply_function(_GateLinear, input, self.weight)
 
 
 class _ScatteredExperts(torch.autograd.Function):
@@ -201,7 +202,8 @@ def scattered_experts(
     int32[E + 1] exclusive prefix sums the kernels read; the former is converted on the device."""
 
     expert_offsets = exclusive_offsets(expert_offsets, expert_weights.size(0))
-    return _ScatteredExperts.apply(
+    return apply_function(
+        _ScatteredExperts,
         inputs,
         expert_weights,
         k,
@@ -533,7 +535,8 @@ class MoE(XMAModule):
         # biases: torch path only in the reference (xma/layers/moe/__init__.py:54,79,104); here both pipelines take them
         activation = fused_activation_name(self.act, self.is_glu)
         if activation is not None:
-            return _FusedExperts.apply(
+            return apply_function(
+                _FusedExperts,
                 hidden_states,
                 self.c_fc.weight,
                 self.c_proj.weight,

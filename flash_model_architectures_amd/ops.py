@@ -19,7 +19,7 @@ import ctypes
 import torch
 
 from . import _native as nat
-from .custom_op import xma_op
+from .custom_op import direct_xma_op
 
 
 def _i64(t: torch.Tensor | None) -> int:
@@ -110,7 +110,7 @@ def offsets_from_sorted(sorted_expert_idxs: torch.Tensor, E: int) -> torch.Tenso
 # ------------------------------------------------------------------------------------------------
 # routing
 # ------------------------------------------------------------------------------------------------
-@xma_op(mutates_args={"output"})
+@direct_xma_op(mutates_args={"output"})
 def continuous_count_rocm(x: torch.Tensor, output: torch.Tensor, E: int) -> None:
     """output[e] = number of elements of x equal to e, e in [0, E); replaces continuous_count_cuda."""
 
@@ -129,7 +129,7 @@ def continuous_count_rocm(x: torch.Tensor, output: torch.Tensor, E: int) -> None
     )
 
 
-@xma_op(mutates_args={"counts", "expert_offsets", "sorted_expert_idxs", "sorted_scattered_idxs"})
+@direct_xma_op(mutates_args={"counts", "expert_offsets", "sorted_expert_idxs", "sorted_scattered_idxs"})
 def route_build_rocm(
     selected_experts: torch.Tensor,
     counts: torch.Tensor,
@@ -168,7 +168,7 @@ def route_build_rocm(
     )
 
 
-@xma_op(mutates_args={"weights", "indices"})
+@direct_xma_op(mutates_args={"weights", "indices"})
 def topk_softmax_rocm(logits: torch.Tensor, weights: torch.Tensor, indices: torch.Tensor, k: int) -> None:
     """Top-k (ties: lower index first) and softmax over the selected logits, one row per token."""
 
@@ -192,7 +192,7 @@ def topk_softmax_rocm(logits: torch.Tensor, weights: torch.Tensor, indices: torc
     )
 
 
-@xma_op(mutates_args={"d_logits"})
+@direct_xma_op(mutates_args={"d_logits"})
 def topk_softmax_backward_rocm(
     logits: torch.Tensor, d_weights: torch.Tensor, indices: torch.Tensor, d_logits: torch.Tensor
 ) -> None:
@@ -222,7 +222,7 @@ def topk_softmax_backward_rocm(
 # ------------------------------------------------------------------------------------------------
 # row moves
 # ------------------------------------------------------------------------------------------------
-@xma_op(mutates_args={"out"})
+@direct_xma_op(mutates_args={"out"})
 def group(
     A: torch.Tensor,
     sorted_expert_idxs: torch.Tensor,
@@ -258,7 +258,7 @@ def group(
     )
 
 
-@xma_op(mutates_args={"out"})
+@direct_xma_op(mutates_args={"out"})
 def ungroup(A: torch.Tensor, index: torch.Tensor, out: torch.Tensor) -> None:
     """out[index[p]] = A[p]: the inverse row permutation of `group`.  Rows of `out` that no index names keep
     their contents; a row that several name receives one of them."""
@@ -286,7 +286,7 @@ def ungroup(A: torch.Tensor, index: torch.Tensor, out: torch.Tensor) -> None:
     )
 
 
-@xma_op(mutates_args={"out"})
+@direct_xma_op(mutates_args={"out"})
 def combine_topk(expanded: torch.Tensor, out: torch.Tensor, k: int, gates: torch.Tensor | None = None) -> None:
     """out[t] = sum_j gates[t, j] * expanded[t*k + j] (plain sum when gates is None)."""
 
@@ -313,7 +313,7 @@ def combine_topk(expanded: torch.Tensor, out: torch.Tensor, k: int, gates: torch
     )
 
 
-@xma_op(mutates_args={"d_gates"})
+@direct_xma_op(mutates_args={"d_gates"})
 def gate_grad(expanded: torch.Tensor, grad_out: torch.Tensor, d_gates: torch.Tensor) -> None:
     """d_gates[t, j] = <expanded[t*k + j], grad_out[t]>."""
 
@@ -352,7 +352,7 @@ def router_weight_grad_supported(x: torch.Tensor, d_logits: torch.Tensor) -> boo
     return True
 
 
-@xma_op(mutates_args={"d_weight"})
+@direct_xma_op(mutates_args={"d_weight"})
 def router_weight_grad(x: torch.Tensor, d_logits: torch.Tensor, d_weight: torch.Tensor) -> None:
     """d_weight[E, H] = d_logits[T, E]^T x[T, H] with fp32 accumulation: the weight gradient of the gate's linear layer
     (xma/layers/moe/__init__.py:148,192).  Shapes the kernel does not take (`router_weight_grad_supported`) are one
@@ -390,7 +390,7 @@ def router_weight_grad(x: torch.Tensor, d_logits: torch.Tensor, d_weight: torch.
     )
 
 
-@xma_op(mutates_args={"y"})
+@direct_xma_op(mutates_args={"y"})
 def add_expert_bias(
     y: torch.Tensor, bias: torch.Tensor, sorted_expert_idxs: torch.Tensor, out_index: torch.Tensor | None = None
 ) -> None:
@@ -422,7 +422,7 @@ def add_expert_bias(
     )
 
 
-@xma_op(mutates_args={"out"})
+@direct_xma_op(mutates_args={"out"})
 def expert_colsum(src: torch.Tensor, expert_offsets: torch.Tensor, out: torch.Tensor) -> None:
     """out[e] = sum of the grouped rows of expert e of `src` (fp32 accumulation, fixed order)."""
 
@@ -452,7 +452,7 @@ def expert_colsum(src: torch.Tensor, expert_offsets: torch.Tensor, out: torch.Te
 # ------------------------------------------------------------------------------------------------
 # sequence packing
 # ------------------------------------------------------------------------------------------------
-@xma_op(mutates_args={"output"})
+@direct_xma_op(mutates_args={"output"})
 def pack_unpack_sequence_rocm(
     x: torch.Tensor, output: torch.Tensor, cu_seqlens: torch.Tensor, padding_side: str, pack: bool
 ) -> None:
@@ -490,7 +490,7 @@ def pack_unpack_sequence_rocm(
 # ------------------------------------------------------------------------------------------------
 # swiglu
 # ------------------------------------------------------------------------------------------------
-@xma_op(mutates_args={"y"})
+@direct_xma_op(mutates_args={"y"})
 def swiglu_forward_rocm(g: torch.Tensor, u: torch.Tensor, y: torch.Tensor) -> None:
     nat.require_device(g, u, y)
     assert g.shape == u.shape == y.shape and g.dtype == u.dtype == y.dtype
@@ -511,7 +511,7 @@ def swiglu_forward_rocm(g: torch.Tensor, u: torch.Tensor, y: torch.Tensor) -> No
     )
 
 
-@xma_op(mutates_args={"dg", "du"})
+@direct_xma_op(mutates_args={"dg", "du"})
 def swiglu_backward_rocm(
     g: torch.Tensor, u: torch.Tensor, dy: torch.Tensor, dg: torch.Tensor, du: torch.Tensor
 ) -> None:
@@ -618,7 +618,7 @@ def _weight_layout(W: torch.Tensor) -> tuple[int, int]:
     raise ValueError(f"expert weights need one unit stride among the last two dims, got strides {W.stride()}")
 
 
-@xma_op(mutates_args={"out"})
+@direct_xma_op(mutates_args={"out"})
 def scatter2scatter(
     X: torch.Tensor,
     W: torch.Tensor,
@@ -678,7 +678,7 @@ def scatter2scatter(
         add_expert_bias(y=out, bias=bias, sorted_expert_idxs=sorted_expert_idxs, out_index=None if y_grouped else idx)
 
 
-@xma_op(mutates_args={"DW"})
+@direct_xma_op(mutates_args={"DW"})
 def group_bwd_W(
     DY: torch.Tensor,
     X: torch.Tensor,
@@ -755,7 +755,7 @@ def group_bwd_W(
         raise ValueError(f"DW needs one unit stride among the last two dims, got strides {DW.stride()}")
 
 
-@xma_op(mutates_args={"act", "preact"})
+@direct_xma_op(mutates_args={"act", "preact"})
 def up_projection_fused(
     X: torch.Tensor,
     W: torch.Tensor,
@@ -801,7 +801,7 @@ def up_projection_fused(
     )
 
 
-@xma_op(mutates_args={"d_preact"})
+@direct_xma_op(mutates_args={"d_preact"})
 def down_projection_dgrad_fused(
     DY: torch.Tensor,
     W: torch.Tensor,
