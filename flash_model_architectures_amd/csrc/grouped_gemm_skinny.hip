@@ -10,13 +10,17 @@
 // unit), and the four partial tiles are added in wave order through LDS.  Many small work-groups keep HBM busy
 // whatever the number of experts that are hit.
 //
-// Measured against the 256 x 256 kernel, up + down projection, inputs changing from call to call: H 2048, I 1024, E 64,
-// k 6, one token (6 experts, 75 MB of weights) 21 us instead of 82; 16 tokens 112 us instead of 192 (5.7 TB/s of
-// weights); H 4096, I 14336, E 8, k 2, 8 tokens 418 us instead of 594 (5.6 TB/s), 32 tokens 560 us instead of 667.
-// In fp32 (the 128 x 128 register-staged kernel before) one token 38 us instead of 248.
-// What was chosen by measurement: four waves (eight: 2-5 % slower); U = 2 for 2 x 1 blocks (4: 5-10 % slower at
-// H 2048, 8: 40 % slower, the registers of the longer batches cost wavefronts); streaming loads of the weights 7-10 %
-// slower.
+// A lane loads two adjacent 16-byte chunks, so that the four lanes of a weight row touch a whole 128-byte line with
+// each of the two loads; one chunk per 64-byte half line (either half by a load of its own) held 5.0 TB/s where this
+// holds 5.9.  A kernel that only reads reaches 6.2.
+//
+// Measured against the 256 x 256 kernel, up + down projection: H 2048, I 1024, E 64, k 6, one token (6 experts, 75 MB
+// of weights) 21 us instead of 82; 16 tokens 117 us instead of 207 (5.6 TB/s of weights); H 4096, I 14336, E 8, k 2,
+// 32 tokens 467 us instead of 653 (6.0 TB/s), 64 tokens 484 us instead of 666.  In fp32 (a 128 x 128 register-staged
+// kernel before) one token 36 us instead of 248, 16 tokens 225 us with whole lines and 247 with half lines.
+// What was chosen by measurement: four waves (eight: 2-5 % slower); U = 2 (4: no gain at 32 x 16 blocks of H 4096, 20 %
+// slower at I 768); streaming loads of the weights 7-10 % slower; 64 x 16 blocks only for many columns (3 % there, 20-30 %
+// slower for the smallest layers).
 //
 // Which rows a work-group has is found by each wave on its own from the expert offsets (RowTileScan), so there is
 // no table to build in a launch of its own.
@@ -88,6 +92,7 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(const GemmParams P
     constexpr int NF_OUT = PAIRED ? NF / 2 : NF;  // blocks of output columns
     constexpr int BM = 16 * RF, BN_OUT = 16 * NF_OUT;
     static_assert(!PAIRED || NF % 2 == 0, "a gated tile pairs blocks");
+    static_assert(U % 2 == 0, "a batch is whole 128-byte lines");
     __shared__ __attribute__((aligned(16))) f32x4_t partial[WAVES][NF * RF][kWaveSize];
 
     const int lane = lane_id();
@@ -113,20 +118,20 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(const GemmParams P
     const int row16 = lane & 15, quarter = lane >> 4;
 
     // Rows past the end of the tile or of the weights read an existing row: their results are dropped.
-    const T* xp[RF];
+    const T* xp[RF];  // rows' starts
     const T* wp[NF];
 #pragma unroll
     for (int r = 0; r < RF; ++r) {
         int64_t p = m_begin + r * 16 + row16;
         p = p < m_end ? p : m_end - 1;
         const int64_t src = P.in_index ? source_row(P, p) : p;
-        xp[r] = A + src * P.lda + quarter * PV;
+        xp[r] = A + src * P.lda;
     }
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
         int64_t n = n0 + (f % NF_OUT) * 16 + row16;
         n = n < n_out ? n : n_out - 1;
-        wp[f] = W + (n + (f >= NF_OUT ? n_out : 0)) * P.ldb + quarter * PV;
+        wp[f] = W + (n + (f >= NF_OUT ? n_out : 0)) * P.ldb;
     }
 
     f32x4_t acc[NF][RF];
@@ -147,7 +152,8 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(const GemmParams P
     auto load_batch = [&](int set, int step) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int64_t k = (int64_t)(step + u) * STEP;
+            // a lane takes two adjacent chunks of a 128-byte line, so either load touches the whole of it
+            const int64_t k = (int64_t)(step + (u & ~1)) * STEP + (quarter * 2 + (u & 1)) * PV;
 #pragma unroll
             for (int f = 0; f < NF; ++f) w[set][u][f] = *reinterpret_cast<const uint4*>(wp[f] + k);
 #pragma unroll
@@ -173,8 +179,8 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(const GemmParams P
     }
     // the remaining steps one by one; elements past the end of the reduction are zero in both operands
     for (int s = first + batches * U; s < last; ++s) {
-        const int64_t k = (int64_t)s * STEP;
-        const bool exists = k + quarter * PV < P.k;
+        const int64_t k = (int64_t)s * STEP + quarter * PV;
+        const bool exists = k < P.k;
         const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
         uint4 wv[NF], xv[RF];
 #pragma unroll
@@ -253,23 +259,39 @@ static int launch(const GemmParams& params, int64_t rows, hipStream_t stream) {
     return check_launch("xma_grouped_gemm");
 }
 
+// work-groups of the 128 x 64 form when every expert has one row tile
+static int64_t wide_tiles(const xma_grouped_gemm_args& a) { return a.n / 128 * a.num_experts; }
+
 template <typename T>
 static int dispatch(const xma_grouped_gemm_args& a, const GemmParams& P, hipStream_t stream) {
     int shape = EPI_PLAIN, act = ACT_NONE;
     split_epilogue(a.epilogue, shape, act);
-    const bool one_block = a.rows <= kSkinnyOneBlock * (int64_t)a.num_experts;
-    if (shape == EPI_PAIRED)
-        return one_block ? launch<T, 2, 1, EPI_PAIRED, 2>(P, a.rows, stream)
-                         : launch<T, 4, 2, EPI_PAIRED, 1>(P, a.rows, stream);
-    return one_block ? launch<T, 2, 1, EPI_PLAIN, 2>(P, a.rows, stream)
-                     : launch<T, 4, 2, EPI_PLAIN, 1>(P, a.rows, stream);
+    constexpr bool FP32 = std::is_same<T, float>::value;
+#define XMA_SKINNY(NF, RF)                                                             \
+    (shape == EPI_PAIRED ? launch<T, NF, RF, EPI_PAIRED, 2>(P, a.rows, stream)          \
+                         : launch<T, NF, RF, EPI_PLAIN, 2>(P, a.rows, stream))
+    if (a.rows <= kSkinnyOneBlock * (int64_t)a.num_experts) {
+        if (!FP32 && a.n >= kSkinnyWideColumns) return XMA_SKINNY(4, 1);
+        return XMA_SKINNY(2, 1);
+    }
+    if constexpr (!FP32) {
+        if (a.rows > kSkinnyTwoBlocks * (int64_t)a.num_experts)
+            return wide_tiles(a) >= kSkinnyWideTiles ? XMA_SKINNY(8, 4) : XMA_SKINNY(4, 4);
+    }
+    return XMA_SKINNY(4, 2);
+#undef XMA_SKINNY
 }
 
 }  // namespace skinny
 
 bool skinny_gemm_supports(const xma_grouped_gemm_args& a) {
-    return a.kind == XMA_GEMM_TN && a.k > 0 && a.num_experts <= kMaxScannedExperts &&
-           a.rows <= kSkinnyRows * (int64_t)a.num_experts;
+    if (a.kind != XMA_GEMM_TN || a.k <= 0 || a.num_experts > kMaxScannedExperts) return false;
+    const int64_t experts = a.num_experts;
+    if (a.dtype == XMA_F32) return a.rows <= kSkinnyRowsF32 * experts;
+    if (a.rows <= kSkinnyTwoBlocks * experts) return true;
+    if (a.rows > kSkinnyRows * experts) return false;
+    if (a.k < kSkinnyLongReduction) return ceil_div(a.n, 256) * experts <= kSkinnyTiledRound;
+    return a.n < 4096 || skinny::wide_tiles(a) >= kSkinnyWideTiles;
 }
 
 int launch_skinny_gemm(const xma_grouped_gemm_args& a, hipStream_t stream) {

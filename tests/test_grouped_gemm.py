@@ -192,6 +192,9 @@ FEW_ROWS = [
     ([15, 33, 1, 32, 31] + [0] * 70 + [7], 520, 144),  # beyond 64 experts; reduction ends inside a step
     ([20, 24, 9, 31, 5], 424, 80),  # row tiles of 32; reduction shorter than two steps of every wave
     ([100, 3], 1096, 112),  # many row tiles of one expert
+    ([1, 0, 17, 8], 1112, 16400),  # many columns: 64 weight rows over 16 routed rows; the last column tile is a quarter full
+    ([64, 1, 18, 65], 424, 80),  # the same tiles over a short reduction
+    ([40, 64, 65, 17, 0, 3], 2056, 144),  # row tiles of 64 (16-bit types): one exactly, one row more; a half line at the end
 ]
 
 
@@ -300,6 +303,37 @@ def test_fp32_tiles(sizes, K, N):
         dw = torch.full((E, N, K), float("nan"), device=dev)
         ops.group_bwd_W(dy, source, off, dw.permute(0, 2, 1), E, index)
         assert_close(dw, want, TOL[dt], "MT", elem_tol=elem)
+
+
+@pytest.mark.parametrize("gated", [True, False])
+def test_few_rows_and_many_columns(gated):
+    """The widest tile of the weight-streaming kernel (128 weight rows over 64 routed rows): 16-bit types, 21 to 40
+    rows per expert on average, reductions from 2048 on and enough columns to fill the device."""
+
+    sizes, K, N, dev = [1, 64, 65, 0, 16, 48, 17, 33], 2056, 16400, "cuda"
+    E, M = len(sizes), sum(sizes)
+    g = torch.Generator(dev).manual_seed(5)
+    off_list = [0] + torch.tensor(sizes).cumsum(0).tolist()
+    off = torch.tensor(off_list, dtype=torch.int32, device=dev)
+    idx = torch.randperm(M, generator=g, device=dev)
+    x = torch.randn(M, K, generator=g, device=dev).bfloat16()
+    w = torch.randn(E, N, K, generator=g, device=dev, dtype=torch.bfloat16) * 0.05
+    rows = x[idx]
+    product = torch.cat([rows[off_list[e] : off_list[e + 1]].float() @ w[e].float().T for e in range(E)])
+    elem = GEMM_ELEM_TOL[torch.bfloat16]
+    if gated:
+        act = torch.empty(M, N // 2, dtype=x.dtype, device=dev)
+        pre = torch.full((M, N), float("nan"), dtype=x.dtype, device=dev)
+        ops.up_projection_fused(x, w, idx.int(), off, act, pre, 1, "swiglu")
+        assert_close(pre, product.cpu(), TOL[x.dtype], "pre-activation, many columns", elem_tol=elem)
+        assert_close(act, to.swiglu_packed(pre.float().cpu()), TOL[x.dtype], "swiglu, many columns")
+    else:
+        out = torch.full((M, N), float("nan"), dtype=x.dtype, device=dev)
+        se = torch.repeat_interleave(torch.arange(E), torch.tensor(sizes)).to(dev).int()
+        ops.scatter2scatter(rows, w.permute(0, 2, 1), se, idx.int(), out, 1, True, False, off)
+        want = torch.empty_like(product)
+        want[idx] = product
+        assert_close(out, want.cpu(), TOL[x.dtype], "scattered rows, many columns", elem_tol=elem)
 
 
 def test_full_length_reductions_dense():
