@@ -9,7 +9,8 @@
 // over the experts turn the rows into the first output slot of every (unit, expert) pair; (3) the
 // unit is walked again in order, equal ids inside each 64-wide batch are ranked with ballots, and
 // the permutation is written.  For the sizes of an MoE layer a unit belongs to a block of four
-// waves (a quarter each) and steps (2) and (3) are one kernel; beyond, a unit belongs to one wave.
+// waves (a quarter each) and steps (2) and (3) are one kernel; longer streams take larger units, put in order in LDS
+// before they are written; beyond kStageExperts experts a unit belongs to four waves again, or to one.
 #include <mutex>
 
 #include "common.h"
@@ -135,9 +136,8 @@ __device__ __forceinline__ void load_chunk(const IdT* __restrict__ ids, int64_t 
 // One 64-wide batch of the placement: lanes holding the same expert id find each other with log2(E) ballots, the
 // first of them takes popcount(peers) consecutive slots from next[e], and every lane's slot follows from its rank
 // among its peers, so equal ids keep their order.
-template <typename OutT>
-__device__ __forceinline__ void place_batch(int64_t e64, int64_t i, int E, int nbits, int lane, uint32_t* next,
-                                            OutT* __restrict__ sorted_ids, OutT* __restrict__ perm) {
+template <typename Write>
+__device__ __forceinline__ void rank_batch(int64_t e64, int E, int nbits, int lane, uint32_t* next, Write write) {
     const bool ok = e64 >= 0 && e64 < E;
     const uint32_t e = ok ? (uint32_t)e64 : 0u;
     uint64_t peers = __ballot(ok);
@@ -150,11 +150,15 @@ __device__ __forceinline__ void place_batch(int64_t e64, int64_t i, int E, int n
     const int leader = ok ? (int)__ffsll((unsigned long long)peers) - 1 : lane;
     if (ok && leader == lane) base = atomicAdd(&next[e], (uint32_t)__popcll(peers));  // one LDS round trip, not two
     base = __shfl(base, leader, kWaveSize);
-    if (ok) {
-        const uint32_t pos = base + (uint32_t)__popcll(peers & (((uint64_t)1 << lane) - 1));
+    if (ok) write(base + (uint32_t)__popcll(peers & (((uint64_t)1 << lane) - 1)), e);
+}
+template <typename OutT>
+__device__ __forceinline__ void place_batch(int64_t e64, int64_t i, int E, int nbits, int lane, uint32_t* next,
+                                            OutT* __restrict__ sorted_ids, OutT* __restrict__ perm) {
+    rank_batch(e64, E, nbits, lane, next, [&](uint32_t pos, uint32_t e) {
         perm[pos] = (OutT)i;
         sorted_ids[pos] = (OutT)e;
-    }
+    });
 }
 
 template <typename IdT>
@@ -376,6 +380,166 @@ __global__ __launch_bounds__(256) void place_quarters_kernel(const IdT* __restri
         place_batch(v[j], begin + j * kWaveSize + lane, E, nbits, lane, next, sorted_ids, perm);
 }
 
+// The counting sort of a long stream into up to kStageExperts experts: units of kStage ids, a block of 16 waves each,
+// three launches (stage_hist_kernel, stage_scan_kernel, stage_place_kernel).  What bounds the placement is its writes:
+// straight from the ranks they are a few adjacent words per expert (n / units / E of them), each a partial line that
+// several XCDs' L2 caches hold pieces of.  Four times as many ids per unit, put in order in LDS first, are written in
+// runs of kStage / E words by consecutive lanes, and the table of unit histograms that is scanned in between shrinks to a
+// quarter.  2^20 ids, 256 experts: 20 us against 34 us for units of 1024 (histograms, scan, offsets, placement straight
+// from the ranks), 2^22 ids 40 against 106, 70000 ids 14 against 23; 8 experts, 2^22 ids 34 against 72.  With more than
+// 256 experts it takes as many ids to be ahead (384: 5000 ids 13.6 against 12.7, 2^17 equal, 2^22 43 against 112).
+constexpr int kStage = 4096;
+constexpr int kStageThreads = 1024;
+constexpr int kStageWaves = kStageThreads / kWaveSize;
+constexpr int kStageBatches = kStage / kStageThreads;  // 64-wide batches per wave
+constexpr int64_t kStageManyIds = (int64_t)1 << 17;    // from here on with more than kScanExperts experts
+constexpr int kStageExperts = 512;                     // 16 rows of E words and the staged unit fit in 64 KiB of LDS
+
+template <typename IdT>
+__global__ __launch_bounds__(kStageThreads) void stage_hist_kernel(const IdT* __restrict__ ids, int64_t n, int E,
+                                                                    uint32_t* __restrict__ unit_hist) {
+    extern __shared__ uint32_t lds_hist[];  // [4][E]: waves w, w + 4, ... share a row
+    const int wave = threadIdx.x / kWaveSize;
+    const int64_t unit = blockIdx.x;
+    const int64_t begin = unit * kStage + wave * (kStageBatches * kWaveSize);
+    int64_t v[kStageBatches];
+    load_chunk(ids, begin, n, lane_id(), v);
+    for (int i = threadIdx.x; i < 4 * E; i += kStageThreads) lds_hist[i] = 0;
+    __syncthreads();
+    uint32_t* mine = lds_hist + (wave & 3) * E;
+#pragma unroll
+    for (int j = 0; j < kStageBatches; ++j)
+        if (v[j] >= 0 && v[j] < E) atomicAdd(&mine[v[j]], 1u);
+    __syncthreads();
+    uint32_t* row = unit_hist + unit * E;
+    for (int i = threadIdx.x; i < E; i += kStageThreads)
+        row[i] = lds_hist[i] + lds_hist[E + i] + lds_hist[2 * E + i] + lds_hist[3 * E + i];
+}
+
+// One block per 16 experts: thread = (expert column, one of 64 segments of the units).  In place: unit_hist[u][e]
+// becomes the number of ids equal to e in units before u; the column totals go to counts[e].
+constexpr int kStageColumns = 16;
+__global__ __launch_bounds__(kStageThreads) void stage_scan_kernel(uint32_t* __restrict__ unit_hist, int64_t units, int E,
+                                                                    uint32_t* __restrict__ counts) {
+    constexpr int kSegments = kStageThreads / kStageColumns;
+    constexpr int kInFlight = 16;
+    __shared__ uint32_t seg_sum[kSegments][kStageColumns];
+    const int c = threadIdx.x % kStageColumns, segment = threadIdx.x / kStageColumns;
+    const int e = blockIdx.x * kStageColumns + c;
+    const int64_t per = (units + kSegments - 1) / kSegments;
+    const int64_t u0 = segment * per < units ? segment * per : units;
+    const int64_t u1 = u0 + per < units ? u0 + per : units;
+    uint32_t v[kInFlight];  // a segment of up to kInFlight units stays in registers between the two passes
+    auto load = [&](int64_t u) {
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) v[j] = e < E && u + j < u1 ? unit_hist[(u + j) * E + e] : 0u;
+    };
+    uint32_t sum = 0;
+    for (int64_t u = u0; u < u1; u += kInFlight) {
+        load(u);
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) sum += v[j];
+    }
+    seg_sum[segment][c] = sum;
+    __syncthreads();
+    uint32_t base = 0;
+    for (int s = 0; s < segment; ++s) base += seg_sum[s][c];
+    if (e >= E) return;
+    for (int64_t u = u0; u < u1; u += kInFlight) {
+        if (per > kInFlight) load(u);
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) {
+            if (u + j < u1) unit_hist[(u + j) * E + e] = base;
+            base += v[j];
+        }
+    }
+    if (segment == kSegments - 1) counts[e] = base;
+}
+
+template <typename IdT, typename OutT>
+__global__ __launch_bounds__(kStageThreads) void stage_place_kernel(const IdT* __restrict__ ids, int64_t n, int E,
+                                                                     int nbits, const uint32_t* __restrict__ unit_prefix,
+                                                                     const uint32_t* __restrict__ counts,
+                                                                     int32_t* __restrict__ offsets,
+                                                                     OutT* __restrict__ sorted_ids,
+                                                                     OutT* __restrict__ perm) {
+    // next[16][E]: a wave's histogram, then its next free staged slots; shift[E]: an expert's first output slot minus its
+    // first staged slot; staged[kStage]: (expert << 16 | id's place in the unit) in output order
+    extern __shared__ uint32_t lds_hist[];
+    uint32_t* shift = lds_hist + kStageWaves * E;
+    uint32_t* staged = shift + E;
+    __shared__ uint32_t wave_counts[kStageWaves], wave_locals[kStageWaves];
+    const int wave = threadIdx.x / kWaveSize;
+    const int lane = lane_id();
+    const int64_t unit = blockIdx.x;
+    const int in_unit = wave * (kStageBatches * kWaveSize);
+    int64_t v[kStageBatches];
+    load_chunk(ids, unit * kStage + in_unit, n, lane, v);  // -1 past the end
+    const int e_mine = threadIdx.x;
+    const uint32_t count = e_mine < E ? counts[e_mine] : 0u;
+    const uint32_t before = e_mine < E ? unit_prefix[unit * E + e_mine] : 0u;
+    for (int i = threadIdx.x; i < kStageWaves * E; i += kStageThreads) lds_hist[i] = 0;
+    __syncthreads();
+    uint32_t* next = lds_hist + wave * E;
+#pragma unroll
+    for (int j = 0; j < kStageBatches; ++j)
+        if (v[j] >= 0 && v[j] < E) atomicAdd(&next[v[j]], 1u);
+    __syncthreads();
+
+    // thread e: expert e's ids in this unit, then exclusive scans over the experts of these and of the totals
+    uint32_t local = 0;
+    if (e_mine < E)
+        for (int w = 0; w < kStageWaves; ++w) local += lds_hist[w * E + e_mine];
+    uint32_t sum_counts = count, sum_locals = local;
+#pragma unroll
+    for (int d = 1; d < kWaveSize; d <<= 1) {
+        const uint32_t a = __shfl_up(sum_counts, d, kWaveSize), b = __shfl_up(sum_locals, d, kWaveSize);
+        if (lane >= d) {
+            sum_counts += a;
+            sum_locals += b;
+        }
+    }
+    if (lane == kWaveSize - 1) {
+        wave_counts[wave] = sum_counts;
+        wave_locals[wave] = sum_locals;
+    }
+    __syncthreads();
+    uint32_t first = sum_counts - count, slot = sum_locals - local;
+    uint32_t placed = 0;  // valid ids of the unit
+    for (int w = 0; w < kStageWaves; ++w) {
+        if (w < wave) {
+            first += wave_counts[w];
+            slot += wave_locals[w];
+        }
+        placed += wave_locals[w];
+    }
+    if (e_mine < E) {
+        if (unit == 0) {
+            offsets[e_mine] = (int32_t)first;
+            if (e_mine == E - 1) offsets[E] = (int32_t)(first + count);
+        }
+        shift[e_mine] = first + before - slot;  // (modulo 2^32)
+        for (int w = 0; w < kStageWaves; ++w) {
+            const uint32_t own = lds_hist[w * E + e_mine];
+            lds_hist[w * E + e_mine] = slot;
+            slot += own;
+        }
+    }
+    __syncthreads();
+
+#pragma unroll
+    for (int j = 0; j < kStageBatches; ++j)
+        rank_batch(v[j], E, nbits, lane, next,
+                   [&](uint32_t pos, uint32_t e) { staged[pos] = e << 16 | (uint32_t)(in_unit + j * kWaveSize + lane); });
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < placed; i += kStageThreads) {
+        const uint32_t entry = staged[i], e = entry >> 16;
+        const uint32_t pos = shift[e] + i;
+        perm[pos] = (OutT)(unit * kStage + (entry & 0xffffu));
+        sorted_ids[pos] = (OutT)e;
+    }
+}
+
 // Column sums of the table of per-unit histograms, by one block of 256 threads: total[e] += all units, before[e] +=
 // the units before `unit`.  A thread handles V adjacent experts (one 4 * V-byte load per unit) of the units r,
 // r + rows, ...; the number of thread columns is E / V rounded up to a power of two, so consecutive lanes read
@@ -425,6 +589,7 @@ __device__ __forceinline__ void sum_table(const uint32_t* __restrict__ unit_hist
 // which it requested before the scan began and counted for itself while the table was on its way (a wave's ids
 // start after those of the waves before it).  Block 0 also writes counts and offsets.
 constexpr int kFusedScanValues = 16384;
+constexpr int kScanExperts = 256;  // a block of 256 threads scans them, one each
 template <typename IdT, typename OutT>
 __global__ __launch_bounds__(256) void scan_place_kernel(const IdT* __restrict__ ids, int64_t n, int E, int nbits,
                                                           int64_t units, const uint32_t* __restrict__ unit_hist,
@@ -862,7 +1027,7 @@ static int route_build_launch(const void* ids, int ids_is_i64, int64_t n, int32_
     }
     const int64_t units = ceil_div(n, kChunk);
     uint32_t* unit_hist = (uint32_t*)workspace;
-    if (units * E <= kFusedScanValues && E <= 256) {  // two launches: histograms, then scan and placement in one
+    if (units * E <= kFusedScanValues && E <= kScanExperts) {  // two launches: histograms, then scan and placement in one
         const size_t hist_lds = (size_t)4 * E * sizeof(uint32_t);
         if (ids_is_i64)
             hipLaunchKernelGGL(block_hist_kernel<int64_t>, dim3((unsigned)units), dim3(256), hist_lds, stream,
@@ -889,12 +1054,39 @@ static int route_build_launch(const void* ids, int ids_is_i64, int64_t n, int32_
 #undef XMA_SCAN_PLACE
         return check_launch("xma_route_build");
     }
+    if (E <= kScanExperts || (E <= kStageExperts && n >= kStageManyIds)) {
+        const int64_t stages = ceil_div(n, kStage);
+        const size_t hist_lds = (size_t)4 * E * sizeof(uint32_t);
+        const size_t place_lds = ((size_t)(kStageWaves + 1) * E + kStage) * sizeof(uint32_t);
+        if (ids_is_i64)
+            hipLaunchKernelGGL(stage_hist_kernel<int64_t>, dim3((unsigned)stages), dim3(kStageThreads), hist_lds, stream,
+                               (const int64_t*)ids, n, (int)E, unit_hist);
+        else
+            hipLaunchKernelGGL(stage_hist_kernel<int32_t>, dim3((unsigned)stages), dim3(kStageThreads), hist_lds, stream,
+                               (const int32_t*)ids, n, (int)E, unit_hist);
+        hipLaunchKernelGGL(stage_scan_kernel, dim3((unsigned)ceil_div(E, kStageColumns)), dim3(kStageThreads), 0, stream,
+                           unit_hist, stages, (int)E, counts);
+#define XMA_STAGE_PLACE(IdT, OutT)                                                                                    \
+    hipLaunchKernelGGL((stage_place_kernel<IdT, OutT>), dim3((unsigned)stages), dim3(kStageThreads), place_lds, stream, \
+                       (const IdT*)ids, n, (int)E, nbits, (const uint32_t*)unit_hist, (const uint32_t*)counts,        \
+                       offsets, (OutT*)sorted_ids, (OutT*)perm)
+        if (ids_is_i64) {
+            if (out_is_i64)
+                XMA_STAGE_PLACE(int64_t, int64_t);
+            else
+                XMA_STAGE_PLACE(int64_t, int32_t);
+        } else {
+            if (out_is_i64)
+                XMA_STAGE_PLACE(int32_t, int64_t);
+            else
+                XMA_STAGE_PLACE(int32_t, int32_t);
+        }
+#undef XMA_STAGE_PLACE
+        return check_launch("xma_route_build");
+    }
     // four launches: histograms, column scan over the units, scan over the experts, placement; a unit belongs to a
     // block of four waves while four rows of E words fit in LDS, to one wave beyond
     const bool quarters = E <= kQuarterMaxExperts;
-    // (measured: 2^17 ids x 1024 experts 8.5 us against 19.2 us for the placement; 2^20 x 256 17.3 against 15.3 us,
-    // where a wave that walks 1024 ids writes four adjacent slots per expert)
-    const bool place_in_quarters = quarters && E > 256;
     const int wpb = sort_waves_per_block(E);
     const unsigned blocks = (unsigned)ceil_div(units, wpb);
     const size_t lds = (size_t)wpb * E * sizeof(uint32_t);
@@ -918,7 +1110,7 @@ static int route_build_launch(const void* ids, int ids_is_i64, int64_t n, int32_
     hipLaunchKernelGGL(offsets_kernel, dim3(1), dim3(1024), 0, stream, (const uint32_t*)counts, (int)E, offsets);
 #define XMA_PLACE(IdT, OutT)                                                                                       \
     do {                                                                                                           \
-        if (place_in_quarters)                                                                                     \
+        if (quarters)                                                                                     \
             hipLaunchKernelGGL((place_quarters_kernel<IdT, OutT>), dim3((unsigned)units), dim3(256), quarter_lds,  \
                                stream, (const IdT*)ids, n, (int)E, nbits, (const uint32_t*)unit_hist,              \
                                (const int32_t*)offsets, (OutT*)sorted_ids, (OutT*)perm);                           \

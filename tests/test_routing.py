@@ -39,6 +39,27 @@ def test_route_matches_oracle(n, E, dtype):
     _check_route(ids, E, index_dtype=torch.int64 if dtype == torch.int64 else torch.int32)
 
 
+@pytest.mark.parametrize("n,E", [(131073, 512), (140001, 300), (66001, 256), (4096 * 17, 256), (4096 * 80, 64), (4300001, 8)])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("invalid", [False, True])
+def test_route_staged(n, E, dtype, invalid):
+    """The counting sort that puts units of 4096 ids in order before it writes them: one id more than a unit, unit
+    edges, more than sixteen units per segment of the scan, the most experts it takes; ids outside [0, E) are left out."""
+
+    g = torch.Generator().manual_seed(n + E)
+    ids = torch.randint(-3 if invalid else 0, E + (3 if invalid else 0), (n,), generator=g, dtype=dtype)
+    ids[ids == 3] = 5  # an empty group in the middle
+    index_dtype = torch.int32 if dtype == torch.int64 else torch.int64
+    valid = ((ids >= 0) & (ids < E)).nonzero().squeeze(1)
+    order = valid[torch.argsort(ids[valid], stable=True)]
+    counts = torch.bincount(ids[valid], minlength=E)
+    r = xma.route_tokens(ids.cuda(), E, index_dtype=index_dtype)
+    assert torch.equal(r.expert_frequency.cpu().to(torch.int64), counts)
+    assert r.expert_offsets.tolist() == [0] + counts.cumsum(0).tolist()
+    assert torch.equal(r.sorted_scattered_idxs[: valid.numel()].cpu(), order.to(index_dtype))
+    assert torch.equal(r.sorted_expert_idxs[: valid.numel()].cpu(), ids[order].to(index_dtype))
+
+
 def test_route_edge_cases():
     _check_route(torch.zeros(3000, dtype=torch.int64), 8)  # everything on the first expert
     _check_route(torch.full((3000,), 7, dtype=torch.int32), 8)  # ... on the last
