@@ -106,6 +106,28 @@ PROTOTYPES: dict[str, tuple] = {
         c_int,
         [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int32, c_int64, c_int, c_void_p],
     ),
+    "xma_invert_index": (c_int, [c_void_p, c_int, c_int64, c_void_p, c_void_p]),
+    "xma_spread_rows": (
+        c_int,
+        [
+            c_void_p,
+            c_int64,
+            c_void_p,
+            c_int64,
+            c_void_p,
+            c_int,
+            c_void_p,
+            c_int64,
+            c_int32,
+            c_int64,
+            c_int,
+            c_void_p,
+            c_void_p,
+            c_int64,
+            c_void_p,
+            c_void_p,
+        ],
+    ),
     "xma_router_weight_grad_workspace_bytes": (c_int64, [c_int64, c_int32, c_int64]),
     "xma_router_weight_grad": (
         c_int,

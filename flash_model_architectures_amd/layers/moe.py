@@ -32,8 +32,10 @@ from ..ops import (
     gate_grad,
     group,
     group_bwd_W,
+    invert_index,
     router_weight_grad,
     scatter2scatter,
+    spread_rows,
     up_projection_fused,
 )
 from ..utils import XMAModule
@@ -286,11 +288,21 @@ class _FusedExperts(torch.autograd.Function):
         if not grad_out.is_contiguous():  # e.g. the expanded (stride 0) gradient of y.sum() or y.mean(0)
             grad_out = grad_out.contiguous()
 
-        d_gates = torch.empty_like(gates, memory_format=torch.contiguous_format)
-        gate_grad(expanded=expanded, grad_out=grad_out, d_gates=d_gates)
+        # routed row of every (token, slot): the row moves below walk the tokens
+        inverse = torch.empty(M, device=x.device, dtype=torch.int32)
+        invert_index(index=idx, inverse=inverse)
 
+        d_gates = torch.empty_like(gates, memory_format=torch.contiguous_format)
         grouped_grad = torch.empty(M, H, device=x.device, dtype=x.dtype)
-        group(A=grad_out, sorted_expert_idxs=idx, out=grouped_grad, coeff=gates.flatten(), fan_out=k)
+        spread_rows(
+            A=grad_out,
+            index=idx,
+            inverse=inverse,
+            out=grouped_grad,
+            gates=gates,
+            expanded=expanded,
+            d_gates=d_gates,
+        )
 
         d_b_down = None
         if ctx.has_bias[1] and ctx.needs_input_grad[7]:
@@ -316,15 +328,13 @@ class _FusedExperts(torch.autograd.Function):
             expert_colsum(src=d_preact, expert_offsets=expert_offsets, out=d_b_up)
 
         d_w_up = torch.empty_like(w_up)
-        group_bwd_W(
-            DY=d_preact,
-            X=x,
-            expert_offsets=expert_offsets,
-            DW=d_w_up.permute(0, 2, 1),
-            E=E,
-            x_index=idx,
-            x_fan_out=k,
-        )
+        if x.dtype == torch.float32:  # the kernel gathers the tokens itself
+            inputs = dict(X=x, x_index=idx, x_fan_out=k)
+        else:
+            grouped_x = torch.empty(M, H, device=x.device, dtype=x.dtype)
+            spread_rows(A=x, index=idx, inverse=inverse, out=grouped_x)
+            inputs = dict(X=grouped_x)
+        group_bwd_W(DY=d_preact, expert_offsets=expert_offsets, DW=d_w_up.permute(0, 2, 1), E=E, **inputs)
 
         d_expanded = torch.empty(M, H, device=x.device, dtype=x.dtype)
         scatter2scatter(

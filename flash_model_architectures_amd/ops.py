@@ -337,6 +337,66 @@ def gate_grad(expanded: torch.Tensor, grad_out: torch.Tensor, d_gates: torch.Ten
     )
 
 
+@direct_xma_op(mutates_args={"inverse"})
+def invert_index(index: torch.Tensor, inverse: torch.Tensor) -> None:
+    """inverse[index[p]] = p for a permutation `index` of 0 .. len - 1; entries outside are ignored."""
+
+    nat.require_device(index, inverse)
+    index = index.contiguous()
+    assert inverse.dtype == torch.int32 and inverse.is_contiguous() and inverse.numel() == index.numel()
+    nat.call("xma_invert_index", index.data_ptr(), _i64(index), index.numel(), inverse.data_ptr(), nat.stream())
+
+
+@direct_xma_op(mutates_args={"out", "d_gates"})
+def spread_rows(
+    A: torch.Tensor,
+    index: torch.Tensor,
+    inverse: torch.Tensor,
+    out: torch.Tensor,
+    gates: torch.Tensor | None = None,
+    expanded: torch.Tensor | None = None,
+    d_gates: torch.Tensor | None = None,
+) -> None:
+    """out[inverse[t*k + j]] = A[t], i.e. `group` with a fan-out of k, walked by token; `inverse` is `invert_index` of
+    `index`.  With `gates`, A is the gradient of the combined output: the rows are scaled by gates[t, j], and
+    d_gates[t, j] = <expanded[t*k + j], A[t]> (`gate_grad`) in the same pass."""
+
+    nat.require_device(A, index, inverse, out, gates, expanded, d_gates)
+    T, cols = A.shape
+    index = index.contiguous()
+    rows = index.numel()
+    k = rows // T if T else 1
+    assert rows == T * k and out.shape == (rows, cols) and out.dtype == A.dtype
+    assert inverse.dtype == torch.int32 and inverse.is_contiguous() and inverse.numel() == rows
+    assert (gates is None) == (expanded is None) == (d_gates is None)
+    if T == 0:
+        return
+    if gates is not None:
+        gates = gates.contiguous()
+        assert gates.numel() == rows and gates.dtype == expanded.dtype == d_gates.dtype == A.dtype
+        assert expanded.shape == (rows, cols) and d_gates.numel() == rows and d_gates.is_contiguous()
+    nat.call(
+        "xma_spread_rows",
+        A.data_ptr(),
+        _row_stride(A),
+        out.data_ptr(),
+        _row_stride(out),
+        index.data_ptr(),
+        _i64(index),
+        inverse.data_ptr(),
+        T,
+        k,
+        cols,
+        nat.dtype_code(A),
+        nat.ptr(gates),
+        nat.ptr(expanded),
+        0 if expanded is None else _row_stride(expanded),
+        nat.ptr(d_gates),
+        nat.stream(),
+        nbytes=(A.numel() + out.numel() + (0 if expanded is None else expanded.numel())) * A.element_size(),
+    )
+
+
 def router_weight_grad_supported(x: torch.Tensor, d_logits: torch.Tensor) -> bool:
     """True when the hand-written kernel behind `router_weight_grad` takes these operands (16-bit element types, E a
     multiple of 8 up to 256, H a multiple of 8, 16-byte aligned rows); other shapes go to the library's GEMM."""

@@ -227,6 +227,21 @@ int xma_gate_grad(const void* y_exp, int64_t ld_exp, const void* dy, int64_t ld_
                   int64_t T, int32_t k, int64_t cols, int dtype, void* stream);
 
 /*
+ * inverse[index[p]] = p for a permutation `index` of 0 .. rows - 1; entries outside that range are ignored.
+ */
+int xma_invert_index(const void* index, int idx_is_i64, int64_t rows, void* inverse, void* stream);
+
+/*
+ * Token rows to their routed rows, walked by token: dst[inverse[t*k + j], :] = src[t, :].  `inverse` is
+ * xma_invert_index of `index` (int32 or int64 [T*k]); entries that `index` does not confirm are skipped.
+ * With gates, expanded and d_gates (all three or none) src is dy: the rows are scaled by gates[t*k + j] and
+ * d_gates[t*k + j] = <expanded[t*k + j, :], dy[t, :]> (xma_gate_grad) is computed in the same pass.
+ */
+int xma_spread_rows(const void* src, int64_t ld_src, void* dst, int64_t ld_dst, const void* index, int idx_is_i64,
+                    const void* inverse, int64_t T, int32_t k, int64_t cols, int dtype, const void* gates,
+                    const void* expanded, int64_t ld_exp, void* d_gates, void* stream);
+
+/*
  * Weight gradient of the router's linear layer: dw[E, H] = d_logits[T, E]^T x[T, H], fp32 accumulation in a
  * fixed order (the token range is split over many blocks; the partial sums are added in split order).
  * XMA_BF16 / XMA_F16 only; E a multiple of 8, at most 256; H a multiple of 8; ldx, ldd multiples of 8 and

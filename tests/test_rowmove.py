@@ -115,3 +115,45 @@ def test_permute_round_trip_full_size():
     ops.ungroup(gathered, perm, restored)
     del gathered
     assert torch.equal(restored.view(torch.int16), act.view(torch.int16))
+
+
+@pytest.mark.parametrize("T,k,cols,dtype", [
+    (257, 6, 2048, torch.bfloat16),  # one trip of four chunks per lane
+    (33, 2, 4104, torch.float16),  # two trips and a chunk
+    (64, 17, 72, torch.bfloat16),  # more slots than waves, fewer chunks than lanes
+    (50, 1, 512, torch.float32),
+    (40, 3, 37, torch.bfloat16),  # not a whole number of vectors
+    (1, 8, 8, torch.float32),
+])
+@pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
+def test_spread_rows_equals_the_gather(T, k, cols, dtype, index_dtype):
+    """Walking the tokens writes the rows and gate gradients that the gather and `gate_grad` give, bit for bit."""
+
+    g = torch.Generator("cuda").manual_seed(T + k)
+    M = T * k
+    wide = torch.randn(T, cols + 8, generator=g, device="cuda").to(dtype)
+    dy, expanded = wide[:, :cols], torch.randn(M, cols, generator=g, device="cuda").to(dtype)
+    gates = torch.rand(T, k, generator=g, device="cuda").to(dtype)
+    idx = torch.randperm(M, generator=g, device="cuda").to(index_dtype)
+    inverse = torch.empty(M, dtype=torch.int32, device="cuda")
+    ops.invert_index(idx, inverse)
+    assert torch.equal(idx[inverse.long()].long(), torch.arange(M, device="cuda"))
+
+    want, got = (torch.full((M, cols), 7.0, dtype=dtype, device="cuda") for _ in range(2))
+    ops.group(dy, idx, want, None, k)
+    ops.spread_rows(dy, idx, inverse, got)
+    assert torch.equal(got, want)
+
+    want_gates, got_gates = torch.empty_like(gates), torch.empty_like(gates)
+    ops.group(dy, idx, want, gates.flatten(), k)
+    ops.gate_grad(expanded, dy, want_gates)
+    ops.spread_rows(dy, idx, inverse, got, gates, expanded, got_gates)
+    assert torch.equal(got, want) and torch.equal(got_gates, want_gates)
+
+    # entries of `inverse` that `index` does not confirm are skipped
+    inverse[0], inverse[-1] = -5, M + 3
+    got.fill_(7.0)
+    ops.spread_rows(dy, idx, inverse, got)
+    skipped = (idx == 0) | (idx == M - 1)
+    ops.group(dy, idx, want, None, k)
+    assert torch.equal(got[~skipped], want[~skipped]) and bool((got[skipped] == 7.0).all())
