@@ -386,7 +386,7 @@ __global__ __launch_bounds__(256) void place_quarters_kernel(const IdT* __restri
 // several XCDs' L2 caches hold pieces of.  Four times as many ids per unit, put in order in LDS first, are written in
 // runs of kStage / E words by consecutive lanes, and the table of unit histograms that is scanned in between shrinks to a
 // quarter.  2^20 ids, 256 experts: 20 us against 34 us for units of 1024 (histograms, scan, offsets, placement straight
-// from the ranks), 2^22 ids 40 against 106, 70000 ids 14 against 23; 8 experts, 2^22 ids 34 against 72.  With more than
+// from the ranks), 2^22 ids 40 against 106; 8 experts, 2^22 ids 34 against 72.  With more than
 // 256 experts it takes as many ids to be ahead (384: 5000 ids 13.6 against 12.7, 2^17 equal, 2^22 43 against 112).
 constexpr int kStage = 4096;
 constexpr int kStageThreads = 1024;
@@ -580,15 +580,21 @@ __device__ __forceinline__ void sum_table(const uint32_t* __restrict__ unit_hist
     }
 }
 
-// Second and last launch of the counting sort for the sizes of an MoE layer (units * E <= kFusedScanValues, E <= 256;
+// Second and last launch of the counting sort for the sizes of an MoE layer (units * E <= kFusedScanValues, E <= 256, units
+// <= kFusedUnits;
 // the first launch is block_hist_kernel).  One work-group moves data at a small fraction of the device's rate, so
 // the ids are spread over many small blocks, one unit of four waves each, and every block repeats the scan for
-// itself: it reads the whole table of per-unit histograms (at most 64 KiB, L2-resident) and adds up, per expert,
+// itself: it reads the whole table of per-unit histograms (at most 192 KiB, L2-resident) and adds up, per expert,
 // all units (the expert's total) and the units before its own (where its ids start inside the expert's range);
 // thread e scans the totals into the offsets with wave shuffles; then every wave places its quarter of the unit,
 // which it requested before the scan began and counted for itself while the table was on its way (a wave's ids
 // start after those of the waves before it).  Block 0 also writes counts and offsets.
-constexpr int kFusedScanValues = 16384;
+// Where the line lies, both launches against the three of the staged sort: 131072 ids x 256 experts 12.0 / 14.9 us, 262144
+// x 256 15.8 / 16.9, 400000 x 256 22 / 17; 262144 x 128 12.0 / 16.1, 400000 x 128 15.9 / 16.1, 524288 x 128 17.3 / 16.8;
+// with few experts the table stays small and the number of blocks that read it decides: 500000 x 8 10.4 / 16.0, 2^20 x 8
+// equal, 2 * 10^6 x 8 31 / 22.
+constexpr int kFusedScanValues = 49152;
+constexpr int64_t kFusedUnits = 1024;
 constexpr int kScanExperts = 256;  // a block of 256 threads scans them, one each
 template <typename IdT, typename OutT>
 __global__ __launch_bounds__(256) void scan_place_kernel(const IdT* __restrict__ ids, int64_t n, int E, int nbits,
@@ -1027,7 +1033,7 @@ static int route_build_launch(const void* ids, int ids_is_i64, int64_t n, int32_
     }
     const int64_t units = ceil_div(n, kChunk);
     uint32_t* unit_hist = (uint32_t*)workspace;
-    if (units * E <= kFusedScanValues && E <= kScanExperts) {  // two launches: histograms, then scan and placement in one
+    if (units * E <= kFusedScanValues && units <= kFusedUnits && E <= kScanExperts) {  // two launches: histograms, then scan and placement in one
         const size_t hist_lds = (size_t)4 * E * sizeof(uint32_t);
         if (ids_is_i64)
             hipLaunchKernelGGL(block_hist_kernel<int64_t>, dim3((unsigned)units), dim3(256), hist_lds, stream,

@@ -39,7 +39,7 @@ def test_route_matches_oracle(n, E, dtype):
     _check_route(ids, E, index_dtype=torch.int64 if dtype == torch.int64 else torch.int32)
 
 
-@pytest.mark.parametrize("n,E", [(131073, 512), (140001, 300), (66001, 256), (4096 * 17, 256), (4096 * 80, 64), (4300001, 8)])
+@pytest.mark.parametrize("n,E", [(131073, 512), (140001, 300), (200001, 256), (4096 * 50, 256), (4096 * 200, 64), (4300001, 8)])
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 @pytest.mark.parametrize("invalid", [False, True])
 def test_route_staged(n, E, dtype, invalid):
