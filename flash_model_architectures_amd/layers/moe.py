@@ -36,6 +36,7 @@ from ..ops import (
     router_weight_grad,
     scatter2scatter,
     spread_rows,
+    spread_rows_gate_grad,
     up_projection_fused,
 )
 from ..utils import XMAModule
@@ -294,7 +295,7 @@ class _FusedExperts(torch.autograd.Function):
 
         d_gates = torch.empty_like(gates, memory_format=torch.contiguous_format)
         grouped_grad = torch.empty(M, H, device=x.device, dtype=x.dtype)
-        spread_rows(
+        spread_rows_gate_grad(
             A=grad_out,
             index=idx,
             inverse=inverse,

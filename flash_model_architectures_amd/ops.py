@@ -347,20 +347,15 @@ def invert_index(index: torch.Tensor, inverse: torch.Tensor) -> None:
     nat.call("xma_invert_index", index.data_ptr(), _i64(index), index.numel(), inverse.data_ptr(), nat.stream())
 
 
-@direct_xma_op(mutates_args={"out", "d_gates"})
-def spread_rows(
+def _spread_rows(
     A: torch.Tensor,
     index: torch.Tensor,
     inverse: torch.Tensor,
     out: torch.Tensor,
-    gates: torch.Tensor | None = None,
-    expanded: torch.Tensor | None = None,
-    d_gates: torch.Tensor | None = None,
+    gates: torch.Tensor | None,
+    expanded: torch.Tensor | None,
+    d_gates: torch.Tensor | None,
 ) -> None:
-    """out[inverse[t*k + j]] = A[t], i.e. `group` with a fan-out of k, walked by token; `inverse` is `invert_index` of
-    `index`.  With `gates`, A is the gradient of the combined output: the rows are scaled by gates[t, j], and
-    d_gates[t, j] = <expanded[t*k + j], A[t]> (`gate_grad`) in the same pass."""
-
     nat.require_device(A, index, inverse, out, gates, expanded, d_gates)
     T, cols = A.shape
     index = index.contiguous()
@@ -368,8 +363,7 @@ def spread_rows(
     k = rows // T if T else 1
     assert rows == T * k and out.shape == (rows, cols) and out.dtype == A.dtype
     assert inverse.dtype == torch.int32 and inverse.is_contiguous() and inverse.numel() == rows
-    assert (gates is None) == (expanded is None) == (d_gates is None)
-    if T == 0:
+    if rows == 0:
         return
     if gates is not None:
         gates = gates.contiguous()
@@ -393,8 +387,33 @@ def spread_rows(
         0 if expanded is None else _row_stride(expanded),
         nat.ptr(d_gates),
         nat.stream(),
+        tag="xma_spread_rows" if gates is None else "xma_spread_rows(gate grad)",
         nbytes=(A.numel() + out.numel() + (0 if expanded is None else expanded.numel())) * A.element_size(),
     )
+
+
+@direct_xma_op(mutates_args={"out"})
+def spread_rows(A: torch.Tensor, index: torch.Tensor, inverse: torch.Tensor, out: torch.Tensor) -> None:
+    """out[inverse[t*k + j]] = A[t], i.e. `group` with a fan-out of k, walked by token; `inverse` is `invert_index` of
+    `index`."""
+
+    _spread_rows(A, index, inverse, out, None, None, None)
+
+
+@direct_xma_op(mutates_args={"out", "d_gates"})
+def spread_rows_gate_grad(
+    A: torch.Tensor,
+    index: torch.Tensor,
+    inverse: torch.Tensor,
+    out: torch.Tensor,
+    gates: torch.Tensor,
+    expanded: torch.Tensor,
+    d_gates: torch.Tensor,
+) -> None:
+    """`spread_rows` of the combined output's gradient, scaled by gates[t, j], and in the same pass
+    d_gates[t, j] = <expanded[t*k + j], A[t]> (`gate_grad`)."""
+
+    _spread_rows(A, index, inverse, out, gates, expanded, d_gates)
 
 
 def router_weight_grad_supported(x: torch.Tensor, d_logits: torch.Tensor) -> bool:

@@ -147,7 +147,7 @@ def test_spread_rows_equals_the_gather(T, k, cols, dtype, index_dtype):
     want_gates, got_gates = torch.empty_like(gates), torch.empty_like(gates)
     ops.group(dy, idx, want, gates.flatten(), k)
     ops.gate_grad(expanded, dy, want_gates)
-    ops.spread_rows(dy, idx, inverse, got, gates, expanded, got_gates)
+    ops.spread_rows_gate_grad(dy, idx, inverse, got, gates, expanded, got_gates)
     assert torch.equal(got, want) and torch.equal(got_gates, want_gates)
 
     # entries of `inverse` that `index` does not confirm are skipped
