@@ -322,6 +322,7 @@ class _FusedExperts(torch.autograd.Function):
             d_preact=d_preact,
             activation=ctx.activation,
         )
+        del grouped_grad  # buffers of routed rows are the largest there are: each is given back after its last reader
 
         d_b_up = None
         if ctx.has_bias[0] and ctx.needs_input_grad[6]:
@@ -335,7 +336,9 @@ class _FusedExperts(torch.autograd.Function):
             grouped_x = torch.empty(M, H, device=x.device, dtype=x.dtype)
             spread_rows(A=x, index=idx, inverse=inverse, out=grouped_x)
             inputs = dict(X=grouped_x)
+            del grouped_x
         group_bwd_W(DY=d_preact, expert_offsets=expert_offsets, DW=d_w_up.permute(0, 2, 1), E=E, **inputs)
+        del inputs
 
         d_expanded = torch.empty(M, H, device=x.device, dtype=x.dtype)
         scatter2scatter(

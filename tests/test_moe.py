@@ -416,3 +416,29 @@ def test_expert_biases(T, H, I, dtype, activation):
     assert_close(moe.c_fc.bias.grad, bu.grad, tol, "d bias up")
     assert_close(moe.c_proj.bias.grad, bd.grad, tol, "d bias down")
     assert_close(moe.gate.weight.grad, go.grad, 5 * tol, "dW gate")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_peak_memory_of_the_backward_pass(dtype):
+    """A row buffer lives as long as it is read.  The most a backward pass holds beyond the forward's tensors: the
+    routed rows of the output's gradient and of the pre-activation's, one more buffer of routed rows (the gathered
+    tokens, then the input gradient of every row), the gradients it returns and small index tensors."""
+
+    T, H, I, E, k = 2048, 2048, 256, 4, 4
+    moe = xma.MoE(E, k, H, I, xma.swiglu_packed, True, False, 0.02).to(dtype).cuda()
+    x = torch.randn(T, H, device="cuda", dtype=dtype, requires_grad=True)
+    dy = torch.randn(T, H, device="cuda", dtype=dtype)
+    moe(x)[0].backward(dy)  # workspaces
+    x.grad = None
+    moe.zero_grad(set_to_none=True)
+
+    y, _ = moe(x)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    y.backward(dy)
+    grown = torch.cuda.max_memory_allocated() - before
+    rows, element = T * k * H, dtype.itemsize
+    held = 2 * rows + T * k * 2 * I + 3 * E * H * I + T * H
+    small = 4 << 20  # indices, gates, router gradients, rounding of the allocator
+    assert grown <= held * element + small, f"{grown / 2**20:.1f} MiB, expected at most {(held * element + small) / 2**20:.1f}"
