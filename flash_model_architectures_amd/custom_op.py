@@ -8,7 +8,9 @@ tensors.  `CustomOp` is the autograd.Function base whose `run()` resolves the ba
 
 from __future__ import annotations
 
+import ctypes
 import inspect
+import os
 from functools import lru_cache
 from typing import Any, Callable, Iterable, Sequence
 
@@ -80,16 +82,33 @@ _DIRECT_TYPES = {
 }
 
 
+def _callback_query() -> Callable[[], bool]:
+    """`at::hasCallbacks()` of ATen/record_function.h, which has no name in Python: whether any profiler, execution trace
+    or other observer of operator calls is registered, for this thread or for all.  A library without it counts as
+    observed.  (0.1 us a call)"""
+
+    try:
+        library = ctypes.PyDLL(os.path.join(os.path.dirname(torch.__file__), "lib", "libtorch_cpu.so"))
+        query = library._ZN2at12hasCallbacksEv
+    except (OSError, AttributeError):
+        return lambda: True
+    query.restype, query.argtypes = ctypes.c_bool, []
+    return query
+
+
+_observed = _callback_query()
+
+
 def _eager() -> bool:
-    """True when nothing observes or transforms operator calls: no compiler, tracer, profiler, dispatch or function
-    mode, functorch transform (vmap, grad, jvp, functionalization) or forward-mode level is active."""
+    """True when nothing observes or transforms operator calls: no compiler, tracer, profiler or other observer, dispatch
+    or function mode, functorch transform (vmap, grad, jvp, functionalization) or forward-mode level is active."""
 
     return not (
         torch.compiler.is_compiling()
         or torch._C._len_torch_dispatch_stack()
         or torch._C._len_torch_function_stack()
         or torch._C._functorch.peek_interpreter_stack() is not None
-        or torch._C._autograd._profiler_enabled()
+        or _observed()
         or torch.autograd.forward_ad._current_level >= 0
         or torch._C._get_tracing_state() is not None
     )

@@ -32,6 +32,31 @@ def test_observed_calls_are_not_direct(mode):
     assert _eager()
 
 
+@contextlib.contextmanager
+def _execution_trace(path):
+    observer = torch.profiler.ExecutionTraceObserver().register_callback(str(path))
+    observer.start()
+    try:
+        yield
+    finally:
+        observer.stop()
+        observer.unregister_callback()
+
+
+def test_execution_trace_holds_every_call(tmp_path):
+    """An execution trace observes calls through a callback of its own, without a profiler being enabled."""
+
+    path = tmp_path / "trace.json"
+    with _execution_trace(path):
+        assert not torch._C._autograd._profiler_enabled() and not _eager()
+        apply_function(_Double, torch.ones(3))
+        with pytest.raises(RuntimeError, match="ROCm device"):  # the operator is reached, and refuses the host tensor
+            ops.swiglu_forward_rocm(*(torch.ones(1, 8) for _ in range(3)))
+    trace = path.read_text()
+    assert "_Double" in trace and "xma::swiglu_forward_rocm" in trace
+    assert _eager()
+
+
 def test_transformed_calls_are_not_direct():
     seen = []
 
