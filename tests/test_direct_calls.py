@@ -10,7 +10,7 @@ from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
 from flash_model_architectures_amd import ops
-from flash_model_architectures_amd.custom_op import _eager, apply_function
+from flash_model_architectures_amd.custom_op import _eager, apply_function, direct_xma_op
 from flash_model_architectures_amd.functional.routing import _TopkSoftmax
 
 
@@ -122,6 +122,47 @@ def test_direct_call_equals_the_operator(kind, positional):
     version = y._version
     assert (ops.swiglu_forward_rocm(g, u, y) if positional else ops.swiglu_forward_rocm(y=y, g=g, u=u)) is None
     assert torch.equal(y, want) and y._version - version == bump == 1
+
+
+def _register_in_library(key):
+    def register(op, kernel):
+        library = torch.library.Library("xma", "IMPL")
+        library.impl(op.__name__, kernel, key)
+        return library._destroy
+
+    return register
+
+
+def _register_in_definition(device):
+    return lambda op, kernel: op._custom_op.register_kernel(device)(kernel)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(
+    "name,register",
+    [
+        ("library_device", _register_in_library("CUDA")),
+        ("library_autograd", _register_in_library("AutogradCUDA")),
+        ("definition", _register_in_definition(None)),
+        ("definition_device", _register_in_definition("cuda")),
+    ],
+)
+def test_registered_kernel_is_called(name, register):
+    """A kernel that a program registers for an operator is called, and no longer once its library is gone."""
+
+    def copy(x: "torch.Tensor", y: "torch.Tensor") -> None:
+        y.copy_(x)
+
+    copy.__name__ = f"test_copy_{name}"
+    op, calls = direct_xma_op(mutates_args={"y"})(copy), []
+    x, y = torch.ones(4, device="cuda"), torch.zeros(4, device="cuda")
+    undo = register(op, lambda x, y: calls.append(y))
+    op(x, y)
+    assert len(calls) == 1 and not y.any()
+    if name.startswith("library"):
+        undo()
+        op(x, y)
+        assert len(calls) == 1 and torch.equal(x, y)
 
 
 @pytest.mark.gpu
