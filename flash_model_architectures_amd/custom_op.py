@@ -100,11 +100,28 @@ def _callback_query() -> Callable[[], bool]:
 _observed = _callback_query()
 
 
+def _predicates_known() -> bool:
+    """Whether this torch has every name without a public counterpart that the short ways rest on; without one of them no
+    call is direct."""
+
+    try:
+        torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack, torch._C._get_tracing_state
+        torch._C._functorch.peek_interpreter_stack, torch.autograd.forward_ad._current_level
+        torch._C._dispatch_keys, torch._C._dispatch_has_kernel_for_any_dispatch_key
+        torch.autograd.graph.increment_version
+    except AttributeError:
+        return False
+    return True
+
+
+_KNOWN = _predicates_known()
+
+
 def _eager() -> bool:
     """True when nothing observes or transforms operator calls: no compiler, tracer, profiler or other observer, dispatch
     or function mode, functorch transform (vmap, grad, jvp, functionalization) or forward-mode level is active."""
 
-    return not (
+    return _KNOWN and not (
         torch.compiler.is_compiling()
         or torch._C._len_torch_dispatch_stack()
         or torch._C._len_torch_function_stack()
@@ -181,7 +198,9 @@ def direct_xma_op(mutates_args: Iterable[str]) -> Callable:
     def decorator(func: Callable) -> Callable:
         op = xma_op(mutates_args=mutates_args)(func)
         qualified_name = f"{LIBRARY_NAME}::{func.__name__}"
-        kernels = op._custom_op._backend_fns  # of the operator's definition, by device
+        kernels = getattr(op._custom_op, "_backend_fns", None)  # of the operator's definition, by device
+        if kernels is None:
+            return op
         own_kernels = dict(kernels)
 
         parameters = inspect.signature(func).parameters

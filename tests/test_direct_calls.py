@@ -2,6 +2,9 @@
 operator in everything a caller can see."""
 
 import contextlib
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -55,6 +58,24 @@ def test_execution_trace_holds_every_call(tmp_path):
     trace = path.read_text()
     assert "_Double" in trace and "xma::swiglu_forward_rocm" in trace
     assert _eager()
+
+
+@pytest.mark.parametrize("name", ["_len_torch_dispatch_stack", "_dispatch_has_kernel_for_any_dispatch_key"])
+def test_unknown_predicate_makes_no_call_direct(name):
+    """A torch without one of the names that the short way asks: every call takes the long way."""
+
+    program = (
+        f"import torch; del torch._C.{name}\n"
+        "from flash_model_architectures_amd import ops\n"
+        "from flash_model_architectures_amd.custom_op import _eager\n"
+        "assert not _eager()\n"
+        "try: ops.swiglu_forward_rocm(*(torch.ones(1, 8) for _ in range(3)))\n"
+        "except RuntimeError as error: assert 'ROCm device' in str(error)\n"
+        "else: raise SystemExit('not refused')\n"
+    )
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    done = subprocess.run([sys.executable, "-c", program], cwd=root, capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0, done.stderr
 
 
 def test_transformed_calls_are_not_direct():
