@@ -115,6 +115,24 @@ def test_apply_function_records_a_graph_when_one_is_needed():
         torch.func.grad(lambda t: apply_function(_Double, t).sum())(x.detach())
 
 
+class _LongWay(Exception):
+    pass
+
+
+def _refuse(*args, **kwargs):
+    raise _LongWay
+
+
+def test_apply_function_takes_the_short_way(monkeypatch):
+    x = torch.ones(3, requires_grad=True)
+    monkeypatch.setattr(_Double, "apply", _refuse)
+    assert torch.equal(apply_function(_Double, x.detach()), torch.full((3,), 2.0))
+    with torch.no_grad():
+        assert torch.equal(apply_function(_Double, x), torch.full((3,), 2.0))
+    with pytest.raises(_LongWay):
+        apply_function(_Double, x)
+
+
 def _swiglu_arguments(kind: str):
     g = torch.randn(5, 24, device="cuda", dtype=torch.float32, generator=torch.Generator("cuda").manual_seed(1))
     u, y = g.flip(0), torch.zeros_like(g)
@@ -143,6 +161,36 @@ def test_direct_call_equals_the_operator(kind, positional):
     version = y._version
     assert (ops.swiglu_forward_rocm(g, u, y) if positional else ops.swiglu_forward_rocm(y=y, g=g, u=u)) is None
     assert torch.equal(y, want) and y._version - version == bump == 1
+
+
+@pytest.mark.gpu
+def test_operator_takes_the_short_way(monkeypatch):
+    """Which calls reach the operator and which do not."""
+
+    arguments = {kind: _swiglu_arguments(kind) for kind in ("plain", "strided", "parameter", "negated")}
+    with torch.inference_mode():
+        created_in_inference = tuple(t.clone() for t in arguments["plain"])
+    monkeypatch.setattr(type(ops.swiglu_forward_rocm._custom_op), "__call__", _refuse)
+    for kind in ("plain", "strided", "parameter"):
+        ops.swiglu_forward_rocm(*arguments[kind])
+        ops.swiglu_forward_rocm(**dict(zip("guy", arguments[kind])))
+    g, u, y = arguments["plain"]
+    with torch.inference_mode():
+        ops.swiglu_forward_rocm(*arguments["plain"])
+        ops.swiglu_forward_rocm(*created_in_inference)
+    differentiable = g.clone().requires_grad_()
+    with torch.no_grad():
+        ops.swiglu_forward_rocm(differentiable, u, y)
+    for long in (
+        lambda: ops.swiglu_forward_rocm(*arguments["negated"]),
+        lambda: ops.swiglu_forward_rocm(differentiable, u, y),
+        lambda: ops.swiglu_forward_rocm(*created_in_inference),  # outputs of inference mode outside it
+        lambda: ops.swiglu_forward_rocm(g, u.cpu(), y),
+        lambda: ops.swiglu_forward_rocm(g, u, 1.0),
+        lambda: ops.swiglu_forward_rocm(g, u, y, y),
+    ):
+        with pytest.raises(_LongWay):
+            long()
 
 
 def _register_in_library(key):
