@@ -19,7 +19,7 @@ _lib: ctypes.CDLL | None = None
 
 DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
-ABI_VERSION = 3  # XMA_ABI_VERSION of include/xma_hip.h these bindings were written against
+ABI_VERSION = 4  # XMA_ABI_VERSION of include/xma_hip.h these bindings were written against
 
 GEMM_TN, GEMM_NN, GEMM_MT = 0, 1, 2
 EPI_NONE, EPI_SWIGLU, EPI_SWIGLU_BWD, EPI_GLU, EPI_GLU_BWD, EPI_GELU_TANH, EPI_GELU_TANH_BWD = 0, 1, 2, 3, 4, 5, 6
@@ -196,7 +196,11 @@ def load() -> ctypes.CDLL:
                 "`python -m flash_model_architectures_amd.build` (needs hipcc); there is no fallback path"
             )
         lib = ctypes.CDLL(_LIB_PATH)
-        if not hasattr(lib, "xma_abi_version") or lib.xma_abi_version() != ABI_VERSION:
+        if (
+            not hasattr(lib, "xma_abi_version")
+            or lib.xma_abi_version() != ABI_VERSION
+            or not all(hasattr(lib, name) for name in PROTOTYPES)
+        ):
             raise RuntimeError(
                 f"{_LIB_PATH} was built from another revision of include/xma_hip.h than these bindings "
                 f"(ABI version {ABI_VERSION} expected): rebuild it with `python -m flash_model_architectures_amd.build`"

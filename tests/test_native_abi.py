@@ -4,6 +4,8 @@ the Python surface that mirrors the reference, and loud failure off-device."""
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 
 import pytest
 import torch
@@ -54,6 +56,23 @@ def test_library_loads_and_exports_every_declared_symbol():
     for name in _declared_symbols():
         assert hasattr(lib, name), f"{name} is declared in include/xma_hip.h but not exported"
     assert sorted(_native.PROTOTYPES) == _declared_symbols()  # the Python binding covers the header exactly
+
+
+@pytest.mark.parametrize("version", [_native.ABI_VERSION - 1, _native.ABI_VERSION])
+def test_library_of_another_revision_is_refused(version, tmp_path, monkeypatch):
+    """A library left from an earlier build, by its version or by an entry point that it lacks: the message says what to
+    do.  (Version 3 did not have xma_invert_index and xma_spread_rows.)"""
+
+    if shutil.which("gcc") is None:
+        pytest.skip("no C compiler")
+    old = sorted(set(_native.PROTOTYPES) - {"xma_abi_version", "xma_invert_index", "xma_spread_rows"})
+    source, library = tmp_path / "old.c", tmp_path / "libold.so"
+    source.write_text(f"int xma_abi_version(void) {{ return {version}; }}\n" + "".join(f"int {n}(void) {{ return 0; }}\n" for n in old))
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(library), str(source)], check=True)
+    monkeypatch.setattr(_native, "_LIB_PATH", str(library))
+    monkeypatch.setattr(_native, "_lib", None)
+    with pytest.raises(RuntimeError, match="rebuild it"):
+        _native.load()
 
 
 def test_identification_and_error_channel():
@@ -222,9 +241,6 @@ def test_product_sources_never_touch_the_oracle():
 def test_header_is_plain_c_and_links(tmp_path):
     """The boundary is a C ABI: the header compiles as C99 with no extension, and a C program linked against the
     library reads the same interface version as the header it was compiled with (no GPU call)."""
-
-    import shutil
-    import subprocess
 
     if shutil.which("gcc") is None:
         pytest.skip("no C compiler")
