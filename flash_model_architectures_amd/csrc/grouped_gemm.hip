@@ -562,6 +562,53 @@ constexpr int lds_bytes() {
     return stages > ctile ? stages : ctile;
 }
 
+// Row-tile list: expert e owns ceil(count_e / BM) consecutive tiles.
+static __global__ __launch_bounds__(1024) void build_row_tiles_kernel(const int32_t* __restrict__ offsets, int E, int BM,
+                                                                int32_t* __restrict__ tile_expert,
+                                                                int32_t* __restrict__ tile_row0,
+                                                                int32_t* __restrict__ tile_count,
+                                                                int32_t* __restrict__ split_counters) {
+    __shared__ int32_t part[1024];
+    if (split_counters != nullptr && threadIdx.x < kSplitSlots) split_counters[threadIdx.x] = 0;
+    const int per = (E + 1023) / 1024;
+    const int e0 = threadIdx.x * per;
+    int32_t s = 0;
+    for (int i = 0; i < per; ++i) {
+        const int e = e0 + i;
+        if (e < E) s += (offsets[e + 1] - offsets[e] + BM - 1) / BM;
+    }
+    part[threadIdx.x] = s;
+    __syncthreads();
+    for (int d = 1; d < 1024; d <<= 1) {
+        const int32_t v = threadIdx.x >= d ? part[threadIdx.x - d] : 0;
+        __syncthreads();
+        part[threadIdx.x] += v;
+        __syncthreads();
+    }
+    int32_t t = part[threadIdx.x] - s;
+    for (int i = 0; i < per; ++i) {
+        const int e = e0 + i;
+        if (e < E) {
+            const int32_t begin = offsets[e], end = offsets[e + 1];
+            for (int32_t r = begin; r < end; r += BM) {
+                tile_expert[t] = e;
+                tile_row0[t] = r;
+                ++t;
+            }
+        }
+    }
+    if (threadIdx.x == 1023) tile_count[0] = part[1023];
+}
+
+void launch_build_row_tiles(const xma_grouped_gemm_args& a, int BM, int64_t row_tiles, GemmParams& P, hipStream_t stream) {
+    int32_t* ws = reinterpret_cast<int32_t*>(a.workspace);
+    P.tile_count = ws;
+    P.tile_expert = ws + 4;
+    P.tile_row0 = ws + 4 + row_tiles;
+    hipLaunchKernelGGL(build_row_tiles_kernel, dim3(1), dim3(1024), 0, stream, a.expert_offsets, a.num_experts, BM, ws + 4,
+                       ws + 4 + row_tiles, ws, P.split_counters);
+}
+
 template <typename T, int KIND, int EPI, bool RAGGED>
 static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
     using Cfg = TileCfg<T>;
@@ -581,14 +628,7 @@ static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
         const int64_t n_out = EPI == EPI_PAIRED ? a.n / 2 : a.n;
         P.col_tiles = (int32_t)ceil_div(n_out, bn_out);
         grid = grid_for_tiles(rt, P.col_tiles);
-        if (a.num_experts > kMaxScannedExperts) {
-            int32_t* ws = reinterpret_cast<int32_t*>(a.workspace);
-            P.tile_count = ws;
-            P.tile_expert = ws + 4;
-            P.tile_row0 = ws + 4 + rt;
-            hipLaunchKernelGGL(build_row_tiles_kernel, dim3(1), dim3(1024), 0, stream, a.expert_offsets, a.num_experts,
-                               Cfg::BM, ws + 4, ws + 4 + rt, ws, nullptr);
-        }
+        if (a.num_experts > kMaxScannedExperts) launch_build_row_tiles(a, Cfg::BM, rt, P, stream);
     }
     XMA_REQUIRE(grid < ((int64_t)1 << 31), "xma_grouped_gemm: %lld tiles exceed the grid limit", (long long)grid);
     (void)PV;
@@ -632,6 +672,8 @@ void fill_params(const xma_grouped_gemm_args& a, GemmParams& P) {
     P.tile_expert = nullptr;
     P.tile_row0 = nullptr;
     P.tile_count = nullptr;
+    P.split_counters = nullptr;
+    P.split_partials = nullptr;
     P.row_tiles_max = 0;
     P.col_tiles = 0;
 }

@@ -80,80 +80,15 @@ inline int64_t split_region_bytes() {
 // rank sort for up to kMaxOrderedExperts experts, natural order beyond.
 constexpr int kMaxOrderedExperts = 1024;
 inline int64_t expert_order_bytes(int64_t E) { return 4 * E * (int64_t)sizeof(int32_t); }
-static __global__ __launch_bounds__(1024) void build_expert_order_kernel(const int32_t* __restrict__ offsets, int E,
-                                                                         int32_t* __restrict__ records) {
-    __shared__ int32_t count[kMaxOrderedExperts];
-    if (E > kMaxOrderedExperts) {
-        for (int e = threadIdx.x; e < E; e += blockDim.x) {
-            records[4 * e] = e;
-            records[4 * e + 1] = offsets[e];
-            records[4 * e + 2] = offsets[e + 1];
-            records[4 * e + 3] = 0;
-        }
-        return;
-    }
-    const int e = threadIdx.x;
-    int32_t begin = 0, end = 0;
-    if (e < E) {
-        begin = offsets[e];
-        end = offsets[e + 1];
-        count[e] = end - begin;
-    }
-    __syncthreads();
-    if (e < E) {
-        const int32_t mine = end - begin;
-        int slot = 0;
-        for (int o = 0; o < E; ++o) slot += (count[o] > mine || (count[o] == mine && o < e)) ? 1 : 0;
-        records[4 * slot] = e;
-        records[4 * slot + 1] = begin;
-        records[4 * slot + 2] = end;
-        records[4 * slot + 3] = 0;
-    }
-}
 
 // routed row p -> source row of the gathered operand (indices are < 2^31, so divide in 32 bits)
 __device__ __forceinline__ int64_t source_row(const GemmParams& P, int64_t p) {
     return (int64_t)((uint32_t)load_index(P.in_index, P.idx_is_i64, p) / (uint32_t)P.in_fan_out);
 }
 
-// Row-tile list for the row-grouped kinds: expert e owns ceil(count_e / BM) consecutive tiles.
-static __global__ __launch_bounds__(1024) void build_row_tiles_kernel(const int32_t* __restrict__ offsets, int E, int BM,
-                                                                int32_t* __restrict__ tile_expert,
-                                                                int32_t* __restrict__ tile_row0,
-                                                                int32_t* __restrict__ tile_count,
-                                                                int32_t* __restrict__ split_counters) {
-    __shared__ int32_t part[1024];
-    if (split_counters != nullptr && threadIdx.x < kSplitSlots) split_counters[threadIdx.x] = 0;
-    const int per = (E + 1023) / 1024;
-    const int e0 = threadIdx.x * per;
-    int32_t s = 0;
-    for (int i = 0; i < per; ++i) {
-        const int e = e0 + i;
-        if (e < E) s += (offsets[e + 1] - offsets[e] + BM - 1) / BM;
-    }
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
-        const int32_t v = threadIdx.x >= d ? part[threadIdx.x - d] : 0;
-        __syncthreads();
-        part[threadIdx.x] += v;
-        __syncthreads();
-    }
-    int32_t t = part[threadIdx.x] - s;
-    for (int i = 0; i < per; ++i) {
-        const int e = e0 + i;
-        if (e < E) {
-            const int32_t begin = offsets[e], end = offsets[e + 1];
-            for (int32_t r = begin; r < end; r += BM) {
-                tile_expert[t] = e;
-                tile_row0[t] = r;
-                ++t;
-            }
-        }
-    }
-    if (threadIdx.x == 1023) tile_count[0] = part[1023];
-}
-
+// Row-tile list for the row-grouped kinds beyond kMaxScannedExperts experts (grouped_gemm.hip): fills P.tile_count,
+// tile_expert and tile_row0 in the workspace, for up to `row_tiles` tiles of BM rows, and clears P.split_counters if set.
+void launch_build_row_tiles(const xma_grouped_gemm_args& a, int BM, int64_t row_tiles, GemmParams& P, hipStream_t stream);
 
 // Work-group -> (row tile, column tile).  Tiles are numbered in bands of kBandTiles row tiles x all column
 // tiles, row tile fastest, so that work-groups running at the same time share A row panels and B column
@@ -370,7 +305,6 @@ struct Mma<float> {
 
 // a launch splits the tiles of its last round only when a part keeps kSplitMinStages stages
 inline bool may_split(int64_t reduction) { return (reduction + 63) / 64 >= 2 * kSplitMinStages; }
-static __global__ void clear_split_counters_kernel(int32_t* counters) { counters[threadIdx.x] = 0; }
 
 // Fills the fields of GemmParams that do not depend on the tile shape.
 void fill_params(const xma_grouped_gemm_args& a, GemmParams& P);

@@ -1005,6 +1005,39 @@ static int compute_units() {
     return count / kNumXcd * kNumXcd;
 }
 
+static __global__ __launch_bounds__(1024) void build_expert_order_kernel(const int32_t* __restrict__ offsets, int E,
+                                                                         int32_t* __restrict__ records) {
+    __shared__ int32_t count[kMaxOrderedExperts];
+    if (E > kMaxOrderedExperts) {
+        for (int e = threadIdx.x; e < E; e += blockDim.x) {
+            records[4 * e] = e;
+            records[4 * e + 1] = offsets[e];
+            records[4 * e + 2] = offsets[e + 1];
+            records[4 * e + 3] = 0;
+        }
+        return;
+    }
+    const int e = threadIdx.x;
+    int32_t begin = 0, end = 0;
+    if (e < E) {
+        begin = offsets[e];
+        end = offsets[e + 1];
+        count[e] = end - begin;
+    }
+    __syncthreads();
+    if (e < E) {
+        const int32_t mine = end - begin;
+        int slot = 0;
+        for (int o = 0; o < E; ++o) slot += (count[o] > mine || (count[o] == mine && o < e)) ? 1 : 0;
+        records[4 * slot] = e;
+        records[4 * slot + 1] = begin;
+        records[4 * slot + 2] = end;
+        records[4 * slot + 3] = 0;
+    }
+}
+
+static __global__ void clear_split_counters_kernel(int32_t* counters) { counters[threadIdx.x] = 0; }
+
 template <typename T, int KIND, int EPI, typename Pipe>
 static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
     GemmParams P;
@@ -1022,7 +1055,6 @@ static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
         }
     } else {
         const int64_t rt = max_row_tiles(a.rows, a.num_experts, BM);
-        int32_t* ws = reinterpret_cast<int32_t*>(a.workspace);
         P.row_tiles_max = (int32_t)rt;
         // the split-K region is the tail of the workspace
         char* split = reinterpret_cast<char*>(a.workspace) +
@@ -1035,11 +1067,7 @@ static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
         P.col_tiles = (int32_t)ceil_div(n_out, bn_out);
         grid = grid_for_work(rt * P.col_tiles);
         if (a.num_experts > kMaxScannedExperts) {
-            P.tile_count = ws;
-            P.tile_expert = ws + 4;
-            P.tile_row0 = ws + 4 + rt;
-            hipLaunchKernelGGL(build_row_tiles_kernel, dim3(1), dim3(1024), 0, stream, a.expert_offsets, a.num_experts,
-                               BM, ws + 4, ws + 4 + rt, ws, P.split_counters);
+            launch_build_row_tiles(a, BM, rt, P, stream);
         } else if (may_split(a.k)) {
             hipLaunchKernelGGL(clear_split_counters_kernel, dim3(1), dim3(kSplitSlots), 0, stream, P.split_counters);
         }

@@ -449,14 +449,7 @@ static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
         P.row_tiles_max = (int32_t)rt;
         P.col_tiles = (int32_t)(EPI == EPI_PAIRED ? ceil_div(a.n / 2, BN / 2) : ceil_div(a.n, BN));
         grid = grid_for_tiles(rt, P.col_tiles);
-        if (a.num_experts > kMaxScannedExperts) {
-            int32_t* ws = reinterpret_cast<int32_t*>(a.workspace);
-            P.tile_count = ws;
-            P.tile_expert = ws + 4;
-            P.tile_row0 = ws + 4 + rt;
-            hipLaunchKernelGGL(build_row_tiles_kernel, dim3(1), dim3(1024), 0, stream, a.expert_offsets, a.num_experts,
-                               BM, ws + 4, ws + 4 + rt, ws, nullptr);
-        }
+        if (a.num_experts > kMaxScannedExperts) launch_build_row_tiles(a, BM, rt, P, stream);
     }
     XMA_REQUIRE(grid < ((int64_t)1 << 31), "xma_grouped_gemm: %lld tiles exceed the grid limit", (long long)grid);
     hipLaunchKernelGGL((gemm_kernel<MB, KIND, EPI>), dim3((unsigned)grid), dim3(THREADS), 0, stream, P);

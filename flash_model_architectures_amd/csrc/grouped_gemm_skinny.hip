@@ -85,7 +85,7 @@ __device__ __forceinline__ void load4(const T* p, float (&v)[4]) {
 // NF: 16-row blocks of weights per work-group; a gated tile (EPI_PAIRED) takes NF / 2 blocks of each half.
 // RF: 16-row blocks of routed rows.  U: 64-byte steps of every row requested together.
 template <typename T, int NF, int RF, int EPI, int U>
-__global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(const GemmParams P, int64_t rows) {
+__global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(const GemmParams P) {
     constexpr int PV = Elem<T>::kPerVec;
     constexpr int STEP = 4 * PV;  // reduction elements of one 64-byte step
     constexpr bool PAIRED = EPI == EPI_PAIRED;
@@ -102,14 +102,9 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(const GemmParams P
 
     int expert = 0;
     int32_t m_begin, m_end;
-    if (P.offsets == nullptr) {  // one group: a plain product
-        m_begin = row_tile * BM;
-        m_end = m_begin + BM < rows ? m_begin + BM : (int32_t)rows;
-    } else {
-        const RowTileScan tiles(P.offsets, P.num_experts, BM, lane);
-        if (row_tile >= tiles.total) return;  // (the same for every wave of the work-group)
-        tiles.find(row_tile, expert, m_begin, m_end);
-    }
+    const RowTileScan tiles(P.offsets, P.num_experts, BM, lane);
+    if (row_tile >= tiles.total) return;  // (the same for every wave of the work-group)
+    tiles.find(row_tile, expert, m_begin, m_end);
 
     const T* A = reinterpret_cast<const T*>(P.a);
     const T* W = reinterpret_cast<const T*>(P.b) + (int64_t)expert * P.b_expert_stride;
@@ -251,11 +246,10 @@ static int launch(const GemmParams& params, int64_t rows, hipStream_t stream) {
     GemmParams P = params;
     const int64_t n_out = EPI == EPI_PAIRED ? P.n / 2 : P.n;
     P.col_tiles = (int32_t)ceil_div(n_out, EPI == EPI_PAIRED ? 8 * NF : 16 * NF);
-    const int64_t row_tiles =
-        P.offsets == nullptr ? ceil_div(rows, 16 * RF) : rows / (16 * RF) + (rows < P.num_experts ? rows : P.num_experts);
+    const int64_t row_tiles = rows / (16 * RF) + (rows < P.num_experts ? rows : P.num_experts);
     const int64_t grid = row_tiles * P.col_tiles;
     XMA_REQUIRE(grid < ((int64_t)1 << 31), "xma_grouped_gemm: %lld tiles exceed the grid limit", (long long)grid);
-    hipLaunchKernelGGL((skinny_gemm_kernel<T, NF, RF, EPI, U>), dim3((unsigned)grid), dim3(THREADS), 0, stream, P, rows);
+    hipLaunchKernelGGL((skinny_gemm_kernel<T, NF, RF, EPI, U>), dim3((unsigned)grid), dim3(THREADS), 0, stream, P);
     return check_launch("xma_grouped_gemm");
 }
 
@@ -271,7 +265,8 @@ static int dispatch(const xma_grouped_gemm_args& a, const GemmParams& P, hipStre
     (shape == EPI_PAIRED ? launch<T, NF, RF, EPI_PAIRED, 2>(P, a.rows, stream)          \
                          : launch<T, NF, RF, EPI_PLAIN, 2>(P, a.rows, stream))
     if (a.rows <= kSkinnyOneBlock * (int64_t)a.num_experts) {
-        if (!FP32 && a.n >= kSkinnyWideColumns) return XMA_SKINNY(4, 1);
+        if constexpr (!FP32)
+            if (a.n >= kSkinnyWideColumns) return XMA_SKINNY(4, 1);
         return XMA_SKINNY(2, 1);
     }
     if constexpr (!FP32) {
