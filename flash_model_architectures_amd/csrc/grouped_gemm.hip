@@ -698,6 +698,26 @@ static int dispatch_kind(const xma_grouped_gemm_args& a, bool ragged, hipStream_
     }
 }
 
+// Sizes that are multiples of the vector width (8 elements of a 16-bit type, 4 of fp32) and 16-byte aligned rows
+// take the vector kernels.  Anything else takes the element-wise form of the register-staged kernel: correct for
+// every size and alignment, at a fraction of the speed.
+static GemmForm choose_form(const xma_grouped_gemm_args& a) {
+    const int pv = a.dtype == XMA_F32 ? 4 : 8;
+    const bool ragged = a.n % pv != 0 || a.k % pv != 0 || a.lda % pv != 0 || a.ldb % pv != 0 || a.ldc % pv != 0 ||
+                        a.b_expert_stride % pv != 0 || a.c_expert_stride % pv != 0 || a.ld_aux % pv != 0 ||
+                        (a.bias != nullptr && a.ld_bias % pv != 0) || !aligned16(a.a) || !aligned16(a.b) ||
+                        !aligned16(a.c) || !aligned16(a.aux) || !aligned16(a.bias);
+    // a gated tile of the vector kernels pairs whole 16-byte chunks of the two halves
+    const bool paired_tail = (a.epilogue == XMA_EPI_SWIGLU || a.epilogue == XMA_EPI_GLU) && a.n % (2 * pv) != 0;
+    const int staged_rows = a.dtype == XMA_F32 ? TileCfg<float>::BM : TileCfg<bf16_t>::BM;
+    const int staged_cols = a.dtype == XMA_F32 ? TileCfg<float>::BN : TileCfg<bf16_t>::BN;
+    if (ragged || paired_tail) return {XMA_FORM_ELEMENTWISE, staged_rows, staged_cols};
+    if (skinny_gemm_supports(a)) return skinny_gemm_form(a);
+    if (a.dtype == XMA_F32) return f32_gemm_form(a);
+    if (dma_gemm_supports(a)) return {XMA_FORM_TILED, 256, 256};
+    return {XMA_FORM_STAGED, staged_rows, staged_cols};
+}
+
 }  // namespace xma
 
 using namespace xma;
@@ -709,6 +729,18 @@ int64_t xma_grouped_gemm_workspace_bytes(int32_t num_experts, int64_t rows) {
     // tile tables (sized for the smallest tile height of any kernel), then the split-K counters and partials
     const int64_t rt = max_row_tiles(rows, num_experts, kSmallestTileRows);
     return tile_table_bytes(rt) + split_region_bytes();
+}
+
+int xma_grouped_gemm_form(const xma_grouped_gemm_args* args, int32_t* kernel, int32_t* tile_rows, int32_t* tile_cols) {
+    XMA_REQUIRE(args && kernel && tile_rows && tile_cols, "xma_grouped_gemm_form: null pointer");
+    XMA_REQUIRE(args->struct_size == sizeof(xma_grouped_gemm_args) && valid_dtype(args->dtype) &&
+                    args->kind >= XMA_GEMM_TN && args->kind <= XMA_GEMM_MT && args->num_experts >= 1,
+                "xma_grouped_gemm_form: bad arguments");
+    const GemmForm form = choose_form(*args);
+    *kernel = form.kernel;
+    *tile_rows = form.tile_rows;
+    *tile_cols = form.tile_cols;
+    return 0;
 }
 
 int xma_grouped_gemm(const xma_grouped_gemm_args* args, void* stream_) {
@@ -730,18 +762,10 @@ int xma_grouped_gemm(const xma_grouped_gemm_args* args, void* stream_) {
                 a.num_experts);
     XMA_REQUIRE(a.rows >= 0 && a.rows < ((int64_t)1 << 31) && a.n >= 0 && a.k >= 0, "xma_grouped_gemm: bad sizes");
     XMA_REQUIRE(a.expert_offsets != nullptr, "xma_grouped_gemm: expert_offsets is null");
-    // Sizes that are multiples of the vector width (8 elements of a 16-bit type, 4 of fp32) and 16-byte aligned rows
-    // take the vector kernels.  Anything else takes the element-wise form of the register-staged kernel: correct for
-    // every size and alignment, at a fraction of the speed.
-    const int pv = a.dtype == XMA_F32 ? 4 : 8;
     const int64_t elem = a.dtype == XMA_F32 ? 4 : 2;
     auto elem_aligned = [&](const void* p) { return (reinterpret_cast<uintptr_t>(p) % elem) == 0; };
     XMA_REQUIRE(elem_aligned(a.a) && elem_aligned(a.b) && elem_aligned(a.c) && elem_aligned(a.aux) && elem_aligned(a.bias),
                 "xma_grouped_gemm: operands must be aligned to their element size");
-    const bool ragged = a.n % pv != 0 || a.k % pv != 0 || a.lda % pv != 0 || a.ldb % pv != 0 || a.ldc % pv != 0 ||
-                        a.b_expert_stride % pv != 0 || a.c_expert_stride % pv != 0 || a.ld_aux % pv != 0 ||
-                        (a.bias != nullptr && a.ld_bias % pv != 0) || !aligned16(a.a) || !aligned16(a.b) ||
-                        !aligned16(a.c) || !aligned16(a.aux) || !aligned16(a.bias);
     const bool mt = a.kind == XMA_GEMM_MT;
     if (mt) {
         XMA_REQUIRE(a.epilogue == XMA_EPI_NONE && a.bias == nullptr, "xma_grouped_gemm: MT takes no epilogue and no bias");
@@ -790,12 +814,10 @@ int xma_grouped_gemm(const xma_grouped_gemm_args* args, void* stream_) {
     // (without rows the weight-gradient kind still writes its zeros; its operands, which may then be null, are never read)
     XMA_REQUIRE(a.c && (a.rows == 0 || (a.a && a.b)), "xma_grouped_gemm: null operand");
     hipStream_t stream = (hipStream_t)stream_;
-    // a gated tile of the vector kernels pairs whole 16-byte chunks of the two halves
-    const bool paired_tail = (a.epilogue == XMA_EPI_SWIGLU || a.epilogue == XMA_EPI_GLU) && a.n % (2 * pv) != 0;
-    const bool elementwise = ragged || paired_tail;
-    if (!elementwise && skinny_gemm_supports(a)) return launch_skinny_gemm(a, stream);
-    if (!elementwise && a.dtype == XMA_F32) return launch_f32_gemm(a, stream);
-    if (!elementwise && dma_gemm_supports(a)) return launch_dma_gemm(a, stream);
+    const GemmForm form = choose_form(a);
+    if (form.kernel == XMA_FORM_STREAMING) return launch_skinny_gemm(a, stream);
+    if (form.kernel == XMA_FORM_TILED) return a.dtype == XMA_F32 ? launch_f32_gemm(a, stream) : launch_dma_gemm(a, stream);
+    const bool elementwise = form.kernel == XMA_FORM_ELEMENTWISE;
     switch (a.dtype) {
         case XMA_F32:
             return dispatch_kind<float>(a, true, stream);

@@ -309,38 +309,24 @@ inline bool may_split(int64_t reduction) { return (reduction + 63) / 64 >= 2 * k
 // Fills the fields of GemmParams that do not depend on the tile shape.
 void fill_params(const xma_grouped_gemm_args& a, GemmParams& P);
 
+// Which kernel takes a call, and the rows and columns of its (tallest) tile.  The launch functions and
+// xma_grouped_gemm_form() ask the same functions.
+struct GemmForm {
+    int kernel;  // enum xma_gemm_form
+    int tile_rows, tile_cols;
+};
+
 // The LDS-DMA pipelined kernel for 16-bit element types (grouped_gemm_dma.hip).
 bool dma_gemm_supports(const xma_grouped_gemm_args& a);
 int launch_dma_gemm(const xma_grouped_gemm_args& a, hipStream_t stream);
 
 // The kernel for fp32 operands in whole, aligned vectors (grouped_gemm_f32.hip).
+GemmForm f32_gemm_form(const xma_grouped_gemm_args& a);
 int launch_f32_gemm(const xma_grouped_gemm_args& a, hipStream_t stream);
 
 // The weight-streaming kernel for few routed rows per expert (grouped_gemm_skinny.hip).
-// With every further row tile of an expert its weights are streamed once more, so the tiles grow with the average
-// number of routed rows per expert.  Measured, bf16, up / down projection in us, each form and the 256 x 256 kernel:
-//   16 rows (up to kSkinnyOneBlock on average)     H 4096, I 14336, E 8, at 8 rows: 318 / 160; 439 / 215
-//   32 rows (up to kSkinnyTwoBlocks)               the same layer at 16 rows: 316 / 168; 443 / 223
-//   64 rows (up to kSkinnyRows)                    the same up-projection at 32 / 40 rows: 360 / 366; 436 / 436.
-//                                                  H 2048, I 1024, E 64, up at 28 / 39 rows: 116 / 124; 155 / 156
-// Beyond 40 rows some experts need two tiles of 64 and the difference is gone (128 experts at 64 rows: 255; 223).
-// The 64-row form is left to the tiled kernel where that is faster: for short reductions, unless the tiled kernel's
-// work-groups do not fill the device (k 768 and 1024, 512 and more tiles: 116 and 76 us against 106 and 67; H 512, I 1024, E 4:
-// 8.5 / 11.6 us against 20 / 25), and where the wide tiles are so few that the additional row tiles of a skewed
-// routing make a second round of work-groups (H 4096, I 14336, E 8, down, skewed: 288 us against 217).
-// fp32 streams up to kSkinnyRowsF32 rows, by tiles of 16 and 32: at 19 / 28 rows 421 / 504 us against 562 / 405 us.
-constexpr int kSkinnyRows = 40;
-constexpr int kSkinnyRowsF32 = 24;
-constexpr int kSkinnyOneBlock = 8;
-constexpr int kSkinnyTwoBlocks = 20;
-constexpr int64_t kSkinnyLongReduction = 2048;
-constexpr int64_t kSkinnyTiledRound = 256;
-// Weight rows per work-group: 32 at 16 routed rows, 64 where one expert has four work-groups of 32 for each compute
-// unit (n = 28672: 307 us against 318); 64 at 32 routed rows; at 64 routed rows 128 where the device still gets four
-// work-groups per compute unit (n = 28672, 32 rows: 360 us against 366; at 48 rows 371 against 409), 64 otherwise.
-constexpr int64_t kSkinnyWideColumns = 16384;
-constexpr int64_t kSkinnyWideTiles = 1024;
 bool skinny_gemm_supports(const xma_grouped_gemm_args& a);
+GemmForm skinny_gemm_form(const xma_grouped_gemm_args& a);
 int launch_skinny_gemm(const xma_grouped_gemm_args& a, hipStream_t stream);
 
 }  // namespace xma

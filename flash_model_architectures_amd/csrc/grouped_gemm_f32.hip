@@ -459,17 +459,26 @@ static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
 // The tallest tile that still gives every compute unit two work-groups to run side by side.  At half and a quarter of
 // that bound, 2048 rows, K 256, 64 output columns per tile: 25 and 28 us instead of 21 us for the up projection; taller
 // tiles move fewer operand bytes per FLOP (64-row tiles on a large call: 125 instead of 146 TFLOP/s).
+static int row_blocks(const xma_grouped_gemm_args& a) {
+    int shape = EPI_PLAIN, act = ACT_NONE;
+    split_epilogue(a.epilogue, shape, act);
+    const bool mt = a.kind == XMA_GEMM_MT;
+    const int64_t cols = mt ? ceil_div(a.k, BN) : shape == EPI_PAIRED ? ceil_div(a.n / 2, BN / 2) : ceil_div(a.n, BN);
+    const int64_t rows = mt ? a.n * a.num_experts : a.rows;
+    return rows * cols >= kFullDeviceTiles * 128 ? 4 : rows * cols >= kFullDeviceTiles * 64 ? 2 : 1;
+}
 template <int KIND, int EPI>
 static int launch_for_size(const xma_grouped_gemm_args& a, hipStream_t stream) {
-    const int64_t cols = KIND == XMA_GEMM_MT ? ceil_div(a.k, BN)
-                                             : (EPI == EPI_PAIRED ? ceil_div(a.n / 2, BN / 2) : ceil_div(a.n, BN));
-    const int64_t rows = KIND == XMA_GEMM_MT ? a.n * a.num_experts : a.rows;
-    if (rows * cols >= kFullDeviceTiles * 128) return launch<4, KIND, EPI>(a, stream);
-    if (rows * cols >= kFullDeviceTiles * 64) return launch<2, KIND, EPI>(a, stream);
-    return launch<1, KIND, EPI>(a, stream);
+    switch (row_blocks(a)) {
+        case 4: return launch<4, KIND, EPI>(a, stream);
+        case 2: return launch<2, KIND, EPI>(a, stream);
+        default: return launch<1, KIND, EPI>(a, stream);
+    }
 }
 
 }  // namespace f32
+
+GemmForm f32_gemm_form(const xma_grouped_gemm_args& a) { return {XMA_FORM_TILED, 32 * f32::row_blocks(a), f32::BN}; }
 
 int launch_f32_gemm(const xma_grouped_gemm_args& a, hipStream_t stream) {
     int shape = EPI_PLAIN, act = ACT_NONE;

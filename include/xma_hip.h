@@ -317,6 +317,19 @@ int xma_expert_colsum(const void* src, int64_t ld, const int32_t* expert_offsets
 int64_t xma_grouped_gemm_workspace_bytes(int32_t num_experts, int64_t rows);
 int xma_grouped_gemm(const xma_grouped_gemm_args* args, void* stream);
 
+/*
+ * Which kernel xma_grouped_gemm would take for these arguments (enum xma_gemm_form; sizes, strides, types, alignments and
+ * whether pointers are null are looked at, nothing is read or launched), and the rows and columns of its largest tile.
+ * The streaming kernel's columns are weight rows.  For tests and for reading profiles.
+ */
+enum xma_gemm_form {
+    XMA_FORM_ELEMENTWISE = 0, /* any size and alignment */
+    XMA_FORM_STAGED = 1,      /* register-staged: 16-bit weight gradient with a fused row gather */
+    XMA_FORM_STREAMING = 2,   /* few routed rows per expert: the weights are streamed */
+    XMA_FORM_TILED = 3        /* LDS-DMA tiles */
+};
+int xma_grouped_gemm_form(const xma_grouped_gemm_args* args, int32_t* kernel, int32_t* tile_rows, int32_t* tile_cols);
+
 #ifdef __cplusplus
 }
 #endif

@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import torch
@@ -124,3 +125,26 @@ def make_moe_inputs(T, H, I, E, seed=0, dtype=torch.float32, with_grad=True):
     d_y = torch.randn(T, H, generator=g) if with_grad else None
     cast = lambda t: None if t is None else t.to(dtype)
     return cast(x), cast(w_gate), cast(w_up), cast(w_down), cast(d_y)
+
+
+FORM_NAMES = ("element-wise", "staged", "streaming", "tiled")  # enum xma_gemm_form
+
+
+def gemm_form(kind: str, dtype, experts: int, rows: int, n: int, k: int, epilogue: int = 0, gathered: bool = False) -> tuple:
+    """(kernel, rows, columns of its largest tile) that the library takes for contiguous, aligned operands."""
+
+    from flash_model_architectures_amd import _native
+
+    args = _native.GroupedGemmArgs()
+    args.struct_size = ctypes.sizeof(args)
+    args.kind = {"TN": 0, "NN": 1, "MT": 2}[kind]
+    args.dtype = _native.DTYPE_CODE[dtype]
+    args.num_experts, args.rows, args.n, args.k, args.epilogue = experts, rows, n, k, epilogue
+    somewhere = ctypes.c_void_p(1 << 20)
+    args.a = args.b = args.c = somewhere
+    if gathered:
+        args.in_index = somewhere
+    out = [ctypes.c_int32() for _ in range(3)]
+    status = _native.load().xma_grouped_gemm_form(ctypes.byref(args), *(ctypes.byref(v) for v in out))
+    assert status == 0, _native.last_error()
+    return FORM_NAMES[out[0].value], out[1].value, out[2].value

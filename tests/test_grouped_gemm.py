@@ -8,7 +8,7 @@ import torch
 from flash_model_architectures_amd import ops
 from oracle import torch_oracle as to
 
-from .helpers import GEMM_ELEM_TOL, TOL, assert_close
+from .helpers import GEMM_ELEM_TOL, TOL, assert_close, gemm_form
 
 pytestmark = pytest.mark.gpu
 
@@ -191,7 +191,7 @@ FEW_ROWS = [
     ([0, 1, 0, 16, 0, 17, 2], 2048, 272),  # empty experts in between; one block exactly, one row more
     ([15, 33, 1, 32, 31] + [0] * 70 + [7], 520, 144),  # beyond 64 experts; reduction ends inside a step
     ([20, 24, 9, 31, 5], 424, 80),  # row tiles of 32; reduction shorter than two steps of every wave
-    ([100, 3], 1096, 112),  # many row tiles of one expert
+    ([100, 3], 1096, 112),  # more than 40 rows per expert: the tiled kernels
     ([1, 0, 17, 8], 1112, 16400),  # many columns: 64 weight rows over 16 routed rows; the last column tile is a quarter full
     ([64, 1, 18, 65], 424, 80),  # the same tiles over a short reduction
     ([40, 64, 65, 17, 0, 3], 2056, 144),  # row tiles of 64 (16-bit types): one exactly, one row more; a half line at the end
@@ -201,9 +201,41 @@ FEW_ROWS = [
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("sizes,K,N", FEW_ROWS)
 def test_forward_with_few_rows_per_expert(sizes, K, N, dtype):
-    """The weight-streaming kernel of the forward projections at the edges of its row tiles (16 and 32), of its
-    64-byte steps and of its 16-column blocks: gathered rows and gated epilogue, scattered rows with a bias."""
+    """Forward projections of few rows at the edges of 16-row blocks, of 64-byte steps of the reduction and of 16-column
+    blocks: gathered rows and gated epilogue, scattered rows with a bias."""
 
+    _check_forward(sizes, K, N, dtype)
+
+
+NONE = [0] * 40
+STREAMING = [
+    # rows and weight rows of the tile, rows per expert, reduction, columns of the gated projection
+    (16, 32, torch.bfloat16, [9, 0, 1, 6], 2056, 48),  # one tile per expert
+    (16, 32, torch.bfloat16, [16, 17, 33, 1, 100] + NONE, 520, 272),  # many tiles of one expert
+    (16, 64, torch.float16, [9, 0, 7], 264, 16400),
+    (32, 32, torch.float16, [33, 64, 1, 16, 17, 100] + NONE, 1032, 272),  # one and two blocks of 16 rows in the last tile
+    (32, 64, torch.bfloat16, [130, 31, 32, 33, 16, 17, 1, 300] + NONE + NONE, 520, 144),
+    (32, 64, torch.float16, [33, 20, 1, 64, 16, 17, 0, 0, 0], 1096, 112),
+    (64, 64, torch.bfloat16, [130, 1, 16, 17, 48, 33, 64, 65] + NONE[:12], 2056, 144),  # one, two, three and four blocks
+    (64, 64, torch.float16, [40, 64, 65, 17, 0, 3, 130, 0], 2056, 144),
+    (64, 128, torch.bfloat16, [1, 64, 129, 0, 16, 48, 17, 33], 2056, 16400),
+    (16, 32, torch.float32, [9, 0, 1, 6], 1028, 48),
+    (32, 32, torch.float32, [33, 64, 1, 16, 17, 100] + NONE, 516, 272),
+    (32, 64, torch.float32, [20, 33, 1, 16, 40, 0, 17], 424, 80),
+]
+
+
+@pytest.mark.parametrize("rows,columns,dtype,sizes,K,N", STREAMING)
+def test_streaming_tiles(rows, columns, dtype, sizes, K, N):
+    """Every tile of the weight-streaming kernel, with experts of several tiles and last tiles of each number of 16-row
+    blocks, the last tile of columns part full."""
+
+    for epilogue in (0, 1):
+        assert gemm_form("TN", dtype, len(sizes), sum(sizes), N, K, epilogue) == ("streaming", rows, columns)
+    _check_forward(sizes, K, N, dtype)
+
+
+def _check_forward(sizes, K, N, dtype):
     E, M, dev = len(sizes), sum(sizes), "cuda"
     g = torch.Generator().manual_seed(M + K + N)
     off_list = [0] + torch.tensor(sizes).cumsum(0).tolist()
