@@ -387,12 +387,15 @@ __global__ __launch_bounds__(256) void place_quarters_kernel(const IdT* __restri
 // runs of kStage / E words by consecutive lanes, and the table of unit histograms that is scanned in between shrinks to a
 // quarter.  2^20 ids, 256 experts: 20 us against 34 us for units of 1024 (histograms, scan, offsets, placement straight
 // from the ranks), 2^22 ids 40 against 106; 8 experts, 2^22 ids 34 against 72.  With more than
-// 256 experts it takes as many ids to be ahead (384: 5000 ids 13.6 against 12.7, 2^17 equal, 2^22 43 against 112).
+// 256 experts it has to be ahead of four launches whose smaller units spread over four times as many compute units, which
+// shows where most of a unit's ids are equal and their counters are one address: 384 experts, us against those four,
+// even ids and all equal: 2^17 ids 16.4 / 16.5, 21.7 / 16.8; 2^18 18.5 / 18.7, 23.4 / 17.5; 2^19 19.6 / 27.0, 23.8 / 21.5;
+// 512 experts, 2^20: 23 / 43, 25 / 31.  (256 experts, 2 * 10^5: 17 / 25, 22 / 25.)
 constexpr int kStage = 4096;
 constexpr int kStageThreads = 1024;
 constexpr int kStageWaves = kStageThreads / kWaveSize;
 constexpr int kStageBatches = kStage / kStageThreads;  // 64-wide batches per wave
-constexpr int64_t kStageManyIds = (int64_t)1 << 17;    // from here on with more than kScanExperts experts
+constexpr int64_t kStageManyIds = (int64_t)1 << 19;    // from here on with more than kScanExperts experts
 constexpr int kStageExperts = 512;                     // 16 rows of E words and the staged unit fit in 64 KiB of LDS
 
 template <typename IdT>

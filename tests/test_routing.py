@@ -39,12 +39,16 @@ def test_route_matches_oracle(n, E, dtype):
     _check_route(ids, E, index_dtype=torch.int64 if dtype == torch.int64 else torch.int32)
 
 
-@pytest.mark.parametrize("n,E", [(131073, 512), (140001, 300), (200001, 256), (4096 * 50, 256), (4096 * 200, 64), (4300001, 8)])
+@pytest.mark.parametrize("n,E", [
+    (524289, 512), (524288, 257), (200001, 256), (4096 * 50, 256), (4096 * 200, 64), (4300001, 8),
+    (131073, 512), (140001, 300), (524287, 512),  # four launches
+])
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 @pytest.mark.parametrize("invalid", [False, True])
 def test_route_staged(n, E, dtype, invalid):
     """The counting sort that puts units of 4096 ids in order before it writes them: one id more than a unit, unit
-    edges, more than sixteen units per segment of the scan, the most experts it takes; ids outside [0, E) are left out."""
+    edges, more than sixteen units per segment of the scan, the most experts it takes, and streams of as many experts that
+    are left to four launches; ids outside [0, E) are left out."""
 
     g = torch.Generator().manual_seed(n + E)
     ids = torch.randint(-3 if invalid else 0, E + (3 if invalid else 0), (n,), generator=g, dtype=dtype)
