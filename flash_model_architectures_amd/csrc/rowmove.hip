@@ -240,7 +240,11 @@ __global__ __launch_bounds__(1024) void gate_grad_kernel(const T* __restrict__ y
 // against 172, and 196 against 89 + 175.  8192 tokens of 4096, k = 2 (rows the caches hold): 42 against 46, 54 against 31 + 41.
 // `inverse` holds for each scattered position its grouped position; an entry that `index` does not confirm (an index
 // that is no permutation leaves some unwritten) is skipped.
-template <typename T, bool GRAD, bool VEC>
+// FOUR: rows of at least 4 * 64 chunks, four of them in flight per lane.  The registers for it halve the waves of a compute
+// unit, which short rows need more: GRAD, bf16, 16384 tokens, without / with it and by gate_grad_kernel and the gather,
+// k = 6, 256 columns 54 / 86 / 66 us; k = 8, 576 columns 98 / 134 / 128; k = 4, 1544 columns 97 / 137 / 137; k = 6,
+// 2048 columns 160 / 154 / 200.
+template <typename T, bool GRAD, bool VEC, bool FOUR>
 __global__ __launch_bounds__(1024) void spread_rows_kernel(const T* __restrict__ src, int64_t ld_src, T* __restrict__ dst,
                                                            int64_t ld_dst, const void* __restrict__ index, int idx_is_i64,
                                                            const int32_t* __restrict__ inverse,
@@ -280,7 +284,7 @@ __global__ __launch_bounds__(1024) void spread_rows_kernel(const T* __restrict__
                     if (live) store_stream(out + chunk * PV, result);
                 };
                 // four chunks (of both rows) in flight per lane
-                for (; c + 3 * kWaveSize < chunks; c += 4 * kWaveSize) {
+                for (; FOUR && c + 3 * kWaveSize < chunks; c += 4 * kWaveSize) {
                     uint4 raw[4], other[4];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
@@ -486,8 +490,8 @@ int xma_spread_rows(const void* src, int64_t ld_src, void* dst, int64_t ld_dst, 
                 "xma_spread_rows: gates, expanded and d_gates come together");
     if (T == 0) return 0;
     XMA_REQUIRE(src && dst && index && inverse, "xma_spread_rows: null pointer");
-#define XMA_SPREAD(G, V)                                                                                              \
-    hipLaunchKernelGGL((spread_rows_kernel<T_, G, V>), grid, block, 0, stream, (const T_*)src, ld_src, (T_*)dst, ld_dst, \
+#define XMA_SPREAD(G, V, F)                                                                                           \
+    hipLaunchKernelGGL((spread_rows_kernel<T_, G, V, F>), grid, block, 0, stream, (const T_*)src, ld_src, (T_*)dst, ld_dst, \
                        index, idx_is_i64, (const int32_t*)inverse, (const T_*)gates, (const T_*)expanded, ld_exp,     \
                        (T_*)d_gates, T, (int)k, cols)
     XMA_DISPATCH_DTYPE(
@@ -496,11 +500,12 @@ int xma_spread_rows(const void* src, int64_t ld_src, void* dst, int64_t ld_dst, 
                          (!grad || (aligned16(expanded) && ld_exp % Elem<T_>::kPerVec == 0));
         const dim3 grid(row_grid(T)), block((unsigned)(kWaveSize * (k < 16 ? k : 16)));
         if (grad) {
-            if (vec) XMA_SPREAD(true, true);
-            else XMA_SPREAD(true, false);
+            if (vec && cols >= 4 * kWaveSize * Elem<T_>::kPerVec) XMA_SPREAD(true, true, true);
+            else if (vec) XMA_SPREAD(true, true, false);
+            else XMA_SPREAD(true, false, false);
         } else {
-            if (vec) XMA_SPREAD(false, true);
-            else XMA_SPREAD(false, false);
+            if (vec) XMA_SPREAD(false, true, true);
+            else XMA_SPREAD(false, false, false);
         })
 #undef XMA_SPREAD
     return check_launch("xma_spread_rows");

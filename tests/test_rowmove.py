@@ -122,6 +122,9 @@ def test_permute_round_trip_full_size():
     (33, 2, 4104, torch.float16),  # two trips and a chunk
     (64, 17, 72, torch.bfloat16),  # more slots than waves, fewer chunks than lanes
     (50, 1, 512, torch.float32),
+    (30, 3, 1544, torch.bfloat16),  # three trips of one chunk per lane and a chunk
+    (30, 3, 2056, torch.float16),
+    (30, 2, 1024, torch.float32),
     (40, 3, 37, torch.bfloat16),  # not a whole number of vectors
     (1, 8, 8, torch.float32),
 ])
