@@ -575,7 +575,7 @@ static __global__ __launch_bounds__(1024) void build_row_tiles_kernel(const int3
     int32_t s = 0;
     for (int i = 0; i < per; ++i) {
         const int e = e0 + i;
-        if (e < E) s += (offsets[e + 1] - offsets[e] + BM - 1) / BM;
+        if (e < E) s += (int32_t)(((uint32_t)(offsets[e + 1] - offsets[e]) + (uint32_t)BM - 1u) / (uint32_t)BM);
     }
     part[threadIdx.x] = s;
     __syncthreads();
@@ -589,11 +589,13 @@ static __global__ __launch_bounds__(1024) void build_row_tiles_kernel(const int3
     for (int i = 0; i < per; ++i) {
         const int e = e0 + i;
         if (e < E) {
-            const int32_t begin = offsets[e], end = offsets[e + 1];
-            for (int32_t r = begin; r < end; r += BM) {
+            const int32_t begin = offsets[e], rows = offsets[e + 1] - begin;
+            for (int32_t r = 0; r < rows;) {
                 tile_expert[t] = e;
-                tile_row0[t] = r;
+                tile_row0[t] = begin + r;
                 ++t;
+                if (rows - r <= BM) break;  // (r + BM may be beyond 2^31 - 1)
+                r += BM;
             }
         }
     }

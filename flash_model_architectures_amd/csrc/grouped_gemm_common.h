@@ -217,7 +217,10 @@ struct RowTileScan {
     int upto;        // first_tile + the run's tiles
     int total;
 
-    __device__ __forceinline__ int tiles_of(int32_t begin, int32_t end) const { return (end - begin + bm - 1) / bm; }
+    // (up to 2^31 - 1 rows: no sum of a row and a tile's height is taken in signed 32 bits)
+    __device__ __forceinline__ int tiles_of(int32_t begin, int32_t end) const {
+        return (int)(((uint32_t)(end - begin) + (uint32_t)bm - 1u) / (uint32_t)bm);
+    }
     __device__ __forceinline__ RowTileScan(const int32_t* __restrict__ expert_offsets, int E, int tile_rows, int lane)
         : offsets(expert_offsets), experts(E), per_lane((E + kWaveSize - 1) / kWaveSize), bm(tile_rows) {
         const int e0 = lane * per_lane;
@@ -247,7 +250,7 @@ struct RowTileScan {
         // (the compiler does not see that these are the same in every lane)
         expert = __builtin_amdgcn_readfirstlane(expert);
         row0 = __builtin_amdgcn_readfirstlane(begin + (tile - before) * bm);
-        row_end = __builtin_amdgcn_readfirstlane(row0 + bm < end ? row0 + bm : end);
+        row_end = __builtin_amdgcn_readfirstlane(end - row0 > bm ? row0 + bm : end);
     }
 };
 

@@ -532,7 +532,7 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
             tile_expert = P.tile_expert[row_tile];
             row0 = P.tile_row0[row_tile];
             const int32_t last = P.offsets[tile_expert + 1];
-            row_end = row0 + BM < last ? row0 + BM : last;
+            row_end = last - row0 > BM ? row0 + BM : last;
         } else {
             tiles.find(row_tile, tile_expert, row0, row_end);
         }

@@ -368,6 +368,29 @@ def test_few_rows_and_many_columns(gated):
         assert_close(out, want.cpu(), TOL[x.dtype], "scattered rows, many columns", elem_tol=elem)
 
 
+def test_last_rows_of_the_longest_call():
+    """Rows are counted in 32 bits up to 2^31 - 1: the last tile of one expert that holds nearly all of them, where the
+    end of a whole tile would be beyond.  (80 GiB)"""
+
+    rows, K, N, dev = 2**31 - 100, 8, 8, "cuda"
+    if torch.cuda.mem_get_info()[0] < 100 * 2**30:
+        pytest.skip("needs 100 GiB of device memory")
+    dt = torch.bfloat16
+    g = torch.Generator(dev).manual_seed(1)
+    w = torch.randn(1, N, K, generator=g, device=dev).to(dt)
+    x, out = (torch.zeros(rows, K, dtype=dt, device=dev) for _ in range(2))
+    last = torch.randn(400, K, generator=g, device=dev).to(dt)
+    x[-400:] = last
+    off = torch.tensor([0, rows], dtype=torch.int32, device=dev)
+    index = torch.zeros(rows, dtype=torch.int32, device=dev)  # not read: rows in and out in grouped order
+    ops.scatter2scatter(x, w.permute(0, 2, 1), index, index, out, 1, True, True, off)
+    del index
+    assert_close(out[-400:], (last.float() @ w[0].float().T).cpu(), TOL[dt], "last rows", elem_tol=GEMM_ELEM_TOL[dt])
+    assert not out[:-400:100003].any()
+    del x, out
+    torch.cuda.empty_cache()
+
+
 def test_full_length_reductions_dense():
     """Every layout once at the row counts of the benchmark layer (16384 routed rows over 8 experts, about 2048 per
     expert) with DENSE operands, so that the weight-gradient kernel's reductions run over ~2048 non-zero rows (32
