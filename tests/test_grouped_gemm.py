@@ -270,15 +270,15 @@ def _check_forward(sizes, K, N, dtype):
 def test_row_tiles_of_many_experts(E, dtype):
     """More experts than lanes in a wave (two and three per lane in the prefix sum that finds a work-group's rows) and
     more than the kernels look up themselves (a table of tiles), with empty experts and one many tiles long, at row
-    counts the tiled kernels take (more than 24 per expert on average)."""
+    counts that the tiled kernels take."""
 
     dev, K, N = "cuda", 64, 72
     g = torch.Generator().manual_seed(E)
-    sizes = torch.randint(0, 60, (E,), generator=g)
+    sizes = torch.randint(0, 120, (E,), generator=g)
     sizes[::7] = 0
     sizes[E // 2], sizes[E - 1] = 2000, 1
-    assert int(sizes.sum()) > 24 * E
     M = int(sizes.sum())
+    assert gemm_form("TN", dtype, E, M, N, K)[0] == "tiled"
     off_list = [0] + sizes.cumsum(0).tolist()
     off = torch.tensor(off_list, dtype=torch.int32, device=dev)
     x = torch.randn(M, K, generator=g).to(dtype)
@@ -291,21 +291,26 @@ def test_row_tiles_of_many_experts(E, dtype):
 
 
 FP32_TILES = [
-    # rows per expert, K, N: tiles of 32 rows (few of them), of 64 and of 128 (enough output columns to fill the device)
-    ([1, 0, 31, 32, 33], 4, 4),
-    ([65, 40, 2], 36, 200),
-    ([64, 65, 129, 300], 68, 8192),
-    ([127, 128, 129, 97, 33, 0, 700], 100, 8196),
-    ([257, 900], 32, 8320),
+    # rows per expert, K, N, rows of the tiles of the three layouts (a forward projection of few rows is streamed)
+    ([1, 0, 31, 32, 33], 4, 4, ("streaming", 32, 32)),
+    ([65, 40, 2], 36, 200, (32, 32, 32)),
+    ([64, 65, 129, 300], 68, 8192, (64, 32, 64)),
+    ([127, 128, 129, 97, 33, 0, 700], 100, 8196, (128, 32, 64)),
+    ([257, 900], 32, 8320, (128, 32, 32)),
+    ([198, 33, 256, 96, 300, 129, 188], 388, 4100, (64, 32, 128)),
 ]
 
 
-@pytest.mark.parametrize("sizes,K,N", FP32_TILES)
-def test_fp32_tiles(sizes, K, N):
-    """The fp32 kernel at the edges of its tile heights (32, 64, 128 rows; 32-row blocks left out of an expert's last
+@pytest.mark.parametrize("sizes,K,N,heights", FP32_TILES)
+def test_fp32_tiles(sizes, K, N, heights):
+    """The fp32 kernel at the edges of its tile heights (32, 64 and 128 rows; 32-row blocks left out of an expert's last
     tile), of its 32-deep stages (one, a partial one, two and three of them) and of its 128 columns, in all three
-    layouts, the weight gradient with and without the fused row gather.  Checker: float64 products."""
+    layouts, the weight gradient with and without the fused row gather.  Checker: float64 products.  (Tall tiles of the
+    input gradient: below.)"""
 
+    for kind, n, k, height in zip(("TN", "NN", "MT"), (N, K, N), (K, N, K), heights):
+        kernel, rows, _ = gemm_form(kind, torch.float32, len(sizes), sum(sizes), n, k)
+        assert height == (rows if kernel == "tiled" else kernel)
     E, M, dev, dt = len(sizes), sum(sizes), "cuda", torch.float32
     g = torch.Generator().manual_seed(M + K + N)
     off_list = [0] + torch.tensor(sizes).cumsum(0).tolist()
@@ -337,6 +342,55 @@ def test_fp32_tiles(sizes, K, N):
         assert_close(dw, want, TOL[dt], "MT", elem_tol=elem)
 
 
+@pytest.mark.parametrize("height,columns", [(64, 3584), (128, 7040)])
+@pytest.mark.parametrize("activation", [None, "swiglu", "gelu_tanh"])
+def test_fp32_tall_tiles(height, columns, activation):
+    """Tall tiles of the fp32 kernel's input gradient, plain and through an activation's backward, and of its gated
+    forward projection, with last tiles of one to four 32-row blocks (65 to 96 rows: three).  Checker: float64."""
+
+    sizes, k, dev, dt = [198, 33, 256, 96, 300, 129, 188], 36, "cuda", torch.float32
+    E, M = len(sizes), sum(sizes)
+    epilogue = {None: 0, "swiglu": 2, "gelu_tanh": 6}[activation]
+    assert gemm_form("NN", dt, E, M, columns, k, epilogue) == ("tiled", height, 128)
+    g = torch.Generator(dev).manual_seed(height)
+    ends = torch.tensor(sizes).cumsum(0).tolist()
+    off = torch.tensor([0] + ends, dtype=torch.int32, device=dev)
+    rows = [slice(end - size, end) for end, size in zip(ends, sizes)]
+    idx = torch.randperm(M, generator=g, device=dev).int()
+    dy = torch.randn(M, k, generator=g, device=dev)
+    w = torch.randn(E, k, columns, generator=g, device=dev)
+    product = torch.cat([dy[r].double() @ w[e].double() for e, r in enumerate(rows)])
+    elem = GEMM_ELEM_TOL[dt]
+    if activation is None:
+        dx = torch.full((M, columns), float("nan"), device=dev)
+        ops.scatter2scatter(dy, w, idx, idx, dx, 1, True, False, off)
+        want = torch.empty_like(product)
+        want[idx.long()] = product
+        assert_close(dx, want.float(), TOL[dt], "NN", elem_tol=elem)
+        return
+    module = to.swiglu_packed if activation == "swiglu" else torch.nn.GELU(approximate="tanh")
+    width = 2 * columns if activation == "swiglu" else columns
+    pre = torch.randn(M, width, generator=g, device=dev)
+    d_pre = torch.full((M, width), float("nan"), device=dev)
+    ops.down_projection_dgrad_fused(dy, w, pre, off, d_pre, activation)
+    leaf = pre.double().requires_grad_()
+    module(leaf).backward(product)
+    assert_close(d_pre, leaf.grad.float(), TOL[dt], f"{activation} backward")
+
+    if activation == "swiglu":
+        n = columns  # of both halves together
+        assert gemm_form("TN", dt, E, M, n, k, 1) == ("tiled", height, 128)
+        x = torch.randn(M, k, generator=g, device=dev)
+        w1 = torch.randn(E, n, k, generator=g, device=dev)
+        act = torch.full((M, n // 2), float("nan"), device=dev)
+        h = torch.full((M, n), float("nan"), device=dev)
+        ops.up_projection_fused(x, w1, idx, off, act, h, 1, activation)
+        gathered = x[idx.long()]
+        want = torch.cat([gathered[r].double() @ w1[e].double().T for e, r in enumerate(rows)])
+        assert_close(h, want.float(), TOL[dt], "gated TN", elem_tol=elem)
+        assert_close(act, module(h.double()).float(), TOL[dt], "gated activation")
+
+
 @pytest.mark.parametrize("gated", [True, False])
 def test_few_rows_and_many_columns(gated):
     """The widest tile of the weight-streaming kernel (128 weight rows over 64 routed rows): 16-bit types, 21 to 40
@@ -344,6 +398,7 @@ def test_few_rows_and_many_columns(gated):
 
     sizes, K, N, dev = [1, 64, 65, 0, 16, 48, 17, 33], 2056, 16400, "cuda"
     E, M = len(sizes), sum(sizes)
+    assert gemm_form("TN", torch.bfloat16, E, M, N, K, int(gated)) == ("streaming", 64, 128)
     g = torch.Generator(dev).manual_seed(5)
     off_list = [0] + torch.tensor(sizes).cumsum(0).tolist()
     off = torch.tensor(off_list, dtype=torch.int32, device=dev)
