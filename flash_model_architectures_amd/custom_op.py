@@ -13,7 +13,7 @@ import inspect
 import os
 from functools import lru_cache
 from itertools import chain
-from typing import Any, Callable, Iterable, Sequence
+from typing import Any, Callable, Iterable, NamedTuple, Sequence
 
 import torch
 
@@ -100,21 +100,15 @@ def _callback_query() -> Callable[[], bool]:
 _observed = _callback_query()
 
 
-def _predicates_known() -> bool:
-    """Whether this torch has every name without a public counterpart that the short ways rest on; without one of them no
-    call is direct."""
-
-    try:
-        torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack, torch._C._get_tracing_state
-        torch._C._functorch.peek_interpreter_stack, torch.autograd.forward_ad._current_level
-        torch._C._dispatch_keys, torch._C._dispatch_has_kernel_for_any_dispatch_key
-        torch.autograd.graph.increment_version
-    except AttributeError:
-        return False
-    return True
-
-
-_KNOWN = _predicates_known()
+# Names without a public counterpart that the short ways rest on; without one of them no call is direct.
+try:
+    _dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+    _interpreter, _tracing = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
+    _dispatch_keys, _has_kernel = torch._C._dispatch_keys, torch._C._dispatch_has_kernel_for_any_dispatch_key
+    _increment_version = torch.autograd.graph.increment_version
+    _KNOWN = hasattr(torch.autograd.forward_ad, "_current_level")
+except AttributeError:
+    _KNOWN = False
 
 
 def _eager() -> bool:
@@ -123,30 +117,34 @@ def _eager() -> bool:
 
     return _KNOWN and not (
         torch.compiler.is_compiling()
-        or torch._C._len_torch_dispatch_stack()
-        or torch._C._len_torch_function_stack()
-        or torch._C._functorch.peek_interpreter_stack() is not None
+        or _dispatch_modes()
+        or _function_modes()
+        or _interpreter() is not None
         or _observed()
         or torch.autograd.forward_ad._current_level >= 0
-        or torch._C._get_tracing_state() is not None
+        or _tracing() is not None
     )
 
 
+class _PlainKeys(NamedTuple):
+    """Dispatch keys of an ordinary dense device tensor, created outside inference mode or in it, and the keys by which the
+    dispatcher finds a kernel for one (but for ADInplaceOrView, where every operator that mutates an argument has a kernel
+    of its definition's)."""
+
+    normal: int
+    inference: int
+    kernels: "torch._C.DispatchKeySet"
+
+
 @lru_cache
-def _plain_keys(inference: bool) -> "torch._C.DispatchKeySet":
-    """Dispatch keys of an ordinary dense device tensor (created in inference mode or outside it)."""
+def _plain_keys() -> _PlainKeys:
+    def keys(inference: bool):
+        with torch.inference_mode(inference):
+            return _dispatch_keys(torch.empty(0, device="cuda"))
 
-    with torch.inference_mode(inference):
-        return torch._C._dispatch_keys(torch.empty(0, device="cuda"))
-
-
-@lru_cache
-def _device_kernel_keys() -> "torch._C.DispatchKeySet":
-    """Keys by which the dispatcher finds a kernel for such a tensor, but for ADInplaceOrView, where every operator that
-    mutates an argument has a kernel of its definition's."""
-
-    keys = torch._C.DispatchKey
-    return _plain_keys(False).remove(keys.ADInplaceOrView).add(keys.BackendSelect)
+    key = torch._C.DispatchKey
+    kernels = keys(False).remove(key.ADInplaceOrView).add(key.BackendSelect)
+    return _PlainKeys(keys(False).raw_repr(), keys(True).raw_repr(), kernels)
 
 
 class _NoGraph:
@@ -211,34 +209,34 @@ def direct_xma_op(mutates_args: Iterable[str]) -> Callable:
             """True when the dispatcher or the definition holds a kernel for the device besides the function.  (1 us; a
             kernel that takes the place of the operator's default one by force, `allow_override`, is not seen)"""
 
-            return kernels != own_kernels or torch._C._dispatch_has_kernel_for_any_dispatch_key(
-                qualified_name, _device_kernel_keys()
-            )
+            return kernels != own_kernels or _has_kernel(qualified_name, _plain_keys().kernels)
 
         def written_tensors(args: tuple, kwargs: dict) -> list[torch.Tensor] | None:
             """The mutated tensors of a call that may run directly, None when it has to go through the operator."""
 
             if len(args) > len(names):
                 return None
-            grad, inference = torch.is_grad_enabled(), torch.is_inference_mode_enabled()
-            written = []
-            dispatch_keys = torch._C._dispatch_keys
+            grad = torch.is_grad_enabled()
+            plain, written = None, []
             for name, value in chain(zip(names, args), kwargs.items()) if args else kwargs.items():
                 kind = type(value)
                 if kind not in types.get(name, ()):
                     return None
                 if kind in _TENSORS:
-                    if not value.is_cuda or (grad and value.requires_grad):
-                        return None
-                    keys = dispatch_keys(value)
-                    is_inference = keys != _plain_keys(False)
-                    if is_inference and keys != _plain_keys(True):
-                        return None
-                    if name in mutated:
-                        if not is_inference:
-                            written.append(value)
-                        elif not inference:  # refused by the operator
+                    if plain is None:
+                        if not value.is_cuda:
                             return None
+                        plain = _plain_keys()
+                    if grad and value.requires_grad:
+                        return None
+                    keys = _dispatch_keys(value).raw_repr()
+                    if keys == plain.normal:
+                        if name in mutated:
+                            written.append(value)
+                    elif keys != plain.inference:
+                        return None
+                    elif name in mutated and not torch.is_inference_mode_enabled():  # refused by the operator
+                        return None
             return written
 
         def call(*args, **kwargs):
@@ -247,7 +245,7 @@ def direct_xma_op(mutates_args: Iterable[str]) -> Callable:
                 if written is not None and not others_registered():
                     func(*args, **kwargs)
                     if written:
-                        torch.autograd.graph.increment_version(written)
+                        _increment_version(written)
                     return None
             return op(*args, **kwargs)
 
