@@ -175,6 +175,7 @@ PROTOTYPES: dict[str, tuple] = {
     "xma_grouped_gemm_workspace_bytes": (c_int64, [c_int32, c_int64]),
     "xma_grouped_gemm": (c_int, [POINTER(GroupedGemmArgs), c_void_p]),
     "xma_grouped_gemm_form": (c_int, [POINTER(GroupedGemmArgs), c_void_p, c_void_p, c_void_p]),
+    "xma_grouped_gemm_tile": (c_int, [POINTER(GroupedGemmArgs), c_void_p, c_void_p]),
 }
 
 

@@ -745,6 +745,17 @@ int xma_grouped_gemm_form(const xma_grouped_gemm_args* args, int32_t* kernel, in
     return 0;
 }
 
+int xma_grouped_gemm_tile(const xma_grouped_gemm_args* args, int32_t* tile_rows, int32_t* tile_cols) {
+    int32_t kernel = 0;
+    const int status = xma_grouped_gemm_form(args, &kernel, tile_rows, tile_cols);
+    if (status == 0 && kernel == XMA_FORM_TILED && args->dtype != XMA_F32) {
+        const DmaTile tile = dma_gemm_tile(*args);
+        *tile_rows = tile.rows;
+        *tile_cols = tile.cols;
+    }
+    return status;
+}
+
 int xma_grouped_gemm(const xma_grouped_gemm_args* args, void* stream_) {
     XMA_REQUIRE(args != nullptr, "xma_grouped_gemm: null args");
     // The caller says how long its revision of the struct is; fields it does not know are zero / NULL.

@@ -35,7 +35,8 @@ struct GemmParams {
     // split-K of the last, partly filled round of tiles (16-bit TN/NN kernels)
     int32_t* split_counters;  // [kSplitSlots] arrivals per split tile, zero at launch
     float* split_partials;    // [kSplitSlots][tile] fp32 accumulators of the parts
-    int32_t num_cu;
+    int32_t tile_rows;  // rows of the tallest tile (16-bit TN/NN)
+    int32_t round_tiles;      // tiles that run at a time on the whole device, a multiple of kNumXcd
     // MT: experts in descending order of their row counts, one record {expert, first row, end row, 0} per slot;
     // nullptr: slot e is expert e
     const int32_t* expert_order;
@@ -128,9 +129,9 @@ __device__ __forceinline__ bool locate_tile(int row_tiles, int col_tiles, int& r
     return col_tile < col_tiles;
 }
 
-// Row-grouped kinds with split-K of the remainder.  With T tiles on a device of C compute units the first
-// floor(T / C) * C tiles fill whole rounds; the R = T mod C tiles of the last round would leave C - R units idle
-// for a whole tile time, so each of them is cut along the reduction into S = min(kMaxSplit, C / R,
+// Row-grouped kinds with split-K of the remainder.  With T tiles on a device that runs C of them at a time (round_tiles: one
+// per compute unit of 256 x 256 tiles, two of the smaller ones) the first floor(T / C) * C tiles fill whole rounds; the
+// R = T mod C tiles of the last round would leave C - R places idle for a whole tile time, so each of them is cut along the reduction into S = min(kMaxSplit, C / R,
 // stages / kSplitMinStages) parts that run side by side.  Only when the launch has fewer than kSplitMaxRounds
 // rounds (the idle units of a last round matter less the more rounds there are), and only while a part keeps
 // kSplitMinStages stages: every part parks a 256 KiB tile of fp32 sums in memory and the last one reads them all
@@ -144,13 +145,13 @@ struct TileWork {
     int split_tile;   // index of the tile among the split ones
     int split_tiles;
 };
-__device__ __forceinline__ bool locate_work(int row_tiles, int col_tiles, int num_cu, int64_t stages, TileWork& w) {
+__device__ __forceinline__ bool locate_work(int row_tiles, int col_tiles, int round_tiles, int64_t stages, TileWork& w) {
     const int xcd = blockIdx.x % kNumXcd;
     const int local = blockIdx.x / kNumXcd;
     const int total = row_tiles * col_tiles;
-    const int whole = total / num_cu * num_cu;  // num_cu is a multiple of kNumXcd
+    const int whole = total / round_tiles * round_tiles;
     const int rem = total - whole;
-    int parts = rem > 0 && total < kSplitMaxRounds * num_cu ? num_cu / rem : 1;
+    int parts = rem > 0 && total < kSplitMaxRounds * round_tiles ? round_tiles / rem : 1;
     parts = parts > kMaxSplit ? kMaxSplit : parts;
     parts = parts > stages / kSplitMinStages ? (int)(stages / kSplitMinStages) : parts;
     parts = parts < 1 ? 1 : parts;
@@ -182,7 +183,7 @@ __device__ __forceinline__ bool locate_work(int row_tiles, int col_tiles, int nu
     return true;
 }
 // number of work-groups that covers every case of locate_work() for up to `tiles` tiles
-inline int64_t grid_for_work(int64_t tiles) { return (ceil_div(tiles, kNumXcd) + kSplitSlots / kNumXcd + 1) * kNumXcd; }
+inline int64_t grid_for_work(int64_t tiles, int round_tiles) { return (ceil_div(tiles, kNumXcd) + round_tiles / kNumXcd + 1) * kNumXcd; }
 
 // number of work-groups that covers up to `row_tiles` x `col_tiles` under either dealing of locate_tile()
 inline int64_t grid_for_tiles(int64_t row_tiles, int64_t col_tiles) {
@@ -321,6 +322,10 @@ struct GemmForm {
 
 // The LDS-DMA pipelined kernel for 16-bit element types (grouped_gemm_dma.hip).
 bool dma_gemm_supports(const xma_grouped_gemm_args& a);
+struct DmaTile {
+    int rows, cols;  // the tallest tile of the launch
+};
+DmaTile dma_gemm_tile(const xma_grouped_gemm_args& a);
 int launch_dma_gemm(const xma_grouped_gemm_args& a, hipStream_t stream);
 
 // The kernel for fp32 operands in whole, aligned vectors (grouped_gemm_f32.hip).

@@ -16,12 +16,16 @@
 // Ring64x5), and the 32 tiles an XCD runs at a time share their operand panels in its L2 as long as they walk
 // the reduction in step (see Kernel::phase).
 //
-// LDS is a pool of five 32 KiB slabs (all 160 KiB of the compute unit).
+// The same body runs tiles of 32, 64, 128 and 192 rows of 128 columns with half the LDS and half the registers, two
+// work-groups on a compute unit, for calls whose experts have few rows or that have few tiles (see dma_gemm_tile).  They are
+// bound by the L2 too: 15.5 TB/s of operand lines at the fine-grained layer (128 x 128, counted), where 256 x 256 asks for 9.8.
+//
+// LDS is a pool of five 32 KiB slabs (all 160 KiB of the compute unit), or of 80 KiB in slabs of 16 and 8 KiB.
 // Tile layouts inside a slab:
-//   K-contiguous operand (A in TN/NN, W in TN): [256 tile rows][BK k]; the 16-byte chunks of a row are
+//   K-contiguous operand (A in TN/NN, W in TN): [tile rows][BK k]; the 16-byte chunks of a row are
 //     XOR-swizzled by the row number so that the 16 rows a quarter-wave reads in one ds_read_b128 cover all
 //     64 banks.
-//   K-strided operand (W in NN, both operands in MT): [BK k][256 tile rows], 512 bytes per k row; chunk c
+//   K-strided operand (W in NN, both operands in MT): [BK k][tile rows], 512 or 256 bytes per k row; chunk c
 //     of k row r sits at c ^ ((r & 3) << 2), so that the four k rows one transposing read touches fall
 //     into different bank groups.
 // A DMA load writes lane l's 16 bytes at (wave-uniform LDS base) + 16*l, so the swizzles are applied
@@ -34,29 +38,65 @@
 namespace xma {
 namespace dma {
 
-constexpr int BM = 256, BN = 256, THREADS = 256, NUM_WAVES = THREADS / 64;
-constexpr int WAVES_N = 2, WM = 128, WN = 128, MI = WM / 16, NI = WN / 16;  // 8 x 8 blocks of 16 x 16 per wave
-constexpr int OUT_SLABS = 4;  // the epilogue stages the tile through LDS 64 rows (one slab) at a time
-constexpr int SLAB_BYTES = 32768;
-static_assert(BM == BN, "both operands use the same tile height");
+constexpr int THREADS = 256, NUM_WAVES = THREADS / 64, WAVES_N = 2;
 
-__shared__ __attribute__((aligned(1024))) char slab0[SLAB_BYTES];
-__shared__ __attribute__((aligned(1024))) char slab1[SLAB_BYTES];
-__shared__ __attribute__((aligned(1024))) char slab2[SLAB_BYTES];
-__shared__ __attribute__((aligned(1024))) char slab3[SLAB_BYTES];
-__shared__ __attribute__((aligned(1024))) char slab4[SLAB_BYTES];
+__shared__ __attribute__((aligned(1024))) char slab0[32768];
+__shared__ __attribute__((aligned(1024))) char slab1[32768];
+__shared__ __attribute__((aligned(1024))) char slab2[32768];
+__shared__ __attribute__((aligned(1024))) char slab3[32768];
+__shared__ __attribute__((aligned(1024))) char slab4[32768];
+__shared__ __attribute__((aligned(1024))) char half_slab0[16384];
+__shared__ __attribute__((aligned(1024))) char half_slab1[16384];
+__shared__ __attribute__((aligned(1024))) char half_slab2[16384];
+__shared__ __attribute__((aligned(1024))) char half_slab3[16384];
+__shared__ __attribute__((aligned(1024))) char half_slab4[16384];
+__shared__ __attribute__((aligned(1024))) char extra_slab0[8192];
+__shared__ __attribute__((aligned(1024))) char extra_slab1[8192];
 
-// The slabs are distinct arrays on purpose: the compiler can then prove that a fragment read of
-// one slab does not alias the DMA writes still in flight to the others, and does not drain them.
-template <int I>
-__device__ __forceinline__ char* slab() {
-    static_assert(I >= 0 && I < 5, "slab index");
-    if constexpr (I == 0) return slab0;
-    if constexpr (I == 1) return slab1;
-    if constexpr (I == 2) return slab2;
-    if constexpr (I == 3) return slab3;
-    return slab4;
-}
+// A tile of BM rows and BN columns, four waves as 2 x 2.  256 x 256 has the compute unit to itself; the tiles of 128
+// columns take half its LDS, so that two work-groups share it.
+template <int BM_, int BN_>
+struct Tile {
+    static constexpr int BM = BM_, BN = BN_, WM = BM / 2, WN = BN / 2;
+    static constexpr int MI = WM / 16, NI = WN / 16;  // blocks of 16 x 16 per wave
+    static_assert((BM == 256 && BN == 256) || ((BM == 192 || BM == 128 || BM == 64 || BM == 32) && BN == 128), "tile size");
+    // The epilogue stages the tile through LDS, SLAB_BLOCKS blocks of 16 rows of each wave row at a time.
+    static constexpr int SLAB_BLOCKS = MI < 2 ? 1 : 2;
+    static constexpr int OUT_SLABS = MI / SLAB_BLOCKS;
+    // A tile row of 192 rows does not fit one slab: rows 128..191 live in a slab of their own, and a wave row's blocks
+    // 4 and 5 are theirs, so that the slab of a block is known at compile time.
+    static constexpr bool EXTRA = BM == 192;
+    static constexpr int MAIN_BLOCKS = EXTRA ? 4 : MI;
+    // first tile row of block mi of wave row wr
+    __device__ static __forceinline__ int block_row(int wr, int mi) {
+        return mi < MAIN_BLOCKS ? wr * (MAIN_BLOCKS * 16) + mi * 16 : 128 + wr * 32 + (mi - MAIN_BLOCKS) * 16;
+    }
+
+    // The slabs are distinct arrays on purpose: the compiler can then prove that a fragment read of
+    // one slab does not alias the DMA writes still in flight to the others, and does not drain them.
+    template <int I>
+    __device__ static __forceinline__ char* slab() {
+        static_assert(I >= 0 && I < 7, "slab index");
+        if constexpr (I == 5) return extra_slab0;
+        if constexpr (I == 6) return extra_slab1;
+        if constexpr (BN == 256) {
+            if constexpr (I == 0) return slab0;
+            if constexpr (I == 1) return slab1;
+            if constexpr (I == 2) return slab2;
+            if constexpr (I == 3) return slab3;
+            return slab4;
+        } else {
+            if constexpr (I == 0) return half_slab0;
+            if constexpr (I == 1) return half_slab1;
+            if constexpr (I == 2) return half_slab2;
+            if constexpr (I == 3) return half_slab3;
+            return half_slab4;
+        }
+    }
+};
+constexpr int groups_per_cu(int BN) { return BN == 256 ? 1 : 2; }
+// fp32 sums of the tallest tile of BN columns: what a part of a split tile parks in the workspace
+constexpr int split_tile_floats(int BN) { return BN == 256 ? 256 * 256 : 192 * 128; }
 
 __device__ __attribute__((aligned(16))) uint32_t g_zero_page[4];  // zero-initialised
 
@@ -111,13 +151,15 @@ __device__ __forceinline__ void pin(V& v) {
 __device__ __forceinline__ void batch_fence() { __builtin_amdgcn_sched_barrier(0); }
 
 // ---- tile geometry for a stage depth of BK reduction elements ---------------------------------------
-template <int BK>
+// (of an operand tile of ROWS rows)
+template <int ROWS, int BK>
 struct Geometry {
     static constexpr int CPR = BK / 8;            // 16-byte chunks per K-contiguous row
     static constexpr int ROW_BYTES = BK * 2;
     static constexpr int ROWS_PER_LOAD = 64 / CPR;  // tile rows one DMA instruction covers
-    static constexpr int LOADS = BK / 2 / NUM_WAVES;  // DMA instructions per wave, operand and stage
-    static constexpr int TILE_BYTES = BM * BK * 2;
+    static constexpr int LOADS = ROWS * BK * 2 / 1024 / NUM_WAVES;  // DMA instructions per wave, operand and stage
+    static constexpr int KROW_CHUNKS = ROWS / 8;             // 16-byte chunks per K-strided row
+    static constexpr int KROWS_PER_LOAD = 64 / KROW_CHUNKS;  // reduction rows one DMA instruction covers
     static_assert(BK == 32 || BK == 64, "stage depth");
 
     __device__ static __forceinline__ int swizzle(int row) { return BK == 32 ? (row >> 2) & 3 : (row >> 1) & 7; }
@@ -137,15 +179,15 @@ struct Geometry {
         const int col = col0 + 4 * (i & 3);
         const int krow0 = kb * 32 + 8 * group + (i >> 2);
         const int chunk = (col >> 3) ^ ((krow0 & 3) << 2);  // (krow0 + 4) & 3 == krow0 & 3
-        return krow0 * (BN * 2) + (chunk << 4) + ((col & 4) << 1);
+        return krow0 * (ROWS * 2) + (chunk << 4) + ((col & 4) << 1);
     }
 };
 
-template <bool STRIDED>
+template <bool STRIDED, int ROWS>
 __device__ __forceinline__ u32x4_t read_fragment(const char* slab_base, int offset) {
     if constexpr (STRIDED) {
         const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(XMA_LDS_S4(slab_base + offset));
-        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(XMA_LDS_S4(slab_base + (offset + 4 * (BN * 2))));
+        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(XMA_LDS_S4(slab_base + (offset + 4 * (ROWS * 2))));
         const u32x2_t a = __builtin_bit_cast(u32x2_t, lo), b = __builtin_bit_cast(u32x2_t, hi);
         return u32x4_t{a.x, a.y, b.x, b.y};
     } else {
@@ -158,7 +200,8 @@ __device__ __forceinline__ u32x4_t read_fragment(const char* slab_base, int offs
 //   K-contiguous tile: tile rows [R * (i * NUM_WAVES + w), +R), R = ROWS_PER_LOAD; lane l -> row + l / CPR,
 //     physical chunk l % CPR (the logical chunk it fetches is the XOR-swizzled one, and because R * NUM_WAVES
 //     is a multiple of the swizzle period it is the same for every i);
-//   K-strided tile: k rows {2 * (i * NUM_WAVES + w), +1}; lane l -> k row + l / 32, physical chunk l % 32.
+//   K-strided tile: k rows [K * (i * NUM_WAVES + w), +K), K = KROWS_PER_LOAD; lane l -> k row + l / KROW_CHUNKS, physical
+//     chunk l % KROW_CHUNKS.
 // Three address plans:
 //   ROWS     one pointer per instruction (rows that are gathered through an index table or end anywhere),
 //   UNIFORM  K-contiguous rows at a constant stride, with one extra jump in the middle of the tile
@@ -166,11 +209,11 @@ __device__ __forceinline__ u32x4_t read_fragment(const char* slab_base, int offs
 //   STRIDED  K-strided tile: one pointer, constant stride between instructions.
 enum LoadPlan { PLAN_ROWS, PLAN_UNIFORM, PLAN_STRIDED };
 
-template <typename T, int BK, LoadPlan PLAN>
+template <typename T, int ROWS, int BK, LoadPlan PLAN>
 struct OperandLoads {
-    using G = Geometry<BK>;
+    using G = Geometry<ROWS, BK>;
     static constexpr int LOADS = G::LOADS;
-    static constexpr int RED_STRIDE = PLAN == PLAN_STRIDED ? 2 * NUM_WAVES : 0;  // reduction rows between i and i+1
+    static constexpr int RED_STRIDE = PLAN == PLAN_STRIDED ? G::KROWS_PER_LOAD * NUM_WAVES : 0;  // reduction rows between i and i+1
     const T* ptr[PLAN == PLAN_ROWS ? LOADS : 1];  // HBM address of this lane's chunk in stage 0
     bool valid[PLAN == PLAN_STRIDED ? 1 : LOADS];  // false: always the zero page (row / column outside the operand)
     int64_t load_stride, mid_jump;  // UNIFORM / STRIDED: elements from instruction i to i+1; UNIFORM: extra at LOADS/2
@@ -196,7 +239,7 @@ struct OperandLoads {
         wave_lds = wave * 1024;
     }
 
-    // UNIFORM: tile row r lives at base + r * ld (+ jump for r >= 128); rows_fn(tile row) says whether it exists.
+    // UNIFORM: tile row r lives at base + r * ld (+ jump in the lower half of the tile); rows_fn(tile row) says whether it exists.
     template <typename ValidFn>
     __device__ __forceinline__ void setup_uniform(int wave, int lane, const T* base, int64_t ld, int64_t jump,
                                                   ValidFn valid_fn) {
@@ -217,11 +260,11 @@ struct OperandLoads {
     // from there; ld = row stride.
     __device__ __forceinline__ void setup_strided(int wave, int lane, const T* base, int64_t ld, int64_t cols_left) {
         static_assert(PLAN == PLAN_STRIDED, "plan");
-        const int krow = wave * 2 + (lane >> 5);
-        const int chunk = (lane & 31) ^ ((krow & 3) << 2);  // 2 * NUM_WAVES is a multiple of 4: same for every i
+        const int krow = wave * G::KROWS_PER_LOAD + lane / G::KROW_CHUNKS;
+        const int chunk = (lane % G::KROW_CHUNKS) ^ ((krow & 3) << 2);  // RED_STRIDE is a multiple of 4: same for every i
         valid[0] = chunk * 8 < cols_left;
         ptr[0] = valid[0] ? base + (int64_t)krow * ld + chunk * 8 : zero_page();
-        load_stride = 2 * NUM_WAVES * ld;
+        load_stride = RED_STRIDE * ld;
         mid_jump = 0;
         red0 = krow;
         step = (int64_t)BK * ld;
@@ -289,82 +332,122 @@ struct OperandLoads {
 // take the B tile of stage s+2 (during the rest of the step) and the A tile of stage s+3 (during the first phase of
 // the next step): every load is issued between one and a half and two and a half phases before the barrier that
 // needs it.
+template <typename TL_>
 struct Ring64x5 {
+    using TL = TL_;
     static constexpr int BK = 64, CYCLE = 5, KK = 2;
-    static constexpr int L = Geometry<BK>::LOADS;
-    static constexpr int PHASE_LOADS = L;
-    static constexpr int WAIT = L;               // loads that may stay in flight at a step's barrier
-    static constexpr int PROLOGUE_WAIT = 2 * L;  // ... and when the first stage is needed
+    static constexpr int LA = Geometry<TL::BM, BK>::LOADS, LB = Geometry<TL::BN, BK>::LOADS;
+    static constexpr int WAIT = LA;                // loads that may stay in flight at a step's barrier
+    static constexpr int PROLOGUE_WAIT = LA + LB;  // ... and when the first stage is needed
+    static constexpr int phase_loads(int phase) { return phase == 0 ? LA : LB; }
     template <int P> struct At {
         static constexpr int A_SLAB = (2 * P) % 5, A_OFF = 0, B_SLAB = (2 * P + 1) % 5, B_OFF = 0;
     };
     static constexpr int LOOKAHEAD = 2;  // a step at stage s issues loads of stages up to s + LOOKAHEAD
     template <typename K> __device__ static __forceinline__ void prologue(K& k) {
-        k.template issue_a<0, 0, L, true>(0); k.template issue_b<0, 0, L, true>(0);
-        k.template issue_a<1, 0, L, true>(1); k.template issue_b<1, 0, L, true>(1);
+        k.template issue_a<0, 0, LA, true>(0); k.template issue_b<0, 0, LB, true>(0);
+        k.template issue_a<1, 0, LA, true>(1); k.template issue_b<1, 0, LB, true>(1);
     }
-    // load number I (0 <= I < PHASE_LOADS) of phase PH of the step at ring position P on stage s
+    // load number I (0 <= I < phase_loads(PH)) of phase PH of the step at ring position P on stage s
     template <int P, int PH, int I, bool MASKED, typename K> __device__ static __forceinline__ void issue_one(K& k, int64_t s) {
         if constexpr (PH == 0) k.template issue_a<(P + 2) % CYCLE, I, I + 1, MASKED>(s + 2);
         else k.template issue_b<(P + 2) % CYCLE, I, I + 1, MASKED>(s + 2);
     }
 };
 
+// Ring64x2: two whole stages, for tiles of 128 columns: 192 rows need 40 KiB a stage.  All loads of stage s+2 go out in the second phase of step s, one to two phases before
+// the barrier that needs them.
+template <typename TL_>
+struct Ring64x2 {
+    using TL = TL_;
+    static constexpr int BK = 64, CYCLE = 2, KK = 2;
+    static constexpr int LA = Geometry<TL::BM, BK>::LOADS, LB = Geometry<TL::BN, BK>::LOADS;
+    static constexpr int WAIT = 0, PROLOGUE_WAIT = LA + LB;
+    static constexpr int phase_loads(int phase) { return phase == 0 ? 0 : LA + LB; }
+    template <int P> struct At {
+        static constexpr int A_SLAB = 2 * P, A_OFF = 0, B_SLAB = 2 * P + 1, B_OFF = 0;
+        static constexpr int EXTRA_SLAB = 5 + P;
+    };
+    static constexpr int LOOKAHEAD = 2;
+    template <typename K> __device__ static __forceinline__ void prologue(K& k) {
+        k.template issue_a<0, 0, LA, true>(0); k.template issue_b<0, 0, LB, true>(0);
+        k.template issue_a<1, 0, LA, true>(1); k.template issue_b<1, 0, LB, true>(1);
+    }
+    template <int P, int PH, int I, bool MASKED, typename K> __device__ static __forceinline__ void issue_one(K& k, int64_t s) {
+        static_assert(PH == 1, "no loads in the first phase");
+        if constexpr (I < LA) k.template issue_a<P, I, I + 1, MASKED>(s + 2);
+        else k.template issue_b<P, I - LA, I - LA + 1, MASKED>(s + 2);
+    }
+};
+
 template <typename T, int KIND, int EPI, typename Pipe>
 struct Kernel {
     static constexpr int BK = Pipe::BK;
-    using G = Geometry<BK>;
+    using TL = typename Pipe::TL;
+    static constexpr int BM = TL::BM, BN = TL::BN, WM = TL::WM, WN = TL::WN, MI = TL::MI, NI = TL::NI;
     static constexpr bool A_STRIDED = KIND == XMA_GEMM_MT;
     static constexpr bool B_STRIDED = KIND != XMA_GEMM_TN;
     static constexpr int BN_OUT = EPI == EPI_PAIRED ? BN / 2 : BN;
 
-    OperandLoads<T, BK, A_STRIDED ? PLAN_STRIDED : PLAN_ROWS> la;
-    OperandLoads<T, BK, B_STRIDED ? PLAN_STRIDED : PLAN_UNIFORM> lb;
+    OperandLoads<T, BM, BK, A_STRIDED ? PLAN_STRIDED : PLAN_ROWS> la;
+    OperandLoads<T, BN, BK, B_STRIDED ? PLAN_STRIDED : PLAN_UNIFORM> lb;
     int64_t red_len;
     int wave, lane;
-    int a_off[4], b_off[4];  // variable parts of the fragment offsets (see fragment_offsets)
+    int a_off[4], b_off[4], extra_off[4];  // variable parts of the fragment offsets (see fragment_offsets)
     u32x4_t fa[2][MI], fb[2][NI];  // fragments: the 32-deep block being multiplied and the one being read
 
     template <int P, int I0, int I1, bool MASKED> __device__ __forceinline__ void issue_a(int64_t stage) {
-        la.template issue<I0, I1, MASKED>(slab<Pipe::template At<P>::A_SLAB>(), Pipe::template At<P>::A_OFF, stage, red_len);
+        using At = typename Pipe::template At<P>;
+        constexpr int MAIN = TL::EXTRA ? 4 : I1, M1 = I1 < MAIN ? I1 : MAIN;  // a load covers 32 tile rows over the waves
+        if constexpr (I0 < M1) la.template issue<I0, M1, MASKED>(TL::template slab<At::A_SLAB>(), At::A_OFF, stage, red_len);
+        if constexpr (TL::EXTRA && I1 > 4)
+            la.template issue<(I0 < 4 ? 4 : I0), I1, MASKED>(TL::template slab<At::EXTRA_SLAB>(), -4 * NUM_WAVES * 1024, stage, red_len);
     }
     template <int P, int I0, int I1, bool MASKED> __device__ __forceinline__ void issue_b(int64_t stage) {
-        lb.template issue<I0, I1, MASKED>(slab<Pipe::template At<P>::B_SLAB>(), Pipe::template At<P>::B_OFF, stage, red_len);
+        lb.template issue<I0, I1, MASKED>(TL::template slab<Pipe::template At<P>::B_SLAB>(), Pipe::template At<P>::B_OFF, stage, red_len);
     }
 
     // Byte offsets of this lane's fragments inside an operand tile.  Only the part that is not a
     // compile-time constant goes through opaque(): for the K-contiguous layout the 16-row block adds a
     // constant (the swizzle repeats every 16 rows); for the K-strided layout the 32-deep block adds 16 KiB and
     // the odd 16-column block of a 32-column pair adds 32 bytes (two chunks; the swizzle leaves that bit alone).
-    template <bool STRIDED>
+    template <bool STRIDED, int ROWS>
     __device__ __forceinline__ void fragment_offsets(int row0, int (&var)[4]) const {
+        using G = Geometry<ROWS, BK>;
         if constexpr (STRIDED) {
 #pragma unroll
-            for (int b = 0; b < 4; ++b) var[b] = opaque(G::kstrided_offset(row0 + b * 32, 0, lane));
+            for (int b = 0; b < ROWS / 64; ++b) var[b] = opaque(G::kstrided_offset(row0 + b * 32, 0, lane));
         } else {
 #pragma unroll
             for (int kb = 0; kb < BK / 32; ++kb) var[kb] = opaque(G::kcontig_offset(row0 + (lane & 15), kb, lane >> 4));
         }
     }
-    template <bool STRIDED>
+    template <bool STRIDED, int ROWS>
     __device__ static __forceinline__ int fragment_offset(const int (&var)[4], int block, int kb) {
-        return STRIDED ? var[block >> 1] + (block & 1) * 32 + kb * (32 * BN * 2) : var[kb] + block * (16 * G::ROW_BYTES);
+        return STRIDED ? var[block >> 1] + (block & 1) * 32 + kb * (32 * ROWS * 2) : var[kb] + block * (16 * Geometry<ROWS, BK>::ROW_BYTES);
     }
     __device__ __forceinline__ void init_fragments() {
-        fragment_offsets<A_STRIDED>((wave / WAVES_N) * WM, a_off);
-        fragment_offsets<B_STRIDED>((wave % WAVES_N) * WN, b_off);
+        fragment_offsets<A_STRIDED, BM>(TL::block_row(wave / WAVES_N, 0), a_off);
+        if constexpr (TL::EXTRA) fragment_offsets<A_STRIDED, BM>(TL::block_row(wave / WAVES_N, TL::MAIN_BLOCKS) - 128, extra_off);
+        fragment_offsets<B_STRIDED, BN>((wave % WAVES_N) * WN, b_off);
     }
 
     // One fragment of the 32-deep block kb of the stage held at ring position P: A block mi / B block ni.
     template <int P>
     __device__ __forceinline__ u32x4_t read_a(int kb, int mi) const {
         using At = typename Pipe::template At<P>;
-        return read_fragment<A_STRIDED>(slab<At::A_SLAB>(), At::A_OFF + fragment_offset<A_STRIDED>(a_off, mi, kb));
+        if constexpr (TL::EXTRA) {
+            static_assert(!A_STRIDED, "rows that do not fit one slab");
+            if (mi >= TL::MAIN_BLOCKS)
+                return read_fragment<false, BM>(TL::template slab<At::EXTRA_SLAB>(),
+                                                fragment_offset<false, BM>(extra_off, mi - TL::MAIN_BLOCKS, kb));
+        }
+        return read_fragment<A_STRIDED, BM>(TL::template slab<At::A_SLAB>(), At::A_OFF + fragment_offset<A_STRIDED, BM>(a_off, mi, kb));
     }
     template <int P>
     __device__ __forceinline__ u32x4_t read_b(int kb, int ni) const {
         using At = typename Pipe::template At<P>;
-        return read_fragment<B_STRIDED>(slab<At::B_SLAB>(), At::B_OFF + fragment_offset<B_STRIDED>(b_off, ni, kb));
+        return read_fragment<B_STRIDED, BN>(TL::template slab<At::B_SLAB>(), At::B_OFF + fragment_offset<B_STRIDED, BN>(b_off, ni, kb));
     }
     // All fragments of a block.
     template <int P>
@@ -401,16 +484,19 @@ struct Kernel {
     // (8 tail tiles among 67 at the benchmark shape).
     template <int RP, int LP, int LPH, bool MASKED>
     __device__ __forceinline__ void phase(int rkb, int cur, int64_t s, f32x4_t (&acc)[MI][NI]) {
-        constexpr int SLOTS = 4 * MI;  // 32
+        constexpr int IN_SLOT = MI < 2 ? 1 : 2, SLOTS = MI * NI / IN_SLOT, PER_B = MI / IN_SLOT;
+        constexpr int READS = MI + NI, LOADS = Pipe::phase_loads(LPH);
         const int nxt = cur ^ 1;
 #pragma unroll
         for (int slot = 0; slot < SLOTS; ++slot) {
-            const int ni = slot / 4, m0 = (slot & 3) * 2;
-            Mma16<T>::run(fb[cur][ni], fa[cur][m0], acc[m0][ni]);
-            Mma16<T>::run(fb[cur][ni], fa[cur][m0 + 1], acc[m0 + 1][ni]);
-            if (slot % 2 == 1) {
-                const int r = slot / 2;  // the r-th of the 16 fragment blocks of the next phase
-                if constexpr (KIND == XMA_GEMM_NN) {
+            const int ni = slot / PER_B, m0 = (slot % PER_B) * IN_SLOT;
+#pragma unroll
+            for (int i = 0; i < IN_SLOT; ++i) Mma16<T>::run(fb[cur][ni], fa[cur][m0 + i], acc[m0 + i][ni]);
+#pragma unroll
+            for (int r = 0; r < READS; ++r) {  // the r-th fragment block of the next phase
+                const int last = (r + 1) * SLOTS / READS - 1;
+                if (slot != (last < 0 ? 0 : last)) continue;
+                if constexpr (KIND == XMA_GEMM_NN && MI == NI) {
                     if (r % 2 == 0) fa[nxt][r / 2] = read_a<RP>(rkb, r / 2);
                     else fb[nxt][r / 2] = read_b<RP>(rkb, r / 2);
                 } else {
@@ -418,22 +504,30 @@ struct Kernel {
                     else fb[nxt][r - MI] = read_b<RP>(rkb, r - MI);
                 }
             }
-            if (slot % 4 == 0) issue_slot<LP, LPH, MASKED>(slot / 4, s);
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i)
+                if (slot == i * SLOTS / LOADS) issue_slot<LP, LPH, MASKED>(i, s);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
     template <int LP, int LPH, bool MASKED>
     __device__ __forceinline__ void issue_slot(int i, int64_t s) {
-        // i is a constant after unrolling; the loads of a phase are numbered 0 .. PHASE_LOADS - 1
+        // i is a constant after unrolling
+        auto one = [&](auto tag) {
+            constexpr int I = decltype(tag)::value;
+            if constexpr (I < Pipe::phase_loads(LPH)) Pipe::template issue_one<LP, LPH, I, MASKED>(*this, s);
+        };
         switch (i) {
-            case 0: Pipe::template issue_one<LP, LPH, 0, MASKED>(*this, s); break;
-            case 1: Pipe::template issue_one<LP, LPH, 1, MASKED>(*this, s); break;
-            case 2: Pipe::template issue_one<LP, LPH, 2, MASKED>(*this, s); break;
-            case 3: Pipe::template issue_one<LP, LPH, 3, MASKED>(*this, s); break;
-            case 4: Pipe::template issue_one<LP, LPH, 4, MASKED>(*this, s); break;
-            case 5: Pipe::template issue_one<LP, LPH, 5, MASKED>(*this, s); break;
-            case 6: Pipe::template issue_one<LP, LPH, 6, MASKED>(*this, s); break;
-            default: Pipe::template issue_one<LP, LPH, 7, MASKED>(*this, s); break;
+            case 0: one(std::integral_constant<int, 0>{}); break;
+            case 1: one(std::integral_constant<int, 1>{}); break;
+            case 2: one(std::integral_constant<int, 2>{}); break;
+            case 3: one(std::integral_constant<int, 3>{}); break;
+            case 4: one(std::integral_constant<int, 4>{}); break;
+            case 5: one(std::integral_constant<int, 5>{}); break;
+            case 6: one(std::integral_constant<int, 6>{}); break;
+            case 7: one(std::integral_constant<int, 7>{}); break;
+            case 8: one(std::integral_constant<int, 8>{}); break;
+            default: one(std::integral_constant<int, 9>{}); break;
         }
     }
     // One pipeline step at ring position P on stage s.  On entry the fragments of the stage's first block are in
@@ -445,7 +539,7 @@ struct Kernel {
     // flight the same at every step and lets the compiler see that the loop needs no other wait on vector memory.
     template <int P, bool MASKED>
     __device__ __forceinline__ void step(int64_t s, f32x4_t (&acc)[MI][NI]) {
-        static_assert(Pipe::KK == 2 && Pipe::PHASE_LOADS == 8, "two phases of eight loads");
+        static_assert(Pipe::KK == 2 && Pipe::phase_loads(0) <= 10 && Pipe::phase_loads(1) <= 10, "two phases of up to ten loads");
         phase<P, P, 0, MASKED>(1, 0, s, acc);
         wait_vmcnt_and_lds<Pipe::WAIT>();
         block_barrier();
@@ -501,9 +595,20 @@ struct Kernel {
     }
 };
 
+// What a work-group multiplies.
+struct TilePlace {
+    int expert;
+    int64_t m_begin, m_end;  // the tile's routed rows; MT: the expert's, which are reduced over
+    int64_t i0, n0;          // first row (MT) and column of the result
+    TileWork work;
+};
+
 template <typename T, int KIND, int EPI, typename Pipe>
-__global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmParams P) {
+__device__ __forceinline__ void multiply_tile(const GemmParams& P, const TilePlace& place) {
     using K = Kernel<T, KIND, EPI, Pipe>;
+    using TL = typename Pipe::TL;
+    constexpr int BM = TL::BM, BN = TL::BN, WM = TL::WM, WN = TL::WN, MI = TL::MI, NI = TL::NI;
+    constexpr int OUT_SLABS = TL::OUT_SLABS, SLAB_BLOCKS = TL::SLAB_BLOCKS;
     constexpr int PV = 8;
     constexpr int BN_OUT = K::BN_OUT;
 
@@ -511,59 +616,12 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
     K k;
     k.lane = tid & 63;
     k.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-    int row_tile, col_tile;
-    int tile_expert = 0;
-    int64_t m_begin, m_end, tile_i0 = 0, n0;
-    TileWork work;
-    work.parts = 1;
-    if constexpr (KIND == XMA_GEMM_MT) {
-        if (!locate_tile<true>(P.row_tiles_max * P.num_experts, P.col_tiles, row_tile, col_tile)) return;
-    } else {
-        // the row tiles present and this one's rows: from the table, or from the offsets when there is none
-        const bool table = P.tile_count != nullptr;
-        const RowTileScan tiles(P.offsets, table ? 0 : P.num_experts, BM, k.lane);
-        const int64_t stages = (P.k + K::BK - 1) / K::BK;
-        if (!locate_work(table ? P.tile_count[0] : tiles.total, P.col_tiles, P.num_cu, stages, work)) return;
-        row_tile = work.row_tile;
-        col_tile = work.col_tile;
-        int32_t row0, row_end;
-        if (table) {
-            tile_expert = P.tile_expert[row_tile];
-            row0 = P.tile_row0[row_tile];
-            const int32_t last = P.offsets[tile_expert + 1];
-            row_end = last - row0 > BM ? row0 + BM : last;
-        } else {
-            tiles.find(row_tile, tile_expert, row0, row_end);
-        }
-        m_begin = row0;
-        m_end = row_end;
-    }
-
+    const int expert = place.expert;
+    const int64_t m_begin = place.m_begin, m_end = place.m_end, tile_i0 = place.i0, n0 = place.n0;
+    const TileWork& work = place.work;
+    k.red_len = KIND == XMA_GEMM_MT ? m_end - m_begin : P.k;
     const T* A = reinterpret_cast<const T*>(P.a);
     const T* B = reinterpret_cast<const T*>(P.b);
-
-    int expert;
-    if constexpr (KIND == XMA_GEMM_MT) {
-        const int slot = row_tile / P.row_tiles_max;
-        tile_i0 = (int64_t)(row_tile % P.row_tiles_max) * BM;
-        if (P.expert_order != nullptr) {  // experts in descending order of their row counts
-            const int32_t* record = P.expert_order + 4 * slot;
-            expert = record[0];
-            m_begin = record[1];
-            m_end = record[2];
-        } else {
-            expert = slot;
-            m_begin = P.offsets[expert];
-            m_end = P.offsets[expert + 1];
-        }
-        k.red_len = m_end - m_begin;
-        n0 = (int64_t)col_tile * BN;
-    } else {
-        expert = tile_expert;
-        k.red_len = P.k;
-        n0 = (int64_t)col_tile * BN_OUT;
-    }
 
     // ---- operand load plans ----
     if constexpr (KIND == XMA_GEMM_MT) {
@@ -648,7 +706,7 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
             // atomics are never merged, widened or hoisted across them.
             auto part_buffer = [&](int part) {
                 return reinterpret_cast<uint64_t*>(P.split_partials +
-                                                   (int64_t)(part * work.split_tiles + work.split_tile) * kSplitTileFloats);
+                                                   (int64_t)(part * work.split_tiles + work.split_tile) * split_tile_floats(BN));
             };
             uint64_t* mine = part_buffer(work.part);
 #pragma unroll
@@ -663,7 +721,7 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
                     }
             wait_vmcnt<0>();  // this wave's partial sums have reached memory ...
             __syncthreads();  // ... and so have everybody else's, before the arrival is counted
-            int* arrivals = reinterpret_cast<int*>(slab<0>());
+            int* arrivals = reinterpret_cast<int*>(TL::template slab<0>());
             if (tid == 0)
                 arrivals[0] = __hip_atomic_fetch_add(P.split_counters + work.split_tile, 1, __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_AGENT);
@@ -680,32 +738,32 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
             for (int part = 0; part < work.parts; ++part) {
                 const uint64_t* src = part_buffer(part);
 #pragma unroll
-                for (int m2 = 0; m2 < MI / 2; ++m2) {
-                    uint64_t v[2][NI][2];
+                for (int m2 = 0; m2 < OUT_SLABS; ++m2) {
+                    uint64_t v[SLAB_BLOCKS][NI][2];
 #pragma unroll
-                    for (int h = 0; h < 2; ++h)
+                    for (int h = 0; h < SLAB_BLOCKS; ++h)
 #pragma unroll
                         for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
                             for (int g = 0; g < 2; ++g)
-                                v[h][ni][g] = __hip_atomic_load(src + (((2 * m2 + h) * NI + ni) * 2 + g) * THREADS + tid,
+                                v[h][ni][g] = __hip_atomic_load(src + (((SLAB_BLOCKS * m2 + h) * NI + ni) * 2 + g) * THREADS + tid,
                                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     batch_fence();
 #pragma unroll
-                    for (int h = 0; h < 2; ++h)
+                    for (int h = 0; h < SLAB_BLOCKS; ++h)
 #pragma unroll
                         for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
                             for (int g = 0; g < 2; ++g) pin(v[h][ni][g]);
 #pragma unroll
-                    for (int h = 0; h < 2; ++h)
+                    for (int h = 0; h < SLAB_BLOCKS; ++h)
 #pragma unroll
                         for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
                             for (int g = 0; g < 2; ++g) {
                                 const float2 f = __builtin_bit_cast(float2, v[h][ni][g]);
-                                acc[2 * m2 + h][ni][2 * g] += f.x;
-                                acc[2 * m2 + h][ni][2 * g + 1] += f.y;
+                                acc[SLAB_BLOCKS * m2 + h][ni][2 * g] += f.x;
+                                acc[SLAB_BLOCKS * m2 + h][ni][2 * g + 1] += f.y;
                             }
                     batch_fence();
                 }
@@ -713,15 +771,16 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
         }
     }
 
-    // ---- epilogue: accumulators -> LDS (slab mi holds the 64 tile rows {wr*128 + mi*32 + 0..31}) -> HBM ----
+    // ---- epilogue: accumulators -> LDS (slab mi holds the 64 tile rows of each wave row from mi * SLAB_ROWS / 2) -> HBM ----
     // Store phase: each thread owns one 16-byte chunk column (cc) and, per slab, the IT buffer rows
     // tid / 32 + 8 * it.  What the rows need from HBM (scatter indices, the saved pre-activation of the
     // activation backward) is requested in batches before it is used: the indices of all four slabs before the
     // accumulators are packed (and waited for after that), a slab's pre-activations one slab ahead.
     T* C = reinterpret_cast<T*>(P.c);
-    constexpr int C_CHUNKS = BN / PV;             // 32
-    constexpr int ROW_STEP = THREADS / C_CHUNKS;  // 8
-    constexpr int IT = 64 / ROW_STEP;             // 8
+    constexpr int C_CHUNKS = BN / PV;             // 32 or 16
+    constexpr int ROW_STEP = THREADS / C_CHUNKS;  // 8 or 16
+    constexpr int SLAB_ROWS = 32 * SLAB_BLOCKS;   // buffer rows of a slab, half of them of each wave row
+    constexpr int IT = SLAB_ROWS / ROW_STEP;      // 8, 4 or 2
     // Per-lane coordinates are derived from a fresh, opaque copy of the thread index: derived from `tid` they
     // would be the values computed before the main loop, which the compiler then keeps in scratch memory
     // across the loop and reloads in the middle of the epilogue's batched requests.
@@ -733,10 +792,10 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
     const int cc = etid & (C_CHUNKS - 1);
     const int r0 = (etid / C_CHUNKS) & (ROW_STEP - 1);
     auto buffer_row = [&](int it) { return r0 + it * ROW_STEP; };
-    // tile row of buffer row r0 + 8 * it of slab mi, less r0: buffer rows 0..31 are tile rows mi*32 + 0..31, buffer
-    // rows 32..63 the same rows of the lower wave row (+128)
-    auto row_base = [](int mi, int it) { return (it >> 2) * 128 + mi * 32 + (it & 3) * ROW_STEP; };
-    const int rows_here = (int)(m_end - m_begin);  // 1..256
+    // tile row of buffer row r0 + ROW_STEP * it of slab mi, less r0: the upper half of the buffer rows are tile
+    // rows from mi * SLAB_ROWS / 2, the lower half the same rows of the lower wave row (+WM)
+    auto row_base = [](int mi, int it) { return TL::block_row(it / (IT / 2), mi * SLAB_BLOCKS) + (it % (IT / 2)) * ROW_STEP; };
+    const int rows_here = (int)(m_end - m_begin);  // 1..BM
     auto row_exists = [&](int mi, int it) { return r0 < rows_here - row_base(mi, it); };
     // a row of the tile that exists: the wanted one or, past the end, the last one
     auto safe_row = [&](int mi, int it) {
@@ -784,15 +843,14 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
     if constexpr (SWBWD) load_saved(0, hu[0], hg[0]);
 
     // MFMA result register r of lane l in block (mi, ni): tile row 16*mi + l%16, tile column 16*ni + 4*(l/16) + r.
-    // Slab s holds the tile rows {wr*128 + s*32 + 0..31} of both wave rows as buffer rows wr*32 + 0..31, i.e. the
-    // blocks mi = 2s and 2s+1.  A 512-byte LDS row holds 32 chunks of 8 columns; chunk c of buffer row br sits at
-    // c ^ (br & 31).
+    // Slab s holds the blocks mi = SLAB_BLOCKS * s + h of both wave rows wr as buffer rows wr * SLAB_ROWS / 2 + 16 * h + 0..15.  An LDS row holds C_CHUNKS chunks of 8 columns; chunk c of buffer row br sits at
+    // c ^ (br % C_CHUNKS).
     {
         const int wn0 = (k.wave % WAVES_N) * WN;
-        const int br0 = (k.wave / WAVES_N) * 32 + (etid & 15);  // buffer row of the even block of a slab
+        const int br0 = (k.wave / WAVES_N) * (SLAB_ROWS / 2) + (etid & 15);  // buffer row of the first block of a slab
         const int quarter = (etid >> 4) & 3;
         // Forward kinds: the expert's bias row, added to the fp32 sums before they are rounded.  Tile column c is
-        // weight row n0 + c, or for a gated tile n0 + c (c < 128) and N/2 + n0 + c - 128 (c >= 128).
+        // weight row n0 + c, or for a gated tile n0 + c (c < BN/2) and N/2 + n0 + c - BN/2 (c >= BN/2).
         float bias[KIND == XMA_GEMM_TN ? NI : 1][KIND == XMA_GEMM_TN ? 4 : 1];
         bool with_bias = false;
         if constexpr (KIND == XMA_GEMM_TN) {
@@ -823,15 +881,16 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
         // (the bias is a copy of the code of its own: a wave alone on its SIMD pays for every instruction, and as
         // one copy the compiler adds a selected zero to every sum of a launch that has no bias)
         auto write_rows = [&](char* buf, const f32x4_t (&even)[NI], const f32x4_t (&odd)[NI], auto bias_tag) {
+            // (a slab of one block has no odd one)
             constexpr bool BIAS = decltype(bias_tag)::value;
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
+            for (int h = 0; h < SLAB_BLOCKS; ++h) {
                 const int br = br0 + 16 * h;
 #pragma unroll
                 for (int ni = 0; ni < NI; ++ni) {
                     const f32x4_t& a = h == 0 ? even[ni] : odd[ni];
                     const int c = wn0 + ni * 16 + 4 * quarter;
-                    const int chunk = (c >> 3) ^ (br & 31);
+                    const int chunk = (c >> 3) ^ (br & (C_CHUNKS - 1));
                     float v[4] = {a[0], a[1], a[2], a[3]};
                     if constexpr (BIAS) {
 #pragma unroll
@@ -843,10 +902,10 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
             }
         };
         auto write_all = [&](auto bias_tag) {
-            write_rows(slab<0>(), acc[0], acc[1], bias_tag);
-            write_rows(slab<1>(), acc[2], acc[3], bias_tag);
-            write_rows(slab<2>(), acc[4], acc[5], bias_tag);
-            write_rows(slab<3>(), acc[6], acc[7], bias_tag);
+            write_rows(TL::template slab<0>(), acc[0], acc[SLAB_BLOCKS - 1], bias_tag);
+            if constexpr (OUT_SLABS >= 2) write_rows(TL::template slab<1>(), acc[2], acc[3], bias_tag);
+            if constexpr (OUT_SLABS >= 3) write_rows(TL::template slab<2>(), acc[4], acc[5], bias_tag);
+            if constexpr (OUT_SLABS >= 4) write_rows(TL::template slab<3>(), acc[6], acc[7], bias_tag);
         };
         if (KIND == XMA_GEMM_TN && with_bias) write_all(std::true_type{});
         else write_all(std::false_type{});
@@ -863,7 +922,7 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
     auto store_rows = [&](const char* buf, auto mi_tag, const int32_t (&out_row)[IT]) {
         constexpr int mi = decltype(mi_tag)::value;
         auto chunk_at = [&](int br, int c) {
-            return *reinterpret_cast<const u32x4_t*>(buf + br * (BN * 2) + ((c ^ (br & 31)) << 4));
+            return *reinterpret_cast<const u32x4_t*>(buf + br * (BN * 2) + ((c ^ (br & (C_CHUNKS - 1))) << 4));
         };
         auto to_uint4 = [](const u32x4_t& v) { return make_uint4(v[0], v[1], v[2], v[3]); };
         // the thread's chunk of each of its IT rows of the slab, requested together
@@ -910,9 +969,9 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
                         __builtin_nontemporal_store(v[it], reinterpret_cast<u32x4_t*>(C + (int64_t)out_row[it] * P.ldc + n));
             }
         } else if constexpr (EPI == EPI_PAIRED) {
-            // The slab row holds 16 chunks of the up half, then the 16 matching chunks of the gate half.  Thread
-            // cc handles chunk pair cc % 16 on every other owned row (even `it` for cc < 16, odd otherwise), so
-            // that every lane computes.
+            // The slab row holds the chunks of the up half, then the matching chunks of the gate half.  Thread cc
+            // handles chunk pair cc % HALF_CHUNKS on every other owned row (even `it` for cc < HALF_CHUNKS, odd
+            // otherwise), so that every lane computes.
             constexpr int HALF_CHUNKS = C_CHUNKS / 2;
             const int64_t half_n = P.n / 2;
             const int pair = cc % HALF_CHUNKS;
@@ -987,10 +1046,62 @@ __global__ __launch_bounds__(THREADS) void grouped_gemm_dma_kernel(const GemmPar
             else rows(std::integral_constant<int, ACT_GELU_TANH>{});
         }
     };
-    store_rows(slab<0>(), std::integral_constant<int, 0>{}, orow[0]);
-    store_rows(slab<1>(), std::integral_constant<int, 1>{}, orow[1]);
-    store_rows(slab<2>(), std::integral_constant<int, 2>{}, orow[2]);
-    store_rows(slab<3>(), std::integral_constant<int, 3>{}, orow[3]);
+    store_rows(TL::template slab<0>(), std::integral_constant<int, 0>{}, orow[0]);
+    if constexpr (OUT_SLABS >= 2) store_rows(TL::template slab<1>(), std::integral_constant<int, 1>{}, orow[1]);
+    if constexpr (OUT_SLABS >= 3) store_rows(TL::template slab<2>(), std::integral_constant<int, 2>{}, orow[2]);
+    if constexpr (OUT_SLABS >= 4) store_rows(TL::template slab<3>(), std::integral_constant<int, 3>{}, orow[3]);
+}
+
+template <typename T, int KIND, int EPI, int BM, int BN>
+__global__ __launch_bounds__(THREADS, groups_per_cu(BN)) void grouped_gemm_dma_kernel(const GemmParams P) {
+    TilePlace place;
+    place.i0 = 0;
+    place.work.parts = 1;
+    if constexpr (KIND == XMA_GEMM_MT) {
+        int row_tile, col_tile;
+        if (!locate_tile<true>(P.row_tiles_max * P.num_experts, P.col_tiles, row_tile, col_tile)) return;
+        const int slot = row_tile / P.row_tiles_max;
+        place.i0 = (int64_t)(row_tile % P.row_tiles_max) * BM;
+        if (P.expert_order != nullptr) {  // experts in descending order of their row counts
+            const int32_t* record = P.expert_order + 4 * slot;
+            place.expert = record[0];
+            place.m_begin = record[1];
+            place.m_end = record[2];
+        } else {
+            place.expert = slot;
+            place.m_begin = P.offsets[slot];
+            place.m_end = P.offsets[slot + 1];
+        }
+        place.n0 = (int64_t)col_tile * BN;
+    } else {
+        // the row tiles present and this one's rows: from the table, or from the offsets when there is none
+        const bool table = P.tile_count != nullptr;
+        const RowTileScan tiles(P.offsets, table ? 0 : P.num_experts, P.tile_rows, threadIdx.x & 63);
+        const int64_t stages = (P.k + 63) / 64;
+        TileWork& work = place.work;
+        if (!locate_work(table ? P.tile_count[0] : tiles.total, P.col_tiles, P.round_tiles, stages, work)) return;
+        int32_t row0, row_end;
+        if (table) {
+            place.expert = P.tile_expert[work.row_tile];
+            row0 = P.tile_row0[work.row_tile];
+            const int32_t last = P.offsets[place.expert + 1];
+            row_end = last - row0 > P.tile_rows ? row0 + P.tile_rows : last;
+        } else {
+            tiles.find(work.row_tile, place.expert, row0, row_end);
+        }
+        place.m_begin = row0;
+        place.m_end = row_end;
+        place.n0 = (int64_t)work.col_tile * (EPI == EPI_PAIRED ? BN / 2 : BN);
+    }
+    if constexpr (BN == 256 || KIND == XMA_GEMM_MT) {
+        multiply_tile<T, KIND, EPI, Ring64x5<Tile<BM, BN>>>(P, place);
+    } else {
+        const int64_t rows = place.m_end - place.m_begin;
+        if (rows > 128) multiply_tile<T, KIND, EPI, Ring64x2<Tile<BM, BN>>>(P, place);
+        else if (rows > 64) multiply_tile<T, KIND, EPI, Ring64x2<Tile<128, BN>>>(P, place);
+        else if (rows > 32) multiply_tile<T, KIND, EPI, Ring64x2<Tile<64, BN>>>(P, place);
+        else multiply_tile<T, KIND, EPI, Ring64x2<Tile<32, BN>>>(P, place);
+    }
 }
 
 // Compute units of the current device, rounded down to a multiple of the XCD count and capped at the
@@ -1038,10 +1149,11 @@ static __global__ __launch_bounds__(1024) void build_expert_order_kernel(const i
 
 static __global__ void clear_split_counters_kernel(int32_t* counters) { counters[threadIdx.x] = 0; }
 
-template <typename T, int KIND, int EPI, typename Pipe>
-static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
+template <typename T, int KIND, int EPI, int BM, int BN>
+static int launch(const xma_grouped_gemm_args& a, int tile_rows, hipStream_t stream) {
     GemmParams P;
     fill_params(a, P);
+    P.tile_rows = tile_rows;
     int64_t grid;
     if (KIND == XMA_GEMM_MT) {
         P.row_tiles_max = (int32_t)ceil_div(a.n, BM);
@@ -1054,45 +1166,42 @@ static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
             P.expert_order = records;
         }
     } else {
-        const int64_t rt = max_row_tiles(a.rows, a.num_experts, BM);
+        const int64_t rt = max_row_tiles(a.rows, a.num_experts, tile_rows);
         P.row_tiles_max = (int32_t)rt;
         // the split-K region is the tail of the workspace
         char* split = reinterpret_cast<char*>(a.workspace) +
                       (xma_grouped_gemm_workspace_bytes(a.num_experts, a.rows) - split_region_bytes());
         P.split_counters = reinterpret_cast<int32_t*>(split);
         P.split_partials = reinterpret_cast<float*>(split + kSplitSlots * sizeof(int32_t));
-        P.num_cu = compute_units();
+        P.round_tiles = compute_units() * groups_per_cu(BN);
         const int bn_out = EPI == EPI_PAIRED ? BN / 2 : BN;
         const int64_t n_out = EPI == EPI_PAIRED ? a.n / 2 : a.n;
         P.col_tiles = (int32_t)ceil_div(n_out, bn_out);
-        grid = grid_for_work(rt * P.col_tiles);
+        grid = grid_for_work(rt * P.col_tiles, P.round_tiles);
         if (a.num_experts > kMaxScannedExperts) {
-            launch_build_row_tiles(a, BM, rt, P, stream);
+            launch_build_row_tiles(a, tile_rows, rt, P, stream);
         } else if (may_split(a.k)) {
             hipLaunchKernelGGL(clear_split_counters_kernel, dim3(1), dim3(kSplitSlots), 0, stream, P.split_counters);
         }
     }
     XMA_REQUIRE(grid < ((int64_t)1 << 31), "xma_grouped_gemm: %lld tiles exceed the grid limit", (long long)grid);
-    hipLaunchKernelGGL((grouped_gemm_dma_kernel<T, KIND, EPI, Pipe>), dim3((unsigned)grid), dim3(THREADS), 0, stream, P);
+    hipLaunchKernelGGL((grouped_gemm_dma_kernel<T, KIND, EPI, BM, BN>), dim3((unsigned)grid), dim3(THREADS), 0, stream, P);
     return check_launch("xma_grouped_gemm");
 }
 
-template <typename T>
-static int dispatch(const xma_grouped_gemm_args& a, hipStream_t stream) {
-    using PipeTN = Ring64x5;
-    using PipeNN = Ring64x5;
-    using PipeMT = Ring64x5;
+template <typename T, int BM, int BN>
+static int dispatch(const xma_grouped_gemm_args& a, int tile_rows, hipStream_t stream) {
     int shape = EPI_PLAIN, act = ACT_NONE;
     split_epilogue(a.epilogue, shape, act);
     switch (a.kind) {
         case XMA_GEMM_TN:
-            if (shape == EPI_PAIRED) return launch<T, XMA_GEMM_TN, EPI_PAIRED, PipeTN>(a, stream);
-            return launch<T, XMA_GEMM_TN, EPI_PLAIN, PipeTN>(a, stream);
+            if (shape == EPI_PAIRED) return launch<T, XMA_GEMM_TN, EPI_PAIRED, BM, BN>(a, tile_rows, stream);
+            return launch<T, XMA_GEMM_TN, EPI_PLAIN, BM, BN>(a, tile_rows, stream);
         case XMA_GEMM_NN:
-            if (shape == EPI_BACKWARD) return launch<T, XMA_GEMM_NN, EPI_BACKWARD, PipeNN>(a, stream);
-            return launch<T, XMA_GEMM_NN, EPI_PLAIN, PipeNN>(a, stream);
+            if (shape == EPI_BACKWARD) return launch<T, XMA_GEMM_NN, EPI_BACKWARD, BM, BN>(a, tile_rows, stream);
+            return launch<T, XMA_GEMM_NN, EPI_PLAIN, BM, BN>(a, tile_rows, stream);
         default:
-            return launch<T, XMA_GEMM_MT, EPI_PLAIN, PipeMT>(a, stream);
+            return launch<T, XMA_GEMM_MT, EPI_PLAIN, BN, BN>(a, tile_rows, stream);
     }
 }
 
@@ -1106,8 +1215,123 @@ bool dma_gemm_supports(const xma_grouped_gemm_args& a) {
     return true;
 }
 
+// ---- which tile a call takes ----------------------------------------------------------------------------------------
+//
+// 256 x 256 tiles have a compute unit each: the fewest bytes of operands per operation, but nothing overlaps what a tile
+// does outside its main loop, an expert's last rows cost a whole tile, and a launch with few tiles leaves compute units
+// idle.  Tiles of up to 192 x 128 run two on a compute unit, so that one's set-up and stores run under the other's main
+// loop, and an expert's last rows take a tile of 32, 64, 128 or 192 rows; per operation they ask the L2 for two thirds more.
+//
+// Row-grouped kinds: the time of both forms is estimated from the tiles that experts of 0.9, 1 and 1.1 times the mean
+// number of rows have, in rounds of the device, at the measured cost of a round (us; K in units of 1024):
+//   256 x 256: 10 + 24 K (24 + 24 K with an activation's backward), a partly filled last round costs a whole one or is
+//     split along the reduction;
+//   192, 128, 64, 32 x 128, two per compute unit: 3.5 (10) + 24, 18.6, 13, 10 K.
+// Measured with the L2 and the caches as the benchmark's layers leave them (us, 256 x 256 / up to 192 / up to 128 rows):
+//   16384 tokens, H 2048, I 1024, 64 experts, 6 each: up 784 / 857 / 902, dX 755 / 819 / 858
+//   3000 tokens of the same layer: 228 / 205 / 244 and 217 / 186 / 228; 800 tokens: 143 / 133 / 132 and 114 / 110 / 112
+//   1531 tokens, H 2048, I 768, 128 experts, 8 each, skewed: up 107 / 102 / 99, down 71 / 58 / 57, dX 127 / 106 / 104
+//   3001 tokens, H 512, I 1024, 6 experts, 4 each: up 49 / 42 / 37, down 28 / 23 / 20, dact 41 / 38 / 34, dX 48 / 38 / 30
+//   1000 tokens, H 1024, I 4096, 16 experts, 2 each: up 68 / 60 / 71, down 61 / 40 / 43, dX 98 / 83 / 91
+//   8192 tokens, H 4096, I 14336, 8 experts, 2 each: up 3082 / 3832 / 4256, down 1427 / 1876 / 2146
+// The smaller tiles are taken where they are expected to gain more than the estimate is sure of (7 %).  Over 28 such layers
+// its choices come within 3 % of the fastest of the three; it is wrong by up to a quarter where the
+// experts' rows all lie a little above a multiple of 192 (3000 tokens, 128 experts, 8 each: down 121 / 149).
+//
+// Weight gradients: tiles of 128 x 128 where 256 x 256 fill the device less than twice, or where the reductions (the rows of
+// an expert) are short: 3001 tokens as above 45 / 22 and 50 / 32 us; 8000
+// tokens, H 512, I 576, 32 experts, 4 each (320 tiles of 256 x 256) 58 / 46; 800 tokens of the 64 experts 95 / 82 and 178 / 159,
+// 3000 tokens (281 rows each) 133 / 125 and 253 / 241, 6000 tokens (562 rows each) 178 / 178 and 346 / 392.
+namespace {
+
+constexpr double kSpread[3] = {0.9, 1.0, 1.1};
+
+struct SmallTile {
+    int rows;
+    double per_1024;
+};
+constexpr SmallTile kSmallTiles[] = {{32, 10.0}, {64, 13.0}, {128, 18.6}, {192, 24.0}};
+
+const SmallTile& small_tile_for(double rows) {
+    int i = 0;
+    while (i < 3 && rows > kSmallTiles[i].rows) ++i;
+    return kSmallTiles[i];
+}
+
+double estimate_256(double rows, int64_t experts, int64_t col_tiles, double k1024, bool backward) {
+    double tiles = 0;
+    for (double f : kSpread) tiles += (rows * f < 1 ? rows * f : (double)(int64_t)((rows * f + 255) / 256)) / 3;
+    const double set_up = backward ? 24 : 10, loop = 24 * k1024;
+    const double rounds = tiles * experts * col_tiles / 256;
+    const int64_t full = (int64_t)rounds;
+    const double rest = rounds - full;
+    if (full > 0 && rest < 0.02) return full * (set_up + loop);
+    double parts = 1;
+    if (rounds < kSplitMaxRounds) {
+        parts = (int)(1 / rest < kMaxSplit ? 1 / rest : kMaxSplit);
+        if (parts > k1024 * 16 / kSplitMinStages) parts = (int)(k1024 * 16 / kSplitMinStages);
+        if (parts < 1) parts = 1;
+    }
+    return (full + 1) * set_up + full * loop + loop / parts + (parts > 1 ? 25 : 0);
+}
+
+double estimate_small(double rows, int64_t experts, int64_t col_tiles, double k1024, bool backward, const SmallTile& tallest) {
+    const double set_up = backward ? 10 : 3.5;
+    auto cost = [&](const SmallTile& t) { return set_up * t.rows / 192 + t.per_1024 * k1024; };
+    double tiles = 0, work = 0;
+    for (double f : kSpread) {
+        const double r = rows * f;
+        const int64_t whole = (int64_t)(r / tallest.rows);
+        const double rest = r - (double)whole * tallest.rows;
+        tiles += (whole + (rest > 0)) / 3.0;
+        work += (whole * cost(tallest) + (rest > 0 ? cost(small_tile_for(rest)) : 0)) / 3;
+    }
+    tiles *= (double)experts * col_tiles;
+    work *= (double)experts * col_tiles / 512;
+    const double one = cost(rows >= tallest.rows ? tallest : small_tile_for(rows));
+    const double rounds = work / one;
+    const int64_t full = (int64_t)rounds;
+    const double rest = rounds - full;
+    if (tiles <= 256) {  // fewer than one per compute unit, or split along the reduction
+        double parts = (int)(512 / (tiles < 1 ? 1 : tiles));
+        if (parts > kMaxSplit) parts = kMaxSplit;
+        if (parts > k1024 * 16 / kSplitMinStages) parts = (int)(k1024 * 16 / kSplitMinStages);
+        if (parts >= 2) return (tiles * parts > 256 ? 1.0 : 0.55) * one / parts + 12;
+        return 4 + 0.55 * one;
+    }
+    return full * one + (rest < 0.02 ? 0 : rest <= 0.5 ? 4 + 0.55 * one : one);
+}
+
+}  // namespace
+
+DmaTile dma_gemm_tile(const xma_grouped_gemm_args& a) {
+    const double rows = (double)a.rows / a.num_experts;
+    if (a.kind == XMA_GEMM_MT) {
+        const int64_t tiles = a.num_experts * ceil_div(a.n, 256) * ceil_div(a.k, 256);
+        return tiles < 512 || rows < 448 ? DmaTile{128, 128} : DmaTile{256, 256};
+    }
+    int shape = EPI_PLAIN, act = ACT_NONE;
+    split_epilogue(a.epilogue, shape, act);
+    const double k1024 = (double)a.k / 1024;
+    const bool backward = shape == EPI_BACKWARD;
+    auto estimate = [&](const SmallTile& t) {
+        return estimate_small(rows, a.num_experts, ceil_div(a.n, 128), k1024, backward, t);
+    };
+    const double big = estimate_256(rows, a.num_experts, ceil_div(a.n, 256), k1024, backward);
+    const double tall = estimate(kSmallTiles[3]), flat = estimate(kSmallTiles[2]);
+    if (big < 1.07 * (tall < flat ? tall : flat)) return DmaTile{256, 256};
+    return tall <= flat ? DmaTile{192, 128} : DmaTile{128, 128};
+}
+
+template <typename T>
+static int launch_tiles(const xma_grouped_gemm_args& a, hipStream_t stream) {
+    const DmaTile tile = dma_gemm_tile(a);
+    return tile.cols == 256 ? dma::dispatch<T, 256, 256>(a, tile.rows, stream)
+                            : dma::dispatch<T, 192, 128>(a, tile.rows, stream);
+}
+
 int launch_dma_gemm(const xma_grouped_gemm_args& a, hipStream_t stream) {
-    return a.dtype == XMA_BF16 ? dma::dispatch<bf16_t>(a, stream) : dma::dispatch<f16_t>(a, stream);
+    return a.dtype == XMA_BF16 ? launch_tiles<bf16_t>(a, stream) : launch_tiles<f16_t>(a, stream);
 }
 
 }  // namespace xma

@@ -319,7 +319,8 @@ int xma_grouped_gemm(const xma_grouped_gemm_args* args, void* stream);
 
 /*
  * Which kernel xma_grouped_gemm would take for these arguments (enum xma_gemm_form; sizes, strides, types, alignments and
- * whether pointers are null are looked at, nothing is read or launched), and the rows and columns of its largest tile.
+ * whether pointers are null are looked at, nothing is read or launched), and the rows and columns of its largest tile
+ * (of XMA_FORM_TILED in 16 bits: of any call; xma_grouped_gemm_tile tells what this one takes).
  * The streaming kernel's columns are weight rows.  For tests and for reading profiles.
  */
 enum xma_gemm_form {
@@ -329,6 +330,9 @@ enum xma_gemm_form {
     XMA_FORM_TILED = 3        /* LDS-DMA tiles */
 };
 int xma_grouped_gemm_form(const xma_grouped_gemm_args* args, int32_t* kernel, int32_t* tile_rows, int32_t* tile_cols);
+
+/* Rows and columns of the tallest tile of the launch that xma_grouped_gemm would make for these arguments. */
+int xma_grouped_gemm_tile(const xma_grouped_gemm_args* args, int32_t* tile_rows, int32_t* tile_cols);
 
 #ifdef __cplusplus
 }
