@@ -201,6 +201,17 @@ __device__ __forceinline__ T wave_sum(T v) {
     return v;
 }
 
+// Inclusive prefix sum over the 64 lanes of a wave (data-parallel moves: no LDS round trips).
+__device__ __forceinline__ int32_t wave_inclusive_sum(int32_t v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1, missing lanes read 0
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // index loads that accept int32 or int64 tables
 __device__ __forceinline__ int64_t load_index(const void* table, int is_i64, int64_t i) {
     return is_i64 ? reinterpret_cast<const int64_t*>(table)[i]

@@ -195,17 +195,6 @@ constexpr int kSmallestTileRows = 32;  // of any kernel that may use a table of 
 inline int64_t max_row_tiles(int64_t rows, int E, int BM) { return rows / BM + E; }
 
 // ---- row tiles without a table ---------------------------------------------------------------------------------
-// Inclusive prefix sum over the 64 lanes of a wave (data-parallel moves: no LDS round trips).
-__device__ __forceinline__ int32_t wave_inclusive_sum(int32_t v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1, missing lanes read 0
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
-    return v;
-}
-
 // Expert e owns ceil(count_e / bm) consecutive row tiles.  How many there are and which expert and rows a tile has, found
 // by each wave on its own from the offsets: lane l adds up the tiles of the l-th run of consecutive experts, one prefix
 // sum over the lanes.  Costs a load and some thirty instructions, against a launch of its own (3-6 us and the gap

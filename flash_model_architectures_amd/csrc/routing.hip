@@ -677,79 +677,69 @@ __global__ __launch_bounds__(256) void scan_place_kernel(const IdT* __restrict__
 // scans the column totals into the expert offsets, and the two are added up: row w, column e is then the first
 // output slot of wave w's ids of expert e; (3) every wave walks its run again in order and ranks equal ids inside
 // each 64-wide batch with ballots, as place_kernel does.  No workspace, no other launch.
+// What it spends is latency, barriers above all: the scan is one prefix sum over the lanes of each wave and one barrier, and
+// batches without ids are stepped over (a run is kSingleBatches batches at most, one or none in the smallest calls).
+// us, with a scan through LDS of 1024 slots in twenty barriers and sixteen batches for every wave / so: 6 ids x 64 experts
+// 13.8 / 2.8, 256 x 128 15.3 / 3.1, 2048 x 8 11.2 / 3.9, 4096 x 64 15.0 / 5.9 (4097 x 64 in two launches: 7.8).
+constexpr int kSingleBatches = (int)(kSingleBlockSortIds / 1024);
 template <typename IdT, typename OutT>
 __global__ __launch_bounds__(1024) void route_single_block_kernel(const IdT* __restrict__ ids, int64_t n, int E,
                                                                    int nbits, uint32_t* __restrict__ counts,
                                                                    int32_t* __restrict__ offsets,
                                                                    OutT* __restrict__ sorted_ids,
                                                                    OutT* __restrict__ perm) {
-    extern __shared__ uint32_t lds_hist[];  // [16 waves][E], then [1024] for the scan
+    extern __shared__ uint32_t lds_hist[];  // [16 waves][E], then the totals of 16 waves' experts
     constexpr int kWaves = 1024 / kWaveSize;
-    uint32_t* part = lds_hist + kWaves * E;
-    const int wave = threadIdx.x / kWaveSize;
+    uint32_t* wave_total = lds_hist + kWaves * E;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int lane = lane_id();
+    const int per = (((int)n + kWaves - 1) / kWaves + kWaveSize - 1) / kWaveSize * kWaveSize;  // ids per wave
+    const int begin = wave * per < (int)n ? wave * per : (int)n;
+    const int end = begin + per < (int)n ? begin + per : (int)n;
+    int64_t v[kSingleBatches];  // requested before the first barrier, kept for the placement
+    load_chunk(ids, begin, end, lane, v);
     for (int i = threadIdx.x; i < kWaves * E; i += 1024) lds_hist[i] = 0;
     __syncthreads();
 
-    const int64_t per = ((n + kWaves - 1) / kWaves + kWaveSize - 1) / kWaveSize * kWaveSize;  // ids per wave
-    const int64_t begin = wave * per < n ? wave * per : n;
-    const int64_t end = begin + per < n ? begin + per : n;
     uint32_t* mine = lds_hist + wave * E;
-    int64_t v[kBatches];  // the wave's first chunk stays in registers for the placement
-    load_chunk(ids, begin, end, lane, v);
 #pragma unroll
-    for (int j = 0; j < kBatches; ++j)
+    for (int j = 0; j < kSingleBatches; ++j)
         if (v[j] >= 0 && v[j] < E) atomicAdd(&mine[v[j]], 1u);
-    for (int64_t c0 = begin + kChunk; c0 < end; c0 += kChunk) {
-        int64_t u[kBatches];
-        load_chunk(ids, c0, end, lane, u);
-#pragma unroll
-        for (int j = 0; j < kBatches; ++j)
-            if (u[j] >= 0 && u[j] < E) atomicAdd(&mine[u[j]], 1u);
-    }
     __syncthreads();
 
     // column e: exclusive prefixes over the waves, total -> counts
     const int e_mine = threadIdx.x;
-    uint32_t total = 0;
+    uint32_t before[kWaves], total = 0;
     if (e_mine < E) {
 #pragma unroll
+        for (int w = 0; w < kWaves; ++w) before[w] = lds_hist[w * E + e_mine];
+#pragma unroll
         for (int w = 0; w < kWaves; ++w) {
-            const uint32_t c = lds_hist[w * E + e_mine];
-            lds_hist[w * E + e_mine] = total;
+            const uint32_t c = before[w];
+            before[w] = total;
             total += c;
         }
         counts[e_mine] = total;
     }
-    // exclusive scan of the totals over the experts (Hillis-Steele over 1024 slots)
-    part[threadIdx.x] = total;
+    // exclusive scan of the totals over the experts
+    const uint32_t upto = (uint32_t)wave_inclusive_sum((int32_t)total);
+    if (lane == kWaveSize - 1) wave_total[wave] = upto;
     __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
-        const uint32_t v = threadIdx.x >= d ? part[threadIdx.x - d] : 0;
-        __syncthreads();
-        part[threadIdx.x] += v;
-        __syncthreads();
-    }
-    const uint32_t first_slot = part[threadIdx.x] - total;
+    uint32_t first_slot = upto - total;
+    for (int w = 0; w < wave && w * kWaveSize < E; ++w) first_slot += wave_total[w];
     if (e_mine < E) {
         offsets[e_mine] = (int32_t)first_slot;
+        if (e_mine == E - 1) offsets[E] = (int32_t)(first_slot + total);
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) lds_hist[w * E + e_mine] += first_slot;
+        for (int w = 0; w < kWaves; ++w) lds_hist[w * E + e_mine] = first_slot + before[w];
     }
-    if (threadIdx.x == 1023) offsets[E] = (int32_t)part[1023];
     __syncthreads();
 
     // placement, stable inside the wave's run and across the runs
-    uint32_t* next = mine;
 #pragma unroll
-    for (int j = 0; j < kBatches; ++j)
-        place_batch(v[j], begin + j * kWaveSize + lane, E, nbits, lane, next, sorted_ids, perm);
-    for (int64_t c0 = begin + kChunk; c0 < end; c0 += kChunk) {
-        load_chunk(ids, c0, end, lane, v);
-#pragma unroll
-        for (int j = 0; j < kBatches; ++j)
-            place_batch(v[j], c0 + j * kWaveSize + lane, E, nbits, lane, next, sorted_ids, perm);
-    }
+    for (int j = 0; j < kSingleBatches; ++j)
+        if (begin + j * kWaveSize < end)
+            place_batch(v[j], begin + j * kWaveSize + lane, E, nbits, lane, mine, sorted_ids, perm);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1016,7 +1006,7 @@ static int route_build_launch(const void* ids, int ids_is_i64, int64_t n, int32_
     }
     const int nbits = ceil_log2(E);
     if (n <= kSingleBlockSortIds && E <= kSingleBlockBins) {  // one launch, no workspace
-        const size_t lds_one = ((size_t)E * (1024 / kWaveSize) + 1024) * sizeof(uint32_t);
+        const size_t lds_one = (size_t)(E + 1) * (1024 / kWaveSize) * sizeof(uint32_t);
 #define XMA_ROUTE_ONE(IdT, OutT)                                                                                     \
     hipLaunchKernelGGL((route_single_block_kernel<IdT, OutT>), dim3(1), dim3(1024), lds_one, stream, (const IdT*)ids, \
                        n, (int)E, nbits, counts, offsets, (OutT*)sorted_ids, (OutT*)perm)
