@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from ctypes import POINTER, c_char_p, c_int, c_int32, c_int64, c_void_p
 
 import torch
@@ -59,6 +60,10 @@ class GroupedGemmArgs(ctypes.Structure):
         ("ld_bias", c_int64),
     ]
 
+
+# struct xma_moe_args: struct_size, dtype, epilogue, num_experts, top_k, reserved, three sizes, 18 fields that both directions
+# or the forward one read (the workspace's size the last of them), ten of the backward one
+MOE_ARGS = struct.Struct("=I5i3q17Qq10Q")
 
 # name -> (restype, argtypes); must list every symbol include/xma_hip.h declares
 PROTOTYPES: dict[str, tuple] = {
@@ -175,6 +180,9 @@ PROTOTYPES: dict[str, tuple] = {
     "xma_grouped_gemm_workspace_bytes": (c_int64, [c_int32, c_int64]),
     "xma_grouped_gemm": (c_int, [POINTER(GroupedGemmArgs), c_void_p]),
     "xma_grouped_gemm_form": (c_int, [POINTER(GroupedGemmArgs), c_void_p, c_void_p, c_void_p]),
+    "xma_moe_workspace_bytes": (c_int64, [c_int64, c_int32, c_int32]),
+    "xma_moe_forward": (c_int, [c_char_p, c_void_p]),
+    "xma_moe_backward": (c_int, [c_char_p, c_void_p]),
     "xma_grouped_gemm_tile": (c_int, [POINTER(GroupedGemmArgs), c_void_p, c_void_p]),
 }
 
@@ -246,6 +254,10 @@ _timeline: Timeline | None = None
 def set_timeline(timeline: Timeline | None) -> None:
     global _timeline
     _timeline = timeline
+
+
+def timeline_active() -> bool:
+    return _timeline is not None
 
 
 def call(name: str, *args, tag: str | None = None, flops: float = 0.0, nbytes: float = 0.0) -> None:

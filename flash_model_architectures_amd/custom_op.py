@@ -175,6 +175,28 @@ def apply_function(function: type[torch.autograd.Function], *args) -> Any:
     return function.apply(*args)
 
 
+def plain_calls(operators: Iterable[Callable], tensors: Iterable[torch.Tensor | None]) -> bool:
+    """True when calls of these `direct_xma_op` operators with these tensors would all be direct, so that one native call may
+    stand for them."""
+
+    if not _eager():
+        return False
+    grad = torch.is_grad_enabled()
+    plain = _plain_keys() if torch.cuda.is_initialized() else None
+    for value in tensors:
+        if value is None:
+            continue
+        if plain is None or type(value) not in _TENSORS or not value.is_cuda or (grad and value.requires_grad):
+            return False
+        if _dispatch_keys(value).raw_repr() not in (plain.normal, plain.inference):
+            return False
+    for operator in operators:
+        others_registered = getattr(operator, "_others_registered", None)
+        if others_registered is None or others_registered():
+            return False
+    return True
+
+
 def direct_xma_op(mutates_args: Iterable[str]) -> Callable:
     """`xma_op` for the package's own operators, with a short way past the dispatcher.
 
@@ -253,6 +275,7 @@ def direct_xma_op(mutates_args: Iterable[str]) -> Callable:
         call.__name__ = op.__name__
         call.__doc__ = op.__doc__
         call._custom_op = op._custom_op
+        call._others_registered = others_registered
         return call
 
     return decorator

@@ -21,7 +21,7 @@ import torch
 import torch.nn as nn
 
 from ..accelerator import KernelBackend, resolve_backend
-from ..custom_op import apply_function
+from ..custom_op import _eager, apply_function
 from ..functional.routing import route_tokens, topk_softmax
 from ..functional.swiglu_packed import swiglu_packed
 from ..ops import (
@@ -33,6 +33,8 @@ from ..ops import (
     group,
     group_bwd_W,
     invert_index,
+    layer_backward,
+    layer_forward,
     router_weight_grad,
     scatter2scatter,
     spread_rows,
@@ -238,13 +240,26 @@ class _FusedExperts(torch.autograd.Function):
     [E, 2I or I, H] and [E, H, I]."""
 
     @staticmethod
-    def forward(ctx, x, w_up, w_down, gates, sorted_scattered_idxs, expert_offsets, b_up, b_down, activation):
+    def forward(ctx, x, w_up, w_down, gates, selected, sorted_scattered_idxs, expert_offsets, b_up, b_down, activation):
+        """`sorted_scattered_idxs` and `expert_offsets` are the selection's routing, or both None: it is built here."""
+
         T, H = x.shape
         E, N, _ = w_up.shape
         I = w_down.size(2)
         k = gates.size(1)
         M = T * k
         needs_grad = any(ctx.needs_input_grad)
+        ctx.activation = activation
+        ctx.has_bias = b_up is not None, b_down is not None
+        if sorted_scattered_idxs is None:
+            done = layer_forward(x, w_up, w_down, b_up, b_down, activation, k, None, gates, selected, needs_grad)
+            if done is not None:
+                y, *saved = done
+                if needs_grad:
+                    ctx.save_for_backward(x, w_up, w_down, gates, *saved)
+                return y
+            routing = route_tokens(selected, E)
+            sorted_scattered_idxs, expert_offsets = routing.sorted_scattered_idxs, routing.expert_offsets
         preact = torch.empty(M, N, device=x.device, dtype=x.dtype) if needs_grad else None
         act = torch.empty(M, I, device=x.device, dtype=x.dtype)
         up_projection_fused(
@@ -275,8 +290,6 @@ class _FusedExperts(torch.autograd.Function):
         combine_topk(expanded=expanded, out=y, k=k, gates=gates)
         if needs_grad:
             ctx.save_for_backward(x, w_up, w_down, gates, sorted_scattered_idxs, expert_offsets, preact, act, expanded)
-        ctx.activation = activation
-        ctx.has_bias = b_up is not None, b_down is not None
         return y
 
     @staticmethod
@@ -288,6 +301,14 @@ class _FusedExperts(torch.autograd.Function):
         M = T * k
         if not grad_out.is_contiguous():  # e.g. the expanded (stride 0) gradient of y.sum() or y.mean(0)
             grad_out = grad_out.contiguous()
+        bias_gradients = ctx.has_bias[0] and ctx.needs_input_grad[7], ctx.has_bias[1] and ctx.needs_input_grad[8]
+
+        done = layer_backward(
+            x, w_up, w_down, gates, idx, expert_offsets, preact, act, expanded, grad_out, ctx.activation, *bias_gradients
+        )
+        if done is not None:
+            d_x, d_w_up, d_w_down, d_gates, d_b_up, d_b_down = done
+            return d_x, d_w_up, d_w_down, d_gates, None, None, None, d_b_up, d_b_down, None
 
         # routed row of every (token, slot): the row moves below walk the tokens
         inverse = torch.empty(M, device=x.device, dtype=torch.int32)
@@ -306,7 +327,7 @@ class _FusedExperts(torch.autograd.Function):
         )
 
         d_b_down = None
-        if ctx.has_bias[1] and ctx.needs_input_grad[7]:
+        if bias_gradients[1]:
             d_b_down = torch.empty(E, H, device=x.device, dtype=x.dtype)
             expert_colsum(src=grouped_grad, expert_offsets=expert_offsets, out=d_b_down)
 
@@ -325,7 +346,7 @@ class _FusedExperts(torch.autograd.Function):
         del grouped_grad  # buffers of routed rows are the largest there are: each is given back after its last reader
 
         d_b_up = None
-        if ctx.has_bias[0] and ctx.needs_input_grad[6]:
+        if bias_gradients[0]:
             d_b_up = torch.empty(E, preact.size(1), device=x.device, dtype=x.dtype)
             expert_colsum(src=d_preact, expert_offsets=expert_offsets, out=d_b_up)
 
@@ -354,7 +375,7 @@ class _FusedExperts(torch.autograd.Function):
         )
         d_x = torch.empty_like(x, memory_format=torch.contiguous_format)
         combine_topk(expanded=d_expanded, out=d_x, k=k, gates=None)
-        return d_x, d_w_up, d_w_down, d_gates, None, None, d_b_up, d_b_down, None
+        return d_x, d_w_up, d_w_down, d_gates, None, None, None, d_b_up, d_b_down, None
 
 
 class Experts(XMAModule):
@@ -519,6 +540,24 @@ class MoE(XMAModule):
         original_shape = hidden_states.shape
         hidden_states = hidden_states.reshape(-1, self.hidden_size)
 
+        if not torch.is_grad_enabled() and self._steps_are_own() and _eager():
+            # one native call for all that follows the gate, where the operators it stands for would be called directly
+            activation = fused_activation_name(self.act, self.is_glu)
+            if activation is not None and kernel_backend in (None, KernelBackend.rocm):
+                router_logits = self.gate(hidden_states)
+                resolve_backend(kernel_backend, "MoE")
+                done = layer_forward(
+                    hidden_states, self.c_fc.weight, self.c_proj.weight, self.c_fc.bias, self.c_proj.bias, activation,
+                    self.top_k, router_logits,
+                )  # fmt: skip
+                if done is not None:
+                    return done[0].view(original_shape), router_logits
+                router_weights, selected_experts = topk_softmax(router_logits, self.top_k, kernel_backend=kernel_backend)
+                hidden_states = self._compute_experts(
+                    hidden_states, router_weights, selected_experts, kernel_backend=kernel_backend
+                )
+                return hidden_states.view(original_shape), router_logits
+
         router_logits, router_weights, selected_experts = self._compute_routing_weights(
             hidden_states, kernel_backend=kernel_backend
         )
@@ -526,6 +565,17 @@ class MoE(XMAModule):
             hidden_states, router_weights, selected_experts, kernel_backend=kernel_backend
         )
         return hidden_states.view(original_shape), router_logits
+
+    def _steps_are_own(self) -> bool:
+        """False when a subclass or a patched instance has steps of its own, which then are called."""
+
+        own = type(self)
+        return (
+            own._compute_routing_weights is MoE._compute_routing_weights
+            and own._compute_experts is MoE._compute_experts
+            and "_compute_routing_weights" not in self.__dict__
+            and "_compute_experts" not in self.__dict__
+        )
 
     def _compute_routing_weights(
         self, hidden_states: torch.Tensor, *, kernel_backend: KernelBackend | None = None
@@ -544,10 +594,10 @@ class MoE(XMAModule):
     ) -> torch.Tensor:
         resolve_backend(kernel_backend, "MoE")
 
-        routing = route_tokens(selected_experts, self.num_experts)
-
         # biases: torch path only in the reference (xma/layers/moe/__init__.py:54,79,104); here both pipelines take them
         activation = fused_activation_name(self.act, self.is_glu)
+        # (a plain call of the fused pipeline builds the routing with its other launches)
+        routing = None if activation is not None and _eager() else route_tokens(selected_experts, self.num_experts)
         if activation is not None:
             return apply_function(
                 _FusedExperts,
@@ -555,8 +605,9 @@ class MoE(XMAModule):
                 self.c_fc.weight,
                 self.c_proj.weight,
                 router_weights,
-                routing.sorted_scattered_idxs,
-                routing.expert_offsets,
+                selected_experts,
+                None if routing is None else routing.sorted_scattered_idxs,
+                None if routing is None else routing.expert_offsets,
                 self.c_fc.bias,
                 self.c_proj.bias,
                 activation,

@@ -19,7 +19,7 @@ import ctypes
 import torch
 
 from . import _native as nat
-from .custom_op import direct_xma_op
+from .custom_op import direct_xma_op, plain_calls
 
 
 def _i64(t: torch.Tensor | None) -> int:
@@ -914,3 +914,180 @@ def down_projection_dgrad_fused(
         aux=preact,
         ld_aux=_row_stride(preact),
     )
+
+
+# ------------------------------------------------------------------------------------------------
+# every launch of the experts of a layer from one native call
+# ------------------------------------------------------------------------------------------------
+# The operators that a native call stands for.  (Between two launches of a small layer the host spends 10-20 us in Python.
+# Operators one by one / one call: one decoded token, H 2048, I 1024, 64 experts, 6 each, 126 / 62 us; a full-precision forward
+# pass of 1024 tokens, H 256, I 512, 131 / 64; a training step of 3001 tokens, H 512, I 1024, 610 / 427.)
+_FORWARD_OPERATORS = (route_build_rocm, up_projection_fused, scatter2scatter, combine_topk)
+_SELECTION_OPERATORS = (topk_softmax_rocm, *_FORWARD_OPERATORS)
+_BACKWARD_OPERATORS = (
+    invert_index, spread_rows_gate_grad, spread_rows, expert_colsum, group_bwd_W, down_projection_dgrad_fused, scatter2scatter,
+    combine_topk,
+)  # fmt: skip
+
+
+def _layer_sizes(x, w_up, w_down, b_up, b_down, activation: str) -> tuple[int, int, int, int, int] | None:
+    """(T, H, N, I, E) of a layer whose tensors are all contiguous, of one type and of sizes that belong together; None: the
+    operators judge."""
+
+    if x.dim() != 2 or w_up.dim() != 3 or w_down.dim() != 3 or x.dtype not in nat.DTYPE_CODE:
+        return None
+    T, H = x.shape
+    E, N, _ = w_up.shape
+    I = w_down.size(2)
+    if N != (2 * I if FUSED_ACTIVATIONS[activation][2] else I) or min(T, H, I, E) < 1:
+        return None
+    if w_up.size(2) != H or w_down.shape != (E, H, I):
+        return None
+    for t, shape in ((x, None), (w_up, None), (w_down, None), (b_up, (E, N)), (b_down, (E, H))):
+        if t is not None and (t.dtype != x.dtype or not t.is_contiguous() or (shape is not None and t.shape != shape)):
+            return None
+    return T, H, N, I, E
+
+
+def layer_forward(
+    x: torch.Tensor,
+    w_up: torch.Tensor,
+    w_down: torch.Tensor,
+    b_up: torch.Tensor | None,
+    b_down: torch.Tensor | None,
+    activation: str,
+    k: int,
+    logits: torch.Tensor | None = None,
+    gates: torch.Tensor | None = None,
+    selected: torch.Tensor | None = None,
+    keep: bool = False,
+) -> tuple | None:
+    """The experts of a layer, from the router's logits or from the selection already made: (y, perm, expert_offsets, preact,
+    act, expanded), of which only y is there unless `keep`.  None when the operators have to be called one by one: when
+    something observes or transforms them, or for tensors that are not contiguous."""
+
+    if nat.timeline_active():
+        return None
+    operators = _FORWARD_OPERATORS if logits is None else _SELECTION_OPERATORS
+    if not plain_calls(operators, (x, w_up, w_down, b_up, b_down, logits, gates, selected)):
+        return None
+    sizes = _layer_sizes(x, w_up, w_down, b_up, b_down, activation)
+    if sizes is None:
+        return None
+    T, H, N, I, E = sizes
+    M, device, dtype = T * k, x.device, x.dtype
+    if k < 1 or k > E:
+        return None
+    if logits is not None:
+        if logits.shape != (T, E) or logits.dtype != dtype or not logits.is_contiguous():
+            return None
+    elif (
+        gates.shape != (T, k)
+        or selected.shape != (T, k)
+        or gates.dtype != dtype
+        or selected.dtype != torch.int64
+        or not gates.is_contiguous()
+        or not selected.is_contiguous()
+    ):
+        return None
+
+    size = x.element_size()
+    y = torch.empty(T, H, device=device, dtype=dtype)
+    # counts, offsets, experts of the routed rows, permutation: one buffer, each part on a multiple of 256 bytes
+    e_words, m_words = (E + 64) // 64 * 64, (M + 63) // 64 * 64
+    words = 2 * e_words + 2 * m_words
+    preact = act = expanded = None
+    if keep:
+        table = torch.empty(words, device=device, dtype=torch.int32)
+        preact = torch.empty(M, N, device=device, dtype=dtype)
+        act = torch.empty(M, I, device=device, dtype=dtype)
+        expanded = torch.empty(M, H, device=device, dtype=dtype)
+        base, act_ptr, expanded_ptr, preact_ptr = table.data_ptr(), act.data_ptr(), expanded.data_ptr(), preact.data_ptr()
+        end = 0
+    else:  # everything goes with the call: one buffer
+        act_at = (4 * words + 255) // 256 * 256
+        expanded_at = act_at + (M * I * size + 255) // 256 * 256
+        end = expanded_at + (M * H * size + 255) // 256 * 256
+        table = torch.empty(end + (0 if logits is None else (M * size + 255) // 256 * 256 + 8 * M), device=device, dtype=torch.uint8)
+        base = table.data_ptr()
+        act_ptr, expanded_ptr, preact_ptr = base + act_at, base + expanded_at, 0
+    offsets_at, experts_at, perm_at = e_words, 2 * e_words, 2 * e_words + m_words
+    if logits is None:
+        logits_ptr, gates_ptr, selected_ptr = 0, gates.data_ptr(), selected.data_ptr()
+    else:
+        assert not keep
+        logits_ptr, gates_ptr = logits.data_ptr(), base + end
+        selected_ptr = gates_ptr + (M * size + 255) // 256 * 256
+    lib = nat.load()
+    workspace = _workspace(device, lib.xma_moe_workspace_bytes(T, E, k))
+    args = nat.MOE_ARGS.pack(
+        nat.MOE_ARGS.size, nat.DTYPE_CODE[dtype], FUSED_ACTIVATIONS[activation][0], E, k, 0, T, H, I,
+        x.data_ptr(), w_up.data_ptr(), w_down.data_ptr(), gates_ptr, base + 4 * offsets_at, base + 4 * perm_at,
+        preact_ptr, act_ptr, expanded_ptr,
+        logits_ptr, selected_ptr, base, base + 4 * experts_at,
+        0 if b_up is None else b_up.data_ptr(), 0 if b_down is None else b_down.data_ptr(),
+        y.data_ptr(), workspace.data_ptr(), workspace.numel(),
+        0, 0, 0, 0, 0, 0, 0, 0, 0, 0,
+    )  # fmt: skip
+    if lib.xma_moe_forward(args, nat.stream()) != 0:
+        raise RuntimeError(f"xma_moe_forward failed: {nat.last_error()}")
+    if not keep:
+        return y, None, None, None, None, None
+    return y, table[perm_at : perm_at + M], table[offsets_at : offsets_at + E + 1], preact, act, expanded
+
+
+def layer_backward(
+    x: torch.Tensor,
+    w_up: torch.Tensor,
+    w_down: torch.Tensor,
+    gates: torch.Tensor,
+    perm: torch.Tensor,
+    expert_offsets: torch.Tensor,
+    preact: torch.Tensor,
+    act: torch.Tensor,
+    expanded: torch.Tensor,
+    d_y: torch.Tensor,
+    activation: str,
+    with_b_up: bool,
+    with_b_down: bool,
+) -> tuple | None:
+    """(d_x, d_w_up, d_w_down, d_gates, d_b_up, d_b_down) of `layer_forward`, or None as there."""
+
+    if nat.timeline_active():
+        return None
+    if not plain_calls(_BACKWARD_OPERATORS, (x, w_up, w_down, gates, perm, expert_offsets, preact, act, expanded, d_y)):
+        return None
+    sizes = _layer_sizes(x, w_up, w_down, None, None, activation)
+    if sizes is None:
+        return None
+    T, H, N, I, E = sizes
+    k = gates.size(1)
+    M, device, dtype = T * k, x.device, x.dtype
+    for t, shape, kind in (
+        (gates, (T, k), dtype), (perm, (M,), torch.int32), (expert_offsets, (E + 1,), torch.int32), (preact, (M, N), dtype),
+        (act, (M, I), dtype), (expanded, (M, H), dtype), (d_y, (T, H), dtype),
+    ):  # fmt: skip
+        if t.shape != shape or t.dtype != kind or not t.is_contiguous():
+            return None
+
+    def empty(*shape):
+        return torch.empty(shape, device=device, dtype=dtype)
+
+    d_x, d_w_up, d_w_down, d_gates = empty(T, H), empty(E, N, H), empty(E, H, I), empty(T, k)
+    d_b_up, d_b_down = empty(E, N) if with_b_up else None, empty(E, H) if with_b_down else None
+    d_preact, rows = empty(M, N), empty(M, H)
+    inverse = torch.empty(M, device=device, dtype=torch.int32)
+    lib = nat.load()
+    workspace = _workspace(device, lib.xma_moe_workspace_bytes(T, E, k))
+    args = nat.MOE_ARGS.pack(
+        nat.MOE_ARGS.size, nat.DTYPE_CODE[dtype], FUSED_ACTIVATIONS[activation][0], E, k, 0, T, H, I,
+        x.data_ptr(), w_up.data_ptr(), w_down.data_ptr(), gates.data_ptr(), expert_offsets.data_ptr(), perm.data_ptr(),
+        preact.data_ptr(), act.data_ptr(), expanded.data_ptr(),
+        0, 0, 0, 0, 0, 0, 0, workspace.data_ptr(), workspace.numel(),
+        d_y.data_ptr(), d_x.data_ptr(), d_gates.data_ptr(), d_w_up.data_ptr(), d_w_down.data_ptr(),
+        0 if d_b_up is None else d_b_up.data_ptr(), 0 if d_b_down is None else d_b_down.data_ptr(),
+        d_preact.data_ptr(), rows.data_ptr(), inverse.data_ptr(),
+    )  # fmt: skip
+    if lib.xma_moe_backward(args, nat.stream()) != 0:
+        raise RuntimeError(f"xma_moe_backward failed: {nat.last_error()}")
+    return d_x, d_w_up, d_w_down, d_gates, d_b_up, d_b_down

@@ -334,6 +334,55 @@ int xma_grouped_gemm_form(const xma_grouped_gemm_args* args, int32_t* kernel, in
 /* Rows and columns of the tallest tile of the launch that xma_grouped_gemm would make for these arguments. */
 int xma_grouped_gemm_tile(const xma_grouped_gemm_args* args, int32_t* tile_rows, int32_t* tile_cols);
 
+/*
+ * The experts of an MoE layer with one of the fused activations, every launch of a pass from one call: the entry points
+ * above in the order of the layer, with the same results.  All tensors are contiguous; T tokens of H, E experts, k per token,
+ * M = T * k routed rows, I intermediate, N = 2 * I for the gated activations and I for tanh-GELU.
+ */
+typedef struct xma_moe_args {
+    uint32_t struct_size; /* sizeof(xma_moe_args) */
+    int32_t dtype;        /* enum xma_dtype of every floating-point tensor */
+    int32_t epilogue;     /* XMA_EPI_SWIGLU, XMA_EPI_GLU or XMA_EPI_GELU_TANH */
+    int32_t num_experts;
+    int32_t top_k;
+    int32_t reserved; /* 0 */
+    int64_t tokens, hidden, intermediate;
+    /* both directions */
+    const void* x;      /* [T, H] */
+    const void* w_up;   /* [E, N, H] */
+    const void* w_down; /* [E, H, I] */
+    void* gates;        /* [T, k] routing weights: an output of the forward direction when `logits` is given */
+    int32_t* expert_offsets; /* [E + 1] */
+    int32_t* perm;      /* [M] grouped position -> scattered position */
+    void* preact;       /* [M, N]; forward: NULL when nothing is kept for backward */
+    void* act;          /* [M, I] */
+    void* expanded;     /* [M, H] down-projected rows in scattered order */
+    /* forward */
+    const void* logits; /* [T, E] or NULL: the selection is made here */
+    int64_t* selected;  /* [T, k] chosen experts, an output when `logits` is given */
+    uint32_t* counts;   /* [E] */
+    int32_t* sorted_experts; /* [M] */
+    const void* b_up;   /* [E, N] or NULL */
+    const void* b_down; /* [E, H] or NULL */
+    void* y;            /* [T, H] */
+    void* workspace;    /* xma_moe_workspace_bytes(T, E, k) bytes, both directions */
+    int64_t workspace_bytes;
+    /* backward */
+    const void* d_y;    /* [T, H] */
+    void* d_x;          /* [T, H] */
+    void* d_gates;      /* [T, k] */
+    void* d_w_up;       /* [E, N, H] */
+    void* d_w_down;     /* [E, H, I] */
+    void* d_b_up;       /* [E, N] or NULL */
+    void* d_b_down;     /* [E, H] or NULL */
+    void* d_preact;     /* [M, N] scratch */
+    void* rows;         /* [M, H] scratch */
+    int32_t* inverse;   /* [M] scratch */
+} xma_moe_args;
+int64_t xma_moe_workspace_bytes(int64_t tokens, int32_t num_experts, int32_t top_k);
+int xma_moe_forward(const xma_moe_args* args, void* stream);
+int xma_moe_backward(const xma_moe_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,145 @@
+"""The experts of a layer from one native call: the same results, bit for bit, as the operators one by one, and the operators
+whenever a call is not a plain one."""
+
+import pytest
+import torch
+import torch.nn as nn
+from torch.utils._python_dispatch import TorchDispatchMode
+
+import flash_model_architectures_amd as xma
+from flash_model_architectures_amd import _native, ops
+
+
+ACTIVATIONS = {
+    "swiglu": (xma.swiglu_packed, True),
+    "glu": (nn.GLU(), True),
+    "gelu_tanh": (nn.GELU(approximate="tanh"), False),
+}
+
+
+def _layer(dtype, activation="swiglu", bias=False, experts=6, k=4, hidden=136, intermediate=72):
+    torch.manual_seed(0)
+    function, is_glu = ACTIVATIONS[activation]
+    layer = xma.MoE(experts, k, hidden, intermediate, function, is_glu, bias, 0.05)
+    if bias:
+        with torch.no_grad():
+            layer.c_fc.bias.normal_()
+            layer.c_proj.bias.normal_()
+    return layer.to("cuda").to(dtype)
+
+
+def _train(layer, x, dy):
+    layer.zero_grad(set_to_none=True)
+    x = x.detach().requires_grad_()
+    y, logits = layer(x)
+    y.backward(dy)
+    return [y.detach(), logits.detach(), x.grad, *(p.grad for p in layer.parameters())]
+
+
+class _Calls:
+    """Native entry points called, in order."""
+
+    def __init__(self, monkeypatch, one_by_one=False):
+        self.names = []
+        real = _native.load()
+        calls = self
+
+        class Library:
+            def __getattr__(self, name):
+                if name in ("xma_moe_forward", "xma_moe_backward"):
+                    calls.names.append(name)
+                return getattr(real, name)
+
+        monkeypatch.setattr(_native, "_lib", Library())
+        if one_by_one:
+            monkeypatch.setattr(_native, "_timeline", _native.Timeline())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("activation", list(ACTIVATIONS))
+@pytest.mark.parametrize("tokens,sizes", [(1, {}), (67, {}), (300, dict(k=1)), (40, dict(hidden=33, intermediate=21))])
+def test_same_results(tokens, sizes, activation, bias, dtype, monkeypatch):
+    layer = _layer(dtype, activation, bias, **sizes)
+    x = torch.randn(tokens, layer.hidden_size, device="cuda", dtype=dtype)
+    dy = torch.randn_like(x)
+    results = {}
+    for one_by_one in (False, True):
+        with monkeypatch.context() as patch:
+            calls = _Calls(patch, one_by_one)
+            with torch.no_grad():
+                forward = layer(x)
+            results[one_by_one] = [*forward, *_train(layer, x, dy)]
+            assert calls.names == ([] if one_by_one else ["xma_moe_forward", "xma_moe_forward", "xma_moe_backward"])
+    for a, b in zip(results[False], results[True]):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_calls_that_are_not_plain(monkeypatch):
+    layer = _layer(torch.bfloat16)
+    x = torch.randn(50, layer.hidden_size, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        want = layer(x)[0]
+
+    class Seen(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_dispatch__(self, function, types, args=(), kwargs=None):
+            self.names.append(str(function))
+            return function(*args, **(kwargs or {}))
+
+    calls = _Calls(monkeypatch)
+    with torch.no_grad(), Seen() as seen:
+        assert torch.equal(layer(x)[0], want)
+    assert any("topk_softmax" in name for name in seen.names) and any("up_projection" in name for name in seen.names)
+    assert calls.names == []
+
+    # a step that a program has replaced is called
+    replaced = []
+
+    def routing(hidden_states, *, kernel_backend=None):
+        replaced.append(hidden_states.shape)
+        return xma.MoE._compute_routing_weights(layer, hidden_states, kernel_backend=kernel_backend)
+
+    layer._compute_routing_weights = routing
+    with torch.no_grad():
+        assert torch.equal(layer(x)[0], want)
+    assert replaced == [x.shape]
+    del layer._compute_routing_weights
+
+    # weights that are views of other storage
+    storage = layer.c_fc.weight.detach().transpose(1, 2).contiguous()
+    layer.c_fc.weight = nn.Parameter(storage.transpose(1, 2))
+    calls.names.clear()
+    with torch.no_grad():
+        with pytest.raises(AssertionError):
+            layer(x)  # as the operator has always judged such weights
+    assert calls.names == []
+
+
+@pytest.mark.gpu
+def test_inference_mode_and_streams():
+    layer = _layer(torch.bfloat16)
+    x = torch.randn(50, layer.hidden_size, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        want = layer(x)[0]
+    with torch.inference_mode():
+        assert torch.equal(layer(x.clone())[0], want)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.no_grad(), torch.cuda.stream(side):
+        on_side = [layer(x)[0] for _ in range(3)]
+    torch.cuda.current_stream().wait_stream(side)
+    assert all(torch.equal(y, want) for y in on_side)
+
+
+@pytest.mark.gpu
+def test_bad_arguments_are_refused():
+    args = _native.MOE_ARGS.pack(8, *[0] * (5 + 3 + 17 + 1 + 10))
+    assert _native.load().xma_moe_forward(args, 0) != 0 and "bad args" in _native.last_error()
+    args = _native.MOE_ARGS.pack(_native.MOE_ARGS.size, 0, ops.nat.EPI_SWIGLU, 4, 2, 0, 1, 8, 8, *[0] * (17 + 1 + 10))
+    assert _native.load().xma_moe_backward(args, 0) != 0 and "null pointer" in _native.last_error()
