@@ -40,53 +40,85 @@ __global__ __launch_bounds__(256) void add_expert_bias_kernel(T* __restrict__ y,
     }
 }
 
-// Block (x = column block of 32 chunks, y = expert): 32 row lanes walk the expert's rows in order, each
-// keeps fp32 partial sums of its chunk, the lanes are added in lane order through LDS.  The order of the
-// additions is fixed, so the result is reproducible.
-template <typename T, bool VEC>
+// Block (x = column block of CL chunks, y = expert): 1024 / CL row lanes walk the expert's rows in order, four in flight, and
+// keep fp32 partial sums of their chunk; the lanes are added through LDS in lane order.  The order of the additions is
+// fixed, so the result is reproducible.
+// Few experts are few blocks, and a block waits for memory: with 32 chunks, one row in flight and the 32 lanes added up by
+// one of them, 12004 rows of 512 and 1024 columns over 6 experts in 16 bits took 13 and 39 us; so 5.5 and 12.6.
+template <typename T, bool VEC, int CL>
 __global__ __launch_bounds__(1024) void expert_colsum_kernel(const T* __restrict__ src, int64_t ld,
                                                               const int32_t* __restrict__ offsets,
                                                               T* __restrict__ out, int64_t ld_out, int64_t cols) {
     constexpr int PV = VEC ? Elem<T>::kPerVec : 1;
-    __shared__ float part[32][32 * PV + 1];
-    const int cl = threadIdx.x % 32, rl = threadIdx.x / 32;
+    constexpr int RL = 1024 / CL, COLS = CL * PV, IN_FLIGHT = 4;
+    constexpr int GROUPS = 1024 / COLS < RL ? 1024 / COLS : RL, PER_GROUP = RL / GROUPS;
+    __shared__ float part[RL][COLS + 1];
+    const int cl = threadIdx.x % CL, rl = threadIdx.x / CL;
     const int e = blockIdx.y;
-    const int64_t chunk = (int64_t)blockIdx.x * 32 + cl;
+    const int64_t chunk = (int64_t)blockIdx.x * CL + cl;
     const int64_t chunks = cols / PV;
     const int64_t begin = offsets[e], end = offsets[e + 1];
     float acc[PV];
 #pragma unroll
     for (int q = 0; q < PV; ++q) acc[q] = 0.0f;
     if (chunk < chunks) {
-        for (int64_t r = begin + rl; r < end; r += 32) {
+        const T* column = src + chunk * PV;
+        int64_t r = begin + rl;
+        for (; r + (IN_FLIGHT - 1) * RL < end; r += IN_FLIGHT * RL) {
+            if constexpr (VEC) {
+                uint4 v[IN_FLIGHT];
+#pragma unroll
+                for (int i = 0; i < IN_FLIGHT; ++i) v[i] = load_stream(column + (r + i * RL) * ld);
+#pragma unroll
+                for (int i = 0; i < IN_FLIGHT; ++i) {
+                    float a[PV];
+                    Elem<T>::unpack(v[i], a);
+#pragma unroll
+                    for (int q = 0; q < PV; ++q) acc[q] += a[q];
+                }
+            } else {
+                float v[IN_FLIGHT];
+#pragma unroll
+                for (int i = 0; i < IN_FLIGHT; ++i) v[i] = Elem<T>::load(column + (r + i * RL) * ld);
+#pragma unroll
+                for (int i = 0; i < IN_FLIGHT; ++i) acc[0] += v[i];
+            }
+        }
+        for (; r < end; r += RL) {
             if constexpr (VEC) {
                 float a[PV];
-                Elem<T>::unpack(load_stream(src + r * ld + chunk * PV), a);
+                Elem<T>::unpack(load_stream(column + r * ld), a);
 #pragma unroll
                 for (int q = 0; q < PV; ++q) acc[q] += a[q];
             } else {
-                acc[0] += Elem<T>::load(src + r * ld + chunk);
+                acc[0] += Elem<T>::load(column + r * ld);
             }
         }
     }
 #pragma unroll
     for (int q = 0; q < PV; ++q) part[rl][cl * PV + q] = acc[q];
     __syncthreads();
-    if (rl == 0 && chunk < chunks) {
-        float total[PV];
+    const int c = threadIdx.x % COLS, group = threadIdx.x / COLS;
+    if (group < GROUPS) {
+        float sum = 0.0f;
 #pragma unroll
-        for (int q = 0; q < PV; ++q) total[q] = 0.0f;
-        for (int i = 0; i < 32; ++i)
+        for (int i = 0; i < PER_GROUP; ++i) sum += part[group * PER_GROUP + i][c];
+        part[group * PER_GROUP][c] = sum;
+    }
+    __syncthreads();
+    const int64_t column = (int64_t)blockIdx.x * COLS + c;
+    if (group == 0 && column < cols) {
+        float total = 0.0f;
 #pragma unroll
-            for (int q = 0; q < PV; ++q) total[q] += part[i][cl * PV + q];
-        T* dst = out + (int64_t)e * ld_out + chunk * PV;
-        if constexpr (VEC) {
-            *reinterpret_cast<uint4*>(dst) = Elem<T>::pack(total);
-        } else {
-            Elem<T>::store(dst, total[0]);
-        }
+        for (int g = 0; g < GROUPS; ++g) total += part[g * PER_GROUP][c];
+        Elem<T>::store(out + (int64_t)e * ld_out + column, total);
     }
 }
+
+// Narrow blocks, with four times as many row lanes each, while the wide ones are fewer than one to a compute unit.  us, wide /
+// narrow: 16384 rows of 4096 columns, 8 experts (128 wide blocks) 45 / 25; 98304 x 2048, 64 experts (512) 65 / 74;
+// 131072 x 1536, 128 experts (768) 64 / 78; 16384 x 28672, 8 experts (896) 151 / 165.
+constexpr int64_t kWideColsumBlocks = 256;
 
 }  // namespace xma
 
@@ -135,11 +167,16 @@ int xma_expert_colsum(const void* src, int64_t ld, const int32_t* expert_offsets
         const bool vec = aligned16(src) && aligned16(out) && ld % Elem<T_>::kPerVec == 0 &&
                          ld_out % Elem<T_>::kPerVec == 0 && cols % Elem<T_>::kPerVec == 0;
         const int64_t chunks = vec ? cols / Elem<T_>::kPerVec : cols;
-        const dim3 grid((unsigned)ceil_div(chunks, 32), (unsigned)num_experts), block(1024);
-        if (vec) hipLaunchKernelGGL((expert_colsum_kernel<T_, true>), grid, block, 0, stream, (const T_*)src, ld,
-                                    expert_offsets, (T_*)out, ld_out, cols);
-        else hipLaunchKernelGGL((expert_colsum_kernel<T_, false>), grid, block, 0, stream, (const T_*)src, ld,
-                                expert_offsets, (T_*)out, ld_out, cols))
+        const bool wide = ceil_div(chunks, 32) * num_experts >= kWideColsumBlocks;
+        const dim3 grid((unsigned)ceil_div(chunks, wide ? 32 : 8), (unsigned)num_experts), block(1024);
+#define XMA_COLSUM_LAUNCH(VEC, CL)                                                                                    \
+    hipLaunchKernelGGL((expert_colsum_kernel<T_, VEC, CL>), grid, block, 0, stream, (const T_*)src, ld, expert_offsets, \
+                       (T_*)out, ld_out, cols)
+        if (vec && wide) XMA_COLSUM_LAUNCH(true, 32);
+        else if (vec) XMA_COLSUM_LAUNCH(true, 8);
+        else if (wide) XMA_COLSUM_LAUNCH(false, 32);
+        else XMA_COLSUM_LAUNCH(false, 8))
+#undef XMA_COLSUM_LAUNCH
     return check_launch("xma_expert_colsum");
 }
 
