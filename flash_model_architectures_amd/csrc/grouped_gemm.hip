@@ -647,6 +647,21 @@ static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
     return check_launch("xma_grouped_gemm");
 }
 
+static __global__ void clear_split_counters_kernel(int32_t* counters) { counters[threadIdx.x] = 0; }
+void launch_clear_split_counters(const GemmParams& P, hipStream_t stream) {
+    hipLaunchKernelGGL(clear_split_counters_kernel, dim3(1), dim3(kSplitSlots), 0, stream, P.split_counters);
+}
+
+int compute_units() {
+    // asked of the calling thread's current device on every launch (a host-side attribute lookup)
+    int device = 0, count = 0;
+    if (hipGetDevice(&device) != hipSuccess ||
+        hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count < kNumXcd)
+        count = kSplitSlots;
+    count = count > kSplitSlots ? kSplitSlots : count;
+    return count / kNumXcd * kNumXcd;
+}
+
 void fill_params(const xma_grouped_gemm_args& a, GemmParams& P) {
     P.a = a.a;
     P.b = a.b;

@@ -36,6 +36,7 @@ struct GemmParams {
     int32_t* split_counters;  // [kSplitSlots] arrivals per split tile, zero at launch
     float* split_partials;    // [kSplitSlots][tile] fp32 accumulators of the parts
     int32_t tile_rows;  // rows of the tallest tile (16-bit TN/NN)
+    int32_t most_parts;       // parts of a split tile at most (fp32)
     int32_t round_tiles;      // tiles that run at a time on the whole device, a multiple of kNumXcd
     // MT: experts in descending order of their row counts, one record {expert, first row, end row, 0} per slot;
     // nullptr: slot e is expert e
@@ -131,29 +132,29 @@ __device__ __forceinline__ bool locate_tile(int row_tiles, int col_tiles, int& r
 
 // Row-grouped kinds with split-K of the remainder.  With T tiles on a device that runs C of them at a time (round_tiles: one
 // per compute unit of 256 x 256 tiles, two of the smaller ones) the first floor(T / C) * C tiles fill whole rounds; the
-// R = T mod C tiles of the last round would leave C - R places idle for a whole tile time, so each of them is cut along the reduction into S = min(kMaxSplit, C / R,
-// stages / kSplitMinStages) parts that run side by side.  Only when the launch has fewer than kSplitMaxRounds
-// rounds (the idle units of a last round matter less the more rounds there are), and only while a part keeps
-// kSplitMinStages stages: every part parks a 256 KiB tile of fp32 sums in memory and the last one reads them all
-// back, 40-50 k cycles or about 17 stages of the main loop (measured; reductions of 14336 and 28672 split in three
-// gain 7 % and 5 % of their launches).  Work-groups are dealt per XCD as in
-// locate_tile<false>: XCD x takes the x-th eighth of the whole tiles, then the x-th eighth of the parts
-// (part-major, so neighbours share panels).
+// R = T mod C tiles of the last round would leave C - R places idle for a whole tile time, so each of them is cut along the
+// reduction into min(most_parts, C / R) parts that run side by side.  Only when the launch has fewer than most_rounds rounds
+// (the idle places of a last round matter less the more rounds there are), only for up to most_tiles tiles, and only while a part is worth its exchange
+// (most_parts, which the kernels derive from the reduction): every part parks its fp32 sums in memory and the last one reads
+// them all back.  16-bit kernels: 40-50 k cycles for a 256 x 256 tile, or about 17 stages of the main loop (measured;
+// reductions of 14336 and 28672 split in three gain 7 % and 5 % of their launches), so a part keeps kSplitMinStages stages.
+// Work-groups are dealt per XCD as in locate_tile<false>: XCD x takes the x-th eighth of the whole tiles, then the x-th
+// eighth of the parts (part-major, so neighbours share panels).
 struct TileWork {
     int row_tile, col_tile;
     int part, parts;  // this work-group reduces stages [part * n / parts, (part + 1) * n / parts)
     int split_tile;   // index of the tile among the split ones
     int split_tiles;
 };
-__device__ __forceinline__ bool locate_work(int row_tiles, int col_tiles, int round_tiles, int64_t stages, TileWork& w) {
+__device__ __forceinline__ bool locate_work(int row_tiles, int col_tiles, int round_tiles, int most_parts, int most_rounds,
+                                            int most_tiles, TileWork& w) {
     const int xcd = blockIdx.x % kNumXcd;
     const int local = blockIdx.x / kNumXcd;
     const int total = row_tiles * col_tiles;
     const int whole = total / round_tiles * round_tiles;
     const int rem = total - whole;
-    int parts = rem > 0 && total < kSplitMaxRounds * round_tiles ? round_tiles / rem : 1;
-    parts = parts > kMaxSplit ? kMaxSplit : parts;
-    parts = parts > stages / kSplitMinStages ? (int)(stages / kSplitMinStages) : parts;
+    int parts = rem > 0 && rem <= most_tiles && total < most_rounds * round_tiles ? round_tiles / rem : 1;
+    parts = parts > most_parts ? most_parts : parts;
     parts = parts < 1 ? 1 : parts;
     const int whole_per_xcd = whole / kNumXcd;
     int tile;
@@ -296,7 +297,20 @@ struct Mma<float> {
     }
 };
 
-// a launch splits the tiles of its last round only when a part keeps kSplitMinStages stages
+// Clears P.split_counters, for a launch that may split.
+void launch_clear_split_counters(const GemmParams& P, hipStream_t stream);
+// Compute units of the current device, rounded down to a multiple of the XCD count and capped at the
+// number of split slots (the split-K scheme treats that many tiles as one round).
+int compute_units();
+// The split-K region of the workspace.
+inline void place_split_region(const xma_grouped_gemm_args& a, GemmParams& P) {
+    char* split = reinterpret_cast<char*>(a.workspace) +
+                  (xma_grouped_gemm_workspace_bytes(a.num_experts, a.rows) - split_region_bytes());
+    P.split_counters = reinterpret_cast<int32_t*>(split);
+    P.split_partials = reinterpret_cast<float*>(split + kSplitSlots * sizeof(int32_t));
+}
+
+// a 16-bit launch splits the tiles of its last round only when a part keeps kSplitMinStages stages
 inline bool may_split(int64_t reduction) { return (reduction + 63) / 64 >= 2 * kSplitMinStages; }
 
 // Fills the fields of GemmParams that do not depend on the tile shape.

@@ -1077,9 +1077,12 @@ __global__ __launch_bounds__(THREADS, groups_per_cu(BN)) void grouped_gemm_dma_k
         // the row tiles present and this one's rows: from the table, or from the offsets when there is none
         const bool table = P.tile_count != nullptr;
         const RowTileScan tiles(P.offsets, table ? 0 : P.num_experts, P.tile_rows, threadIdx.x & 63);
-        const int64_t stages = (P.k + 63) / 64;
+        const int most_parts = (int)((P.k + 63) / 64 / kSplitMinStages);
         TileWork& work = place.work;
-        if (!locate_work(table ? P.tile_count[0] : tiles.total, P.col_tiles, P.round_tiles, stages, work)) return;
+        if (!locate_work(table ? P.tile_count[0] : tiles.total, P.col_tiles, P.round_tiles,
+                         most_parts < kMaxSplit ? most_parts : kMaxSplit, kSplitMaxRounds,
+                         kSplitSlots, work))
+            return;
         int32_t row0, row_end;
         if (table) {
             place.expert = P.tile_expert[work.row_tile];
@@ -1102,18 +1105,6 @@ __global__ __launch_bounds__(THREADS, groups_per_cu(BN)) void grouped_gemm_dma_k
         else if (rows > 32) multiply_tile<T, KIND, EPI, Ring64x2<Tile<64, BN>>>(P, place);
         else multiply_tile<T, KIND, EPI, Ring64x2<Tile<32, BN>>>(P, place);
     }
-}
-
-// Compute units of the current device, rounded down to a multiple of the XCD count and capped at the
-// number of split slots (the split-K scheme treats that many tiles as one round).
-static int compute_units() {
-    // asked of the calling thread's current device on every launch (a host-side attribute lookup)
-    int device = 0, count = 0;
-    if (hipGetDevice(&device) != hipSuccess ||
-        hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count < kNumXcd)
-        count = kSplitSlots;
-    count = count > kSplitSlots ? kSplitSlots : count;
-    return count / kNumXcd * kNumXcd;
 }
 
 static __global__ __launch_bounds__(1024) void build_expert_order_kernel(const int32_t* __restrict__ offsets, int E,
@@ -1147,8 +1138,6 @@ static __global__ __launch_bounds__(1024) void build_expert_order_kernel(const i
     }
 }
 
-static __global__ void clear_split_counters_kernel(int32_t* counters) { counters[threadIdx.x] = 0; }
-
 template <typename T, int KIND, int EPI, int BM, int BN>
 static int launch(const xma_grouped_gemm_args& a, int tile_rows, hipStream_t stream) {
     GemmParams P;
@@ -1168,11 +1157,7 @@ static int launch(const xma_grouped_gemm_args& a, int tile_rows, hipStream_t str
     } else {
         const int64_t rt = max_row_tiles(a.rows, a.num_experts, tile_rows);
         P.row_tiles_max = (int32_t)rt;
-        // the split-K region is the tail of the workspace
-        char* split = reinterpret_cast<char*>(a.workspace) +
-                      (xma_grouped_gemm_workspace_bytes(a.num_experts, a.rows) - split_region_bytes());
-        P.split_counters = reinterpret_cast<int32_t*>(split);
-        P.split_partials = reinterpret_cast<float*>(split + kSplitSlots * sizeof(int32_t));
+        place_split_region(a, P);
         P.round_tiles = compute_units() * groups_per_cu(BN);
         const int bn_out = EPI == EPI_PAIRED ? BN / 2 : BN;
         const int64_t n_out = EPI == EPI_PAIRED ? a.n / 2 : a.n;
@@ -1181,7 +1166,7 @@ static int launch(const xma_grouped_gemm_args& a, int tile_rows, hipStream_t str
         if (a.num_experts > kMaxScannedExperts) {
             launch_build_row_tiles(a, tile_rows, rt, P, stream);
         } else if (may_split(a.k)) {
-            hipLaunchKernelGGL(clear_split_counters_kernel, dim3(1), dim3(kSplitSlots), 0, stream, P.split_counters);
+            launch_clear_split_counters(P, stream);
         }
     }
     XMA_REQUIRE(grid < ((int64_t)1 << 31), "xma_grouped_gemm: %lld tiles exceed the grid limit", (long long)grid);

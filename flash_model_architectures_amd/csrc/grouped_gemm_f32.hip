@@ -33,6 +33,15 @@ constexpr int BN = 128, BK = 32, THREADS = 256, WAVES = 4, KK = BK / 8;
 constexpr int kRowBytes = BK * 4;
 constexpr int64_t kFullDeviceTiles = 512;  // two work-groups on every compute unit
 
+// Split of a partly filled last round (see locate_work).  A stage of a 128 x 128 tile takes 3.7 us with two work-groups on a
+// compute unit, so a part of 16 stages (of flatter tiles, as many times more) is already worth an exchange of 64 KiB, and a
+// last round matters up to many rounds.  A last round of more tiles than half the compute units is left alone: a work-group
+// that has a compute unit to itself runs almost at the rate of two.  8192 rows, 8 experts, 2048 columns, us without / with:
+// K 8192 (1088 tiles, 64 of them in the third round) 2412 / 2117, K 16384 5022 / 4366; last rounds of 256 tiles cut in two
+// or three: 1713 / 1820 (K 4096), 314 / 334 (K 2048).
+constexpr int kSplitStages = 16, kSplitParts = 8, kSplitRounds = 32, kSplitTiles = 128;
+constexpr double kSplitFlops = 2e10;  // below that (0.14 ms) the launch that clears the counters costs what a split gains
+
 __device__ __attribute__((aligned(16))) uint32_t zero_chunk[4];  // zero-initialised
 
 __device__ __forceinline__ void wait_loads_and_lds() {
@@ -89,6 +98,11 @@ struct Loads {
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) ptr[i] = exists ? base + (int64_t)(red0 + i * RED_STEP) * ld + chunk * 4 : zeros();
         step[0] = exists ? BK * ld : 0;
+    }
+    // Make stage 0 the stage `first` of the reduction (the parts of a split tile start in the middle).
+    __device__ __forceinline__ void skip_stages(int first) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) ptr[i] += first * step[STRIDED ? 0 : i];
     }
     // Load i of a stage of which the first `left` reduction elements exist (WHOLE: all BK).
     template <bool WHOLE>
@@ -155,7 +169,15 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_kernel(const GemmParams P) {
     const int row_tiles =
         KIND == XMA_GEMM_MT ? P.row_tiles_max * P.num_experts : table ? P.tile_count[0] : tiles.total;
     int row_tile, col_tile;
-    if (!locate_tile<KIND == XMA_GEMM_MT>(row_tiles, P.col_tiles, row_tile, col_tile)) return;
+    TileWork work;
+    work.parts = 1;
+    if constexpr (KIND == XMA_GEMM_MT) {
+        if (!locate_tile<true>(row_tiles, P.col_tiles, row_tile, col_tile)) return;
+    } else {
+        if (!locate_work(row_tiles, P.col_tiles, P.round_tiles, P.most_parts, kSplitRounds, kSplitTiles, work)) return;
+        row_tile = work.row_tile;
+        col_tile = work.col_tile;
+    }
 
     const float* A = reinterpret_cast<const float*>(P.a);
     const float* B = reinterpret_cast<const float*>(P.b);
@@ -212,6 +234,15 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_kernel(const GemmParams P) {
             });
         } else {
             lb.setup_strided(wave, lane, W + n0, P.ldb, P.n - n0);
+        }
+    }
+    if constexpr (KIND != XMA_GEMM_MT) {
+        if (work.parts > 1) {
+            const int64_t all = (red_len + BK - 1) / BK;
+            const int first = (int)(work.part * all / work.parts), end = (int)((work.part + 1) * all / work.parts);
+            la.skip_stages(first);
+            lb.skip_stages(first);
+            red_len = ((int64_t)end * BK < red_len ? (int64_t)end * BK : red_len) - (int64_t)first * BK;
         }
     }
     // MT with a row gather: the source rows of the next stage's loads, requested a stage ahead
@@ -333,6 +364,54 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_kernel(const GemmParams P) {
         run(std::integral_constant<int, 1>{});
     }
 
+    // ---- a split tile: every part parks its sums, the part that arrives last adds them up in part order and goes on ----
+    // (what the exchange between XCDs relies on is written at the same place of the 16-bit kernel)
+    if constexpr (KIND != XMA_GEMM_MT) {
+        if (work.parts > 1) {
+            auto part_buffer = [&](int part) {
+                return reinterpret_cast<uint64_t*>(P.split_partials +
+                                                   (int64_t)(part * work.split_tiles + work.split_tile) * (BM * BN));
+            };
+            uint64_t* mine = part_buffer(work.part);
+#pragma unroll
+            for (int mi = 0; mi < MB; ++mi)
+#pragma unroll
+                for (int g = 0; g < 8; ++g) {
+                    const float2 v{acc[mi][2 * g], acc[mi][2 * g + 1]};
+                    __hip_atomic_store(mine + (mi * 8 + g) * THREADS + tid, __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+                }
+            wait_loads_and_lds();
+            __syncthreads();
+            int* arrivals = reinterpret_cast<int*>(even_stage);
+            if (tid == 0)
+                arrivals[0] = __hip_atomic_fetch_add(P.split_counters + work.split_tile, 1, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            const bool last = arrivals[0] == work.parts - 1;
+            __syncthreads();
+            if (!last) return;
+#pragma unroll
+            for (int mi = 0; mi < MB; ++mi)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[mi][r] = 0.0f;
+            for (int part = 0; part < work.parts; ++part) {
+                const uint64_t* src = part_buffer(part);
+                uint64_t v[MB * 8];
+#pragma unroll
+                for (int i = 0; i < MB * 8; ++i)
+                    v[i] = __hip_atomic_load(src + i * THREADS + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < MB * 8; ++i) {
+                    const float2 f = __builtin_bit_cast(float2, v[i]);
+                    acc[i / 8][2 * (i % 8)] += f.x;
+                    acc[i / 8][2 * (i % 8) + 1] += f.y;
+                }
+            }
+        }
+    }
+
     // ---- epilogue: registers -> LDS [BM][128], 512-byte rows, chunk c of row r at c ^ (r & 31) -> HBM ----
     // Register r of lane (h, i): tile row i (+ 32 mi), tile column 32 wave + 8 (r / 4) + 4 h + r % 4.
     constexpr int HALF_BLOCKS = (MB + 1) / 2;
@@ -448,8 +527,13 @@ static int launch(const xma_grouped_gemm_args& a, hipStream_t stream) {
         const int64_t rt = max_row_tiles(a.rows, a.num_experts, BM);
         P.row_tiles_max = (int32_t)rt;
         P.col_tiles = (int32_t)(EPI == EPI_PAIRED ? ceil_div(a.n / 2, BN / 2) : ceil_div(a.n, BN));
-        grid = grid_for_tiles(rt, P.col_tiles);
+        place_split_region(a, P);
+        P.round_tiles = (MB == 4 ? 2 : MB == 2 ? 3 : 4) * compute_units();  // by their registers
+        const int64_t parts = 2.0 * a.rows * a.n * a.k < kSplitFlops ? 1 : ceil_div(a.k, BK) / (kSplitStages * 4 / MB);
+        P.most_parts = (int32_t)(parts < 1 ? 1 : parts > kSplitParts ? kSplitParts : parts);
+        grid = grid_for_work(rt * P.col_tiles, P.round_tiles);
         if (a.num_experts > kMaxScannedExperts) launch_build_row_tiles(a, BM, rt, P, stream);
+        else if (P.most_parts > 1) launch_clear_split_counters(P, stream);
     }
     XMA_REQUIRE(grid < ((int64_t)1 << 31), "xma_grouped_gemm: %lld tiles exceed the grid limit", (long long)grid);
     hipLaunchKernelGGL((gemm_kernel<MB, KIND, EPI>), dim3((unsigned)grid), dim3(THREADS), 0, stream, P);

@@ -185,3 +185,23 @@ def test_table_of_tiles():
     out = torch.full((M, N), float("nan"), dtype=x.dtype, device="cuda")
     ops.scatter2scatter(x, w.permute(0, 2, 1), index, index, out, 1, True, True, offsets)
     assert_close(out, _products(rows, x, w.transpose(1, 2)).float(), TOL[x.dtype], "table", elem_tol=GEMM_ELEM_TOL[x.dtype])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("experts,columns", [(3, 8), (3, 520), (8, 8192), (8, 8200), (5, 333), (256, 36)])
+def test_column_sums(experts, columns, dtype):
+    """Per-expert column sums in narrow and in wide blocks (from 256 wide ones on), with vectors and without."""
+
+    g = torch.Generator("cuda").manual_seed(columns)
+    sizes = torch.randint(0, 700, (experts,), generator=g, device="cuda")
+    sizes[0], sizes[1] = 0, 1
+    offsets = torch.cat([sizes.new_zeros(1), sizes.cumsum(0)]).int()
+    x = torch.randn(int(offsets[-1]), columns, generator=g, device="cuda").to(dtype)
+    out = torch.full((experts, columns), float("nan"), dtype=dtype, device="cuda")
+    ops.expert_colsum(x, offsets, out)
+    ends = offsets.tolist()
+    want = torch.stack([x[a:b].double().sum(0) for a, b in zip(ends, ends[1:])])
+    # one rounding of the result, and the roundings of up to 700 additions in fp32, whose terms are about one
+    rounding = torch.finfo(dtype).eps / 2
+    assert bool(((out.double() - want).abs() <= rounding * 1.01 * want.abs() + 700 * 2.0**-24 * 30).all())
