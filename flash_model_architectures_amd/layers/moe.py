@@ -540,23 +540,22 @@ class MoE(XMAModule):
         original_shape = hidden_states.shape
         hidden_states = hidden_states.reshape(-1, self.hidden_size)
 
-        if not torch.is_grad_enabled() and self._steps_are_own() and _eager():
+        activation = None if torch.is_grad_enabled() else fused_activation_name(self.act, self.is_glu)
+        if activation is not None and kernel_backend in (None, KernelBackend.rocm) and self._steps_are_own() and _eager():
             # one native call for all that follows the gate, where the operators it stands for would be called directly
-            activation = fused_activation_name(self.act, self.is_glu)
-            if activation is not None and kernel_backend in (None, KernelBackend.rocm):
-                router_logits = self.gate(hidden_states)
-                resolve_backend(kernel_backend, "MoE")
-                done = layer_forward(
-                    hidden_states, self.c_fc.weight, self.c_proj.weight, self.c_fc.bias, self.c_proj.bias, activation,
-                    self.top_k, router_logits,
-                )  # fmt: skip
-                if done is not None:
-                    return done[0].view(original_shape), router_logits
-                router_weights, selected_experts = topk_softmax(router_logits, self.top_k, kernel_backend=kernel_backend)
-                hidden_states = self._compute_experts(
-                    hidden_states, router_weights, selected_experts, kernel_backend=kernel_backend
-                )
-                return hidden_states.view(original_shape), router_logits
+            router_logits = self.gate(hidden_states)
+            resolve_backend(kernel_backend, "MoE")
+            done = layer_forward(
+                hidden_states, self.c_fc.weight, self.c_proj.weight, self.c_fc.bias, self.c_proj.bias, activation, self.top_k,
+                router_logits,
+            )  # fmt: skip
+            if done is not None:
+                return done[0].view(original_shape), router_logits
+            router_weights, selected_experts = topk_softmax(router_logits, self.top_k, kernel_backend=kernel_backend)
+            hidden_states = self._compute_experts(
+                hidden_states, router_weights, selected_experts, kernel_backend=kernel_backend
+            )
+            return hidden_states.view(original_shape), router_logits
 
         router_logits, router_weights, selected_experts = self._compute_routing_weights(
             hidden_states, kernel_backend=kernel_backend
