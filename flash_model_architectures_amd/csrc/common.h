@@ -23,6 +23,10 @@ int check_launch(const char* what);  // reads hipGetLastError(), 0 if clean
         }                                 \
     } while (0)
 
+// inverse[perm[p]] = p, and offsets[p] = perm[p] / fan_out * row_bytes with `padding` zeros behind (rowmove.hip)
+int launch_invert_and_locate(const int32_t* perm, int64_t rows, int32_t fan_out, uint32_t row_bytes, int32_t* inverse,
+                             uint32_t* offsets, int padding, void* stream);
+
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline int dtype_size(int dtype) { return dtype == XMA_F32 ? 4 : 2; }
 inline bool valid_dtype(int dtype) { return dtype == XMA_F32 || dtype == XMA_F16 || dtype == XMA_BF16; }

@@ -35,6 +35,8 @@ struct GemmParams {
     // split-K of the last, partly filled round of tiles (16-bit TN/NN kernels)
     int32_t* split_counters;  // [kSplitSlots] arrivals per split tile, zero at launch
     float* split_partials;    // [kSplitSlots][tile] fp32 accumulators of the parts
+    // MT with gathered rows (16 bits): byte offset of the source row of every routed row, kRowOffsetsPadding entries more
+    const uint32_t* row_offsets;
     int32_t tile_rows;  // rows of the tallest tile (16-bit TN/NN)
     int32_t most_parts;       // parts of a split tile at most (fp32)
     int32_t round_tiles;      // tiles that run at a time on the whole device, a multiple of kNumXcd
@@ -330,6 +332,10 @@ struct DmaTile {
 };
 DmaTile dma_gemm_tile(const xma_grouped_gemm_args& a);
 int launch_dma_gemm(const xma_grouped_gemm_args& a, hipStream_t stream);
+// MT whose B rows are row_offsets[p] bytes behind a.b, for arguments that dma_gemm_supports() and whole vectors.  The table
+// is read up to kRowOffsetsPadding entries past the last routed row; what is read there is not used.
+constexpr int kRowOffsetsPadding = 256;
+int launch_gathered_weight_gradient(const xma_grouped_gemm_args& a, const uint32_t* row_offsets, hipStream_t stream);
 
 // The kernel for fp32 operands in whole, aligned vectors (grouped_gemm_f32.hip).
 GemmForm f32_gemm_form(const xma_grouped_gemm_args& a);

@@ -125,6 +125,13 @@ __device__ __forceinline__ void wait_vmcnt_and_lds() {
     compiler_fence();
 }
 
+// s_waitcnt for every LDS read and scalar load of this wave alone (vmcnt = 63)
+__device__ __forceinline__ void wait_lds() {
+    compiler_fence();
+    __builtin_amdgcn_s_waitcnt(0xF | (7 << 4) | (0 << 8) | (3 << 14));
+    compiler_fence();
+}
+
 __device__ __forceinline__ void block_barrier() {
     compiler_fence();
     __builtin_amdgcn_s_barrier();
@@ -207,18 +214,30 @@ __device__ __forceinline__ u32x4_t read_fragment(const char* slab_base, int offs
 //   UNIFORM  K-contiguous rows at a constant stride, with one extra jump in the middle of the tile
 //            (the up|gate halves of a fused SwiGLU weight tile): one pointer, the rest is scalar arithmetic,
 //   STRIDED  K-strided tile: one pointer, constant stride between instructions.
-enum LoadPlan { PLAN_ROWS, PLAN_UNIFORM, PLAN_STRIDED };
+//   GATHERED K-strided tile whose reduction rows lie anywhere: byte offsets of the rows, which are the same for the lanes that
+//            fetch one row, are read from a table by scalar loads a phase ahead.  (A vector load would do it per lane, but
+//            the compiler waits for vector loads and for the LDS-DMA loads in flight together.)
+enum LoadPlan { PLAN_ROWS, PLAN_UNIFORM, PLAN_STRIDED, PLAN_GATHERED };
+
+typedef __attribute__((address_space(4))) const uint32_t scalar_u32_t;  // read by scalar loads where the address is uniform
 
 template <typename T, int ROWS, int BK, LoadPlan PLAN>
 struct OperandLoads {
     using G = Geometry<ROWS, BK>;
     static constexpr int LOADS = G::LOADS;
-    static constexpr int RED_STRIDE = PLAN == PLAN_STRIDED ? G::KROWS_PER_LOAD * NUM_WAVES : 0;  // reduction rows between i and i+1
+    static constexpr bool KSTRIDED = PLAN == PLAN_STRIDED || PLAN == PLAN_GATHERED;
+    static constexpr int RED_STRIDE = KSTRIDED ? G::KROWS_PER_LOAD * NUM_WAVES : 0;  // reduction rows between i and i+1
     const T* ptr[PLAN == PLAN_ROWS ? LOADS : 1];  // HBM address of this lane's chunk in stage 0
-    bool valid[PLAN == PLAN_STRIDED ? 1 : LOADS];  // false: always the zero page (row / column outside the operand)
+    bool valid[KSTRIDED ? 1 : LOADS];  // false: always the zero page (row / column outside the operand)
     int64_t load_stride, mid_jump;  // UNIFORM / STRIDED: elements from instruction i to i+1; UNIFORM: extra at LOADS/2
     int64_t step;                   // elements to advance per stage
     int32_t red0;                   // reduction index covered by the lane in stage 0, instruction 0
+    // GATHERED: column offset of the lane's chunk, a mask for each of the rows of a load (all ones in the lanes that fetch
+    // it), the table at the wave's first row, and the offsets of the rows of the stage that is requested next
+    static constexpr bool GATHERED = PLAN == PLAN_GATHERED;
+    uint32_t column, row_mask[GATHERED ? G::KROWS_PER_LOAD : 1];
+    scalar_u32_t* table;
+    uint32_t row[GATHERED ? LOADS * G::KROWS_PER_LOAD : 1];
     int wave_lds;                   // byte offset of the wave's first 1 KiB block inside the operand's LDS tile
 
     __device__ static __forceinline__ const T* zero_page() { return reinterpret_cast<const T*>(g_zero_page); }
@@ -271,6 +290,31 @@ struct OperandLoads {
         wave_lds = wave * 1024;
     }
 
+    // GATHERED: `base` points at the first tile column of source row 0, table[r] is the byte offset of reduction row r.
+    __device__ __forceinline__ void setup_gathered(int wave, int lane, const T* base, const uint32_t* offsets, int64_t cols_left) {
+        static_assert(PLAN == PLAN_GATHERED, "plan");
+        const int krow = wave * G::KROWS_PER_LOAD + lane / G::KROW_CHUNKS;
+        const int chunk = (lane % G::KROW_CHUNKS) ^ ((krow & 3) << 2);
+        valid[0] = chunk * 8 < cols_left;
+        ptr[0] = base;
+        column = chunk * 16;
+#pragma unroll
+        for (int j = 0; j < G::KROWS_PER_LOAD; ++j) row_mask[j] = lane / G::KROW_CHUNKS == j ? ~0u : 0u;
+        table = (scalar_u32_t*)offsets + wave * G::KROWS_PER_LOAD;
+        load_stride = mid_jump = 0;
+        red0 = krow;
+        step = 0;
+        wave_lds = wave * 1024;
+    }
+    // Requests the row offsets of a stage; up to a load's rows past the end of the reduction are read from the table.
+    __device__ __forceinline__ void look_up(int64_t stage) {
+        scalar_u32_t* at = table + stage * BK;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+#pragma unroll
+            for (int j = 0; j < G::KROWS_PER_LOAD; ++j) row[i * G::KROWS_PER_LOAD + j] = at[i * RED_STRIDE + j];
+    }
+
     // Make stage 0 the stage `first` of the reduction (split-K parts start in the middle).
     __device__ __forceinline__ void skip_stages(int64_t first) {
 #pragma unroll
@@ -289,10 +333,16 @@ struct OperandLoads {
 #pragma unroll
         for (int i = I0; i < I1; ++i) {
             const T* p;
-            if constexpr (PLAN == PLAN_ROWS) p = ptr[i] + stage_off;
-            else p = ptr[0] + (stage_off + i * load_stride + (i >= LOADS / 2 ? mid_jump : 0));
+            if constexpr (PLAN == PLAN_ROWS) {
+                p = ptr[i] + stage_off;
+            } else if constexpr (GATHERED) {
+                uint32_t off = column;
+#pragma unroll
+                for (int j = 0; j < G::KROWS_PER_LOAD; ++j) off += row[i * G::KROWS_PER_LOAD + j] & row_mask[j];
+                p = reinterpret_cast<const T*>(reinterpret_cast<const char*>(ptr[0]) + off);
+            } else p = ptr[0] + (stage_off + i * load_stride + (i >= LOADS / 2 ? mid_jump : 0));
             if constexpr (MASKED) {
-                const bool ok = valid[PLAN == PLAN_STRIDED ? 0 : i] && (red0 + i * RED_STRIDE < red_left);
+                const bool ok = valid[KSTRIDED ? 0 : i] && (red0 + i * RED_STRIDE < red_left);
                 // computed for every lane and then selected: a branch around the load would make the number of
                 // loads in flight differ between waves
                 asm("" : "+v"(p));
@@ -314,7 +364,7 @@ struct OperandLoads {
     __device__ __forceinline__ bool all_valid() const {
         bool ok = true;
 #pragma unroll
-        for (int i = 0; i < (PLAN == PLAN_STRIDED ? 1 : LOADS); ++i) ok = ok && valid[i];
+        for (int i = 0; i < (KSTRIDED ? 1 : LOADS); ++i) ok = ok && valid[i];
         return ok;
     }
 };
@@ -345,7 +395,9 @@ struct Ring64x5 {
     };
     static constexpr int LOOKAHEAD = 2;  // a step at stage s issues loads of stages up to s + LOOKAHEAD
     template <typename K> __device__ static __forceinline__ void prologue(K& k) {
+        k.look_up(0);
         k.template issue_a<0, 0, LA, true>(0); k.template issue_b<0, 0, LB, true>(0);
+        k.look_up(1);
         k.template issue_a<1, 0, LA, true>(1); k.template issue_b<1, 0, LB, true>(1);
     }
     // load number I (0 <= I < phase_loads(PH)) of phase PH of the step at ring position P on stage s
@@ -380,7 +432,7 @@ struct Ring64x2 {
     }
 };
 
-template <typename T, int KIND, int EPI, typename Pipe>
+template <typename T, int KIND, int EPI, typename Pipe, bool GATHER>
 struct Kernel {
     static constexpr int BK = Pipe::BK;
     using TL = typename Pipe::TL;
@@ -390,7 +442,7 @@ struct Kernel {
     static constexpr int BN_OUT = EPI == EPI_PAIRED ? BN / 2 : BN;
 
     OperandLoads<T, BM, BK, A_STRIDED ? PLAN_STRIDED : PLAN_ROWS> la;
-    OperandLoads<T, BN, BK, B_STRIDED ? PLAN_STRIDED : PLAN_UNIFORM> lb;
+    OperandLoads<T, BN, BK, GATHER ? PLAN_GATHERED : B_STRIDED ? PLAN_STRIDED : PLAN_UNIFORM> lb;
     int64_t red_len;
     int wave, lane;
     int a_off[4], b_off[4], extra_off[4];  // variable parts of the fragment offsets (see fragment_offsets)
@@ -405,6 +457,11 @@ struct Kernel {
     }
     template <int P, int I0, int I1, bool MASKED> __device__ __forceinline__ void issue_b(int64_t stage) {
         lb.template issue<I0, I1, MASKED>(TL::template slab<Pipe::template At<P>::B_SLAB>(), Pipe::template At<P>::B_OFF, stage, red_len);
+    }
+
+    // the gathered rows of the B tile of a stage, ahead of its loads
+    __device__ __forceinline__ void look_up(int64_t stage) {
+        if constexpr (GATHER) lb.look_up(stage);
     }
 
     // Byte offsets of this lane's fragments inside an operand tile.  Only the part that is not a
@@ -485,6 +542,7 @@ struct Kernel {
     template <int RP, int LP, int LPH, bool MASKED>
     __device__ __forceinline__ void phase(int rkb, int cur, int64_t s, f32x4_t (&acc)[MI][NI]) {
         constexpr int IN_SLOT = MI < 2 ? 1 : 2, SLOTS = MI * NI / IN_SLOT, PER_B = MI / IN_SLOT;
+        constexpr int READ_SLOTS = GATHER && LPH == 1 ? SLOTS - SLOTS / 8 : SLOTS;  // (see step)
         constexpr int READS = MI + NI, LOADS = Pipe::phase_loads(LPH);
         const int nxt = cur ^ 1;
 #pragma unroll
@@ -494,7 +552,7 @@ struct Kernel {
             for (int i = 0; i < IN_SLOT; ++i) Mma16<T>::run(fb[cur][ni], fa[cur][m0 + i], acc[m0 + i][ni]);
 #pragma unroll
             for (int r = 0; r < READS; ++r) {  // the r-th fragment block of the next phase
-                const int last = (r + 1) * SLOTS / READS - 1;
+                const int last = (r + 1) * READ_SLOTS / READS - 1;
                 if (slot != (last < 0 ? 0 : last)) continue;
                 if constexpr (KIND == XMA_GEMM_NN && MI == NI) {
                     if (r % 2 == 0) fa[nxt][r / 2] = read_a<RP>(rkb, r / 2);
@@ -540,6 +598,14 @@ struct Kernel {
     template <int P, bool MASKED>
     __device__ __forceinline__ void step(int64_t s, f32x4_t (&acc)[MI][NI]) {
         static_assert(Pipe::KK == 2 && Pipe::phase_loads(0) <= 10 && Pipe::phase_loads(1) <= 10, "two phases of up to ten loads");
+        // Gathered rows: the offsets of the B tile that is requested in the second phase.  Scalar loads share a counter with
+        // the fragment reads and return in any order, so the compiler waits for all of both wherever a fragment is used
+        // while they are on their way.  Hence the reads of a stage's first block are done a few slots early and waited for
+        // here, and nothing else is until the step's barrier.
+        if constexpr (GATHER) {
+            wait_lds();
+            look_up(s + 2);
+        }
         phase<P, P, 0, MASKED>(1, 0, s, acc);
         wait_vmcnt_and_lds<Pipe::WAIT>();
         block_barrier();
@@ -603,9 +669,9 @@ struct TilePlace {
     TileWork work;
 };
 
-template <typename T, int KIND, int EPI, typename Pipe>
+template <typename T, int KIND, int EPI, typename Pipe, bool GATHER = false>
 __device__ __forceinline__ void multiply_tile(const GemmParams& P, const TilePlace& place) {
-    using K = Kernel<T, KIND, EPI, Pipe>;
+    using K = Kernel<T, KIND, EPI, Pipe, GATHER>;
     using TL = typename Pipe::TL;
     constexpr int BM = TL::BM, BN = TL::BN, WM = TL::WM, WN = TL::WN, MI = TL::MI, NI = TL::NI;
     constexpr int OUT_SLABS = TL::OUT_SLABS, SLAB_BLOCKS = TL::SLAB_BLOCKS;
@@ -626,7 +692,8 @@ __device__ __forceinline__ void multiply_tile(const GemmParams& P, const TilePla
     // ---- operand load plans ----
     if constexpr (KIND == XMA_GEMM_MT) {
         k.la.setup_strided(k.wave, k.lane, A + m_begin * P.lda + tile_i0, P.lda, P.n - tile_i0);
-        k.lb.setup_strided(k.wave, k.lane, B + m_begin * P.ldb + n0, P.ldb, P.k - n0);
+        if constexpr (GATHER) k.lb.setup_gathered(k.wave, k.lane, B + n0, P.row_offsets + m_begin, P.k - n0);
+        else k.lb.setup_strided(k.wave, k.lane, B + m_begin * P.ldb + n0, P.ldb, P.k - n0);
     } else {
         // The three ways of finding a row's source are told apart once, outside the per-row code, and rows past
         // the end look up the tile's first row (which always exists) and are then dropped: with a branch per
@@ -1052,7 +1119,7 @@ __device__ __forceinline__ void multiply_tile(const GemmParams& P, const TilePla
     if constexpr (OUT_SLABS >= 4) store_rows(TL::template slab<3>(), std::integral_constant<int, 3>{}, orow[3]);
 }
 
-template <typename T, int KIND, int EPI, int BM, int BN>
+template <typename T, int KIND, int EPI, int BM, int BN, bool GATHER = false>
 __global__ __launch_bounds__(THREADS, groups_per_cu(BN)) void grouped_gemm_dma_kernel(const GemmParams P) {
     TilePlace place;
     place.i0 = 0;
@@ -1097,7 +1164,7 @@ __global__ __launch_bounds__(THREADS, groups_per_cu(BN)) void grouped_gemm_dma_k
         place.n0 = (int64_t)work.col_tile * (EPI == EPI_PAIRED ? BN / 2 : BN);
     }
     if constexpr (BN == 256 || KIND == XMA_GEMM_MT) {
-        multiply_tile<T, KIND, EPI, Ring64x5<Tile<BM, BN>>>(P, place);
+        multiply_tile<T, KIND, EPI, Ring64x5<Tile<BM, BN>>, GATHER>(P, place);
     } else {
         const int64_t rows = place.m_end - place.m_begin;
         if (rows > 128) multiply_tile<T, KIND, EPI, Ring64x2<Tile<BM, BN>>>(P, place);
@@ -1138,11 +1205,12 @@ static __global__ __launch_bounds__(1024) void build_expert_order_kernel(const i
     }
 }
 
-template <typename T, int KIND, int EPI, int BM, int BN>
-static int launch(const xma_grouped_gemm_args& a, int tile_rows, hipStream_t stream) {
+template <typename T, int KIND, int EPI, int BM, int BN, bool GATHER = false>
+static int launch(const xma_grouped_gemm_args& a, int tile_rows, hipStream_t stream, const uint32_t* row_offsets = nullptr) {
     GemmParams P;
     fill_params(a, P);
     P.tile_rows = tile_rows;
+    P.row_offsets = row_offsets;
     int64_t grid;
     if (KIND == XMA_GEMM_MT) {
         P.row_tiles_max = (int32_t)ceil_div(a.n, BM);
@@ -1170,7 +1238,7 @@ static int launch(const xma_grouped_gemm_args& a, int tile_rows, hipStream_t str
         }
     }
     XMA_REQUIRE(grid < ((int64_t)1 << 31), "xma_grouped_gemm: %lld tiles exceed the grid limit", (long long)grid);
-    hipLaunchKernelGGL((grouped_gemm_dma_kernel<T, KIND, EPI, BM, BN>), dim3((unsigned)grid), dim3(THREADS), 0, stream, P);
+    hipLaunchKernelGGL((grouped_gemm_dma_kernel<T, KIND, EPI, BM, BN, GATHER>), dim3((unsigned)grid), dim3(THREADS), 0, stream, P);
     return check_launch("xma_grouped_gemm");
 }
 
@@ -1191,6 +1259,22 @@ static int dispatch(const xma_grouped_gemm_args& a, int tile_rows, hipStream_t s
 }
 
 }  // namespace dma
+
+// Token rows of the up-projection's weight gradient, read where they are instead of from a grouped copy.  us, copy + kernel /
+// kernel that gathers: fine-grained layer (16384 tokens, H 2048, 64 experts, 6 each) 88 + 705 / 775, skewed (128 experts, 8
+// each) 111 + 765 / 825, Mixtral-shaped (8192 tokens, H 4096) 42 + 3160 / 3160; and a buffer of the routed rows less.  The loop
+// has the same instructions but for four vector ones a load; at the fine-grained sizes it waits longer for its rows.
+template <typename T>
+static int launch_gathered(const xma_grouped_gemm_args& a, const uint32_t* row_offsets, hipStream_t stream) {
+    const DmaTile tile = dma_gemm_tile(a);
+    return tile.cols == 256 ? dma::launch<T, XMA_GEMM_MT, EPI_PLAIN, 256, 256, true>(a, tile.rows, stream, row_offsets)
+                            : dma::launch<T, XMA_GEMM_MT, EPI_PLAIN, 128, 128, true>(a, tile.rows, stream, row_offsets);
+}
+
+int launch_gathered_weight_gradient(const xma_grouped_gemm_args& a, const uint32_t* row_offsets, hipStream_t stream) {
+    return a.dtype == XMA_BF16 ? launch_gathered<bf16_t>(a, row_offsets, stream)
+                               : launch_gathered<f16_t>(a, row_offsets, stream);
+}
 
 // 16-bit element types; the weight-gradient layout only without a fused row gather (its reduction rows
 // would need an index lookup per stage).

@@ -1,7 +1,7 @@
 // The experts of an MoE layer from one call (host code only): selection, routing, both projections and the combination, and
 // the backward pass, as calls of the library's entry points.  A layer called from Python otherwise spends more time between
 // its launches than in its kernels when it is small.
-#include "common.h"
+#include "grouped_gemm_common.h"
 
 namespace {
 
@@ -65,16 +65,21 @@ struct Layer {
         g.ld_bias = a.b_down ? a.hidden : 0;
         return run(g);
     }
-    int weight_gradient(const void* d_rows, int64_t n, const void* rows, int64_t k, void* out, bool gathered) const {
+    xma_grouped_gemm_args weight_gradient(const void* d_rows, int64_t n, const void* rows, int64_t k, void* out) const {
         auto g = gemm(XMA_GEMM_MT, n, k);
         g.a = d_rows;
         g.b = rows;
         g.c = out;
-        if (gathered) {
-            g.in_index = a.perm;
-            g.in_fan_out = a.top_k;
-        }
-        return run(g);
+        return g;
+    }
+    // The up-projection's weight gradient reads the tokens where they are.  In 16 bits that takes whole vectors and byte
+    // offsets of 32 bits; otherwise their rows are copied in grouped order first.
+    xma_grouped_gemm_args d_w_up() const { return weight_gradient(a.d_preact, N, a.x, a.hidden, a.d_w_up); }
+    bool gathers_tokens() const {
+        int32_t kernel = 0, tile_rows, tile_cols;
+        const auto g = d_w_up();
+        return a.dtype != XMA_F32 && 2 * a.tokens * a.hidden < ((int64_t)1 << 32) &&
+               xma_grouped_gemm_form(&g, &kernel, &tile_rows, &tile_cols) == 0 && kernel == XMA_FORM_TILED;
     }
     int d_preact() const {
         auto g = gemm(XMA_GEMM_NN, a.intermediate, a.hidden);
@@ -155,21 +160,34 @@ int xma_moe_backward(const xma_moe_args* args, void* stream) {
                 "xma_moe_backward: null pointer");
     const Layer layer(a, stream);
     const int64_t H = a.hidden, I = a.intermediate, N = layer.N;
+    const bool gathers = layer.gathers_tokens();
+    uint32_t* token_offsets = reinterpret_cast<uint32_t*>(a.inverse) + layer.M;
+    if (gathers) {
+        XMA_STEP(launch_invert_and_locate(a.perm, layer.M, a.top_k, (uint32_t)(2 * H), a.inverse, token_offsets, kRowOffsetsPadding,
+                                          stream));
+    } else {
+        XMA_STEP(xma_invert_index(a.perm, 0, layer.M, a.inverse, stream));
+    }
     // the output's gradient in grouped order, and the gates'
-    XMA_STEP(xma_invert_index(a.perm, 0, layer.M, a.inverse, stream));
     XMA_STEP(xma_spread_rows(a.d_y, H, a.rows, H, a.perm, 0, a.inverse, a.tokens, a.top_k, H, a.dtype, a.gates, a.expanded, H,
                              a.d_gates, stream));
     if (a.d_b_down) XMA_STEP(xma_expert_colsum(a.rows, H, a.expert_offsets, a.num_experts, H, a.d_b_down, H, a.dtype, stream));
-    XMA_STEP(layer.weight_gradient(a.rows, H, a.act, I, a.d_w_down, false));
+    XMA_STEP(layer.run(layer.weight_gradient(a.rows, H, a.act, I, a.d_w_down)));
     XMA_STEP(layer.d_preact());
     if (a.d_b_up) XMA_STEP(xma_expert_colsum(a.d_preact, N, a.expert_offsets, a.num_experts, N, a.d_b_up, N, a.dtype, stream));
-    // `rows` holds the output's gradient, then the inputs of the up-projection, then its input gradients
-    if (a.dtype == XMA_F32) {  // the kernel gathers the tokens itself
-        XMA_STEP(layer.weight_gradient(a.d_preact, N, a.x, H, a.d_w_up, true));
+    // `rows` holds the output's gradient, then the inputs of the up-projection where they are copied, then its input gradients
+    auto d_w_up = layer.d_w_up();
+    if (gathers) {
+        XMA_STEP(launch_gathered_weight_gradient(d_w_up, token_offsets, (hipStream_t)stream));
+    } else if (a.dtype == XMA_F32) {  // the kernel looks the tokens up itself
+        d_w_up.in_index = a.perm;
+        d_w_up.in_fan_out = a.top_k;
+        XMA_STEP(layer.run(d_w_up));
     } else {
         XMA_STEP(xma_spread_rows(a.x, H, a.rows, H, a.perm, 0, a.inverse, a.tokens, a.top_k, H, a.dtype, nullptr, nullptr, 0,
                                  nullptr, stream));
-        XMA_STEP(layer.weight_gradient(a.d_preact, N, a.rows, H, a.d_w_up, false));
+        d_w_up.b = a.rows;
+        XMA_STEP(layer.run(d_w_up));
     }
     XMA_STEP(layer.d_rows());
     return xma_combine_topk(a.rows, H, nullptr, a.d_x, H, a.tokens, a.top_k, H, a.dtype, stream);

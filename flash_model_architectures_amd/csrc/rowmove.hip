@@ -105,6 +105,18 @@ __global__ __launch_bounds__(256) void invert_index_kernel(const void* __restric
     if (d >= 0 && d < dst_rows) inverse[d] = (int32_t)p;
 }
 
+// Both tables of the backward pass from the sort permutation: the inverse, and the byte offset of every routed row's token,
+// followed by `padding` zeros.
+__global__ __launch_bounds__(256) void invert_and_locate_kernel(const int32_t* __restrict__ perm, int64_t rows, int32_t fan_out,
+                                                                uint32_t row_bytes, int32_t* __restrict__ inverse,
+                                                                uint32_t* __restrict__ offsets, int padding) {
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= rows + padding) return;
+    const uint32_t d = p < rows ? (uint32_t)perm[p] : 0u;
+    offsets[p] = p < rows && d < (uint32_t)rows ? d / (uint32_t)fan_out * row_bytes : 0u;
+    if (p < rows && d < (uint32_t)rows) inverse[d] = (int32_t)p;
+}
+
 // y[t, :] = sum_j gates[t, j] * y_exp[t*k + j, :]   (GATED) or the plain sum over j.
 // STREAM: the expanded rows are read with streaming loads.  That is the faster way when they come from HBM; rows that
 // the previous kernel has just written and that fit the 256 MiB Infinity Cache are served from there, and plain
@@ -368,6 +380,15 @@ static void launch_move(const void* src, int64_t ld_src, void* dst, int64_t ld_d
 }  // namespace xma
 
 using namespace xma;
+
+namespace xma {
+int launch_invert_and_locate(const int32_t* perm, int64_t rows, int32_t fan_out, uint32_t row_bytes, int32_t* inverse,
+                             uint32_t* offsets, int padding, void* stream) {
+    hipLaunchKernelGGL(invert_and_locate_kernel, dim3((unsigned)ceil_div(rows + padding, 256)), dim3(256), 0, (hipStream_t)stream,
+                       perm, rows, fan_out, row_bytes, inverse, offsets, padding);
+    return check_launch("invert_and_locate");
+}
+}  // namespace xma
 
 extern "C" {
 

@@ -1076,7 +1076,7 @@ def layer_backward(
     d_x, d_w_up, d_w_down, d_gates = empty(T, H), empty(E, N, H), empty(E, H, I), empty(T, k)
     d_b_up, d_b_down = empty(E, N) if with_b_up else None, empty(E, H) if with_b_down else None
     d_preact, rows = empty(M, N), empty(M, H)
-    inverse = torch.empty(M, device=device, dtype=torch.int32)
+    inverse = torch.empty(2 * M + 256, device=device, dtype=torch.int32)
     lib = nat.load()
     workspace = _workspace(device, lib.xma_moe_workspace_bytes(T, E, k))
     args = nat.MOE_ARGS.pack(

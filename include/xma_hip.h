@@ -377,7 +377,7 @@ typedef struct xma_moe_args {
     void* d_b_down;     /* [E, H] or NULL */
     void* d_preact;     /* [M, N] scratch */
     void* rows;         /* [M, H] scratch */
-    int32_t* inverse;   /* [M] scratch */
+    int32_t* inverse;   /* [2 * M + 256] scratch */
 } xma_moe_args;
 int64_t xma_moe_workspace_bytes(int64_t tokens, int32_t num_experts, int32_t top_k);
 int xma_moe_forward(const xma_moe_args* args, void* stream);

@@ -143,3 +143,25 @@ def test_bad_arguments_are_refused():
     assert _native.load().xma_moe_forward(args, 0) != 0 and "bad args" in _native.last_error()
     args = _native.MOE_ARGS.pack(_native.MOE_ARGS.size, 0, ops.nat.EPI_SWIGLU, 4, 2, 0, 1, 8, 8, *[0] * (17 + 1 + 10))
     assert _native.load().xma_moe_backward(args, 0) != 0 and "null pointer" in _native.last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens", [4003, 4800])
+def test_gathered_weight_gradient_of_large_tiles(tokens, dtype, monkeypatch):
+    """The up-projection's weight gradient reads the tokens where they are, in 256 x 256 tiles too (the rest of this file has
+    128 x 128 ones), with part-full last tiles and reductions that end anywhere."""
+
+    layer = _layer(dtype, experts=16, k=2, hidden=1032, intermediate=1032)
+    x = torch.randn(tokens, 1032, device="cuda", dtype=dtype)
+    dy = torch.randn_like(x)
+    want = None
+    for one_by_one in (True, False):
+        with monkeypatch.context() as patch:
+            calls = _Calls(patch, one_by_one)
+            got = _train(layer, x, dy)
+            assert len(calls.names) == (0 if one_by_one else 2)
+        if want is not None:
+            for a, b in zip(got, want):
+                assert torch.equal(a, b)
+        want = got
