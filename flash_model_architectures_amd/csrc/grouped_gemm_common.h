@@ -105,11 +105,11 @@ void launch_build_row_tiles(const xma_grouped_gemm_args& a, int BM, int64_t row_
 //     turn; spreads a run of expensive bands (the weight-gradient tiles of an overloaded expert) over all XCDs and,
 //     when band costs fall monotonically, balances them.
 // `row_tiles` is the number of row tiles actually present.  Returns false when this work-group has no tile.
-template <bool SPREAD>
+template <bool SPREAD, int BAND = kBandTiles>
 __device__ __forceinline__ bool locate_tile(int row_tiles, int col_tiles, int& row_tile, int& col_tile) {
     const int xcd = blockIdx.x % kNumXcd;
     const int local = blockIdx.x / kNumXcd;
-    const int per_band = kBandTiles * col_tiles;
+    const int per_band = BAND * col_tiles;
     int band, in_band;
     if constexpr (SPREAD) {
         // forwards over the XCDs for even groups of eight bands, backwards for odd ones
@@ -124,12 +124,28 @@ __device__ __forceinline__ bool locate_tile(int row_tiles, int col_tiles, int& r
         band = tile / per_band;
         in_band = tile - band * per_band;
     }
-    const int band_first = band * kBandTiles;
+    const int band_first = band * BAND;
     if (band_first >= row_tiles) return false;
-    const int band_rows = row_tiles - band_first < kBandTiles ? row_tiles - band_first : kBandTiles;
+    const int band_rows = row_tiles - band_first < BAND ? row_tiles - band_first : BAND;
     row_tile = band_first + in_band % band_rows;
     col_tile = in_band / band_rows;
     return col_tile < col_tiles;
+}
+
+// The small tiles of the row-grouped kinds differ in cost, and under a skewed routing the tall ones come first: an eighth of
+// the sequence each leaves most of them to a few XCDs.  While the tiles are few they are therefore dealt in bands of two, where
+// that gives every XCD about as many bands; beyond, the panels that neighbouring tiles share in an XCD's L2 are worth more.
+// Four GEMMs of a layer, us, eighths / bands of two: 1531 tokens, 128 experts, 8 each, skewed (89 row tiles) 336 / 322; 1500, 64
+// experts, 6 each, skewed (67) 353 / 316, even (64) 390 / 379; 3000, even (128) 628 / 652; 5000, 128 experts, skewed (248) 865
+// / 894.
+constexpr int kDealtBand = 2, kMostDealtTiles = 104;
+__device__ __forceinline__ bool deal_row_tiles(int row_tiles) {
+    const int bands = (row_tiles + kDealtBand - 1) / kDealtBand, even = (bands + kNumXcd - 1) / kNumXcd * kNumXcd;
+    return row_tiles <= kMostDealtTiles && 4 * even <= 5 * bands;
+}
+inline int64_t grid_for_dealt_tiles(int64_t row_tiles, int64_t col_tiles) {
+    const int64_t rows = row_tiles < kMostDealtTiles ? row_tiles : kMostDealtTiles;
+    return ceil_div(ceil_div(rows, kDealtBand), kNumXcd) * kNumXcd * kDealtBand * col_tiles;
 }
 
 // Row-grouped kinds with split-K of the remainder.  With T tiles on a device that runs C of them at a time (round_tiles: one

@@ -1146,10 +1146,13 @@ __global__ __launch_bounds__(THREADS, groups_per_cu(BN)) void grouped_gemm_dma_k
         const RowTileScan tiles(P.offsets, table ? 0 : P.num_experts, P.tile_rows, threadIdx.x & 63);
         const int most_parts = (int)((P.k + 63) / 64 / kSplitMinStages);
         TileWork& work = place.work;
-        if (!locate_work(table ? P.tile_count[0] : tiles.total, P.col_tiles, P.round_tiles,
-                         most_parts < kMaxSplit ? most_parts : kMaxSplit, kSplitMaxRounds,
-                         kSplitSlots, work))
+        const int row_tiles = table ? P.tile_count[0] : tiles.total;
+        if (BN == 128 && most_parts < 2 && deal_row_tiles(row_tiles)) {
+            if (!locate_tile<true, kDealtBand>(row_tiles, P.col_tiles, work.row_tile, work.col_tile)) return;
+        } else if (!locate_work(row_tiles, P.col_tiles, P.round_tiles, most_parts < kMaxSplit ? most_parts : kMaxSplit,
+                                kSplitMaxRounds, kSplitSlots, work)) {
             return;
+        }
         int32_t row0, row_end;
         if (table) {
             place.expert = P.tile_expert[work.row_tile];
@@ -1231,6 +1234,10 @@ static int launch(const xma_grouped_gemm_args& a, int tile_rows, hipStream_t str
         const int64_t n_out = EPI == EPI_PAIRED ? a.n / 2 : a.n;
         P.col_tiles = (int32_t)ceil_div(n_out, bn_out);
         grid = grid_for_work(rt * P.col_tiles, P.round_tiles);
+        if (BN == 128 && !may_split(a.k)) {
+            const int64_t dealt = grid_for_dealt_tiles(rt, P.col_tiles);
+            grid = grid > dealt ? grid : dealt;
+        }
         if (a.num_experts > kMaxScannedExperts) {
             launch_build_row_tiles(a, tile_rows, rt, P, stream);
         } else if (may_split(a.k)) {
