@@ -158,12 +158,16 @@ inline int64_t grid_for_dealt_tiles(int64_t row_tiles, int64_t col_tiles) {
 // reductions of 14336 and 28672 split in three gain 7 % and 5 % of their launches), so a part keeps kSplitMinStages stages.
 // Work-groups are dealt per XCD as in locate_tile<false>: XCD x takes the x-th eighth of the whole tiles, then the x-th
 // eighth of the parts (part-major, so neighbours share panels).
+// HALVES: tiles of a last round that are not cut along the reduction, and leave half the places free, go to two work-groups
+// by their rows.
 struct TileWork {
     int row_tile, col_tile;
     int part, parts;  // this work-group reduces stages [part * n / parts, (part + 1) * n / parts)
     int split_tile;   // index of the tile among the split ones
     int split_tiles;
+    int half, halves;     // this work-group has the rows of one half of the tile
 };
+template <bool HALVES>
 __device__ __forceinline__ bool locate_work(int row_tiles, int col_tiles, int round_tiles, int most_parts, int most_rounds,
                                             int most_tiles, TileWork& w) {
     const int xcd = blockIdx.x % kNumXcd;
@@ -174,6 +178,9 @@ __device__ __forceinline__ bool locate_work(int row_tiles, int col_tiles, int ro
     int parts = rem > 0 && rem <= most_tiles && total < most_rounds * round_tiles ? round_tiles / rem : 1;
     parts = parts > most_parts ? most_parts : parts;
     parts = parts < 1 ? 1 : parts;
+    const int halves = HALVES && parts == 1 && 2 * rem <= round_tiles ? 2 : 1;
+    w.half = 0;
+    w.halves = 1;
     const int whole_per_xcd = whole / kNumXcd;
     int tile;
     if (local < whole_per_xcd) {
@@ -182,7 +189,7 @@ __device__ __forceinline__ bool locate_work(int row_tiles, int col_tiles, int ro
         w.parts = 1;
         w.split_tile = 0;
     } else {
-        const int items = rem * parts;
+        const int items = rem * parts * halves;
         const int per_xcd = (items + kNumXcd - 1) / kNumXcd;
         const int l = local - whole_per_xcd;
         const int q = xcd * per_xcd + l;
@@ -190,6 +197,11 @@ __device__ __forceinline__ bool locate_work(int row_tiles, int col_tiles, int ro
         w.part = q / rem;
         w.split_tile = q - w.part * rem;
         w.parts = parts;
+        if (halves > 1) {
+            w.half = w.part;
+            w.halves = 2;
+            w.part = 0;
+        }
         tile = whole + w.split_tile;
     }
     w.split_tiles = rem;

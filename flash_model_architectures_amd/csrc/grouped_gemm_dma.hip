@@ -53,13 +53,13 @@ __shared__ __attribute__((aligned(1024))) char half_slab4[16384];
 __shared__ __attribute__((aligned(1024))) char extra_slab0[8192];
 __shared__ __attribute__((aligned(1024))) char extra_slab1[8192];
 
-// A tile of BM rows and BN columns, four waves as 2 x 2.  256 x 256 has the compute unit to itself; the tiles of 128
+// A tile of BM rows and BN columns, four waves as 2 x 2.  The tiles of 256 columns have the compute unit to themselves; those of 128
 // columns take half its LDS, so that two work-groups share it.
 template <int BM_, int BN_>
 struct Tile {
     static constexpr int BM = BM_, BN = BN_, WM = BM / 2, WN = BN / 2;
     static constexpr int MI = WM / 16, NI = WN / 16;  // blocks of 16 x 16 per wave
-    static_assert((BM == 256 && BN == 256) || ((BM == 192 || BM == 128 || BM == 64 || BM == 32) && BN == 128), "tile size");
+    static_assert(((BM == 256 || BM == 128) && BN == 256) || ((BM == 192 || BM == 128 || BM == 64 || BM == 32) && BN == 128), "tile size");
     // The epilogue stages the tile through LDS, SLAB_BLOCKS blocks of 16 rows of each wave row at a time.
     static constexpr int SLAB_BLOCKS = MI < 2 ? 1 : 2;
     static constexpr int OUT_SLABS = MI / SLAB_BLOCKS;
@@ -539,6 +539,11 @@ struct Kernel {
     // finishes early puts its compute unit out of step for the rest of the launch, its requests stop hitting lines
     // its neighbours brought in, and the launch, which is bound by what the L2 has to fetch, gets 13-16 % slower
     // (8 tail tiles among 67 at the benchmark shape).
+    // Tail tiles of up to 128 rows as tiles of 128 x 256, which cost half: the input gradients gain where the reductions are
+    // short, the forward kinds win here and lose there (us, without / with, up, down, dact, dX: 16384 tokens, 64 experts, 6
+    // each, H 2048, I 1024 772 / 762, 431 / 435, 469 / 467, 760 / 737; 128 experts, 8 each, skewed 744 / 734, 470 / 491, 478 /
+    // 467, 797 / 755; 12000 tokens of the first 567 / 584, 314 / 325, 346 / 343, 557 / 554; 8192 tokens, 8 experts, 4 each, I
+    // 8192 1999 / 1990, 819 / 819, 1217 / 1155, 1623 / 1621).  So the input gradients have them.
     template <int RP, int LP, int LPH, bool MASKED>
     __device__ __forceinline__ void phase(int rkb, int cur, int64_t s, f32x4_t (&acc)[MI][NI]) {
         constexpr int IN_SLOT = MI < 2 ? 1 : 2, SLOTS = MI * NI / IN_SLOT, PER_B = MI / IN_SLOT;
@@ -1149,7 +1154,7 @@ __global__ __launch_bounds__(THREADS, groups_per_cu(BN)) void grouped_gemm_dma_k
         const int row_tiles = table ? P.tile_count[0] : tiles.total;
         if (BN == 128 && most_parts < 2 && deal_row_tiles(row_tiles)) {
             if (!locate_tile<true, kDealtBand>(row_tiles, P.col_tiles, work.row_tile, work.col_tile)) return;
-        } else if (!locate_work(row_tiles, P.col_tiles, P.round_tiles, most_parts < kMaxSplit ? most_parts : kMaxSplit,
+        } else if (!locate_work<BN == 256 && KIND == XMA_GEMM_NN>(row_tiles, P.col_tiles, P.round_tiles, most_parts < kMaxSplit ? most_parts : kMaxSplit,
                                 kSplitMaxRounds, kSplitSlots, work)) {
             return;
         }
@@ -1166,8 +1171,20 @@ __global__ __launch_bounds__(THREADS, groups_per_cu(BN)) void grouped_gemm_dma_k
         place.m_end = row_end;
         place.n0 = (int64_t)work.col_tile * (EPI == EPI_PAIRED ? BN / 2 : BN);
     }
-    if constexpr (BN == 256 || KIND == XMA_GEMM_MT) {
+    if constexpr (KIND == XMA_GEMM_MT) {
         multiply_tile<T, KIND, EPI, Ring64x5<Tile<BM, BN>>, GATHER>(P, place);
+    } else if constexpr (BN == 256 && KIND == XMA_GEMM_NN) {
+        // Flat tiles: halves of the tiles of a last round, and an expert's last rows.  (The forward kinds gain nothing from them
+        // on balance, see phase().)
+        if (place.work.halves > 1) {
+            place.m_begin += 128 * place.work.half;
+            if (place.m_begin >= place.m_end) return;
+            place.m_end = place.m_end - place.m_begin > 128 ? place.m_begin + 128 : place.m_end;
+        }
+        if (place.m_end - place.m_begin <= 128) multiply_tile<T, KIND, EPI, Ring64x5<Tile<128, BN>>>(P, place);
+        else multiply_tile<T, KIND, EPI, Ring64x5<Tile<BM, BN>>>(P, place);
+    } else if constexpr (BN == 256) {
+        multiply_tile<T, KIND, EPI, Ring64x5<Tile<BM, BN>>>(P, place);
     } else {
         const int64_t rows = place.m_end - place.m_begin;
         if (rows > 128) multiply_tile<T, KIND, EPI, Ring64x2<Tile<BM, BN>>>(P, place);

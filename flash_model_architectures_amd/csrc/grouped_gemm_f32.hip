@@ -174,7 +174,7 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_kernel(const GemmParams P) {
     if constexpr (KIND == XMA_GEMM_MT) {
         if (!locate_tile<true>(row_tiles, P.col_tiles, row_tile, col_tile)) return;
     } else {
-        if (!locate_work(row_tiles, P.col_tiles, P.round_tiles, P.most_parts, kSplitRounds, kSplitTiles, work)) return;
+        if (!locate_work<false>(row_tiles, P.col_tiles, P.round_tiles, P.most_parts, kSplitRounds, kSplitTiles, work)) return;
         row_tile = work.row_tile;
         col_tile = work.col_tile;
     }

@@ -173,6 +173,32 @@ def test_split_reductions_of_every_height(kind, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize(
+    "sizes,N", [([11200, 129, 128, 127, 257, 384, 385, 1, 0, 10240] * 2, 4104), ([2048, 2049, 4096, 2200], 8200)]
+)
+def test_flat_tiles_of_the_input_gradient(sizes, N):
+    """256 columns: an expert's last rows in tiles of 128, and the halves of the tiles of a last round (124 and 106 tiles).
+    Small integers, bit for bit."""
+
+    dt, K = torch.bfloat16, 2056
+    E, M = len(sizes), sum(sizes)
+    assert gemm_tile("NN", dt, E, M, N, K) == gemm_tile("NN", dt, E, M, N, K, 2) == (256, 256)
+    g, offsets, rows, index = _setup(sizes, M)
+    a = torch.randint(-2, 3, (M, K), generator=g, device="cuda").to(dt)
+    w = torch.randint(-1, 2, (E, K, N), generator=g, device="cuda").to(dt)
+    want = _products(rows, a, w)
+    out = torch.full((M, N), float("nan"), dtype=dt, device="cuda")
+    ops.scatter2scatter(a, w, index, index, out, 1, True, False, offsets)
+    assert torch.equal(out[index.long()], want.to(dt))
+    saved = torch.randn(M, 2 * N, generator=g, device="cuda").to(dt)
+    d_pre = torch.full((M, 2 * N), float("nan"), dtype=dt, device="cuda")
+    ops.down_projection_dgrad_fused(a, w, saved, offsets, d_pre, "swiglu")
+    leaf = saved.float().requires_grad_()
+    to.swiglu_packed(leaf).backward(want.to(dt).float())
+    assert_close(d_pre, leaf.grad, TOL[dt], "swiglu backward in flat tiles")
+
+
+@pytest.mark.gpu
 def test_table_of_tiles():
     """More experts than the kernel looks up itself: the tiles come from a table."""
 
