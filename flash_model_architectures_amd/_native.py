@@ -87,6 +87,13 @@ PROTOTYPES: dict[str, tuple] = {
         c_int,
         [c_void_p, c_int, c_int64, c_int32, c_int32, c_int64, c_void_p, c_void_p, c_int, c_void_p],
     ),
+    "xma_topk_route": (
+        c_int,
+        [
+            c_void_p, c_int, c_int64, c_int32, c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+            c_void_p, c_int64, c_void_p,
+        ],
+    ),  # fmt: skip
     "xma_topk_softmax_bwd": (
         c_int,
         [c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int, c_int64, c_int32, c_int32, c_void_p, c_int64, c_void_p],

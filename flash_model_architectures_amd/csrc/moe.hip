@@ -144,10 +144,13 @@ int xma_moe_forward(const xma_moe_args* args, void* stream) {
     const xma_moe_args& a = *args;
     XMA_REQUIRE(a.selected && a.counts && a.sorted_experts && a.y, "xma_moe_forward: null pointer");
     const Layer layer(a, stream);
-    if (a.logits)
-        XMA_STEP(xma_topk_softmax(a.logits, a.dtype, a.tokens, a.num_experts, a.top_k, a.num_experts, a.gates, a.selected, 1, stream));
-    XMA_STEP(xma_route_build(a.selected, 1, layer.M, a.num_experts, a.counts, a.expert_offsets, a.sorted_experts, a.perm, 0,
-                             a.workspace, a.workspace_bytes, stream));
+    if (a.logits) {
+        XMA_STEP(xma_topk_route(a.logits, a.dtype, a.tokens, a.num_experts, a.top_k, a.num_experts, a.gates, a.selected, a.counts,
+                                a.expert_offsets, a.sorted_experts, a.perm, a.workspace, a.workspace_bytes, stream));
+    } else {
+        XMA_STEP(xma_route_build(a.selected, 1, layer.M, a.num_experts, a.counts, a.expert_offsets, a.sorted_experts, a.perm, 0,
+                                 a.workspace, a.workspace_bytes, stream));
+    }
     XMA_STEP(layer.up());
     XMA_STEP(layer.down());
     return xma_combine_topk(a.expanded, a.hidden, a.gates, a.y, a.hidden, a.tokens, a.top_k, a.hidden, a.dtype, stream);

@@ -682,25 +682,22 @@ __global__ __launch_bounds__(256) void scan_place_kernel(const IdT* __restrict__
 // us, with a scan through LDS of 1024 slots in twenty barriers and sixteen batches for every wave / so: 6 ids x 64 experts
 // 13.8 / 2.8, 256 x 128 15.3 / 3.1, 2048 x 8 11.2 / 3.9, 4096 x 64 15.0 / 5.9 (4097 x 64 in two launches: 7.8).
 constexpr int kSingleBatches = (int)(kSingleBlockSortIds / 1024);
-template <typename IdT, typename OutT>
-__global__ __launch_bounds__(1024) void route_single_block_kernel(const IdT* __restrict__ ids, int64_t n, int E,
-                                                                   int nbits, uint32_t* __restrict__ counts,
-                                                                   int32_t* __restrict__ offsets,
-                                                                   OutT* __restrict__ sorted_ids,
-                                                                   OutT* __restrict__ perm) {
-    extern __shared__ uint32_t lds_hist[];  // [16 waves][E], then the totals of 16 waves' experts
+struct BlockRun {  // the wave's ids
+    int begin, end;
+};
+__device__ __forceinline__ BlockRun run_of_wave(int n, int wave) {
+    constexpr int kWaves = 1024 / kWaveSize;
+    const int per = ((n + kWaves - 1) / kWaves + kWaveSize - 1) / kWaveSize * kWaveSize;
+    const int begin = wave * per < n ? wave * per : n;
+    return {begin, begin + per < n ? begin + per : n};
+}
+// `v` holds the wave's ids, lds_hist [16 waves][E] zeros, then the totals of 16 waves' experts.
+template <typename OutT>
+__device__ __forceinline__ void sort_in_block(const int64_t (&v)[kSingleBatches], BlockRun run, int wave, int lane, int E, int nbits,
+                                              uint32_t* lds_hist, uint32_t* __restrict__ counts, int32_t* __restrict__ offsets,
+                                              OutT* __restrict__ sorted_ids, OutT* __restrict__ perm) {
     constexpr int kWaves = 1024 / kWaveSize;
     uint32_t* wave_total = lds_hist + kWaves * E;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
-    const int lane = lane_id();
-    const int per = (((int)n + kWaves - 1) / kWaves + kWaveSize - 1) / kWaveSize * kWaveSize;  // ids per wave
-    const int begin = wave * per < (int)n ? wave * per : (int)n;
-    const int end = begin + per < (int)n ? begin + per : (int)n;
-    int64_t v[kSingleBatches];  // requested before the first barrier, kept for the placement
-    load_chunk(ids, begin, end, lane, v);
-    for (int i = threadIdx.x; i < kWaves * E; i += 1024) lds_hist[i] = 0;
-    __syncthreads();
-
     uint32_t* mine = lds_hist + wave * E;
 #pragma unroll
     for (int j = 0; j < kSingleBatches; ++j)
@@ -738,8 +735,25 @@ __global__ __launch_bounds__(1024) void route_single_block_kernel(const IdT* __r
     // placement, stable inside the wave's run and across the runs
 #pragma unroll
     for (int j = 0; j < kSingleBatches; ++j)
-        if (begin + j * kWaveSize < end)
-            place_batch(v[j], begin + j * kWaveSize + lane, E, nbits, lane, mine, sorted_ids, perm);
+        if (run.begin + j * kWaveSize < run.end)
+            place_batch(v[j], run.begin + j * kWaveSize + lane, E, nbits, lane, mine, sorted_ids, perm);
+}
+
+template <typename IdT, typename OutT>
+__global__ __launch_bounds__(1024) void route_single_block_kernel(const IdT* __restrict__ ids, int64_t n, int E,
+                                                                   int nbits, uint32_t* __restrict__ counts,
+                                                                   int32_t* __restrict__ offsets,
+                                                                   OutT* __restrict__ sorted_ids,
+                                                                   OutT* __restrict__ perm) {
+    extern __shared__ uint32_t lds_hist[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+    const int lane = lane_id();
+    const BlockRun run = run_of_wave((int)n, wave);
+    int64_t v[kSingleBatches];  // requested before the first barrier, kept for the placement
+    load_chunk(ids, run.begin, run.end, lane, v);
+    for (int i = threadIdx.x; i < 1024 / kWaveSize * E; i += 1024) lds_hist[i] = 0;
+    __syncthreads();
+    sort_in_block(v, run, wave, lane, E, nbits, lds_hist, counts, offsets, sorted_ids, perm);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -783,18 +797,9 @@ __device__ __forceinline__ float group_sum(float v, int width) {
 // with many experts each are cheaper than a whole wave per token (E = 64: 8 lanes x 8 experts).
 // key = (order_key(value) << 32) | (0xffffffff - expert): the maximum picks the largest value
 // and, among equals, the lowest expert index.
-template <typename T, int EPL, typename IdxT>
-__global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__ logits, int64_t Tn, int E, int k, int G,
-                                                            int64_t ld, T* __restrict__ weights,
-                                                            IdxT* __restrict__ idx) {
-    const int lane = lane_id();
-    const int g = lane & (G - 1);
-    const int tokens_per_wave = kWaveSize / G;
-    const int64_t first = ((int64_t)blockIdx.x * (blockDim.x / kWaveSize) + threadIdx.x / kWaveSize) * tokens_per_wave;
-    if (first >= Tn) return;  // whole waves only: every lane of a wave takes part in the exchanges
-    const int64_t t = first + lane / G;
-    const bool live = t < Tn;
-    const T* row = logits + (live ? t : first) * ld;
+// Lane g of the group gets the g-th selection: its index and its weight.
+template <typename T, int EPL>
+__device__ __forceinline__ void select_in_group(const T* row, int E, int k, int G, int g, float& weight, uint32_t& index) {
     uint64_t keys[EPL];
 #pragma unroll
     for (int j = 0; j < EPL; ++j) {
@@ -821,11 +826,65 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
         }
     }
     const float ex = g < k ? expf(my_val - vmax) : 0.0f;
-    const float denom = group_sum(ex, G);
+    weight = ex / group_sum(ex, G);
+    index = my_idx;
+}
+
+template <typename T, int EPL, typename IdxT>
+__global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__ logits, int64_t Tn, int E, int k, int G,
+                                                            int64_t ld, T* __restrict__ weights,
+                                                            IdxT* __restrict__ idx) {
+    const int lane = lane_id();
+    const int g = lane & (G - 1);
+    const int tokens_per_wave = kWaveSize / G;
+    const int64_t first = ((int64_t)blockIdx.x * (blockDim.x / kWaveSize) + threadIdx.x / kWaveSize) * tokens_per_wave;
+    if (first >= Tn) return;  // whole waves only: every lane of a wave takes part in the exchanges
+    const int64_t t = first + lane / G;
+    const bool live = t < Tn;
+    float weight;
+    uint32_t index;
+    select_in_group<T, EPL>(logits + (live ? t : first) * ld, E, k, G, g, weight, index);
     if (live && g < k) {
-        Elem<T>::store(weights + t * k + g, ex / denom);
-        idx[t * k + g] = (IdxT)my_idx;
+        Elem<T>::store(weights + t * k + g, weight);
+        idx[t * k + g] = (IdxT)index;
     }
+}
+
+// Selection and counting sort of a small call in one block: the selected experts go on to the sort through LDS.  Both are
+// chains of latencies, and a launch less is worth more than the other compute units (see kTopkRouteRounds).
+template <typename T, int EPL>
+__global__ __launch_bounds__(1024) void topk_route_kernel(const T* __restrict__ logits, int Tn, int E, int k, int G, int64_t ld,
+                                                          int nbits, T* __restrict__ weights, int64_t* __restrict__ idx,
+                                                          uint32_t* __restrict__ counts, int32_t* __restrict__ offsets,
+                                                          int32_t* __restrict__ sorted_ids, int32_t* __restrict__ perm) {
+    extern __shared__ uint32_t lds_hist[];  // as in sort_in_block, then the selected experts
+    uint32_t* selected = lds_hist + 1024 / kWaveSize * (E + 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+    const int lane = lane_id();
+    const int g = lane & (G - 1), tokens_per_wave = kWaveSize / G;
+    const int first = wave * tokens_per_wave;
+    if (first < Tn) {  // whole waves only
+        const int t = first + lane / G;
+        const bool live = t < Tn;
+        float weight;
+        uint32_t index;
+        select_in_group<T, EPL>(logits + (int64_t)(live ? t : first) * ld, E, k, G, g, weight, index);
+        if (live && g < k) {
+            Elem<T>::store(weights + t * k + g, weight);
+            idx[t * k + g] = (int64_t)index;
+            selected[t * k + g] = index;
+        }
+    }
+    for (int i = threadIdx.x; i < 1024 / kWaveSize * E; i += 1024) lds_hist[i] = 0;
+    __syncthreads();
+    const BlockRun run = run_of_wave(Tn * k, wave);
+    int64_t v[kSingleBatches];
+#pragma unroll
+    for (int j = 0; j < kSingleBatches; ++j) {
+        const int i = run.begin + j * kWaveSize + lane;
+        v[j] = i < run.end ? (int64_t)selected[i] : -1;
+    }
+    sort_in_block(v, run, wave, lane, E, nbits, lds_hist, counts, offsets, sorted_ids, perm);
 }
 
 // Any E <= 16384: one wave per block, ordered keys of the row staged in LDS.
@@ -1181,6 +1240,13 @@ int xma_route_build_static(const void* ids, int ids_is_i64, int64_t n, int32_t E
                               (hipStream_t)stream_);
 }
 
+static int lanes_per_token(int E, int k) {  // at least k (lane s keeps the s-th selection) and enough for eight experts per lane
+    int G = 1;
+    while (G < k) G <<= 1;
+    while (G < kWaveSize && G * 8 < E) G <<= 1;
+    return G;
+}
+
 int xma_topk_softmax(const void* logits, int dtype, int64_t T, int32_t E, int32_t k, int64_t ld, void* weights,
                      void* idx, int idx_is_i64, void* stream_) {
     hipStream_t stream = (hipStream_t)stream_;
@@ -1190,10 +1256,7 @@ int xma_topk_softmax(const void* logits, int dtype, int64_t T, int32_t E, int32_
     XMA_REQUIRE(T >= 0 && ld >= E, "xma_topk_softmax: bad T=%lld or row stride %lld", (long long)T, (long long)ld);
     if (T == 0) return 0;
     XMA_REQUIRE(logits && weights && idx, "xma_topk_softmax: null pointer");
-    // lanes per token: at least k (lane s of a group keeps the s-th selection) and enough for eight experts per lane
-    int G = 1;
-    while (G < k) G <<= 1;
-    while (G < kWaveSize && G * 8 < E) G <<= 1;
+    const int G = lanes_per_token(E, k);
     const int per_lane = (int)ceil_div(E, G);
     const int wpb = 4;
     const unsigned blocks = (unsigned)ceil_div(T, (int64_t)wpb * (kWaveSize / G));
@@ -1217,6 +1280,36 @@ int xma_topk_softmax(const void* logits, int dtype, int64_t T, int32_t E, int32_
 #undef XMA_TOPK_E
 #undef XMA_TOPK
     return check_launch("xma_topk_softmax");
+}
+
+// One block takes the calls whose tokens fit its lanes at once and whose selection is short (rounds times experts per lane).
+// us, two launches / one: 1 token, 64 experts, k 6 7.6 / 6.4; 32 tokens, 8 experts, k 2 5.0 / 3.9; 512 of them 6.1 / 5.2; 64
+// tokens, 64 experts, k 6 9.2 / 8.3, 128 of them 9.5 / 9.3; beyond: 1024 tokens, 8 experts, k 2 6.9 / 7.3; 1000, 6 experts, k 4
+// 8.8 / 13.3; 16, 512 experts, k 8 11.8 / 12.3; 128, 128 experts, k 8 11.6 / 19.3.
+static constexpr int kTopkRouteRounds = 48;
+
+int xma_topk_route(const void* logits, int dtype, int64_t T, int32_t E, int32_t k, int64_t ld, void* weights, int64_t* selected,
+                   uint32_t* counts, int32_t* offsets, int32_t* sorted_ids, int32_t* perm, void* workspace,
+                   int64_t workspace_bytes, void* stream_) {
+    hipStream_t stream = (hipStream_t)stream_;
+    const bool sizes_ok = valid_dtype(dtype) && E >= 1 && E <= kSingleBlockBins && k >= 1 && k <= E && k <= kWaveSize && T >= 1 &&
+                          T * k <= kSingleBlockSortIds && ld >= E;
+    const int G = sizes_ok ? lanes_per_token(E, k) : 1;
+    const int per_lane = sizes_ok ? (int)ceil_div(E, G) : 0;
+    if (!sizes_ok || T * G > 1024 || k * per_lane > kTopkRouteRounds) {
+        const int status = xma_topk_softmax(logits, dtype, T, E, k, ld, weights, selected, 1, stream_);
+        if (status) return status;
+        return xma_route_build(selected, 1, T * k, E, counts, offsets, sorted_ids, perm, 0, workspace, workspace_bytes, stream_);
+    }
+    XMA_REQUIRE(logits && weights && selected && counts && offsets && sorted_ids && perm, "xma_topk_route: null pointer");
+    const size_t lds = ((size_t)(E + 1) * (1024 / kWaveSize) + (size_t)(T * k)) * sizeof(uint32_t);
+#define XMA_TOPK_ROUTE(T_, EPL)                                                                                             \
+    hipLaunchKernelGGL((topk_route_kernel<T_, EPL>), dim3(1), dim3(1024), lds, stream, (const T_*)logits, (int)T, (int)E,    \
+                       (int)k, G, ld, ceil_log2(E), (T_*)weights, selected, counts, offsets, sorted_ids, perm)
+    XMA_DISPATCH_DTYPE(dtype, T_, if (per_lane <= 1) XMA_TOPK_ROUTE(T_, 1); else if (per_lane <= 2) XMA_TOPK_ROUTE(T_, 2);
+                       else if (per_lane <= 4) XMA_TOPK_ROUTE(T_, 4); else XMA_TOPK_ROUTE(T_, 8))
+#undef XMA_TOPK_ROUTE
+    return check_launch("xma_topk_route");
 }
 
 int xma_topk_softmax_bwd(const void* logits, int64_t ld_logits, const void* d_weights, const void* idx,

@@ -175,6 +175,14 @@ int xma_topk_softmax(const void* logits, int dtype, int64_t T, int32_t E, int32_
                      void* weights, void* idx, int idx_is_i64, void* stream);
 
 /*
+ * xma_topk_softmax with int64 indices followed by xma_route_build with int32 outputs, for sizes of a small call in one launch.
+ * The workspace is that of xma_route_build.
+ */
+int xma_topk_route(const void* logits, int dtype, int64_t T, int32_t E, int32_t k, int64_t ld, void* weights, int64_t* selected,
+                   uint32_t* counts, int32_t* offsets, int32_t* sorted_ids, int32_t* perm, void* workspace,
+                   int64_t workspace_bytes, void* stream);
+
+/*
  * Backward of xma_topk_softmax: d_logits[T, E] (row stride ld, fully overwritten) is zero except
  * d_logits[t, idx[t, j]] = w_j * (d_weights[t, j] - sum_i w_i * d_weights[t, i]), where
  * w = softmax(logits[t, idx[t, :]]) is recomputed in fp32.  This is what autograd derives for
