@@ -1317,9 +1317,9 @@ bool dma_gemm_supports(const xma_grouped_gemm_args& a) {
 //
 // Row-grouped kinds: the time of both forms is estimated from the tiles that experts of 0.9, 1 and 1.1 times the mean
 // number of rows have, in rounds of the device, at the measured cost of a round (us; K in units of 1024):
-//   256 x 256: 10 + 24 K (24 + 24 K with an activation's backward), a partly filled last round costs a whole one or is
-//     split along the reduction;
-//   192, 128, 64, 32 x 128, two per compute unit: 3.5 (10) + 24, 18.6, 13, 10 K.
+//   256 x 256: 10 + 24 K (13 with a gated activation, 26 with an activation's backward), a partly filled last round costs a
+//     whole one or is split along the reduction;
+//   192, 128, 64, 32 x 128, two per compute unit: 3.5 (5, 13) + 24, 18.6, 13, 10 K.
 // Measured with the L2 and the caches as the benchmark's layers leave them (us, 256 x 256 / up to 192 / up to 128 rows):
 //   16384 tokens, H 2048, I 1024, 64 experts, 6 each: up 784 / 857 / 902, dX 755 / 819 / 858
 //   3000 tokens of the same layer: 228 / 205 / 244 and 217 / 186 / 228; 800 tokens: 143 / 133 / 132 and 114 / 110 / 112
@@ -1327,14 +1327,15 @@ bool dma_gemm_supports(const xma_grouped_gemm_args& a) {
 //   3001 tokens, H 512, I 1024, 6 experts, 4 each: up 49 / 42 / 37, down 28 / 23 / 20, dact 41 / 38 / 34, dX 48 / 38 / 30
 //   1000 tokens, H 1024, I 4096, 16 experts, 2 each: up 68 / 60 / 71, down 61 / 40 / 43, dX 98 / 83 / 91
 //   8192 tokens, H 4096, I 14336, 8 experts, 2 each: up 3082 / 3832 / 4256, down 1427 / 1876 / 2146
-// The smaller tiles are taken where they are expected to gain more than the estimate is sure of (7 %).  Over 28 such layers
-// its choices come within 3 % of the fastest of the three; it is wrong by up to a quarter where the
-// experts' rows all lie a little above a multiple of 192 (3000 tokens, 128 experts, 8 each: down 121 / 149).
+// The smaller tiles are taken where they are expected to gain more than the estimate is sure of (7 %).  Over 44 such layers
+// its choices cost 1 % more than the fastest of the three on average, and a quarter at the worst: where the experts' rows all
+// lie a little above a multiple of 192 (3000 tokens, 128 experts, 8 each: down 121 / 149), and in the smallest launches.
 //
 // Weight gradients: tiles of 128 x 128 where 256 x 256 fill the device less than twice, or where the reductions (the rows of
 // an expert) are short: 3001 tokens as above 45 / 22 and 50 / 32 us; 8000
 // tokens, H 512, I 576, 32 experts, 4 each (320 tiles of 256 x 256) 58 / 46; 800 tokens of the 64 experts 95 / 82 and 178 / 159,
-// 3000 tokens (281 rows each) 133 / 125 and 253 / 241, 6000 tokens (562 rows each) 178 / 178 and 346 / 392.
+// 3000 tokens (281 rows each) 133 / 125 and 253 / 241, 4000 tokens (375) 149 / 147 and 284 / 286; 375 rows of 128 experts, H
+// 2048, I 768 219 / 227 and 444 / 500; 6000 tokens of the 64 experts (562) 178 / 178 and 346 / 392.
 namespace {
 
 constexpr double kSpread[3] = {0.9, 1.0, 1.1};
@@ -1351,10 +1352,10 @@ const SmallTile& small_tile_for(double rows) {
     return kSmallTiles[i];
 }
 
-double estimate_256(double rows, int64_t experts, int64_t col_tiles, double k1024, bool backward) {
+double estimate_256(double rows, int64_t experts, int64_t col_tiles, double k1024, int shape) {
     double tiles = 0;
     for (double f : kSpread) tiles += (rows * f < 1 ? rows * f : (double)(int64_t)((rows * f + 255) / 256)) / 3;
-    const double set_up = backward ? 24 : 10, loop = 24 * k1024;
+    const double set_up = shape == EPI_BACKWARD ? 26 : shape == EPI_PAIRED ? 13 : 10, loop = 24 * k1024;
     const double rounds = tiles * experts * col_tiles / 256;
     const int64_t full = (int64_t)rounds;
     const double rest = rounds - full;
@@ -1368,8 +1369,8 @@ double estimate_256(double rows, int64_t experts, int64_t col_tiles, double k102
     return (full + 1) * set_up + full * loop + loop / parts + (parts > 1 ? 25 : 0);
 }
 
-double estimate_small(double rows, int64_t experts, int64_t col_tiles, double k1024, bool backward, const SmallTile& tallest) {
-    const double set_up = backward ? 10 : 3.5;
+double estimate_small(double rows, int64_t experts, int64_t col_tiles, double k1024, int shape, const SmallTile& tallest) {
+    const double set_up = shape == EPI_BACKWARD ? 13 : shape == EPI_PAIRED ? 5 : 3.5;
     auto cost = [&](const SmallTile& t) { return set_up * t.rows / 192 + t.per_1024 * k1024; };
     double tiles = 0, work = 0;
     for (double f : kSpread) {
@@ -1401,16 +1402,15 @@ DmaTile dma_gemm_tile(const xma_grouped_gemm_args& a) {
     const double rows = (double)a.rows / a.num_experts;
     if (a.kind == XMA_GEMM_MT) {
         const int64_t tiles = a.num_experts * ceil_div(a.n, 256) * ceil_div(a.k, 256);
-        return tiles < 512 || rows < 448 ? DmaTile{128, 128} : DmaTile{256, 256};
+        return tiles < 512 || rows < 330 ? DmaTile{128, 128} : DmaTile{256, 256};
     }
     int shape = EPI_PLAIN, act = ACT_NONE;
     split_epilogue(a.epilogue, shape, act);
     const double k1024 = (double)a.k / 1024;
-    const bool backward = shape == EPI_BACKWARD;
     auto estimate = [&](const SmallTile& t) {
-        return estimate_small(rows, a.num_experts, ceil_div(a.n, 128), k1024, backward, t);
+        return estimate_small(rows, a.num_experts, ceil_div(a.n, 128), k1024, shape, t);
     };
-    const double big = estimate_256(rows, a.num_experts, ceil_div(a.n, 256), k1024, backward);
+    const double big = estimate_256(rows, a.num_experts, ceil_div(a.n, 256), k1024, shape);
     const double tall = estimate(kSmallTiles[3]), flat = estimate(kSmallTiles[2]);
     if (big < 1.07 * (tall < flat ? tall : flat)) return DmaTile{256, 256};
     return tall <= flat ? DmaTile{192, 128} : DmaTile{128, 128};

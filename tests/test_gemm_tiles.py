@@ -45,10 +45,10 @@ def gemm_tile(kind: str, dtype, experts: int, rows: int, n: int, k: int, epilogu
         ("NN", 6, 12004, 512, 1024, 0, (128, 128)),
         ("TN", 8, 400, 4096, 14336, 0, (192, 128)),
         ("NN", 8, 0, 4096, 4096, 0, (192, 128)),
-        # weight gradients: two rounds of tiles, 448 rows per expert
+        # weight gradients: two rounds of tiles, 330 rows per expert
         ("MT", 8, 16384, 4096, 14336, 0, (256, 256)),
-        ("MT", 8, 3584, 2048, 2048, 0, (256, 256)),
-        ("MT", 8, 3583, 2048, 2048, 0, (128, 128)),
+        ("MT", 8, 2640, 2048, 2048, 0, (256, 256)),
+        ("MT", 8, 2639, 2048, 2048, 0, (128, 128)),
         ("MT", 8, 16384, 2048, 1792, 0, (128, 128)),
     ],
 )
