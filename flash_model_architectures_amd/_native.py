@@ -20,7 +20,7 @@ _lib: ctypes.CDLL | None = None
 
 DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
-ABI_VERSION = 4  # XMA_ABI_VERSION of include/xma_hip.h these bindings were written against
+ABI_VERSION = 5  # XMA_ABI_VERSION of include/xma_hip.h these bindings were written against
 
 GEMM_TN, GEMM_NN, GEMM_MT = 0, 1, 2
 EPI_NONE, EPI_SWIGLU, EPI_SWIGLU_BWD, EPI_GLU, EPI_GLU_BWD, EPI_GELU_TANH, EPI_GELU_TANH_BWD = 0, 1, 2, 3, 4, 5, 6

@@ -66,7 +66,7 @@ enum xma_gemm_epilogue {
 
 /* ABI revision of this header: bumped whenever a struct gains a field, an enum a value or the interface an entry
    point.  A caller may compare it with xma_abi_version() of the library it loaded. */
-#define XMA_ABI_VERSION 4
+#define XMA_ABI_VERSION 5
 
 typedef struct xma_grouped_gemm_args {
     uint32_t struct_size; /* sizeof(xma_grouped_gemm_args) as the CALLER was compiled: fields beyond it are taken as
