@@ -67,7 +67,8 @@ inline void split_epilogue(int epilogue, int& shape, int& act) {
     }
 }
 
-// At most kSplitSlots (tile, part) pairs exist at a time: the split tiles are those of one round of the device.
+// At most kSplitSlots tiles are split, those of one round of the device.  Their parts' sums take kSplitSlots tiles of 256 x 256 at
+// most: as many pairs of a tile and a part exist as places of a round (512 of 192 x 128, or 1024 of 32 x 128).
 constexpr int kSplitSlots = 256;
 constexpr int kMaxSplit = 4;
 constexpr int kSplitMaxRounds = 8;
