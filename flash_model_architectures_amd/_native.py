@@ -16,7 +16,7 @@ import torch
 
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libxma_hip.so")
-_lib: ctypes.CDLL | None = None
+_lib: ctypes.PyDLL | None = None
 
 DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
@@ -202,7 +202,7 @@ def is_built() -> bool:
     return os.path.exists(_LIB_PATH)
 
 
-def load() -> ctypes.CDLL:
+def load() -> ctypes.PyDLL:
     """Load the kernel library once; raises if it has not been built."""
 
     global _lib
@@ -212,7 +212,9 @@ def load() -> ctypes.CDLL:
                 f"{_LIB_PATH} is missing: build the HIP kernels with "
                 "`python -m flash_model_architectures_amd.build` (needs hipcc); there is no fallback path"
             )
-        lib = ctypes.CDLL(_LIB_PATH)
+        # PyDLL: the interpreter lock is held during a call.  The entry points only enqueue, and those that use the workspace of
+        # their stream (ops._workspace) enqueue several launches that must not be mixed with another thread's.
+        lib = ctypes.PyDLL(_LIB_PATH)
         if (
             not hasattr(lib, "xma_abi_version")
             or lib.xma_abi_version() != ABI_VERSION

@@ -64,7 +64,9 @@ def exclusive_offsets(expert_offsets: torch.Tensor, E: int) -> torch.Tensor:
 
 
 # One workspace per (device, stream), grown on demand and reused by every launch on that stream: launches on a
-# stream run in order, and every kernel initialises the part of the workspace it reads.
+# stream run in order, and every kernel initialises the part of the workspace it reads.  An entry point that clears or fills a
+# part in one launch and reads it in a later one is one native call, which holds the interpreter lock (see _native.load), so
+# the launches of two threads on one stream are not mixed.
 #
 # Lifetime and sharing rules:
 #   * a buffer lives until release_workspaces() or the end of the process; a stream that has run a 16-bit grouped GEMM
