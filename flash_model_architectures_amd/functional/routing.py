@@ -89,3 +89,12 @@ def route_tokens(
         E=num_experts,
     )
     return Routing(counts, offsets, sorted_expert_idxs, sorted_scattered_idxs)
+
+
+_OWN_OPERATORS = topk_softmax_rocm, route_build_rocm
+
+
+def operators_are_own() -> bool:
+    """False when a program has given the names by which this module calls its operators another meaning."""
+
+    return (topk_softmax_rocm, route_build_rocm) == _OWN_OPERATORS

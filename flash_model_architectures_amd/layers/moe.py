@@ -22,7 +22,7 @@ import torch.nn as nn
 
 from ..accelerator import KernelBackend, resolve_backend
 from ..custom_op import _eager, apply_function
-from ..functional.routing import route_tokens, topk_softmax
+from ..functional.routing import operators_are_own, route_tokens, topk_softmax
 from ..functional.swiglu_packed import swiglu_packed
 from ..ops import (
     exclusive_offsets,
@@ -252,7 +252,9 @@ class _FusedExperts(torch.autograd.Function):
         ctx.activation = activation
         ctx.has_bias = b_up is not None, b_down is not None
         if sorted_scattered_idxs is None:
-            done = layer_forward(x, w_up, w_down, b_up, b_down, activation, k, None, gates, selected, needs_grad)
+            done = None
+            if _forward_operators() == _OWN_FORWARD_OPERATORS and operators_are_own():
+                done = layer_forward(x, w_up, w_down, b_up, b_down, activation, k, None, gates, selected, needs_grad)
             if done is not None:
                 y, *saved = done
                 if needs_grad:
@@ -303,9 +305,11 @@ class _FusedExperts(torch.autograd.Function):
             grad_out = grad_out.contiguous()
         bias_gradients = ctx.has_bias[0] and ctx.needs_input_grad[7], ctx.has_bias[1] and ctx.needs_input_grad[8]
 
-        done = layer_backward(
-            x, w_up, w_down, gates, idx, expert_offsets, preact, act, expanded, grad_out, ctx.activation, *bias_gradients
-        )
+        done = None
+        if _backward_operators() == _OWN_BACKWARD_OPERATORS:
+            done = layer_backward(
+                x, w_up, w_down, gates, idx, expert_offsets, preact, act, expanded, grad_out, ctx.activation, *bias_gradients
+            )
         if done is not None:
             d_x, d_w_up, d_w_down, d_gates, d_b_up, d_b_down = done
             return d_x, d_w_up, d_w_down, d_gates, None, None, None, d_b_up, d_b_down, None
@@ -372,6 +376,23 @@ class _FusedExperts(torch.autograd.Function):
         d_x = torch.empty_like(x, memory_format=torch.contiguous_format)
         combine_topk(expanded=d_expanded, out=d_x, k=k, gates=None)
         return d_x, d_w_up, d_w_down, d_gates, None, None, None, d_b_up, d_b_down, None
+
+
+# What a native call of a pass stands for, by the names this module calls it by.  A program that gives one of the names another
+# meaning (or replaces a step of the layer, see MoE._steps_are_own) has its own called, with a graph and without.
+def _forward_operators() -> tuple:
+    return route_tokens, up_projection_fused, scatter2scatter, combine_topk
+
+
+def _backward_operators() -> tuple:
+    return (
+        invert_index, spread_rows_gate_grad, spread_rows, expert_colsum, group_bwd_W, down_projection_dgrad_fused,
+        scatter2scatter, combine_topk,
+    )  # fmt: skip
+
+
+_OWN_FORWARD_OPERATORS, _OWN_BACKWARD_OPERATORS = _forward_operators(), _backward_operators()
+_OWN_EXPERTS = _FusedExperts, _FusedExperts.forward, topk_softmax
 
 
 class Experts(XMAModule):
@@ -562,14 +583,20 @@ class MoE(XMAModule):
         return hidden_states.view(original_shape), router_logits
 
     def _steps_are_own(self) -> bool:
-        """False when a subclass or a patched instance has steps of its own, which then are called."""
+        """False when a subclass, a patched class or a patched instance has steps of its own, or a name that the steps call has
+        another meaning: these then are called."""
 
         own = type(self)
         return (
-            own._compute_routing_weights is MoE._compute_routing_weights
-            and own._compute_experts is MoE._compute_experts
+            own._compute_routing_weights is _OWN_STEPS[0]
+            and own._compute_experts is _OWN_STEPS[1]
             and "_compute_routing_weights" not in self.__dict__
             and "_compute_experts" not in self.__dict__
+            and _FusedExperts is _OWN_EXPERTS[0]
+            and _FusedExperts.forward is _OWN_EXPERTS[1]
+            and topk_softmax is _OWN_EXPERTS[2]
+            and _forward_operators() == _OWN_FORWARD_OPERATORS
+            and operators_are_own()
         )
 
     def _compute_routing_weights(
@@ -629,3 +656,6 @@ class MoE(XMAModule):
             grouped_out=False,
         )
         return hidden_states
+
+
+_OWN_STEPS = MoE._compute_routing_weights, MoE._compute_experts

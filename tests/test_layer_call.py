@@ -8,6 +8,8 @@ from torch.utils._python_dispatch import TorchDispatchMode
 
 import flash_model_architectures_amd as xma
 from flash_model_architectures_amd import _native, ops
+from flash_model_architectures_amd.functional import routing as routing_module
+from flash_model_architectures_amd.layers import moe
 
 
 ACTIVATIONS = {
@@ -26,6 +28,10 @@ def _layer(dtype, activation="swiglu", bias=False, experts=6, k=4, hidden=136, i
             layer.c_fc.bias.normal_()
             layer.c_proj.bias.normal_()
     return layer.to("cuda").to(dtype)
+
+
+def _layer_on_cpu():
+    return xma.MoE(4, 2, 16, 8, xma.swiglu_packed, True, False, 0.05)
 
 
 def _train(layer, x, dy):
@@ -165,3 +171,80 @@ def test_gathered_weight_gradient_of_large_tiles(tokens, dtype, monkeypatch):
             for a, b in zip(got, want):
                 assert torch.equal(a, b)
         want = got
+
+
+STEPS = ["_compute_routing_weights", "_compute_experts"]
+# names by which the layer's module calls what a native call stands for, and whether the forward pass calls them
+NAMES = {
+    **dict.fromkeys(["_FusedExperts", "topk_softmax", "route_tokens", "up_projection_fused", "scatter2scatter", "combine_topk"], True),
+    **dict.fromkeys(
+        ["invert_index", "spread_rows_gate_grad", "spread_rows", "expert_colsum", "group_bwd_W", "down_projection_dgrad_fused"], False
+    ),
+}
+BOTH = ("scatter2scatter", "combine_topk")  # called in both directions
+
+
+def test_replaced_steps_are_not_own(monkeypatch):
+    layer = _layer_on_cpu()
+    assert layer._steps_are_own()
+    for name in STEPS:
+        with monkeypatch.context() as patch:
+            patch.setattr(xma.MoE, name, lambda *args, **kwargs: None)
+            assert not layer._steps_are_own()
+    for name, forward in NAMES.items():
+        with monkeypatch.context() as patch:
+            patch.setattr(moe, name, object())
+            assert layer._steps_are_own() is not forward
+            assert (moe._backward_operators() == moe._OWN_BACKWARD_OPERATORS) is (forward and name not in BOTH)
+    for name in ("topk_softmax_rocm", "route_build_rocm"):
+        with monkeypatch.context() as patch:
+            patch.setattr(routing_module, name, object())
+            assert not layer._steps_are_own()
+    assert layer._steps_are_own()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("step", STEPS)
+def test_steps_replaced_on_the_class(step, monkeypatch):
+    layer = _layer(torch.bfloat16)
+    x = torch.randn(50, layer.hidden_size, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        want = layer(x)[0]
+    own, called = getattr(xma.MoE, step), []
+
+    def replaced(self, *args, **kwargs):
+        called.append(step)
+        return own(self, *args, **kwargs)
+
+    monkeypatch.setattr(xma.MoE, step, replaced)
+    with torch.no_grad():
+        assert torch.equal(layer(x)[0], want)
+    assert len(called) == 1
+    assert torch.equal(layer(x)[0], want)
+    assert len(called) == 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", [name for name in NAMES if name != "_FusedExperts"])
+def test_replaced_names_are_called(name, monkeypatch):
+    layer = _layer(torch.bfloat16, bias=True)
+    x = torch.randn(50, layer.hidden_size, device="cuda", dtype=torch.bfloat16)
+    dy = torch.randn_like(x)
+    with torch.no_grad():
+        want = layer(x)[0]
+    gradients = _train(layer, x, dy)
+    own, called = getattr(moe, name), []
+
+    def replaced(*args, **kwargs):
+        called.append(name)
+        return own(*args, **kwargs)
+
+    monkeypatch.setattr(moe, name, replaced)
+    if NAMES[name]:
+        with torch.no_grad():
+            assert torch.equal(layer(x)[0], want)
+        assert called
+        called.clear()
+    for a, b in zip(_train(layer, x, dy), gradients):
+        assert torch.equal(a, b)
+    assert called
