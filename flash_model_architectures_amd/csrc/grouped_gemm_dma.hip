@@ -31,6 +31,7 @@
 // A DMA load writes lane l's 16 bytes at (wave-uniform LDS base) + 16*l, so the swizzles are applied
 // by choosing which HBM chunk each lane fetches.  Masked rows / reduction tails are fetched from a
 // 16-byte page of zeros, which keeps every lane active and the outstanding-load count uniform.
+#include <cmath>
 #include <type_traits>
 
 #include "grouped_gemm_common.h"
@@ -1331,11 +1332,19 @@ bool dma_gemm_supports(const xma_grouped_gemm_args& a) {
 // its choices cost 1 % more than the fastest of the three on average, and a quarter at the worst: where the experts' rows all
 // lie a little above a multiple of 192 (3000 tokens, 128 experts, 8 each: down 121 / 149), and in the smallest launches.
 //
-// Weight gradients: tiles of 128 x 128 where 256 x 256 fill the device less than twice, or where the reductions (the rows of
-// an expert) are short: 3001 tokens as above 45 / 22 and 50 / 32 us; 8000
-// tokens, H 512, I 576, 32 experts, 4 each (320 tiles of 256 x 256) 58 / 46; 800 tokens of the 64 experts 95 / 82 and 178 / 159,
-// 3000 tokens (281 rows each) 133 / 125 and 253 / 241, 4000 tokens (375) 149 / 147 and 284 / 286; 375 rows of 128 experts, H
-// 2048, I 768 219 / 227 and 444 / 500; 6000 tokens of the 64 experts (562) 178 / 178 and 346 / 392.
+// Weight gradients: tiles of 128 x 128 where 256 x 256 leave much of the device idle, or where the reductions (the rows of an
+// expert) are short.  us, 256 x 256 / 128 x 128 (one launch back to back with itself, evenly spread rows):
+//   one round of large tiles, 16 experts, 1024 x 1024: 500 rows 26 / 28, 1000 37 / 39, 2000 59 / 65, 4000 101 / 124, 8000 199 / 267;
+//     8 experts, 2048 x 1024, 16000 rows 375 / 542
+//   a second round of three quarters, 8 experts, 2048 x 1792: 2000 rows 100 / 110, 4000 175 / 204, 16000 696 / 1050
+//   fewer than four bands of row tiles, which leave half the XCDs without work: 4 experts, 768 x 3072: 1500 rows 73 / 43, 4000
+//     165 / 102, 9000 353 / 229; 6 experts, 2048 x 1024, 9000 rows, skewed (an expert's tiles are one band): 411 / 275
+//   two rounds and more: 64 experts, 4096 x 512, 281 rows 133 / 125, 375 149 / 147; 64 experts, 2048 x 2048, 281 253 / 241, 375
+//     284 / 286, 562 346 / 392; 128 experts, 1536 x 2048, 375 444 / 500
+// Long launches of many tiles turn earlier: with 4096 tiles 1.05 times as long in small ones at 390 rows, with 8192 at 300, with
+// 16384 at 220, hence rows^2 * tiles.  Over 4310 calls of 1 to 256 experts, 20 to 20000 evenly spread rows each, the choice costs
+// 0.8 % more than the faster of the two on average, and is within 3 % of 256 x 256 or faster in 97 %.  Under a skewed routing
+// small tiles win for longer (one expert's reductions bound the launch), which the host cannot see.
 namespace {
 
 constexpr double kSpread[3] = {0.9, 1.0, 1.1};
@@ -1396,14 +1405,39 @@ double estimate_small(double rows, int64_t experts, int64_t col_tiles, double k1
     return full * one + (rest < 0.02 ? 0 : rest <= 0.5 ? 4 + 0.55 * one : one);
 }
 
+// Tiles of the XCD that has most of them: bands of kBandTiles row tiles are dealt in turn (locate_tile<true>).
+int64_t busiest_xcd(int64_t row_tiles, int64_t col_tiles) {
+    const int64_t bands = ceil_div(ceil_div(row_tiles, kBandTiles), kNumXcd);
+    return (row_tiles < kBandTiles ? row_tiles : bands * kBandTiles) * col_tiles;
+}
+
+// Rounds of `places` tiles, the last of which takes `part` of a whole one, and more the fuller it is.
+double rounds_of(int64_t tiles, int places, double part) {
+    const int64_t full = tiles / places;
+    const double rest = (double)(tiles % places) / places;
+    const double rounds = rest > 0 ? (double)full + part + (1 - part) * rest : (double)full;
+    return rounds < 1 ? 1 : rounds;
+}
+
+bool small_weight_gradient_tiles(const xma_grouped_gemm_args& a, double rows) {
+    const double tiles = (double)a.num_experts * ceil_div(a.n, 256) * ceil_div(a.k, 256);
+    if (tiles >= 512) return rows < 330 && rows * rows * tiles < 5e8;
+    // 32 compute units of an XCD, two places each for small tiles; us of a round, least squares over the calls of few tiles
+    const int64_t large = busiest_xcd(a.num_experts * ceil_div(a.n, 256), ceil_div(a.k, 256));
+    const int64_t small = busiest_xcd(a.num_experts * ceil_div(a.n, 128), ceil_div(a.k, 128));
+    const double x = rows / 1024;
+    const double time_large = rounds_of(large, 32, 0.8) * (14.4 + 24 * x);
+    const double time_small = rounds_of(small, 64, 0.7) * (6.6 + 13.6 * x * (1 + 0.1 * log2(1 + x)));
+    // (with at most one large tile per compute unit a skewed call takes up to twice as long in large tiles; an even one loses a
+    // seventh at most to the other mistake)
+    return time_small < (large <= 32 ? 1.2 : 1.03) * time_large;
+}
+
 }  // namespace
 
 DmaTile dma_gemm_tile(const xma_grouped_gemm_args& a) {
     const double rows = (double)a.rows / a.num_experts;
-    if (a.kind == XMA_GEMM_MT) {
-        const int64_t tiles = a.num_experts * ceil_div(a.n, 256) * ceil_div(a.k, 256);
-        return tiles < 512 || rows < 330 ? DmaTile{128, 128} : DmaTile{256, 256};
-    }
+    if (a.kind == XMA_GEMM_MT) return small_weight_gradient_tiles(a, rows) ? DmaTile{128, 128} : DmaTile{256, 256};
     int shape = EPI_PLAIN, act = ACT_NONE;
     split_epilogue(a.epilogue, shape, act);
     const double k1024 = (double)a.k / 1024;

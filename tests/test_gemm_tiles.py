@@ -49,12 +49,41 @@ def gemm_tile(kind: str, dtype, experts: int, rows: int, n: int, k: int, epilogu
         ("MT", 8, 16384, 4096, 14336, 0, (256, 256)),
         ("MT", 8, 2640, 2048, 2048, 0, (256, 256)),
         ("MT", 8, 2639, 2048, 2048, 0, (128, 128)),
-        ("MT", 8, 16384, 2048, 1792, 0, (128, 128)),
+        ("MT", 8, 16384, 2048, 1792, 0, (256, 256)),  # 100 us, 110 in small tiles
     ],
 )
 def test_which_calls_take_them(kind, experts, rows, n, k, epilogue, tile):
     for dtype in (torch.bfloat16, torch.float16):
         assert gemm_tile(kind, dtype, experts, rows, n, k, epilogue) == tile
+
+
+@pytest.mark.parametrize(
+    "experts,rows,n,k,large",
+    [
+        # long reductions in one round of large tiles, and in the greater part of a second one
+        (8, 16000, 2048, 1024, True),
+        (16, 8000, 1024, 1024, True),
+        (8, 4000, 2048, 1792, True),
+        (4, 16000, 4096, 1792, True),
+        (2, 8000, 4096, 3584, True),
+        (16, 500, 1024, 1024, False),
+        # half a round, a quarter of a second one, and row tiles that leave XCDs without work
+        (1, 9000, 2048, 1024, False),
+        (6, 2000, 2048, 1408, False),
+        (4, 4000, 768, 3072, False),
+        # two rounds and more: the reduction's length, earlier the longer the launch
+        (64, 281, 4096, 512, False),
+        (64, 400, 4096, 512, True),
+        (128, 230, 1024, 4096, False),
+        (128, 300, 1024, 4096, True),
+        (256, 180, 3584, 4096, True),
+    ],
+)
+def test_tile_of_a_weight_gradient(experts, rows, n, k, large):
+    """Against the times of both tiles (rows: of each expert)."""
+
+    want = (256, 256) if large else (128, 128)
+    assert gemm_tile("MT", torch.bfloat16, experts, experts * rows, n, k) == want
 
 
 def test_tile_of_the_other_kernels():
