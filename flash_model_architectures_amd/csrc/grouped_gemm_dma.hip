@@ -1316,21 +1316,28 @@ bool dma_gemm_supports(const xma_grouped_gemm_args& a) {
 // idle.  Tiles of up to 192 x 128 run two on a compute unit, so that one's set-up and stores run under the other's main
 // loop, and an expert's last rows take a tile of 32, 64, 128 or 192 rows; per operation they ask the L2 for two thirds more.
 //
-// Row-grouped kinds: the time of both forms is estimated from the tiles that experts of 0.9, 1 and 1.1 times the mean
-// number of rows have, in rounds of the device, at the measured cost of a round (us; K in units of 1024):
-//   256 x 256: 10 + 24 K (13 with a gated activation, 26 with an activation's backward), a partly filled last round costs a
-//     whole one or is split along the reduction;
-//   192, 128, 64, 32 x 128, two per compute unit: 3.5 (5, 13) + 24, 18.6, 13, 10 K.
-// Measured with the L2 and the caches as the benchmark's layers leave them (us, 256 x 256 / up to 192 / up to 128 rows):
-//   16384 tokens, H 2048, I 1024, 64 experts, 6 each: up 784 / 857 / 902, dX 755 / 819 / 858
-//   3000 tokens of the same layer: 228 / 205 / 244 and 217 / 186 / 228; 800 tokens: 143 / 133 / 132 and 114 / 110 / 112
-//   1531 tokens, H 2048, I 768, 128 experts, 8 each, skewed: up 107 / 102 / 99, down 71 / 58 / 57, dX 127 / 106 / 104
-//   3001 tokens, H 512, I 1024, 6 experts, 4 each: up 49 / 42 / 37, down 28 / 23 / 20, dact 41 / 38 / 34, dX 48 / 38 / 30
-//   1000 tokens, H 1024, I 4096, 16 experts, 2 each: up 68 / 60 / 71, down 61 / 40 / 43, dX 98 / 83 / 91
-//   8192 tokens, H 4096, I 14336, 8 experts, 2 each: up 3082 / 3832 / 4256, down 1427 / 1876 / 2146
-// The smaller tiles are taken where they are expected to gain more than the estimate is sure of (7 %).  Over 44 such layers
-// its choices cost 1 % more than the fastest of the three on average, and a quarter at the worst: where the experts' rows all
-// lie a little above a multiple of 192 (3000 tokens, 128 experts, 8 each: down 121 / 149), and in the smallest launches.
+// Row-grouped kinds: the cost of each form is estimated from the tiles that experts have whose numbers of rows spread as
+// randomly chosen ones do, and two per cent more, in rounds of the device (K: the reduction in units of 1024):
+//   256 x 256: 20 + 24 K a round (34 where the epilogue has an activation of two halves or its backward); a partly filled last round
+//     costs a whole one, or is split along the reduction for 40 more;
+//   192, 128, 64, 32 x 128, two per compute unit: 7 (10) + 33, 24, 20, 24 K, 1.45 times that where rows do not start at whole
+//     lines of 128 bytes; a last round of half the places or less two thirds of a whole one.
+// These are not times: small tiles take about 0.75 of it, and a remainder of 32 rows costs its neighbour more than itself.  They are
+// the constants whose choice cost least over 11600 calls (1 to 256 experts, 20 to 20000 rows each, 12 layers) timed in all three
+// forms: 1.2 % more than the fastest on average where rows are spread evenly, 4 % under a skewed routing.  94 % of them are within
+// 3 % of 256 x 256 everywhere or faster, on average they take 0.74 of its time.  The worst are experts whose rows lie just above a
+// multiple of 192 or 256, which a few rows more or less decide.
+// us, 256 x 256 / up to 192 / up to 128 rows, evenly spread unless said otherwise:
+//   64 experts, H 2048, I 1024: 1536 rows each, up 784 / 857 / 902, dX 755 / 819 / 858; 281, 228 / 205 / 244 and 217 / 186 / 228; 75,
+//     143 / 133 / 132 and 114 / 110 / 112
+//   128 experts, H 2048, I 768, 96 rows, skewed: up 107 / 102 / 99, down 71 / 58 / 57, dX 127 / 106 / 104; even, 200 rows, dact 143
+//     / 173 / 159
+//   6 experts, H 512, I 1024, 2000 rows: up 49 / 42 / 37, down 28 / 23 / 20, dact 41 / 38 / 34, dX 48 / 38 / 30
+//   16 experts, H 1024, I 4096, 125 rows: up 68 / 60 / 71, down 61 / 40 / 43, dX 98 / 83 / 91
+//   8 experts, H 4096, I 14336, 2048 rows: up 3082 / 3832 / 4256, down 1427 / 1876 / 2146
+//   one round of 256 x 256, two of the others: 4 experts, H 4096, I 14336, 187 rows, up 231 / 362 / 306, dact 119 / 185 / 162; 8
+//     experts, H 6144, I 2048, 200 rows, down 48 / 74 / 54
+//   rows of 1040 and 15056 bytes: 32 experts, H 520, I 7528, 200 rows, down 140 / 235 / 191, up 299 / 391 / 339
 //
 // Weight gradients: tiles of 128 x 128 where 256 x 256 leave much of the device idle, or where the reductions (the rows of an
 // expert) are short.  us, 256 x 256 / 128 x 128 (one launch back to back with itself, evenly spread rows):
@@ -1347,62 +1354,72 @@ bool dma_gemm_supports(const xma_grouped_gemm_args& a) {
 // small tiles win for longer (one expert's reductions bound the launch), which the host cannot see.
 namespace {
 
-constexpr double kSpread[3] = {0.9, 1.0, 1.1};
+constexpr int kSpreadPoints = 5;
+// the i-th of a few numbers of rows that stand for those of the experts
+int64_t rows_at(double mean, int i) {
+    constexpr double kDeviations[kSpreadPoints] = {-1.4, -0.7, 0, 0.7, 1.4};
+    const double rows = mean + kDeviations[i] * sqrt(mean + 4e-4 * mean * mean);
+    return rows < 0 ? 0 : (int64_t)(rows + 0.5);
+}
 
-struct SmallTile {
-    int rows;
-    double per_1024;
-};
-constexpr SmallTile kSmallTiles[] = {{32, 10.0}, {64, 13.0}, {128, 18.6}, {192, 24.0}};
-
-const SmallTile& small_tile_for(double rows) {
+constexpr int kHeights = 4;
+constexpr int kSmallRows[kHeights] = {32, 64, 128, 192};
+constexpr double kSmallLoop[kHeights] = {24, 20, 24, 33};
+int height_for(int64_t rows) {
     int i = 0;
-    while (i < 3 && rows > kSmallTiles[i].rows) ++i;
-    return kSmallTiles[i];
+    while (i < kHeights - 1 && rows > kSmallRows[i]) ++i;
+    return i;
 }
 
 double estimate_256(double rows, int64_t experts, int64_t col_tiles, double k1024, int shape) {
     double tiles = 0;
-    for (double f : kSpread) tiles += (rows * f < 1 ? rows * f : (double)(int64_t)((rows * f + 255) / 256)) / 3;
-    const double set_up = shape == EPI_BACKWARD ? 26 : shape == EPI_PAIRED ? 13 : 10, loop = 24 * k1024;
-    const double rounds = tiles * experts * col_tiles / 256;
-    const int64_t full = (int64_t)rounds;
-    const double rest = rounds - full;
-    if (full > 0 && rest < 0.02) return full * (set_up + loop);
-    double parts = 1;
+    for (int i = 0; i < kSpreadPoints; ++i) tiles += (double)ceil_div(rows_at(rows, i), 256) / kSpreadPoints;
+    const double set_up = shape == EPI_PLAIN ? 20 : 34, loop = 24 * k1024;
+    const double rounds = tiles * (double)experts * (double)col_tiles / 256;
+    const int64_t full = (int64_t)(rounds + 1e-6);
+    const double rest = rounds - (double)full;
+    if (full > 0 && rest < 1e-5) return full * (set_up + loop);
+    int parts = 1;
     if (rounds < kSplitMaxRounds) {
-        parts = (int)(1 / rest < kMaxSplit ? 1 / rest : kMaxSplit);
+        parts = rest * kMaxSplit < 1 ? kMaxSplit : (int)(1 / rest);
         if (parts > k1024 * 16 / kSplitMinStages) parts = (int)(k1024 * 16 / kSplitMinStages);
-        if (parts < 1) parts = 1;
     }
-    return (full + 1) * set_up + full * loop + loop / parts + (parts > 1 ? 25 : 0);
+    return full * (set_up + loop) + set_up + (parts > 1 ? loop / parts + 40 : loop);
 }
 
-double estimate_small(double rows, int64_t experts, int64_t col_tiles, double k1024, int shape, const SmallTile& tallest) {
-    const double set_up = shape == EPI_BACKWARD ? 13 : shape == EPI_PAIRED ? 5 : 3.5;
-    auto cost = [&](const SmallTile& t) { return set_up * t.rows / 192 + t.per_1024 * k1024; };
-    double tiles = 0, work = 0;
-    for (double f : kSpread) {
-        const double r = rows * f;
-        const int64_t whole = (int64_t)(r / tallest.rows);
-        const double rest = r - (double)whole * tallest.rows;
-        tiles += (whole + (rest > 0)) / 3.0;
-        work += (whole * cost(tallest) + (rest > 0 ? cost(small_tile_for(rest)) : 0)) / 3;
+double estimate_small(double rows, int64_t experts, int64_t col_tiles, double k1024, int shape, bool whole_lines, int tallest) {
+    double count[kHeights] = {};
+    for (int i = 0; i < kSpreadPoints; ++i) {
+        const int64_t r = rows_at(rows, i);
+        count[tallest] += (double)(r / kSmallRows[tallest]) / kSpreadPoints;
+        if (r % kSmallRows[tallest] > 0) count[height_for(r % kSmallRows[tallest])] += 1.0 / kSpreadPoints;
     }
-    tiles *= (double)experts * col_tiles;
-    work *= (double)experts * col_tiles / 512;
-    const double one = cost(rows >= tallest.rows ? tallest : small_tile_for(rows));
-    const double rounds = work / one;
-    const int64_t full = (int64_t)rounds;
-    const double rest = rounds - full;
+    double tiles = 0, work = 0, longest = 0;
+    for (int h = 0; h < kHeights; ++h) {
+        const double cost = ((shape == EPI_PLAIN ? 7 : 10) + kSmallLoop[h] * k1024) * (whole_lines ? 1 : 1.45);
+        tiles += count[h];
+        work += count[h] * cost;
+        if (count[h] > 0) longest = cost;
+    }
+    if (tiles == 0) return 0;
+    const double mean = work / tiles;
+    constexpr double kHalfRound = 0.66;
+    tiles *= (double)experts * (double)col_tiles;
     if (tiles <= 256) {  // fewer than one per compute unit, or split along the reduction
         double parts = (int)(512 / (tiles < 1 ? 1 : tiles));
         if (parts > kMaxSplit) parts = kMaxSplit;
         if (parts > k1024 * 16 / kSplitMinStages) parts = (int)(k1024 * 16 / kSplitMinStages);
-        if (parts >= 2) return (tiles * parts > 256 ? 1.0 : 0.55) * one / parts + 12;
-        return 4 + 0.55 * one;
+        if (parts < 2) parts = 1;
+        return (tiles * parts > 256 ? 1 : kHalfRound) * longest / parts;
     }
-    return full * one + (rest < 0.02 ? 0 : rest <= 0.5 ? 4 + 0.55 * one : one);
+    const double rounds = tiles / 512;
+    const int64_t full = (int64_t)(rounds + 1e-6);
+    const double rest = rounds - (double)full;
+    if (rest < 1e-5) return full * mean;
+    const double part = rest <= 0.5 ? kHalfRound : 1;
+    if (full == 0) return part * longest;
+    const double mixed = part * mean + 0.5 * (longest - mean);
+    return full * mean + (mixed < part * longest ? mixed : part * longest);
 }
 
 // Tiles of the XCD that has most of them: bands of kBandTiles row tiles are dealt in turn (locate_tile<true>).
@@ -1441,12 +1458,13 @@ DmaTile dma_gemm_tile(const xma_grouped_gemm_args& a) {
     int shape = EPI_PLAIN, act = ACT_NONE;
     split_epilogue(a.epilogue, shape, act);
     const double k1024 = (double)a.k / 1024;
-    auto estimate = [&](const SmallTile& t) {
-        return estimate_small(rows, a.num_experts, ceil_div(a.n, 128), k1024, shape, t);
+    const bool whole_lines = a.n % 64 == 0 && a.k % 64 == 0;
+    auto estimate = [&](int tallest) {
+        return estimate_small(rows, a.num_experts, ceil_div(a.n, 128), k1024, shape, whole_lines, tallest);
     };
     const double big = estimate_256(rows, a.num_experts, ceil_div(a.n, 256), k1024, shape);
-    const double tall = estimate(kSmallTiles[3]), flat = estimate(kSmallTiles[2]);
-    if (big < 1.07 * (tall < flat ? tall : flat)) return DmaTile{256, 256};
+    const double tall = estimate(kHeights - 1), flat = estimate(kHeights - 2);
+    if (big < tall && big < flat) return DmaTile{256, 256};
     return tall <= flat ? DmaTile{192, 128} : DmaTile{128, 128};
 }
 

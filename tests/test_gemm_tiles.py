@@ -40,7 +40,7 @@ def gemm_tile(kind: str, dtype, experts: int, rows: int, n: int, k: int, epilogu
         ("TN", 128, 12248, 1536, 2048, 1, (192, 128)),
         ("NN", 128, 12248, 2048, 1536, 0, (192, 128)),
         ("TN", 64, 18000, 2048, 2048, 1, (192, 128)),
-        ("NN", 64, 9000, 2048, 2048, 0, (192, 128)),
+        ("NN", 64, 9000, 2048, 2048, 0, (256, 256)),  # 118-121 us either way
         ("TN", 6, 12004, 512, 1024, 0, (128, 128)),
         ("NN", 6, 12004, 512, 1024, 0, (128, 128)),
         ("TN", 8, 400, 4096, 14336, 0, (192, 128)),
@@ -84,6 +84,35 @@ def test_tile_of_a_weight_gradient(experts, rows, n, k, large):
 
     want = (256, 256) if large else (128, 128)
     assert gemm_tile("MT", torch.bfloat16, experts, experts * rows, n, k) == want
+
+
+@pytest.mark.parametrize(
+    "kind,experts,rows,n,k,epilogue,tile",
+    [
+        # experts' rows a little below and above a multiple of 192, of which small tiles need a second round
+        ("TN", 4, 187, 28672, 4096, 1, (256, 256)),  # 231 us in 256 x 256, 362 in 192 x 128, 306 in 128 x 128
+        ("NN", 4, 187, 14336, 4096, 2, (256, 256)),  # 119, 185, 162
+        ("TN", 32, 187, 1536, 2048, 1, (256, 256)),  # 51, 74, 53
+        ("TN", 8, 200, 6144, 2048, 0, (256, 256)),  # 48, 74, 54
+        ("NN", 64, 200, 768, 2048, 2, (256, 256)),  # 64, 79, 66
+        ("NN", 128, 160, 512, 2048, 0, (256, 256)),  # 72, 93, 91
+        ("NN", 32, 187, 1792, 4096, 2, (256, 256)),  # 123, 178, 166
+        ("TN", 16, 4000, 768, 3072, 0, (256, 256)),  # 236, 288, 316
+        # rows that start in the middle of a line of 128 bytes
+        ("TN", 32, 200, 520, 7528, 0, (256, 256)),  # 140, 235, 191
+        ("TN", 64, 200, 15056, 520, 1, (256, 256)),  # 559, 731, 678
+        ("NN", 128, 1000, 7528, 520, 2, (256, 256)),  # 2557, 2956, 2918
+        # where they pay
+        ("TN", 64, 281, 2048, 2048, 1, (192, 128)),  # 228, 205, 244
+        ("TN", 16, 125, 1024, 4096, 0, (192, 128)),  # 61, 40, 43
+        ("TN", 1, 9000, 1024, 512, 0, (192, 128)),  # 19, 14, 18
+        ("NN", 6, 2000, 512, 1024, 2, (128, 128)),  # 41, 38, 34
+    ],
+)
+def test_tile_of_a_projection(kind, experts, rows, n, k, epilogue, tile):
+    """Against the times of the three tiles, in the comments (rows: of each expert)."""
+
+    assert gemm_tile(kind, torch.bfloat16, experts, experts * rows, n, k, epilogue) == tile
 
 
 def test_tile_of_the_other_kernels():
