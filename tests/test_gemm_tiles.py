@@ -122,8 +122,10 @@ def test_tile_of_the_other_kernels():
 
 # rows per expert: both sides of every height, a full tile and a last one of each height behind it, none
 SIZES = [192, 193, 1, 31, 32, 33, 0, 64, 65, 128, 129, 200, 320, 321, 385, 95, 97, 191, 2, 0, 1, 0]
-# (reduction, columns, tile of TN and of NN): one stage, a last stage of eight, whole ones, a partial last tile of columns
+# (reduction, columns, tile of TN and of NN): one stage, a last stage of eight, whole ones, a partial last tile of columns; the
+# gated epilogues need columns in multiples of 16: halves of 8, 72, 136 and 168, in tiles of 64 and 128
 SMALL = [(8, 8, 192, 192), (72, 136, 192, 192), (320, 264, 192, 192), (456, 328, 192, 192)]
+GATED = [(8, 16, 192, 192), (72, 144, 192, 192), (320, 272, 192, 192), (456, 336, 192, 192)]
 
 
 def _setup(sizes, seed):
@@ -142,7 +144,7 @@ def _products(rows, a, w):  # w[e]: [in, out]
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("sizes", [SIZES, [3, 700]])
-@pytest.mark.parametrize("k,n,tn,nn", SMALL)
+@pytest.mark.parametrize("k,n,tn,nn", SMALL + GATED)
 def test_heights(k, n, tn, nn, sizes, dtype):
     E, M = len(sizes), sum(sizes)
     g, offsets, rows, index = _setup(sizes, k + n)
@@ -173,8 +175,12 @@ def test_heights(k, n, tn, nn, sizes, dtype):
     # the activations' epilogues, gated ones over the halves of the columns
     for activation in ("swiglu", "glu", "gelu_tanh"):
         gated = activation != "gelu_tanh"
-        if gated and n % 16:
+        if gated and (k, n, tn, nn) not in GATED:
             continue
+        if gated and sizes is SIZES:
+            epilogue, _, _ = ops.FUSED_ACTIVATIONS[activation]
+            assert gemm_tile("TN", dtype, E, M, n, k, epilogue) == (tn, 128)
+            assert gemm_tile("NN", dtype, E, M, n // 2, k, epilogue + 1) == (nn, 128)
         act, pre = empty(M, n // 2 if gated else n), empty(M, n)
         ops.up_projection_fused(x, w, index, offsets, act, pre, 1, activation, bias)
         assert_close(pre, with_bias, tol, f"{activation}, pre-activation", elem_tol=elem)

@@ -1,10 +1,13 @@
 """The experts of a layer from one native call: the same results, bit for bit, as the operators one by one, and the operators
 whenever a call is not a plain one."""
 
+import threading
+
 import pytest
 import torch
 import torch.nn as nn
 from torch.utils._python_dispatch import TorchDispatchMode
+from torch.utils.checkpoint import checkpoint
 
 import flash_model_architectures_amd as xma
 from flash_model_architectures_amd import _native, ops
@@ -248,3 +251,112 @@ def test_replaced_names_are_called(name, monkeypatch):
     for a, b in zip(_train(layer, x, dy), gradients):
         assert torch.equal(a, b)
     assert called
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_saved_tensor_hooks_and_checkpoints(dtype, monkeypatch):
+    """What a call keeps for its backward pass may be replaced by copies, or be made again there."""
+
+    layer = _layer(dtype, bias=True)
+    x = torch.randn(77, layer.hidden_size, device="cuda", dtype=dtype)
+    dy = torch.randn_like(x)
+    want = _train(layer, x, dy)
+    packed = []
+
+    def pack(t):
+        packed.append(t.shape)
+        return t.cpu()
+
+    calls = _Calls(monkeypatch)
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+        got = _train(layer, x, dy)
+    assert len(packed) >= 9 and calls.names == ["xma_moe_forward", "xma_moe_backward"]
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    for reentrant in (False, True):
+        calls.names.clear()
+        layer.zero_grad(set_to_none=True)
+        leaf = x.detach().requires_grad_()
+        y, _ = checkpoint(layer, leaf, use_reentrant=reentrant)
+        y.backward(dy)
+        assert calls.names == ["xma_moe_forward", "xma_moe_forward", "xma_moe_backward"]
+        for a, b in zip([y.detach(), leaf.grad, *(p.grad for p in layer.parameters())], [want[0], *want[2:]]):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("forward_on_side", [False, True])
+def test_directions_on_different_streams(forward_on_side):
+    layer = _layer(torch.bfloat16)
+    x = torch.randn(900, layer.hidden_size, device="cuda", dtype=torch.bfloat16)
+    dy = torch.randn_like(x)
+    want = _train(layer, x, dy)
+    main, side = torch.cuda.current_stream(), torch.cuda.Stream()
+    first, second = (side, main) if forward_on_side else (main, side)
+    for _ in range(3):
+        layer.zero_grad(set_to_none=True)
+        leaf = x.detach().requires_grad_()
+        first.wait_stream(main)
+        with torch.cuda.stream(first):
+            y, _ = layer(leaf)
+        second.wait_stream(first)
+        with torch.cuda.stream(second):
+            y.backward(dy)
+        main.wait_stream(side)
+        for a, b in zip([y.detach(), leaf.grad, *(p.grad for p in layer.parameters())], [want[0], *want[2:]]):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_two_threads_train_on_one_stream(dtype):
+    """One thread's forward pass beside the other's backward one, which runs in a thread of autograd's."""
+
+    layers = [_layer(dtype, experts=6, k=2, hidden=512, intermediate=256), _layer(dtype, experts=200, k=4)]
+    work = []
+    for layer in layers:
+        x = torch.randn(1500, layer.hidden_size, device="cuda", dtype=dtype)
+        dy = torch.randn_like(x)
+        work.append((layer, x, dy, _train(layer, x, dy)))
+    failures = []
+
+    def loop(layer, x, dy, want):
+        try:
+            for _ in range(20):
+                assert all(torch.equal(a, b) for a, b in zip(_train(layer, x, dy), want))
+        except BaseException as e:  # noqa: BLE001 (handed to the main thread)
+            failures.append(e)
+
+    threads = [threading.Thread(target=loop, args=w) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [300_001, 540_001])
+def test_many_token_bytes(tokens, monkeypatch):
+    """Token rows more than 2^31 bytes behind the first one, whose offsets fill 32 bits, and beyond 2^32, where the rows are
+    copied."""
+
+    layer = _layer(torch.bfloat16, experts=8, k=1, hidden=4096, intermediate=64)
+    assert (tokens * 4096 * 2 < 2**32) is (tokens == 300_001)
+    x = torch.randn(tokens, 4096, device="cuda", dtype=torch.bfloat16)
+    dy = torch.randn_like(x)
+    want = None
+    for one_by_one in (True, False):
+        with monkeypatch.context() as patch:
+            calls = _Calls(patch, one_by_one)
+            got = _train(layer, x, dy)
+            assert len(calls.names) == (0 if one_by_one else 2)
+        if want is not None:
+            for a, b in zip(got, want):
+                assert torch.equal(a, b)
+        want = got
+    # and the last tokens' part in a weight gradient: their experts' gradients change with them
+    del want
+    x[-1].zero_()
+    assert not all(torch.equal(a, b) for a, b in zip(got[3:], _train(layer, x, dy)[3:]))
