@@ -4,7 +4,7 @@ A "step" is one forward + backward pass of the Mixtral-shaped MoE layer (bf16 wi
 accumulation, hidden 4096, per-expert intermediate 14336, 8 experts, top-2, 8192 tokens) over
 synthetic inputs that are already resident in HBM.  Prints ONE JSON line with the whole-job
 throughput in tokens/s, the roofline position of the dominant kernel (timed with events on the
-launch stream during the timed steps) and a CPU baseline: the torch restatement of the
+launch stream in passes of their own after the timed steps) and a CPU baseline: the torch restatement of the
 reference's torch path (oracle/torch_oracle.py) timed on this host's cores on a bounded sample.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu-baseline] [--no-aux]
@@ -39,6 +39,42 @@ TRAFFIC_ROW_TAGS = {
     (1, 2): "xma_grouped_gemm/NN+swiglu_bwd",
     (1, 0): "xma_grouped_gemm/NN",
 }
+
+
+# Launches are timed in passes of their own: events around every launch need the operators called one by one, while a plain
+# pass, as a user's program makes it and as the steps are timed, is one native call per direction.
+OBSERVED_PASSES = 5
+KERNELS_FROM = (
+    "separate passes with events around every launch, operators one by one; the timed steps make these launches from one native "
+    "call per direction, but in 16 bits the up-projection's weight gradient looks the tokens' rows up instead of reading a grouped copy"
+)
+
+
+def _time_steps(step, steps: int, observe: bool = True) -> tuple[float, dict, int]:
+    """(seconds that `steps` plain steps take, Timeline summary of some more steps, their number)."""
+
+    import torch
+
+    from flash_model_architectures_amd import _native
+
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    for _ in range(steps):
+        step()
+    torch.cuda.synchronize()
+    seconds = time.perf_counter() - t0
+    if not observe:
+        return seconds, {}, 0
+    observed = min(steps, OBSERVED_PASSES)
+    timeline = _native.Timeline()
+    _native.set_timeline(timeline)
+    try:
+        for _ in range(observed):
+            step()
+        torch.cuda.synchronize()
+    finally:
+        _native.set_timeline(None)
+    return seconds, timeline.summary(), observed
 
 
 def _profile_blob_id() -> str | None:
@@ -115,6 +151,8 @@ def _parse() -> argparse.Namespace:
     ap.add_argument("--other-steps", type=int, default=10, help="timed passes of each of the other configurations")
     ap.add_argument("--no-other-dtypes", action="store_true", help="skip the fp16 and fp32 passes of the same layer")
     ap.add_argument("--no-library-gemm", action="store_true", help="skip the loop of library GEMMs of the same shapes")
+    ap.add_argument("--no-kernel-table", action="store_true",
+                    help="skip the passes with events around every launch (a profile then holds the timed steps' kernels alone)")
     ap.add_argument("--only-config", choices=["fine-grained", "skewed"], default=None,
                     help="run only that one of the other configurations (the command its profile is taken with)")
     ap.add_argument("--library-gemm-only", action="store_true",
@@ -193,16 +231,15 @@ def _kernel_table(summary: dict, steps: int) -> list:
     return kernels
 
 
-def _other_config(workload: dict, steps: int, warmup: int) -> dict:
-    """Forward+backward of one of OTHER_WORKLOADS, timed like the headline region (host clock around `steps`
-    passes, events on the launch stream around every native call)."""
+def _other_config(workload: dict, steps: int, warmup: int, observe: bool = True) -> dict:
+    """Forward+backward of one of OTHER_WORKLOADS, timed like the headline region (host clock around `steps` passes, then
+    events on the launch stream around every launch of some more)."""
 
     import math
 
     import torch
 
     import flash_model_architectures_amd as xma
-    from flash_model_architectures_amd import _native
     from flash_model_architectures_amd.utils import skewed_router_bias
 
     dev, dt = torch.device("cuda:0"), torch.bfloat16
@@ -229,15 +266,7 @@ def _other_config(workload: dict, steps: int, warmup: int) -> dict:
 
     for _ in range(warmup):
         step()
-    torch.cuda.synchronize()
-    timeline = _native.Timeline()
-    _native.set_timeline(timeline)
-    t0 = time.perf_counter()
-    for _ in range(steps):
-        step()
-    torch.cuda.synchronize()
-    seconds = time.perf_counter() - t0
-    _native.set_timeline(None)
+    seconds, summary, observed = _time_steps(step, steps, observe)
 
     with torch.no_grad():
         logits = moe.gate(x)
@@ -247,7 +276,7 @@ def _other_config(workload: dict, steps: int, warmup: int) -> dict:
         # experts rests on a tie rule (lower expert index here)
         ranked = torch.sort(logits.float(), dim=-1, descending=True).values
         ties = int((ranked[:, k - 1] == ranked[:, k]).sum()) if E > k else 0
-    kernels = _kernel_table(timeline.summary(), steps)
+    kernels = _kernel_table(summary, observed)
     gemm_ms = sum(kr["ms_per_step"] for kr in kernels if kr["kernel"].startswith("xma_grouped_gemm"))
     flops = 18.0 * T * k * H * I
     ms_per_step = seconds / steps * 1e3
@@ -270,6 +299,7 @@ def _other_config(workload: dict, steps: int, warmup: int) -> dict:
                 "per_expert": counts.tolist(),
             },
             "tokens_with_a_tie_at_the_selection_boundary": ties,
+            "kernels_from": KERNELS_FROM,
             "kernels": kernels,
         }
     )
@@ -278,12 +308,11 @@ def _other_config(workload: dict, steps: int, warmup: int) -> dict:
 
 def _other_dtype(dtype_name: str, steps: int, warmup: int) -> dict:
     """The headline layer (same shape, same seed) in another element type: fp16 through the same LDS-DMA kernels as
-    bf16, fp32 through the register-staged kernel with true-fp32 matrix instructions.  Timed like the headline region."""
+    bf16, fp32 through a kernel of its own with true-fp32 matrix instructions.  Timed like the headline region."""
 
     import torch
 
     import flash_model_architectures_amd as xma
-    from flash_model_architectures_amd import _native
 
     dt, peak = {"fp16": (torch.float16, PEAK_FP16_FLOPS), "fp32": (torch.float32, PEAK_FP32_MATRIX_FLOPS)}[dtype_name]
     dev = torch.device("cuda:0")
@@ -302,16 +331,8 @@ def _other_dtype(dtype_name: str, steps: int, warmup: int) -> dict:
 
     for _ in range(warmup):
         step()
-    torch.cuda.synchronize()
-    timeline = _native.Timeline()
-    _native.set_timeline(timeline)
-    t0 = time.perf_counter()
-    for _ in range(steps):
-        step()
-    torch.cuda.synchronize()
-    seconds = time.perf_counter() - t0
-    _native.set_timeline(None)
-    kernels = _kernel_table(timeline.summary(), steps)
+    seconds, summary, observed = _time_steps(step, steps)
+    kernels = _kernel_table(summary, observed)
     for kr in kernels:  # the table's fraction column assumes the bf16 peak
         if "tflops" in kr:
             kr["frac_of_matrix_peak"] = round(kr["tflops"] * 1e12 / peak, 4)
@@ -531,7 +552,7 @@ def main() -> int:
 
     if args.only_config is not None:
         workload = OTHER_WORKLOADS[0 if args.only_config == "fine-grained" else 1]
-        print(json.dumps({"other_configs": [_other_config(workload, args.other_steps, 2)]}))
+        print(json.dumps({"other_configs": [_other_config(workload, args.other_steps, 2, not args.no_kernel_table)]}))
         return 0
     if args.reduction_sweep:
         print(json.dumps({"reduction_sweep": _reduction_sweep()}))
@@ -561,23 +582,17 @@ def main() -> int:
         torch.cuda.synchronize()
         del src, dst
 
-    timeline = _native.Timeline()
-    _native.set_timeline(timeline)
-    t0 = time.perf_counter()
-    for _ in range(args.steps):
-        step()
-    torch.cuda.synchronize()
-    seconds = time.perf_counter() - t0
-    _native.set_timeline(None)
-
+    seconds, summary, observed = _time_steps(step, args.steps, not args.no_kernel_table)
     ms_per_step = seconds / args.steps * 1e3
     tokens_per_s = T * args.steps / seconds
     gemm_flops = 18.0 * T * k * H * I  # forward 6*M*H*I, backward twice that
 
-    kernels = _kernel_table(timeline.summary(), args.steps)
+    kernels = _kernel_table(summary, observed)
 
-    dominant = kernels[0]
-    if "tflops" in dominant:
+    dominant = kernels[0] if kernels else {}
+    if not dominant:
+        roofline = None
+    elif "tflops" in dominant:
         roofline = {
             "kernel": dominant["kernel"],
             "bound": "mfma",
@@ -621,6 +636,7 @@ def main() -> int:
         "grouped_gemm_tflops": round(gemm_flops / (gemm_ms * 1e-3) / 1e12, 2) if gemm_ms > 0 else None,
         "grouped_gemm_frac_of_bf16_peak": round(gemm_flops / (gemm_ms * 1e-3) / PEAK_BF16_FLOPS, 4) if gemm_ms else None,
         "roofline": roofline,
+        "kernels_from": KERNELS_FROM,
         "kernels": kernels,
     }
     if not args.no_other_configs:
