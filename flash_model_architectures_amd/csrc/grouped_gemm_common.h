@@ -32,14 +32,14 @@ struct GemmParams {
     int32_t num_experts, in_fan_out, idx_is_i64;
     int32_t row_tiles_max;  // upper bound used for the grid (TN/NN); MT: row tiles per expert
     int32_t col_tiles;
-    // split-K of the last, partly filled round of tiles (16-bit TN/NN kernels)
+    // split-K of the last, partly filled round of tiles (TN/NN kernels of 16 and 32 bits)
     int32_t* split_counters;  // [kSplitSlots] arrivals per split tile, zero at launch
     float* split_partials;    // [kSplitSlots][tile] fp32 accumulators of the parts
     // MT with gathered rows (16 bits): byte offset of the source row of every routed row, kRowOffsetsPadding entries more
     const uint32_t* row_offsets;
-    int32_t tile_rows;  // rows of the tallest tile (16-bit TN/NN)
-    int32_t most_parts;       // parts of a split tile at most (fp32)
-    int32_t round_tiles;      // tiles that run at a time on the whole device, a multiple of kNumXcd
+    int32_t tile_rows;    // rows of the tallest tile (16-bit TN/NN)
+    int32_t most_parts;   // parts of a split tile at most (fp32)
+    int32_t round_tiles;  // tiles that run at a time on the whole device, a multiple of kNumXcd
     // MT: experts in descending order of their row counts, one record {expert, first row, end row, 0} per slot;
     // nullptr: slot e is expert e
     const int32_t* expert_order;
@@ -153,9 +153,9 @@ inline int64_t grid_for_dealt_tiles(int64_t row_tiles, int64_t col_tiles) {
 // per compute unit of 256 x 256 tiles, two of the smaller ones) the first floor(T / C) * C tiles fill whole rounds; the
 // R = T mod C tiles of the last round would leave C - R places idle for a whole tile time, so each of them is cut along the
 // reduction into min(most_parts, C / R) parts that run side by side.  Only when the launch has fewer than most_rounds rounds
-// (the idle places of a last round matter less the more rounds there are), only for up to most_tiles tiles, and only while a part is worth its exchange
-// (most_parts, which the kernels derive from the reduction): every part parks its fp32 sums in memory and the last one reads
-// them all back.  16-bit kernels: 40-50 k cycles for a 256 x 256 tile, or about 17 stages of the main loop (measured;
+// (the idle places of a last round matter less the more rounds there are), only for up to most_tiles tiles, and only while a
+// part is worth its exchange (most_parts, which the kernels derive from the reduction): every part parks its fp32 sums in memory
+// and the last one reads them all back.  16-bit kernels: 40-50 k cycles for a 256 x 256 tile, or about 17 stages of the main loop (measured;
 // reductions of 14336 and 28672 split in three gain 7 % and 5 % of their launches), so a part keeps kSplitMinStages stages.
 // Work-groups are dealt per XCD as in locate_tile<false>: XCD x takes the x-th eighth of the whole tiles, then the x-th
 // eighth of the parts (part-major, so neighbours share panels).
@@ -166,7 +166,7 @@ struct TileWork {
     int part, parts;  // this work-group reduces stages [part * n / parts, (part + 1) * n / parts)
     int split_tile;   // index of the tile among the split ones
     int split_tiles;
-    int half, halves;     // this work-group has the rows of one half of the tile
+    int half, halves;  // this work-group has the rows of one half of the tile
 };
 template <bool HALVES>
 __device__ __forceinline__ bool locate_work(int row_tiles, int col_tiles, int round_tiles, int most_parts, int most_rounds,

@@ -408,8 +408,8 @@ struct Ring64x5 {
     }
 };
 
-// Ring64x2: two whole stages, for tiles of 128 columns: 192 rows need 40 KiB a stage.  All loads of stage s+2 go out in the second phase of step s, one to two phases before
-// the barrier that needs them.
+// Ring64x2: two whole stages, for tiles of 128 columns: 192 rows need 40 KiB a stage.  All loads of stage s+2 go out in the
+// second phase of step s, one to two phases before the barrier that needs them.
 template <typename TL_>
 struct Ring64x2 {
     using TL = TL_;
@@ -467,7 +467,7 @@ struct Kernel {
 
     // Byte offsets of this lane's fragments inside an operand tile.  Only the part that is not a
     // compile-time constant goes through opaque(): for the K-contiguous layout the 16-row block adds a
-    // constant (the swizzle repeats every 16 rows); for the K-strided layout the 32-deep block adds 16 KiB and
+    // constant (the swizzle repeats every 16 rows); for the K-strided layout the 32-deep block adds 64 * ROWS bytes and
     // the odd 16-column block of a 32-column pair adds 32 bytes (two chunks; the swizzle leaves that bit alone).
     template <bool STRIDED, int ROWS>
     __device__ __forceinline__ void fragment_offsets(int row0, int (&var)[4]) const {
@@ -518,8 +518,9 @@ struct Kernel {
 
     // One phase = one 32-deep block = MI * NI matrix instructions of 16 cycles.  A wave that is alone on its SIMD
     // has nobody to hide its stalls, so the three instruction streams are interleaved by hand: the phase is cut into
-    // 32 slots of two matrix instructions (one B block against two A blocks).  Every odd slot also reads one block
-    // of the NEXT phase's fragments and every fourth slot issues one DMA load.  The matrix instructions are inline
+    // slots of two matrix instructions (one B block against two A blocks; of one, where the wave has one A block), 32 of them for
+    // a 256 x 256 tile.  The MI + NI reads of the NEXT phase's fragments and the phase's DMA loads are spread evenly over the
+    // slots: for 256 x 256 every odd slot reads one block and every fourth issues one load.  The matrix instructions are inline
     // assembly, which the instruction scheduler cannot classify, so the order is pinned with a scheduling fence
     // after each slot.  RP / RKB: ring position and block of the fragments being read; LP / LPH: the step and phase
     // whose loads go out.
@@ -726,7 +727,7 @@ __device__ __forceinline__ void multiply_tile(const GemmParams& P, const TilePla
         const T* W = B + (int64_t)expert * P.b_expert_stride;
         if constexpr (KIND == XMA_GEMM_TN) {
             if constexpr (EPI == EPI_PAIRED) {
-                // tile rows 0..127: weight rows n0 + r (up half); rows 128..255: P.n / 2 + n0 + r - 128 (gate half)
+                // tile row r < BN_OUT: weight row n0 + r (up half); others: P.n / 2 + n0 + r - BN_OUT (gate half)
                 const int64_t half = P.n / 2;
                 k.lb.setup_uniform(k.wave, k.lane, W + n0 * P.ldb, P.ldb, (half - BN_OUT) * P.ldb,
                                    [&](int r) { return n0 + (r % BN_OUT) < half; });
@@ -844,10 +845,10 @@ __device__ __forceinline__ void multiply_tile(const GemmParams& P, const TilePla
         }
     }
 
-    // ---- epilogue: accumulators -> LDS (slab mi holds the 64 tile rows of each wave row from mi * SLAB_ROWS / 2) -> HBM ----
+    // ---- epilogue: accumulators -> LDS (slab mi holds SLAB_ROWS / 2 tile rows of each wave row, see row_base) -> HBM ----
     // Store phase: each thread owns one 16-byte chunk column (cc) and, per slab, the IT buffer rows
-    // tid / 32 + 8 * it.  What the rows need from HBM (scatter indices, the saved pre-activation of the
-    // activation backward) is requested in batches before it is used: the indices of all four slabs before the
+    // tid / C_CHUNKS + ROW_STEP * it.  What the rows need from HBM (scatter indices, the saved pre-activation of the
+    // activation backward) is requested in batches before it is used: the indices of all slabs before the
     // accumulators are packed (and waited for after that), a slab's pre-activations one slab ahead.
     T* C = reinterpret_cast<T*>(P.c);
     constexpr int C_CHUNKS = BN / PV;             // 32 or 16
@@ -916,8 +917,8 @@ __device__ __forceinline__ void multiply_tile(const GemmParams& P, const TilePla
     if constexpr (SWBWD) load_saved(0, hu[0], hg[0]);
 
     // MFMA result register r of lane l in block (mi, ni): tile row 16*mi + l%16, tile column 16*ni + 4*(l/16) + r.
-    // Slab s holds the blocks mi = SLAB_BLOCKS * s + h of both wave rows wr as buffer rows wr * SLAB_ROWS / 2 + 16 * h + 0..15.  An LDS row holds C_CHUNKS chunks of 8 columns; chunk c of buffer row br sits at
-    // c ^ (br % C_CHUNKS).
+    // Slab s holds the blocks mi = SLAB_BLOCKS * s + h of both wave rows wr as buffer rows wr * SLAB_ROWS / 2 + 16 * h + 0..15.
+    // An LDS row holds C_CHUNKS chunks of 8 columns; chunk c of buffer row br sits at c ^ (br % C_CHUNKS).
     {
         const int wn0 = (k.wave % WAVES_N) * WN;
         const int br0 = (k.wave / WAVES_N) * (SLAB_ROWS / 2) + (etid & 15);  // buffer row of the first block of a slab
@@ -1301,8 +1302,8 @@ int launch_gathered_weight_gradient(const xma_grouped_gemm_args& a, const uint32
                                : launch_gathered<f16_t>(a, row_offsets, stream);
 }
 
-// 16-bit element types; the weight-gradient layout only without a fused row gather (its reduction rows
-// would need an index lookup per stage).
+// 16-bit element types; the weight-gradient layout only without a row index.  (Rows that are looked up take a table of byte
+// offsets and sizes that fit it: launch_gathered_weight_gradient, which a layer's native backward pass calls.)
 bool dma_gemm_supports(const xma_grouped_gemm_args& a) {
     if (a.dtype != XMA_BF16 && a.dtype != XMA_F16) return false;
     if (a.kind == XMA_GEMM_MT && a.in_index != nullptr) return false;
@@ -1318,20 +1319,19 @@ bool dma_gemm_supports(const xma_grouped_gemm_args& a) {
 //
 // Row-grouped kinds: the cost of each form is estimated from the tiles that experts have whose numbers of rows spread as
 // randomly chosen ones do, and two per cent more, in rounds of the device (K: the reduction in units of 1024):
-//   256 x 256: 20 + 24 K a round (34 where the epilogue has an activation of two halves or its backward); a partly filled last round
-//     costs a whole one, or is split along the reduction for 40 more;
+//   256 x 256: 20 + 24 K a round (34 where the epilogue has an activation of two halves or its backward); a partly filled last
+//     round costs a whole one, or is split along the reduction for 40 more;
 //   192, 128, 64, 32 x 128, two per compute unit: 7 (10) + 33, 24, 20, 24 K, 1.45 times that where rows do not start at whole
 //     lines of 128 bytes; a last round of half the places or less two thirds of a whole one.
-// These are not times: small tiles take about 0.75 of it, and a remainder of 32 rows costs its neighbour more than itself.  They are
-// the constants whose choice cost least over 11600 calls (1 to 256 experts, 20 to 20000 rows each, 12 layers) timed in all three
-// forms: 1.2 % more than the fastest on average where rows are spread evenly, 4 % under a skewed routing.  94 % of them are within
-// 3 % of 256 x 256 everywhere or faster, on average they take 0.74 of its time.  The worst are experts whose rows lie just above a
-// multiple of 192 or 256, which a few rows more or less decide.
+// These are not times: small tiles take about 0.75 of it, and a remainder of 32 rows costs its neighbour more than itself.  They
+// are the constants whose choice cost least over 10302 calls (1 to 256 experts, 20 to 20000 rows each, 12 layers) timed in all
+// three forms: 1.2 % more than the fastest on average where rows are spread evenly, 4 % under a skewed routing.  95 % of the
+// former are within 3 % of 256 x 256 everywhere or faster, on average they take 0.74 of its time.  The worst are experts whose
+// rows lie just above a multiple of 192 or 256, which a few rows more or less decide.
 // us, 256 x 256 / up to 192 / up to 128 rows, evenly spread unless said otherwise:
-//   64 experts, H 2048, I 1024: 1536 rows each, up 784 / 857 / 902, dX 755 / 819 / 858; 281, 228 / 205 / 244 and 217 / 186 / 228; 75,
-//     143 / 133 / 132 and 114 / 110 / 112
-//   128 experts, H 2048, I 768, 96 rows, skewed: up 107 / 102 / 99, down 71 / 58 / 57, dX 127 / 106 / 104; even, 200 rows, dact 143
-//     / 173 / 159
+//   64 experts, H 2048, I 1024: 1536 rows each, up 784 / 857 / 902, dX 755 / 819 / 858; 281, 228 / 205 / 244 and 217 / 186 / 228;
+//     75, 143 / 133 / 132 and 114 / 110 / 112
+//   128 experts, H 2048, I 768, 96 rows, skewed: up 107 / 102 / 99, down 71 / 58 / 57, dX 127 / 106 / 104
 //   6 experts, H 512, I 1024, 2000 rows: up 49 / 42 / 37, down 28 / 23 / 20, dact 41 / 38 / 34, dX 48 / 38 / 30
 //   16 experts, H 1024, I 4096, 125 rows: up 68 / 60 / 71, down 61 / 40 / 43, dX 98 / 83 / 91
 //   8 experts, H 4096, I 14336, 2048 rows: up 3082 / 3832 / 4256, down 1427 / 1876 / 2146
@@ -1341,12 +1341,12 @@ bool dma_gemm_supports(const xma_grouped_gemm_args& a) {
 //
 // Weight gradients: tiles of 128 x 128 where 256 x 256 leave much of the device idle, or where the reductions (the rows of an
 // expert) are short.  us, 256 x 256 / 128 x 128 (one launch back to back with itself, evenly spread rows):
-//   one round of large tiles, 16 experts, 1024 x 1024: 500 rows 26 / 28, 1000 37 / 39, 2000 59 / 65, 4000 101 / 124, 8000 199 / 267;
-//     8 experts, 2048 x 1024, 16000 rows 375 / 542
+//   one round of large tiles, 16 experts, 1024 x 1024: 500 rows 26 / 28, 1000 37 / 39, 2000 59 / 65, 4000 101 / 124, 8000
+//     199 / 267; 8 experts, 2048 x 1024, 16000 rows 375 / 542
 //   a second round of three quarters, 8 experts, 2048 x 1792: 2000 rows 100 / 110, 4000 175 / 204, 16000 696 / 1050
 //   fewer than four bands of row tiles, which leave half the XCDs without work: 4 experts, 768 x 3072: 1500 rows 73 / 43, 4000
 //     165 / 102, 9000 353 / 229; 6 experts, 2048 x 1024, 9000 rows, skewed (an expert's tiles are one band): 411 / 275
-//   two rounds and more: 64 experts, 4096 x 512, 281 rows 133 / 125, 375 149 / 147; 64 experts, 2048 x 2048, 281 253 / 241, 375
+//   two rounds and more: 64 experts, 2048 x 1024, 281 rows 133 / 125, 375 149 / 147; 64 experts, 2048 x 2048, 281 253 / 241, 375
 //     284 / 286, 562 346 / 392; 128 experts, 1536 x 2048, 375 444 / 500
 // Long launches of many tiles turn earlier: with 4096 tiles 1.05 times as long in small ones at 390 rows, with 8192 at 300, with
 // 16384 at 220, hence rows^2 * tiles.  Over 4310 calls of 1 to 256 experts, 20 to 20000 evenly spread rows each, the choice costs

@@ -19,7 +19,7 @@
 // each of the two loads; one chunk per 64-byte half line (either half by a load of its own) held 5.0 TB/s where this
 // holds 5.9.  A kernel that only reads reaches 6.2.
 //
-// Measured against the 256 x 256 kernel, up + down projection: H 2048, I 1024, E 64, k 6, one token (6 experts, 75 MB
+// Measured against tiles of 256 x 256, up + down projection (the smaller tiles of that kernel: see skinny_gemm_supports): H 2048, I 1024, E 64, k 6, one token (6 experts, 75 MB
 // of weights) 21 us instead of 82; 16 tokens 117 us instead of 207 (5.6 TB/s of weights); H 4096, I 14336, E 8, k 2,
 // 32 tokens 467 us instead of 653 (6.0 TB/s), 64 tokens 484 us instead of 666.  In fp32 (a 128 x 128 register-staged
 // kernel before) one token 36 us instead of 248, 16 tokens 225 us with whole lines and 247 with half lines.
@@ -320,6 +320,16 @@ static int dispatch(const xma_grouped_gemm_args& a, hipStream_t stream) {
 // not longest (the tiled kernel pays its prologue per tile, and cuts the longest reductions until the device is
 // full) or whose projection is wide, and of the short reductions those of too few tiles of 256 x 256 to fill the device.
 // Beyond kSkinnyRows even calls gain nothing (128 experts at 64 rows: 255 / 223).
+// These lines were drawn against tiles of 256 x 256.  A call that does not stream now takes tiles of up to 192 x 128 where they are
+// faster, and against those it streams for too long.  This kernel / the fastest tiles, up projection, even calls, us by rows:
+//   H 4096, I 14336, E 8: 8 rows 331 / 339, 20 rows 359 / 350, 40 rows 388 / 379; down 8 rows 168 / 173, 20 rows 173 / 167
+//   H 2048, I 1024, E 64: 8 rows 100 / 129, 20 rows 110 / 128, 40 rows 132 / 131; down 44 / 43, 50 / 42
+//   H 2048, I 768, E 128: 8 rows 149 / 156, 20 rows 168 / 192, 40 rows 195 / 162; down 79 / 78, 20 rows 95 / 81; skewed, 20 rows
+//     180 / 213, down 106 / 96, 40 rows up 230 / 197
+//   H 2048, I 8192, E 16: 8 rows 195 / 196, 20 rows 218 / 196, 40 rows 260 / 200; down 115 / 132, 127 / 132, 131 / 131
+//   H 2048, I 1024, E 8: 8 rows 15 / 21, 20 rows 17 / 21, 40 rows 21 / 23
+//   H 1024, I 4096, E 128, down: 8 rows 184 / 190, 20 rows 210 / 192, 40 rows 253 / 196
+// Median over 1270 calls that stream: 0.93 of the fastest tiles at 8 rows, 1.05 at 14, 1.10 at 20, 1.16 at 30, 1.25 at 40.
 constexpr int kSkinnyRows = 40;
 constexpr int kSkinnyTwoBlocks = 20;
 constexpr int kSkinnyOneBlock = 8;

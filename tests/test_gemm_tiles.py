@@ -72,8 +72,8 @@ def test_which_calls_take_them(kind, experts, rows, n, k, epilogue, tile):
         (6, 2000, 2048, 1408, False),
         (4, 4000, 768, 3072, False),
         # two rounds and more: the reduction's length, earlier the longer the launch
-        (64, 281, 4096, 512, False),
-        (64, 400, 4096, 512, True),
+        (64, 281, 2048, 1024, False),
+        (64, 400, 2048, 1024, True),
         (128, 230, 1024, 4096, False),
         (128, 300, 1024, 4096, True),
         (256, 180, 3584, 4096, True),
