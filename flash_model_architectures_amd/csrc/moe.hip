@@ -81,6 +81,11 @@ struct Layer {
         return a.dtype != XMA_F32 && 2 * a.tokens * a.hidden < ((int64_t)1 << 32) &&
                xma_grouped_gemm_form(&g, &kernel, &tile_rows, &tile_cols) == 0 && kernel == XMA_FORM_TILED;
     }
+    // fp32: the kernel that looks the rows up itself waits for the look-up in every stage, so long reductions of wide gradients
+    // pay for a copy.  us, look-up / copy + plain: 8192 rows over 8 experts, N 16384, H 2048 4512 / 14 + 4038; 17728 rows over 64, N
+    // 2048, H 2048 1364 / 1257, N 512 386 / 357, N 256 189 / 196; 35456 rows over 128, N 512, H 576 235 / 229, N 128 76 / 85; 2216
+    // rows over 8, H 576: N 2048 73 / 83, N 512 27 / 29; 256 rows over 8, N 512, H 2048 18 / 21
+    bool copies_tokens() const { return a.dtype != XMA_F32 || (N >= 512 && M * N >= (int64_t)200000 * a.num_experts); }
     int d_preact() const {
         auto g = gemm(XMA_GEMM_NN, a.intermediate, a.hidden);
         g.epilogue = a.epilogue + 1;  // the activation's backward
@@ -182,10 +187,11 @@ int xma_moe_backward(const xma_moe_args* args, void* stream) {
     auto d_w_up = layer.d_w_up();
     if (gathers) {
         XMA_STEP(launch_gathered_weight_gradient(d_w_up, token_offsets, (hipStream_t)stream));
+    } else if (!layer.copies_tokens()) {
+        d_w_up.in_index = a.perm;
+        d_w_up.in_fan_out = a.top_k;
+        XMA_STEP(layer.run(d_w_up));
     } else {
-        // fp32: the kernel that looks the rows up itself waits for the look-up in every stage.  us, look-up / copy + plain: 8192
-        // rows over 8 experts, N 16384, H 2048 4512 / 14 + 4038; 18000 rows over 64 experts, N 2048, H 2048 1381 / 29 + 1241;
-        // 1000 rows over 8, N 8192, H 1024 184 / 5 + 167
         XMA_STEP(xma_spread_rows(a.x, H, a.rows, H, a.perm, 0, a.inverse, a.tokens, a.top_k, H, a.dtype, nullptr, nullptr, 0,
                                  nullptr, stream));
         d_w_up.b = a.rows;

@@ -355,11 +355,16 @@ class _FusedExperts(torch.autograd.Function):
             expert_colsum(src=d_preact, expert_offsets=expert_offsets, out=d_b_up)
 
         d_w_up = torch.empty_like(w_up)
-        # (a copy of the tokens' rows: the fp32 kernel that looks them up itself takes a tenth longer)
-        grouped_x = torch.empty(M, H, device=x.device, dtype=x.dtype)
-        spread_rows(A=x, index=idx, inverse=inverse, out=grouped_x)
-        group_bwd_W(DY=d_preact, X=grouped_x, expert_offsets=expert_offsets, DW=d_w_up.permute(0, 2, 1), E=E)
-        del grouped_x
+        N = preact.size(1)
+        if x.dtype == torch.float32 and (N < 512 or M * N < 200000 * E):  # the kernel looks the tokens' rows up itself
+            inputs = dict(X=x, x_index=idx, x_fan_out=k)
+        else:  # a copy of the rows: look-ups take the fp32 kernel a tenth longer where the reductions are long
+            grouped_x = torch.empty(M, H, device=x.device, dtype=x.dtype)
+            spread_rows(A=x, index=idx, inverse=inverse, out=grouped_x)
+            inputs = dict(X=grouped_x)
+            del grouped_x
+        group_bwd_W(DY=d_preact, expert_offsets=expert_offsets, DW=d_w_up.permute(0, 2, 1), E=E, **inputs)
+        del inputs
 
         d_expanded = torch.empty(M, H, device=x.device, dtype=x.dtype)
         scatter2scatter(

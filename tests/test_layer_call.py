@@ -13,6 +13,9 @@ import flash_model_architectures_amd as xma
 from flash_model_architectures_amd import _native, ops
 from flash_model_architectures_amd.functional import routing as routing_module
 from flash_model_architectures_amd.layers import moe
+from oracle import torch_oracle as to
+
+from .helpers import TOL, assert_close
 
 
 ACTIVATIONS = {
@@ -360,3 +363,37 @@ def test_many_token_bytes(tokens, monkeypatch):
     del want
     x[-1].zero_()
     assert not all(torch.equal(a, b) for a, b in zip(got[3:], _train(layer, x, dy)[3:]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(
+    "tokens,sizes,copied",
+    [
+        (620, dict(intermediate=256), True),  # 413 rows per expert, 512 columns
+        (700, dict(intermediate=252), False),  # 466 rows, 504 columns
+        (160, dict(intermediate=1024), True),  # 107 rows, 2048 columns
+        (560, dict(k=1, intermediate=256), False),  # 93 rows
+    ],
+)
+def test_token_rows_of_the_fp32_weight_gradient(tokens, sizes, copied, monkeypatch):
+    """Long reductions of wide gradients read a copy of the tokens' rows, others look them up: the same sums."""
+
+    sizes = {"intermediate": 256, **sizes}
+    layer = _layer(torch.float32, experts=6, hidden=136, **sizes)
+    rows, columns = tokens * layer.top_k / 6, 2 * sizes["intermediate"]
+    assert copied is (columns >= 512 and rows * columns >= 200000)
+    x = torch.randn(tokens, 136, device="cuda")
+    dy = torch.randn_like(x)
+    want = _train(layer, x, dy)
+    calls = _Calls(monkeypatch, one_by_one=True)
+    got = _train(layer, x, dy)
+    assert calls.names == []
+    launched = [tag for tag, *_ in _native._timeline.records]
+    assert launched.count("xma_spread_rows") == (1 if copied else 0)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    # against float64
+    double = [p.detach().cpu().double().requires_grad_() for p in layer.parameters()]  # gate, up, down
+    y, _ = to.moe_forward(x.cpu().double(), *double, layer.top_k)
+    y.backward(dy.cpu().double())
+    assert_close(got[4].cpu(), double[1].grad.float(), TOL[torch.float32], "dW_up")
