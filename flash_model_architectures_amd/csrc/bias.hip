@@ -40,17 +40,18 @@ __global__ __launch_bounds__(256) void add_expert_bias_kernel(T* __restrict__ y,
     }
 }
 
-// Block (x = column block of CL chunks, y = expert): 1024 / CL row lanes walk the expert's rows in order, four in flight, and
+// Block (x = column block of CL chunks, y = expert): 1024 / CL row lanes walk the expert's rows in order, IN_FLIGHT at a time, and
 // keep fp32 partial sums of their chunk; the lanes are added through LDS in lane order.  The order of the additions is
 // fixed, so the result is reproducible.
 // Few experts are few blocks, and a block waits for memory: with 32 chunks, one row in flight and the 32 lanes added up by
 // one of them, 12004 rows of 512 and 1024 columns over 6 experts in 16 bits took 13 and 39 us; so 5.5 and 12.6.
-template <typename T, bool VEC, int CL>
+// ONE_FROM: from so many rows on they are read one at a time.
+template <typename T, bool VEC, int CL, int IN_FLIGHT, int64_t ONE_FROM>
 __global__ __launch_bounds__(1024) void expert_colsum_kernel(const T* __restrict__ src, int64_t ld,
                                                               const int32_t* __restrict__ offsets,
                                                               T* __restrict__ out, int64_t ld_out, int64_t cols) {
     constexpr int PV = VEC ? Elem<T>::kPerVec : 1;
-    constexpr int RL = 1024 / CL, COLS = CL * PV, IN_FLIGHT = 4;
+    constexpr int RL = 1024 / CL, COLS = CL * PV;
     constexpr int GROUPS = 1024 / COLS < RL ? 1024 / COLS : RL, PER_GROUP = RL / GROUPS;
     __shared__ float part[RL][COLS + 1];
     const int cl = threadIdx.x % CL, rl = threadIdx.x / CL;
@@ -64,7 +65,8 @@ __global__ __launch_bounds__(1024) void expert_colsum_kernel(const T* __restrict
     if (chunk < chunks) {
         const T* column = src + chunk * PV;
         int64_t r = begin + rl;
-        for (; r + (IN_FLIGHT - 1) * RL < end; r += IN_FLIGHT * RL) {
+        const int64_t together = end - begin < ONE_FROM ? end : begin;
+        for (; r + (IN_FLIGHT - 1) * RL < together; r += IN_FLIGHT * RL) {
             if constexpr (VEC) {
                 uint4 v[IN_FLIGHT];
 #pragma unroll
@@ -115,10 +117,23 @@ __global__ __launch_bounds__(1024) void expert_colsum_kernel(const T* __restrict
     }
 }
 
-// Narrow blocks, with four times as many row lanes each, while the wide ones are fewer than one to a compute unit.  us, wide /
-// narrow: 16384 rows of 4096 columns, 8 experts (128 wide blocks) 45 / 25; 98304 x 2048, 64 experts (512) 65 / 74;
-// 131072 x 1536, 128 experts (768) 64 / 78; 16384 x 28672, 8 experts (896) 151 / 165.
-constexpr int64_t kWideColsumBlocks = 256;
+// Few blocks wait for memory, many are bound by it.  By blocks of 32 chunks, us with 32 chunks and one row in flight / 32 and
+// two / 32 and four / 8 and four:
+//   128 blocks, 2048 rows (16384 x 4096 in 16 bits, 8 experts) 41 / 26 / 26 / 24
+//   160, 16 rows (512 x 520 in fp32, 32 experts) 3.1 / 3.1 / 3.1 / 4.2
+//   224, 16384 rows (16384 x 28672 in fp32, one expert) 316 / 273 / 282 / 369
+//   1024, 4096 rows (131072 x 8192 in 16 bits, 32 experts) 322 / 334 / 374 / 349
+// and times the fastest form of each call, from 1024 rows on: 128 blocks 1.59 / 1.05 / 1.09 / 1.01; 160 1.41 / 1.00 / 1.08 / 1.35; 256
+// 1.09 / 1.00 / 1.05 / 1.13; 320 1.00 / 1.16 / 1.07 / 1.26; 512 1.00 / 1.09 / 1.05 / 1.10.  Experts of a hundred rows gain from four
+// in flight there too (one takes 1.11 times as long at 128 rows of 16 bits, 1.05 at 256, 0.99 at 375; 1.03 and 0.99 at 128 and 256
+// in fp32): below kManyRows.
+constexpr int64_t kWideColsumBlocks = 160, kManyColsumBlocks = 320, kAnyRows = (int64_t)1 << 62;
+template <typename T>
+constexpr int64_t kManyRows = Elem<T>::kPerVec * 40;
+// Without vectors a chunk is one element, and narrow blocks read few bytes of a row: 32 / 64 chunks, four rows in flight, times
+// the fastest: 128 blocks 1.00 / 1.40, 256 1.09 / 1.04, 512 1.39 / 1.00 (8 chunks: 2.35, 2.50, 3.38); 32 blocks 1.5 / 2.8, and 16
+// chunks 1.0.
+constexpr int64_t kFewScalarColsumBlocks = 64, kManyScalarColsumBlocks = 256;
 
 }  // namespace xma
 
@@ -167,15 +182,17 @@ int xma_expert_colsum(const void* src, int64_t ld, const int32_t* expert_offsets
         const bool vec = aligned16(src) && aligned16(out) && ld % Elem<T_>::kPerVec == 0 &&
                          ld_out % Elem<T_>::kPerVec == 0 && cols % Elem<T_>::kPerVec == 0;
         const int64_t chunks = vec ? cols / Elem<T_>::kPerVec : cols;
-        const bool wide = ceil_div(chunks, 32) * num_experts >= kWideColsumBlocks;
-        const dim3 grid((unsigned)ceil_div(chunks, wide ? 32 : 8), (unsigned)num_experts), block(1024);
-#define XMA_COLSUM_LAUNCH(VEC, CL)                                                                                    \
-    hipLaunchKernelGGL((expert_colsum_kernel<T_, VEC, CL>), grid, block, 0, stream, (const T_*)src, ld, expert_offsets, \
-                       (T_*)out, ld_out, cols)
-        if (vec && wide) XMA_COLSUM_LAUNCH(true, 32);
-        else if (vec) XMA_COLSUM_LAUNCH(true, 8);
-        else if (wide) XMA_COLSUM_LAUNCH(false, 32);
-        else XMA_COLSUM_LAUNCH(false, 8))
+        const int64_t blocks = ceil_div(chunks, 32) * num_experts;
+#define XMA_COLSUM_LAUNCH(VEC, CL, IN_FLIGHT, ONE_FROM)                                                                     \
+    hipLaunchKernelGGL((expert_colsum_kernel<T_, VEC, CL, IN_FLIGHT, ONE_FROM>),                                            \
+                       dim3((unsigned)ceil_div(chunks, CL), (unsigned)num_experts), dim3(1024), 0, stream, (const T_*)src, ld, \
+                       expert_offsets, (T_*)out, ld_out, cols)
+        if (vec && blocks < kWideColsumBlocks) XMA_COLSUM_LAUNCH(true, 8, 4, kAnyRows);
+        else if (vec && blocks < kManyColsumBlocks) XMA_COLSUM_LAUNCH(true, 32, 2, kAnyRows);
+        else if (vec) XMA_COLSUM_LAUNCH(true, 32, 4, kManyRows<T_>);
+        else if (blocks < kFewScalarColsumBlocks) XMA_COLSUM_LAUNCH(false, 16, 4, kAnyRows);
+        else if (blocks < kManyScalarColsumBlocks) XMA_COLSUM_LAUNCH(false, 32, 4, kAnyRows);
+        else XMA_COLSUM_LAUNCH(false, 64, 4, kAnyRows))
 #undef XMA_COLSUM_LAUNCH
     return check_launch("xma_expert_colsum");
 }

@@ -279,9 +279,11 @@ def test_table_of_tiles():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("experts,columns", [(3, 8), (3, 520), (8, 8192), (8, 8200), (5, 333), (256, 36)])
+@pytest.mark.parametrize(
+    "experts,columns", [(3, 8), (3, 520), (8, 8192), (8, 8200), (5, 333), (256, 36), (8, 16384), (9, 333), (12, 3333)]
+)
 def test_column_sums(experts, columns, dtype):
-    """Per-expert column sums in narrow and in wide blocks (from 256 wide ones on), with vectors and without."""
+    """Per-expert column sums in blocks of every width, with vectors and without."""
 
     g = torch.Generator("cuda").manual_seed(columns)
     sizes = torch.randint(0, 700, (experts,), generator=g, device="cuda")
